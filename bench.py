@@ -39,7 +39,7 @@ SEED = 0xF10E0000
 # has changed since is not reported.  Written by --record-traffic from the counter CSVs.
 TRAFFIC_RECORD = os.path.join(ROOT, "profiles", "traffic.json")
 KERNEL_SOURCES = {"decode_splitkv": "attn_decode.hip", "prefill_mfma": "attn_prefill_mfma.hip",
-                  "prefill_f32": "attn_prefill_f32.hip", "generic": "attn_generic.hip"}
+                  "prefill_f32": "attn_prefill_f32_terms.hip", "generic": "attn_generic.hip"}
 
 
 def source_hash(kernel, source=None):

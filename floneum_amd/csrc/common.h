@@ -55,15 +55,11 @@ struct AttnParams {
     // needs no clearing beforehand (whatever the workspace held, it is not this call's tag, short of a 2^-32
     // coincidence that only costs the fast path).
     int32_t bad_tag;
-    // Tiled f32 prefill only.  Workgroups are numbered longest first.  When the whole grid is resident at once
-    // (two workgroups per CU) nothing is rebalanced at run time, so the second half of the numbers is walked
-    // backwards: a CU's two workgroups are then a long and a short one.  0: off; else the number of CUs.
-    int32_t snake_cus;
     // Tiled prefill kernels: keys split over pf_nsplit workgroups per query block (few query rows on a long
     // cache would otherwise occupy a fraction of the chip).  Split s takes keys [s * pf_chunk, (s + 1) * pf_chunk)
     // and parks (O unnormalised, m, l) per row in `partials` [B, H, Sq, pf_nsplit, pf_pitch]; a merge kernel follows.
     int32_t pf_nsplit, pf_chunk;
-    int32_t pf_pitch;  // floats per (row, share) in `partials`: D + 2, or D + 4 where rows are written in 16-byte pieces
+    int32_t pf_pitch;  // floats per (row, share) in `partials`: D + 4, rows are written in 16-byte pieces
     int32_t pf_pack;   // tiled kernels, set by their launchers: query heads per workgroup of the packed form, or 0
     int32_t pf_rows64; // 16-bit tiled prefill at head_dim 128: the caller forced the 64-rows-per-wavefront form
 };
@@ -132,8 +128,11 @@ int launch_prefill_mfma_rows32(const AttnParams &p, fhip_dtype dtype, hipStream_
 // head_dim 128 on 256-row workgroups of four wavefronts with 64 rows each (FHIP_KERNEL_PREFILL_MFMA_ROWS64: forced only)
 bool prefill_mfma_rows64_takes(int D, float scale);
 int launch_prefill_mfma_rows64(const AttnParams &p, fhip_dtype dtype, hipStream_t stream);
-// f32 arithmetic on the f32 matrix cores; `dtype` is the tensors' storage type (16-bit rows are widened on load)
+// f32 precision; `dtype` is the tensors' storage type (16-bit rows are widened on load)
 int launch_prefill_f32(const AttnParams &p, fhip_dtype dtype, hipStream_t stream);
+// the same precision on the bf16 matrix cores, head dims to 128 (mode: a PF32_... of attn_f32.h); no merge of key shares
+bool prefill_f32_terms_takes(const AttnParams &p);
+int launch_prefill_f32_terms(const AttnParams &p, fhip_dtype dtype, int mode, hipStream_t stream);
 
 // decode planning (host): keys per split and number of splits; `ragged`: per-batch key counts are given;
 // `f32`: the tensors are f32 (vector variant) rather than 16-bit

@@ -47,6 +47,16 @@ __device__ __forceinline__ bf16_t from_float<bf16_t>(float x) {
     return r;
 }
 
+// Values (kernel arguments) that are in scalar registers from here on.
+template <typename V>
+__device__ __forceinline__ void pin_one(V v) {
+    asm volatile("" ::"s"(v));
+}
+template <typename... V>
+__device__ __forceinline__ void pin(V... v) {
+    (pin_one(v), ...);
+}
+
 // Orders this wavefront's LDS writes before its later LDS reads (no workgroup barrier).
 __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

@@ -19,6 +19,7 @@ const SOURCES: &[&str] = &[
     "attn_prefill_mfma_rows32.hip",
     "attn_prefill_mfma_rows64.hip",
     "attn_prefill_f32.hip",
+    "attn_prefill_f32_terms.hip",
     "kv_cache.hip",
     "mask_intervals.hip",
     "rope.hip",
