@@ -252,14 +252,14 @@ static bool decode_eligible(const fhip_attn_args *a) {
 static bool prefill_mfma_eligible(const fhip_attn_args *a) {
     if (a->dtype == FHIP_F32) return false;
     const uint32_t D = a->q.shape[3];
-    // 64 / 96 / 128: attn_prefill_mfma.hip; every other multiple of 8 up to 256 (padded to the next multiple of 32):
-    // attn_prefill_mfma_wide.hip
-    const bool wide = !(D == 64 || D == 96 || D == 128);
+    // 64 / 96 / 128: attn_prefill_mfma.hip only; other multiples of 8 (padded): that kernel to 128, and
+    // attn_prefill_mfma_wide.hip above and for scales it does not take
+    const bool exact = D == 64 || D == 96 || D == 128;
     if (D % 8 != 0 || D < 8 || D > 256) return false;
     if (!rows_vectorizable(a->q, 2) || !rows_vectorizable(a->k, 2) || !rows_vectorizable(a->v, 2)) return false;
-    // the kernel for 64 / 96 / 128 multiplies Q by the power-of-two part of scale * log2(e): that power must be at most
-    // 1 so that no finite element can leave the type's range (the wide-head kernel scales the scores in f32 only)
-    if (!wide && (!(a->scale > 0.0f) || !(a->scale * 1.4426950408889634f < 2.0f))) return false;
+    // that kernel multiplies Q by the power-of-two part of scale * log2(e): the power must be at most 1 so that no finite
+    // element can leave the type's range (the wide-head kernel scales the scores in f32 only)
+    if (exact && (!(a->scale > 0.0f) || !(a->scale * 1.4426950408889634f < 2.0f))) return false;
     // K/V rows are fetched through 32-bit buffer offsets: rows must not overlap and one (batch, kv
     // head) slice must span less than 2 GiB
     const uint64_t Skv = a->k.shape[2];
@@ -335,7 +335,8 @@ static void mfma_split_plan(const fhip_attn_args *a, int cus, int *nsplit, int *
     }
     const bool causal_square = a->analytic.enabled && a->analytic.causal && 2ull * a->q.shape[2] > a->k.shape[2];
     const int Hkv = (int)a->k.shape[1];
-    if (!(a->q.shape[3] == 64 || a->q.shape[3] == 96 || a->q.shape[3] == 128))  // the wide-head form: 128-row query blocks
+    if (!prefill_mfma_rows256_takes((int)a->q.shape[3], a->scale, (int)a->q.shape[0], (int)a->q.shape[1], (int)a->q.shape[2],
+                                    cus > 0 ? cus : 256))  // the wide-head form: 128-row query blocks
         prefill_mfma_wide_plan((int)a->q.shape[0], (int)a->q.shape[1], Hkv ? (int)a->q.shape[1] / Hkv : 1, (int)a->q.shape[2],
                                (int)a->k.shape[2], causal_square, cus > 0 ? cus : 256, nsplit, chunk);
     else
@@ -833,13 +834,14 @@ static void plan_decode_call(fhip_device *dev, const fhip_attn_args *args, AttnP
     }
 }
 
-// the 16-bit tiled prefill kernels: 64 / 96 / 128, and the wide-head form above
+// the 16-bit tiled prefill kernels: head dims to 128, and the wide-head form for those above and for scales the first cannot fold
 static int launch_mfma_by_head_dim(const AttnParams &p, fhip_dtype dtype, hipStream_t stream) {
     // the form of four wavefronts with 64 rows each (attn_prefill_mfma_rows64.hip), when the caller forces it: measured
     // 1-3 % slower than the 256-row form of eight wavefronts on the benchmark prompts (fewer LDS reads and a higher clock,
     // but a lone wavefront per SIMD issues everything in order), so it is never chosen
     if (p.pf_rows64) return launch_prefill_mfma_rows64(p, dtype, stream);
-    return (p.D == 64 || p.D == 96 || p.D == 128) ? launch_prefill_mfma(p, dtype, stream) : launch_prefill_mfma_wide(p, dtype, stream);
+    return prefill_mfma_rows256_takes(p.D, p.scale, p.B, p.H, p.Sq, p.cus > 0 ? p.cus : 256) ? launch_prefill_mfma(p, dtype, stream)
+                                                                                           : launch_prefill_mfma_wide(p, dtype, stream);
 }
 
 int fhip_flash_attention_decode_plan(fhip_stream *s, const fhip_attn_args *args, fhip_decode_plan_info *info) {

@@ -119,7 +119,10 @@ __device__ __forceinline__ float half_swap_sum(float x) {
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-template <typename T, int D, bool KS>
+// D: head_dim rounded up to 64, 96 or 128, the width of the tiles and of O.  QD: the dims contracted in K . Q^T, head_dim
+// rounded up to 16.  PAD: head_dim is less than D; the dims behind it are zero in Q, K and V (their lanes fetch from beyond
+// the buffer) and are not written.
+template <typename T, int D, int QD, bool PAD, bool KS>
 __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnParams p, int nqb, int out_vec) {
     typedef PfCfg<D, KS> C;
     typedef typename Mma<T>::vec8 vec8;
@@ -175,6 +178,7 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnPara
     const int lo_wg = rb.lo_wg, hi_wg = rb.hi_wg, lo_w = rb.lo_w, hi_w = rb.hi_w;
     const int full_lo_w = rb.full_lo_w, full_hi_w = rb.full_hi_w, klo = rb.klo, khi = rb.khi;
     const int qrow = min(query, p.Sq - 1);
+    const int hd = PAD ? p.D : D;  // the head dim itself
     const bool wave_has_rows = qw0 < p.Sq;
 
     // Q^T operand: Q[query][16 kb + 8 h2 .. +8], kept in registers for the whole kernel
@@ -187,12 +191,15 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnPara
     // an error that grows in proportion to the scores.  The S^T accumulators and m are in units of 1 / rr.
     const float pw = __uint_as_float(__float_as_uint(scale2) & 0x7F800000u);
     const float rr = scale2 / pw;
-    vec8 qreg[D / 16];
+    vec8 qreg[QD / 16];
     {
         const uint16_t *qp = (const uint16_t *)p.q + b * p.qs[0] + h * p.qs[1] + (int64_t)qrow * p.qs[2];
 #pragma unroll
-        for (int kb = 0; kb < D / 16; kb++)
-            qreg[kb] = __builtin_bit_cast(vec8, *(const uint4_t *)(qp + 16 * kb + 8 * h2));
+        for (int kb = 0; kb < QD / 16; kb++) {
+            uint4_t raw = {0, 0, 0, 0};
+            if (!PAD || 16 * kb + 8 * h2 < hd) raw = *(const uint4_t *)(qp + 16 * kb + 8 * h2);
+            qreg[kb] = __builtin_bit_cast(vec8, raw);
+        }
     }
 
     const int j_begin = (lo_wg / PF_BN) * PF_BN;
@@ -231,12 +238,13 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnPara
     const int wv = wave & 3;
     auto descriptor = [&](const uint16_t *base, int row_bytes) __attribute__((always_inline)) {
         const uint64_t ptr = (uint64_t)base;
-        return uint4_t{(uint32_t)ptr, (uint32_t)(ptr >> 32) & 0xffffu, (uint32_t)((key_end - 1) * row_bytes + D * 2),
+        return uint4_t{(uint32_t)ptr, (uint32_t)(ptr >> 32) & 0xffffu, (uint32_t)((key_end - 1) * row_bytes + hd * 2),
                        0x00020000u};
     };
     const uint4_t krs = descriptor(kg, krow_bytes), vrs = descriptor(vg, vrow_bytes);
-    const int gofs_k = (16 * (lane / C::CPR) + wv) * krow_bytes + (lane % C::CPR) * 16;
-    const int gofs_v = (16 * (lane / C::CPR) + wv) * vrow_bytes + (lane % C::CPR) * 16;
+    const bool padding = PAD && (lane % C::CPR) * 8 >= hd;
+    const int gofs_k = padding ? 0x7ffffff0 : (16 * (lane / C::CPR) + wv) * krow_bytes + (lane % C::CPR) * 16;
+    const int gofs_v = padding ? 0x7ffffff0 : (16 * (lane / C::CPR) + wv) * vrow_bytes + (lane % C::CPR) * 16;
     // where tile t lives in LDS
     auto k_stage = [&](int t) __attribute__((always_inline)) { return KS ? (t % C::NK) * C::K_BYTES : (t % 3) * STAGE; };
     auto v_stage = [&](int t) __attribute__((always_inline)) {
@@ -297,7 +305,7 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnPara
     auto qk = [&](int i) __attribute__((always_inline)) {
         const int kbase = k_stage(tile_of(i)) + (ln & 15) * C::KG + (ln >> 4) * C::ROWB + h2 * 16;
 #pragma unroll
-        for (int kb = 0; kb < D / 16; kb++) {
+        for (int kb = 0; kb < QD / 16; kb++) {
 #pragma unroll
             for (int t = 0; t < 2; t++) {
                 uint4_t raw = *LDS_PTR(uint4_t, kbase + t * 2 * C::ROWB + kb * 32);
@@ -344,7 +352,7 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnPara
     auto qk_pv = [&](int ip, int ik, auto do_pv, auto prefetched) __attribute__((always_inline)) {
         constexpr bool PV = decltype(do_pv)::value;
         constexpr bool PRE = decltype(prefetched)::value;
-        constexpr int NDB = D / 32, NKB = D / 16;
+        constexpr int NDB = D / 32, NKB = QD / 16;
         const int vstage = v_stage(tile_of(ip)), kstage = k_stage(tile_of(ik));
         const int i16 = lane & 15;
         const int bl = (lane & 31) >> 4;
@@ -560,7 +568,7 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnPara
             issue_tile(0);
         }
 #pragma unroll
-        for (int kb = 0; kb < D / 16; kb++) qreg[kb] = Mma<T>::scaled(qreg[kb], pw);
+        for (int kb = 0; kb < QD / 16; kb++) qreg[kb] = Mma<T>::scaled(qreg[kb], pw);
         wait_tiles(integral_constant<int, 0>{});
         lds_barrier();
         if (group == 0) {
@@ -635,8 +643,8 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnPara
     char *const og = parked ? (char *)(p.partials + (int64_t)ksplit * p.pf_pitch) : (char *)p.out;
     if (parked && query < p.Sq && h2 == 0) {
         float *ws = (float *)og + b * os0 + h * os1 + (int64_t)query * os2;
-        ws[D] = m * rr;  // base-2 exponent units
-        ws[D + 1] = l_tot;
+        ws[hd] = m * rr;  // base-2 exponent units
+        ws[hd + 1] = l_tot;
     }
     if (out_vec || parked) {
         // transpose through a wavefront-private slice of the LDS so that every global store is a
@@ -672,7 +680,7 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnPara
             for (int c = lane; c < rows_per_round * cpr; c += 64) {
                 const int row = c / cpr, col = c % cpr;
                 const int qr = qw0 + row_lo_ + row;
-                if (qr < p.Sq) {
+                if (qr < p.Sq && (!PAD || col * 16 < hd * esz)) {
                     const uint4_t val = *(__attribute__((address_space(3))) uint4_t *)(wbase + row * pitch + col * 16);
                     const int64_t eidx = b * os0 + h * os1 + (int64_t)qr * os2;
                     *(uint4_t *)(og + eidx * esz + col * 16) = val;
@@ -687,6 +695,7 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnPara
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const int dim = 32 * db + 8 * (r >> 2) + 4 * h2 + (r & 3);
+                if (PAD && dim >= hd) continue;
                 const float val = dead ? __builtin_nanf("") : o[db][r] * inv;
                 if (p.out_f32) ((float *)p.out)[obase + dim * p.os[3]] = val;
                 else ((T *)p.out)[obase + dim * p.os[3]] = from_float<T>(val);
@@ -708,6 +717,19 @@ static bool use_key_split_form(const AttnParams &p) {
     return p.Sq <= PF_BM / 2 || 2 * wgs <= cus || (wgs <= cus && nqb >= 8);
 }
 
+// Head dims 64, 96 and 128 are this kernel's own.  The other multiples of 8 above 64 run on it padded, quicker than on
+// the wide-head kernel, whose wavefronts read every LDS operand for half as many matrix instructions (f16, 16 heads, 4096 x 4096 keys without a mask: head_dim
+// 72 149 -> 118 us, 80 150 -> 118, 88 162 -> 120, 104 198 -> 132, 112 199 -> 133, 120 201 -> 139; causal, 80: 163 -> 68;
+// 512-token causal prompt, 32/8 heads, 80: 16.0 -> 15.4).  Below 64 the padding costs what the kernel gains unless the grid
+// fills the chip (head_dim 40: 4096 keys 131 -> 98 us, 512-token prompt 13.9 -> 14.2; head_dim 32: 112 -> 96 and 12.4 ->
+// 14.0), and to 32, where it is half of the work or more, also in short row blocks (300 rows of four sequences 60 -> 64).
+bool prefill_mfma_rows256_takes(int D, float scale, int B, int H, int Sq, int compute_units) {
+    if (!(D % 8 == 0 && D >= 8 && D <= 128 && scale > 0.0f && scale * PF_LOG2E < 2.0f)) return false;
+    if (D >= 64) return true;
+    const long blocks = (long)B * H * ((Sq + PF_BM - 1) / PF_BM);
+    return blocks >= compute_units && (D > 32 || Sq >= 1024);
+}
+
 template <typename T>
 static int launch_t(const AttnParams &p0, hipStream_t stream) {
     AttnParams p = p0;
@@ -726,15 +748,21 @@ static int launch_t(const AttnParams &p0, hipStream_t stream) {
     int out_vec = (p.os[3] == 1 || p.D == 1) && ((uintptr_t)p.out % 16 == 0);
     for (int i = 0; i < 3; i++)
         if ((p.os[i] * oeb) % 16 != 0) out_vec = 0;
-#define PF_LAUNCH(DIM)                                                                                         \
-    if (ks) FHIP_LAUNCH_MAIN((prefill_mfma_kernel<T, DIM, true>), grid, block, stream, p, p, nqb, out_vec);      \
-    else FHIP_LAUNCH_MAIN((prefill_mfma_kernel<T, DIM, false>), grid, block, stream, p, p, nqb, out_vec)
-    switch (p.D) {
-        case 64: PF_LAUNCH(64); break;
-        case 96: PF_LAUNCH(96); break;
-        case 128: PF_LAUNCH(128); break;
-        default: set_error("prefill MFMA kernel: head_dim %d not in {64, 96, 128}", p.D); return FHIP_ERR_UNSUPPORTED;
+#define PF_LAUNCH(DIM, QDIM, PAD)                                                                               \
+    if (ks) FHIP_LAUNCH_MAIN((prefill_mfma_kernel<T, DIM, QDIM, PAD, true>), grid, block, stream, p, p, nqb, out_vec); \
+    else FHIP_LAUNCH_MAIN((prefill_mfma_kernel<T, DIM, QDIM, PAD, false>), grid, block, stream, p, p, nqb, out_vec)
+    if (p.D % 8 != 0 || p.D < 8 || p.D > 128) {
+        set_error("prefill MFMA kernel: head_dim %d is not a multiple of 8 up to 128", p.D);
+        return FHIP_ERR_UNSUPPORTED;
     }
+    if (p.D == 64) { PF_LAUNCH(64, 64, false); }
+    else if (p.D == 96) { PF_LAUNCH(96, 96, false); }
+    else if (p.D == 128) { PF_LAUNCH(128, 128, false); }
+    else if (p.D < 64) { PF_LAUNCH(64, 64, true); }
+    else if (p.D <= 80) { PF_LAUNCH(96, 80, true); }
+    else if (p.D < 96) { PF_LAUNCH(96, 96, true); }
+    else if (p.D <= 112) { PF_LAUNCH(128, 112, true); }
+    else { PF_LAUNCH(128, 128, true); }
 #undef PF_LAUNCH
     FHIP_HIP_CHECK(hipGetLastError());
     if (p.pf_nsplit > 1) return launch_prefill_merge(p, sizeof(T) == 2 && std::is_same<T, half_t>::value ? FHIP_F16 : FHIP_BF16, stream);

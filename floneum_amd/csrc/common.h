@@ -118,8 +118,10 @@ int hip_fail(hipError_t e, const char *what);
 // launchers (each returns a status code, all asynchronous on `stream`)
 int launch_generic(const AttnParams &p, fhip_dtype dtype, hipStream_t stream);
 int launch_decode(const AttnParams &p, fhip_dtype dtype, hipStream_t stream);
+// which calls that kernel takes: head dims to 128, scales times log2(e) below 2
+bool prefill_mfma_rows256_takes(int D, float scale, int B, int H, int Sq, int compute_units);
 int launch_prefill_mfma(const AttnParams &p, fhip_dtype dtype, hipStream_t stream);
-// the same for head dims 160 / 192 / 224 / 256 (four wavefronts per workgroup, 128 query rows, 32-key tiles)
+// the same for every multiple of 8 up to 256 (four wavefronts per workgroup, 128 query rows, 32-key tiles)
 int launch_prefill_mfma_wide(const AttnParams &p, fhip_dtype dtype, hipStream_t stream);
 void prefill_mfma_wide_plan(int B, int H, int G, int Sq, int Skv, bool causal_square, int compute_units, int *nsplit, int *chunk);
 // head dims above 192 on 128-row workgroups of four wavefronts with 32 rows each (one per SIMD, software-pipelined)
