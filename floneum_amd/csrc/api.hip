@@ -946,6 +946,15 @@ int fhip_flash_attention(fhip_stream *s, const fhip_attn_args *args) {
         // f32-arithmetic kernel's mask-adding form (up to head_dim 128), else the general kernel.
         int32_t *bad = (int32_t *)args->workspace;
         int2 *iv = (int2 *)((char *)args->workspace + 16);
+        const bool both_forms = id == FHIP_KERNEL_PREFILL_F32 && f32_serves_both_mask_forms(args);
+        if (both_forms && !args->mask_intervals && prefill_f32_terms_scans(p, args->dtype)) {
+            // a padding mask short enough for every wavefront to look at its own sequence's row
+            AttnParams ps = p;
+            ps.iv_either = 2;
+            rc = launch_prefill_f32(ps, args->dtype, s->s);
+            if (rc == FHIP_OK) FHIP_MARK_MAIN_DONE(p, s->s);
+            return rc;
+        }
         if (args->mask_intervals) {
             // the interval form came with the call (fhip_mask_intervals, computed once for a mask that does not change):
             // no scan
@@ -970,7 +979,6 @@ int fhip_flash_attention(fhip_stream *s, const fhip_attn_args *args) {
         AttnParams pt = p;
         pt.iv = iv;
         pt.iv_bad = bad;
-        const bool both_forms = id == FHIP_KERNEL_PREFILL_F32 && f32_serves_both_mask_forms(args);
         pt.iv_either = both_forms ? 1 : 0;
         rc = id == FHIP_KERNEL_PREFILL_MFMA ? launch_mfma_by_head_dim(pt, args->dtype, s->s) : launch_prefill_f32(pt, args->dtype, s->s);
         if (rc) return rc;

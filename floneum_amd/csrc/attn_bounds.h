@@ -21,10 +21,12 @@ struct RowBounds {
 };
 
 // q0: first row of the workgroup, bm: rows per workgroup, qw0: first row of the wavefront (32 rows,
-// lane ln = lane % 32 owns row qw0 + ln).  iv: the interval form of the mask tensor, or NULL.
-__device__ __forceinline__ RowBounds row_bounds(const AttnParams &p, const int2 *iv, int b, int q0, int bm, int qw0, int lane) {
+// lane ln = lane % 32 owns row qw0 + ln).  iv: the interval form of the mask tensor, or NULL.  span: keys all rows are
+// limited to, where the kernel has found the interval of its sequence's mask row itself.
+__device__ __forceinline__ RowBounds row_bounds(const AttnParams &p, const int2 *iv, int b, int q0, int bm, int qw0, int lane,
+                                                int2 span = int2{0, 0x7fffffff}) {
     const int ln = lane & 31;
-    int kv_lo = 0, kv_hi = p.Skv;
+    int kv_lo = span.x, kv_hi = min(p.Skv, span.y);
     if (p.kv_lens) kv_hi = min(kv_hi, max(p.kv_lens[b], 0));
     if (iv && p.mask_kind == FHIP_MASK_BATCH_KEY) {
         const int2 t = iv[b];

@@ -684,7 +684,7 @@ size_t prefill_f32_workspace_bytes(int B, int H, int Sq, int D, int nsplit) {
 template <typename T>
 static int launch_prefill_f32_t(const AttnParams &p, hipStream_t stream) {
     if (p.D > 128) return launch_wide<T>(p, stream);
-    const int mode = !p.mask ? PF32_INTERVALS : !p.iv ? PF32_BIAS : p.iv_either ? PF32_EITHER : PF32_INTERVALS;
+    const int mode = !p.mask ? PF32_INTERVALS : !p.iv && !p.iv_either ? PF32_BIAS : p.iv_either ? PF32_EITHER : PF32_INTERVALS;
     if (mode == PF32_EITHER && p.D > 64) {
         set_error("internal: the two-form f32 kernel takes head_dim <= 64");
         return FHIP_ERR_UNSUPPORTED;

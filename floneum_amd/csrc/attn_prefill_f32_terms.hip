@@ -40,6 +40,7 @@
 namespace fhip {
 
 constexpr int PT_BN = 32;  // keys per tile
+constexpr int SCAN_KEYS = 1024;  // longest mask row a wavefront looks at itself
 
 #define LDST_PTR(type, byte_off) ((__attribute__((address_space(3))) type *)(lds_base + (byte_off)))
 
@@ -127,6 +128,7 @@ struct TermsLaunch {
     uint32_t g_magic;  // unit / G = (unit * g_magic) >> 32 (0: G is 1)
     int32_t snake;     // workgroups from this one of the last grid dimension on are numbered backwards (0: none)
     int32_t out_vec;   // bytes per store of the result: 16 (f32), 8 (16-bit), or 0: element by element
+    int32_t mask_rows; // an added mask is read four keys at a time through a buffer
 };
 
 template <typename T, int D, int U, int KG, int MODE>
@@ -134,6 +136,12 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
     typedef PtCfg<T, D, U> C;
     constexpr int N = C::N, NDB = D / 32, NKB = D / 16;
     constexpr bool BIAS = MODE != PF32_INTERVALS;
+    // Which phase of the two wavefronts on a SIMD goes first where both could issue: the matrix one at wide heads, the vector
+    // one where a tile's matrix work is short beside it.  D = 64: 12 x 700 rows with added masks 127 us without priorities,
+    // 126 / 122 with the matrix / vector phase first, 2048-row prompt 115, 112 / 110.5; D = 128: 1024-row prompt 79, 76 / 76,
+    // 4096 rows 717, 711 / 718.
+    // Four key groups (few tiles per wavefront) gain nothing from the vector phase: 512-row layer 29.3 against 29.7.
+    constexpr int MATRIX_PRIO = D > 64 || KG == 4 ? 1 : 0;
     __shared__ __attribute__((aligned(16))) char smem[KG * C::G_BYTES > U * KG * C::ROWS_BYTES ? KG * C::G_BYTES : U * KG * C::ROWS_BYTES];
     auto lds_base = (__attribute__((address_space(3))) char *)smem;
 
@@ -142,7 +150,7 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
     pin(p.q, p.k, p.v, p.out, p.mask, p.kv_lens, p.qs[0], p.qs[1], p.qs[2], p.ks[0], p.ks[1], p.ks[2]);
     pin(p.vs[0], p.vs[1], p.vs[2], p.os[0], p.os[1], p.os[2], p.ms0, p.B, p.Hkv, p.G, p.Sq, p.Skv, p.D, p.mask_kind);
     pin(p.analytic, p.causal, p.q_pos_offset, p.window, p.scale, p.iv, p.iv_bad, p.only_if_bad, p.bad_tag, p.pf_nsplit, p.pf_chunk,
-        tl.g_magic, tl.snake);
+        p.iv_either, tl.g_magic, tl.snake, tl.mask_rows);
 
     if constexpr (MODE == PF32_BIAS) {
         if (p.only_if_bad && *p.only_if_bad != p.bad_tag) return;  // the interval form of the mask has served the call
@@ -184,9 +192,45 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
     const int bm = 32 * (over_g(first_unit + U - 1) + 1) - q0;   // rows from there to its last
     const int qw0 = 32 * unit_row;
     const int query = qw0 + ln;
-    // uniform over the launch
-    const bool bias_on = MODE == PF32_BIAS || (MODE == PF32_EITHER && *p.iv_bad == p.bad_tag);
-    RowBounds rb = row_bounds(p, MODE == PF32_BIAS ? nullptr : p.iv, b, q0, bm, qw0, lane);
+    // uniform over the sequence
+    bool bias_on = MODE == PF32_BIAS;
+    int2 span = {0, 0x7fffffff};
+    if constexpr (MODE == PF32_EITHER) {
+        if (p.iv_either == 2) {
+            // What the scan launch would find, of this sequence's row alone (at most SCAN_KEYS keys, in whole pieces): that
+            // launch in front cost 8 x 512 keys 4.7 us, the row's pieces come in about the time its result took to read.
+            const auto row = __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)p.mask + b * p.ms0), 0, p.Skv * (int)sizeof(T), 0x00020000);
+            constexpr int PIECES = SCAN_KEYS / 256;
+            float4_t x[PIECES];
+#pragma unroll
+            for (int i = 0; i < PIECES; i++)
+                if (256 * i < p.Skv) x[i] = buffer_load4<T>(row, lane * 4 * (int)sizeof(T), 256 * i * (int)sizeof(T));
+            int lo = 0x7fffffff, hi = 0, zeros = 0;
+            bool others = false;
+#pragma unroll
+            for (int i = 0; i < PIECES; i++) {
+                if (256 * i >= p.Skv) continue;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int key = 256 * i + 4 * lane + e;
+                    const bool zero = key < p.Skv && x[i][e] == 0.0f;
+                    others |= key < p.Skv && !zero && x[i][e] != -INFINITY;
+                    lo = zero ? min(lo, key) : lo;
+                    hi = zero ? key + 1 : hi;
+                    zeros += zero;
+                }
+            }
+            lo = wave_reduce_i(lo, [](int x, int y) { return min(x, y); });
+            hi = wave_reduce_i(hi, [](int x, int y) { return max(x, y); });
+            zeros = wave_reduce_i(zeros, [](int x, int y) { return x + y; });
+            if (zeros == 0) lo = 0;  // no visible key: the empty interval
+            bias_on = __builtin_amdgcn_ballot_w64(others) != 0 || __builtin_amdgcn_readfirstlane(zeros) != __builtin_amdgcn_readfirstlane(hi - lo);
+            if (!bias_on) span = {lo, hi};
+        } else {
+            bias_on = *p.iv_bad == p.bad_tag;
+        }
+    }
+    RowBounds rb = row_bounds(p, MODE == PF32_BIAS ? nullptr : p.iv, b, q0, bm, qw0, lane, span);
     if constexpr (MODE == PF32_EITHER) {
         if (bias_on) rb = row_bounds(p, nullptr, b, q0, bm, qw0, lane);
     }
@@ -302,6 +346,11 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
     const T *mrow = nullptr;
     if constexpr (BIAS)
         mrow = (const T *)p.mask + (int64_t)(p.mask_kind == FHIP_MASK_QK ? min(query, p.Sq - 1) : b) * p.ms0;
+    // The same as a buffer.  Whole tiles read four keys per load without an address or a test per element, which cost more
+    // than the tile's matrix work: f32, 8 x 512 rows, 12 heads, D = 64 with -10000 on the padding 61 -> 46 us (the scan launch below included).
+    const auto mask_buf = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)((const T *)p.mask + (BIAS && p.mask_kind != FHIP_MASK_QK ? b * p.ms0 : 0)), 0, 0x7fffffff, 0x00020000);
+    const int mask_at = (p.mask_kind == FHIP_MASK_QK ? min(query, p.Sq - 1) * (int)p.ms0 * ES : 0) + 4 * h2 * ES;
 
     float16_t s;
     uint32_t pt[3][8];  // the terms of the tile's probabilities, packed pairs in the operand's order
@@ -313,7 +362,14 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
     auto scores = [&](int j0) __attribute__((always_inline)) {
         float bias[BIAS ? 16 : 1];
         if constexpr (BIAS) {  // requested before the matrix work that hides their latency
-            if (bias_on) {
+            if (bias_on && tl.mask_rows && j0 + PT_BN <= p.Skv) {
+#pragma unroll
+                for (int rq = 0; rq < 4; rq++) {
+                    const float4_t x = buffer_load4<T>(mask_buf, mask_at + 8 * rq * ES, j0 * ES);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) bias[4 * rq + e] = x[e];
+                }
+            } else if (bias_on) {
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
                     const int key = j0 + 8 * (r >> 2) + 4 * h2 + (r & 3);
@@ -329,6 +385,7 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
         auto read_k = [&](int kb, int i) __attribute__((always_inline)) {
             ka[i] = __builtin_bit_cast(bf16x8_t, *LDST_PTR(uint4_t, k_at + i * C::K_PLANE + kb * 32));
         };
+        __builtin_amdgcn_s_setprio(MATRIX_PRIO);
 #pragma unroll
         for (int i = N - 1; i >= 0; i--) read_k(0, i);
 #pragma unroll
@@ -353,6 +410,7 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
                 else __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                 if (kb + 1 < NKB) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
             }
+        __builtin_amdgcn_s_setprio(1 - MATRIX_PRIO);
         if constexpr (N > 1) s += small;
 
         // element r is key j0 + 8 (r / 4) + 4 h2 + r % 4 for query `query`
@@ -468,7 +526,9 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
         if (it > 0) store_rows(st, gbase + C::V_BASE, C::VP, C::V_PLANE);
         if (more) load_rows(st, k_rows, k_row, j0 + KG * PT_BN);
         lds_barrier();
+        __builtin_amdgcn_s_setprio(MATRIX_PRIO);
         if (tile_visible) pv();
+        __builtin_amdgcn_s_setprio(1 - MATRIX_PRIO);
         if (more) {
             store_rows(st, gbase, C::KP, C::K_PLANE);  // the group's next K tile: every wavefront is past S^T of this one
             load_rows(st, v_rows, v_row, j0 + KG * PT_BN);
@@ -610,6 +670,10 @@ static int launch_form(const AttnParams &p_in, hipStream_t stream) {
     tl.out_vec = p.os[3] == 1 && (uintptr_t)p.out % (4 * oeb) == 0 ? 4 * oeb : 0;
     for (int i = 0; i < 3; i++)
         if (p.os[i] % 4 != 0) tl.out_vec = 0;
+    // rows of the mask in 16-byte (f32, element-aligned) or 8-byte pieces, within a buffer's 32-bit offsets
+    const int64_t mask_span = ((p.mask_kind == FHIP_MASK_QK ? (int64_t)(p.Sq - 1) * p.ms0 : 0) + p.Skv) * (int64_t)sizeof(T);
+    tl.mask_rows = p.mask_kind != FHIP_MASK_NONE && p.ms1 == 1 && p.ms0 >= 0 && mask_span < 0x7fffffffLL &&
+                   (sizeof(T) == 4 || ((uintptr_t)p.mask % 8 == 0 && p.ms0 % 4 == 0));
     dim3 grid(nks, groups, nwg), block(64 * U * KG);
     switch ((p.D + 31) / 32 * 32) {  // the kernel's D is head_dim rounded up to a multiple of 32
         case 32: FHIP_LAUNCH_MAIN((prefill_f32_terms_kernel<T, 32, U, KG, MODE>), grid, block, stream, p, p, tl); break;
@@ -664,6 +728,14 @@ bool prefill_f32_terms_takes(const AttnParams &p) {
     if ((int64_t)p.B * p.Hkv > 65535 || units > 65535 || units * p.G > 0x7fffffffLL) return false;
     if (p.qs[2] < 0 || (int64_t)p.Sq * p.qs[2] * 4 >= 0x7fffffffLL) return false;
     return p.D <= 128 && p.ks[2] >= p.D && p.vs[2] >= p.D && rows * p.ks[2] * 4 < 0x7fffffffLL && rows * p.vs[2] * 4 < 0x7fffffffLL;
+}
+
+// A BatchKeyMask whose row every wavefront can look at for itself, four keys per load and all loads at once: no scan launch.
+// Longer rows, rows of a QKMask (each read by all heads) and 16-bit rows, whose last piece a buffer's bounds would cut, are
+// scanned once per call.
+bool prefill_f32_terms_scans(const AttnParams &p, fhip_dtype dtype) {
+    return dtype == FHIP_F32 && p.mask_kind == FHIP_MASK_BATCH_KEY && p.D <= 64 && p.Skv <= SCAN_KEYS && p.ms1 == 1 &&
+           prefill_f32_terms_takes(p);
 }
 
 int launch_prefill_f32_terms(const AttnParams &p, fhip_dtype dtype, int mode, hipStream_t stream) {

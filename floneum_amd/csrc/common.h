@@ -48,6 +48,7 @@ struct AttnParams {
     const int2 *iv;
     // With iv_either set the f32-arithmetic tiled kernel (head_dim <= 64) serves the call whatever the scan found: it
     // masks by interval when *iv_bad != bad_tag and adds the mask values otherwise, and no second kernel is queued.
+    // 2: there was no scan; the kernel looks at its sequence's row of the mask itself (prefill_f32_terms_scans).
     int32_t iv_either;
     const int32_t *iv_bad;
     const int32_t *only_if_bad;
@@ -134,6 +135,7 @@ int launch_prefill_mfma_rows64(const AttnParams &p, fhip_dtype dtype, hipStream_
 int launch_prefill_f32(const AttnParams &p, fhip_dtype dtype, hipStream_t stream);
 // the same precision on the bf16 matrix cores, head dims to 128 (mode: a PF32_... of attn_f32.h); no merge of key shares
 bool prefill_f32_terms_takes(const AttnParams &p);
+bool prefill_f32_terms_scans(const AttnParams &p, fhip_dtype dtype);  // no scan launch is needed: iv_either may be 2
 int launch_prefill_f32_terms(const AttnParams &p, fhip_dtype dtype, int mode, hipStream_t stream);
 
 // decode planning (host): keys per split and number of splits; `ragged`: per-batch key counts are given;
