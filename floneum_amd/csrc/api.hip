@@ -914,7 +914,7 @@ int fhip_flash_attention(fhip_stream *s, const fhip_attn_args *args) {
         if (part && usable && args->workspace_bytes >= off + part) {
             p.pf_nsplit = ns;
             p.pf_chunk = chunk;
-            p.pf_pitch = p.D + 4;  // rows of the partials are written in 16-byte pieces
+            p.pf_pitch = p.D + 2;
             p.partials = (float *)((char *)args->workspace + off);
         }
     }

@@ -634,16 +634,23 @@ void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_s
     *chunk = Skv;
     if (D <= 128) {
         // attn_prefill_f32_terms.hip, whose forms with key groups give a CU eight wavefronts in one workgroup: one workgroup
-        // per CU, shares of at least 256 keys, or 128 while that leaves CUs idle.  (The same for a causal descriptor and for
-        // a mask tensor: a square prompt keeps its plan, and with it its bits.)
+        // per CU, shares of at least 256 keys, or 128 while 256-key shares of all units are fewer than the CUs.  (The same
+        // for a causal descriptor and for a mask tensor: a square prompt keeps its plan, and with it its bits.)
         const bool few_rows = 2L * Sq <= Skv;
-        const int U = D > 64 && (few_rows || Skv >= 768) ? 4 : 2;
-        const long wgs = (long)B * (H / G) * ((G * ((Sq + 31) / 32) + U - 1) / U);
-        if (wgs == 0 || 2 * wgs > compute_units) return;
-        const long want = compute_units / wgs;
+        const long units = (long)G * ((Sq + 31) / 32), kv_heads = (long)B * (H / G);
         long most = Skv / 256;
-        if (few_rows && (want < most ? want : most) * wgs < compute_units) most = Skv / 128;
-        const long ns = want < most ? want : most;
+        if (few_rows && most * kv_heads * units < compute_units) most = Skv / 128;
+        auto shares = [&](int U) {
+            const long wgs = kv_heads * ((units + U - 1) / U);
+            if (wgs == 0 || 2 * wgs > compute_units) return 1L;
+            const long want = compute_units / wgs;
+            return want < most ? want : most;
+        };
+        long ns = shares(D > 64 && (few_rows || Skv >= 768) ? 4 : 2);
+        // Partials beyond 16 MiB: half the shares for workgroups of half the units, so that a call's workspace stays within
+        // about what its caller may have set aside for it (32/8 heads, 128 rows on 8192 keys: 4 shares 125 us, 8 shares 97).
+        constexpr size_t MOST_PARTIALS = (size_t)16 << 20;
+        if (few_rows && D > 64 && prefill_f32_workspace_bytes(B, H, Sq, D, (int)ns) > MOST_PARTIALS) ns = shares(2);
         if (ns < 2) return;
         const long c = ((Skv + ns - 1) / ns + 31) / 32 * 32;
         *chunk = (int)c;
@@ -678,7 +685,7 @@ void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_s
 
 size_t prefill_f32_workspace_bytes(int B, int H, int Sq, int D, int nsplit) {
     if (nsplit <= 1) return 0;
-    return (size_t)B * H * Sq * nsplit * (size_t)(D + 4) * sizeof(float);
+    return (size_t)B * H * Sq * nsplit * (size_t)(D + 2) * sizeof(float);
 }
 
 template <typename T>

@@ -40,6 +40,7 @@
 namespace fhip {
 
 constexpr int PT_BN = 32;  // keys per tile
+typedef float4_t __attribute__((aligned(8))) float4_at8_t;  // a row of the partials is D + 2 floats
 constexpr int SCAN_KEYS = 1024;  // longest mask row a wavefront looks at itself
 
 #define LDST_PTR(type, byte_off) ((__attribute__((address_space(3))) type *)(lds_base + (byte_off)))
@@ -622,7 +623,7 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
                 if (q >= p.Sq || dim >= p.D) continue;
                 const float4_t v = *LDST_PTR(float4_t, mine + row * C::OUT_PITCH + (lane & 7) * 16);
                 if (parked) {
-                    *(float4_t *)(part + q * part_row + dim) = v;
+                    *(float4_at8_t *)(part + q * part_row + dim) = v;
                 } else if (sizeof(T) == 4 || tl.out_vec == 16) {
                     *(float4_t *)((float *)p.out + ob + (int64_t)q * p.os[2] + dim) = v;
                 } else if constexpr (sizeof(T) == 2) {
@@ -713,7 +714,7 @@ static int launch_terms(const AttnParams &p, hipStream_t stream) {
             if (uneven && 2 * w4 <= 5L * cus) return launch_form<T, 2, 2, MODE>(p, stream);
             if (!uneven && w4 <= cus) return launch_form<T, 4, 2, MODE>(p, stream);
         } else {
-            if (!few_rows && 2 * w2 <= 3L * cus) return launch_form<T, 2, 2, MODE>(p, stream);
+            if (2 * w2 <= (few_rows ? 2L : 3L) * cus) return launch_form<T, 2, 2, MODE>(p, stream);
             if (w4 < 2L * cus) return launch_form<T, 4, 2, MODE>(p, stream);
         }
     }

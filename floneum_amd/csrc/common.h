@@ -60,7 +60,7 @@ struct AttnParams {
     // cache would otherwise occupy a fraction of the chip).  Split s takes keys [s * pf_chunk, (s + 1) * pf_chunk)
     // and parks (O unnormalised, m, l) per row in `partials` [B, H, Sq, pf_nsplit, pf_pitch]; a merge kernel follows.
     int32_t pf_nsplit, pf_chunk;
-    int32_t pf_pitch;  // floats per (row, share) in `partials`: D + 4, rows are written in 16-byte pieces
+    int32_t pf_pitch;  // floats per (row, share) in `partials`: D + 2, or D + 4 where 16-byte pieces of rows are to be aligned
     int32_t pf_pack;   // tiled kernels, set by their launchers: query heads per workgroup of the packed form, or 0
     int32_t pf_rows64; // 16-bit tiled prefill at head_dim 128: the caller forced the 64-rows-per-wavefront form
 };
