@@ -7,7 +7,8 @@
 // the f32 accumulation; the other six are formed: 6 / 16 of the f32 instruction's matrix time.  16-bit tensors, which
 // this kernel serves where their own one does not (finite mask values), have two terms (f16) or one (bf16); the
 // probabilities are f32 values and always have three.
-// Infinities: an element of Q, K or V that is +-inf (or beyond 3.39e38, bf16's largest) makes its products NaN.
+// Infinities: an element of Q, K or V that is +-inf (or beyond 3.39e38, bf16's largest) makes its products NaN.  Rows whose
+// sums are not finite at the end are formed once more without terms (plain_row).
 //
 // A unit is 32 query rows of one head; a wavefront owns one.  A workgroup holds U units that share a KV head (the heads of
 // a GQA group first, then further rows) and walks the keys they see in tiles of 32 rows, which are split into terms on the
@@ -131,6 +132,51 @@ struct TermsLaunch {
     int32_t out_vec;   // bytes per store of the result: 16 (f32), 8 (16-bit), or 0: element by element
     int32_t mask_rows; // an added mask is read four keys at a time through a buffer
 };
+
+// One row by plain f32 sums over its keys [lo, hi): exponent, sum and (in acc) the unnormalised result, whose dims lane and
+// lane + 64 a lane holds.  For rows that met an element without a finite bf16 term, so only its answer matters: lanes split
+// the keys for the scores and the dims for P.V.  q_at: LDS space for head_dim floats; mrow: mask values to add, or NULL.
+struct PlainRow {
+    float m, l, acc[2];
+};
+template <typename T>
+__device__ __forceinline__ PlainRow plain_row(const AttnParams &p, __attribute__((address_space(3))) char *q_at, const T *q, const T *k,
+                                              const T *v, const T *mrow, int lo, int hi, int lane) {
+    auto q_lds = (__attribute__((address_space(3))) float *)q_at;
+    wave_lds_sync();
+    for (int d = lane; d < p.D; d += 64) q_lds[d] = to_float(q[d]);
+    wave_lds_sync();
+    PlainRow r = {-INFINITY, 0.0f, {0.0f, 0.0f}};
+    for (int j0 = lo; j0 < hi; j0 += 64) {
+        float s = -INFINITY;
+        if (j0 + lane < hi) {
+            const T *kr = k + (j0 + lane) * p.ks[2];
+            float dot = 0.0f;
+            for (int d = 0; d < p.D; d++) dot = __builtin_fmaf(q_lds[d], to_float(kr[d]), dot);
+            s = dot * p.scale;
+            if (mrow) s += to_float(mrow[(j0 + lane) * p.ms1]);
+            s *= PF32_LOG2E;
+        }
+        // fmaxf passes NaN by: a score that is NaN leaves the exponent alone and makes the sums NaN; with no other score than
+        // -inf and NaN the exponent stays -inf and -inf - 0 gives 0, NaN gives NaN
+        const float m_new = fmaxf(r.m, wave_max(s)), base = m_new == -INFINITY ? 0.0f : m_new;
+        const float pj = __builtin_amdgcn_exp2f(s - base), corr = __builtin_amdgcn_exp2f(r.m - base);
+        r.m = m_new;
+        r.l = r.l * corr + wave_sum(pj);
+        const int n = min(64, hi - j0);
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const int d = lane + 64 * t;
+            float a = r.acc[t] * corr;
+            for (int jj = 0; jj < n; jj++) {
+                const float w = read_lane(pj, jj);
+                if (d < p.D) a = __builtin_fmaf(w, to_float(v[(j0 + jj) * p.vs[2] + d]), a);
+            }
+            r.acc[t] = a;
+        }
+    }
+    return r;
+}
 
 template <typename T, int D, int U, int KG, int MODE>
 __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG == 1 && D == 64 && MODE == PF32_INTERVALS ? 3 : 2) void prefill_f32_terms_kernel(AttnParams p, TermsLaunch tl) {
@@ -585,6 +631,14 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
     // ---- out[query][dim] = O^T[dim][query] / l; with the keys split over workgroups this share's state is parked and
     // the merge kernel normalises
     const float l_tot = half_swap_sum32(l);
+    // rows with a sum that is not finite: 0 x inf and 0 x NaN are NaN
+    float zero[4] = {l * 0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int db = 0; db < NDB; db++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) zero[r & 3] = __builtin_fmaf(o[db][r], 0.0f, zero[r & 3]);
+    const uint64_t odd = __builtin_amdgcn_ballot_w64(!(zero[0] + zero[1] + (zero[2] + zero[3]) == 0.0f));
+    uint32_t odd_rows = (uint32_t)odd | (uint32_t)(odd >> 32);
     const bool parked = nks > 1;
     float *const part = p.partials + (((int64_t)b * p.H + h) * p.Sq * nks + ksplit) * p.pf_pitch;
     const int64_t part_row = (int64_t)nks * p.pf_pitch;
@@ -605,9 +659,9 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
             }
     }
     const int64_t ob = b * p.os[0] + h * p.os[1];
-    if (parked || tl.out_vec) {
-        // through a wavefront's own part of LDS (with key groups: where this wavefront alone has just read), 32 dims at a time
-        const int mine = KG > 1 ? wave * (4 * NDB + 1) * 1024 : wave * C::ROWS_BYTES;
+    // a wavefront's own part of LDS (with key groups: where this wavefront alone has just read)
+    const int mine = KG > 1 ? wave * (4 * NDB + 1) * 1024 : wave * C::ROWS_BYTES;
+    if (parked || tl.out_vec) {  // through LDS, 32 dims at a time
 #pragma unroll
         for (int db = 0; db < NDB; db++) {
             wave_lds_sync();
@@ -634,16 +688,33 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
                 }
             }
         }
-        return;
+    } else if (query < p.Sq) {
+#pragma unroll
+        for (int db = 0; db < NDB; db++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int dim = 32 * db + 8 * (r >> 2) + 4 * h2 + (r & 3);
+                if (dim < p.D) store_out<T>(p, ob + (int64_t)query * p.os[2] + dim * p.os[3], o[db][r]);
+            }
     }
-    if (query >= p.Sq) return;
+    if (odd_rows == 0) return;
+    __threadfence();  // the stores above come first
+    for (; odd_rows; odd_rows &= odd_rows - 1) {
+        const int row = __builtin_ctz(odd_rows), q = qw0 + row;
+        if (q >= p.Sq) return;
+        const T *bias_row = bias_on ? (const T *)p.mask + (int64_t)(p.mask_kind == FHIP_MASK_QK ? q : b) * p.ms0 : nullptr;
+        const PlainRow x = plain_row<T>(p, lds_base + mine, (const T *)p.q + b * p.qs[0] + h * p.qs[1] + q * p.qs[2],
+                                        (const T *)p.k + b * p.ks[0] + g * p.ks[1], (const T *)p.v + b * p.vs[0] + g * p.vs[1],
+                                        bias_row, __builtin_amdgcn_readlane(rb.klo, row), __builtin_amdgcn_readlane(rb.khi, row), lane);
+        if (parked && lane == 0) part[q * part_row + p.D] = x.m, part[q * part_row + p.D + 1] = x.l;
 #pragma unroll
-    for (int db = 0; db < NDB; db++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int dim = 32 * db + 8 * (r >> 2) + 4 * h2 + (r & 3);
-            if (dim < p.D) store_out<T>(p, ob + (int64_t)query * p.os[2] + dim * p.os[3], o[db][r]);
+        for (int t = 0; t < 2; t++) {
+            const int dim = lane + 64 * t;
+            if (dim >= p.D) continue;
+            if (parked) part[q * part_row + dim] = x.acc[t];
+            else store_out<T>(p, ob + (int64_t)q * p.os[2] + dim * p.os[3], x.acc[t] / x.l);
         }
+    }
 }
 
 // workgroups of the form with U units each
