@@ -257,8 +257,9 @@ static bool prefill_mfma_eligible(const fhip_attn_args *a) {
     const bool exact = D == 64 || D == 96 || D == 128;
     if (D % 8 != 0 || D < 8 || D > 256) return false;
     if (!rows_vectorizable(a->q, 2) || !rows_vectorizable(a->k, 2) || !rows_vectorizable(a->v, 2)) return false;
-    // that kernel multiplies Q by the power-of-two part of scale * log2(e): the power must be at most 1 so that no finite
-    // element can leave the type's range (the wide-head kernel scales the scores in f32 only)
+    // in bf16 that kernel multiplies Q by the power-of-two part of scale * log2(e): the power must be at most 1 so that no
+    // finite element can leave the type's range (f16 and the padded head dims are scaled in f32 only, and so is the wide-head
+    // kernel; f16 keeps the same limit)
     if (exact && (!(a->scale > 0.0f) || !(a->scale * 1.4426950408889634f < 2.0f))) return false;
     // K/V rows are fetched through 32-bit buffer offsets: rows must not overlap and one (batch, kv
     // head) slice must span less than 2 GiB

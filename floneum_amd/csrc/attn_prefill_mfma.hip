@@ -4,9 +4,8 @@
 // Keys/values are walked in tiles of 64 rows that go from global memory straight into a three-stage
 // LDS ring (direct-to-LDS buffer loads, no staging registers).  Per tile and wavefront:
 //   S^T (64 keys x 32 queries)  = K_tile . Q^T      v_mfma_f32_32x32x16  (A = K from LDS, B = Q in registers)
-//   Q is multiplied once by the power-of-two part of scale * log2(e) (exact); the rest, a factor rr in [1, 2),
-//   multiplies the scores in f32: a probability is exp2(fma(s, rr, -m * rr)), one fused multiply-add and one
-//   exponential per score, with m the row's reference exponent
+//   scale * log2(e) (rr) multiplies the scores in f32: a probability is exp2(fma(s, rr, -m * rr)), one fused
+//   multiply-add and one exponential per score, with m the row's reference exponent
 //   online softmax down the key axis: with S^T every lane owns ONE query column and 16 keys of it per 32-key
 //   block, so row sums are in-lane folds (the two half-rows are added once, at the end).  No maximum is taken
 //   per tile: the reference m is the maximum the row had when it was last set, and it is moved (and l and O
@@ -60,11 +59,6 @@ struct Mma<half_t> {
     static __device__ __forceinline__ uint32_t pack2(float x, float y) {
         half2_t h = {(half_t)x, (half_t)y};
         return __builtin_bit_cast(uint32_t, h);
-    }
-    static __device__ __forceinline__ vec8 scaled(vec8 q, float c) {
-#pragma unroll
-        for (int e = 0; e < 8; e++) q[e] = (half_t)((float)q[e] * c);
-        return q;
     }
 };
 template <>
@@ -182,15 +176,18 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnPara
     const bool wave_has_rows = qw0 < p.Sq;
 
     // Q^T operand: Q[query][16 kb + 8 h2 .. +8], kept in registers for the whole kernel
-    // (the loads are issued here, the scaling waits until the first K/V tiles are on their way too)
+    // (the loads are issued here; whatever scaling they take waits until the first K/V tiles are on their way too)
     const float scale2 = p.scale * PF_LOG2E;
-    // scale2 = pw * rr with pw a power of two and rr in [1, 2).  Q takes pw, which is exact in f16 and bf16 alike, and
     // rr multiplies every score in f32 right before exp2: the scores are then the f32 dot product times the scale, one
-    // rounding, as the reference computes them (fusor-ml/fusor/src/composite/flash_attention.rs:145).  Folding all of
-    // scale2 into Q instead would save that multiply but round Q's elements a second time (11 bits in f16, 8 in bf16),
-    // an error that grows in proportion to the scores.  The S^T accumulators and m are in units of 1 / rr.
-    const float pw = __uint_as_float(__float_as_uint(scale2) & 0x7F800000u);
-    const float rr = scale2 / pw;
+    // rounding, as the reference computes them (fusor-ml/fusor/src/composite/flash_attention.rs:145).  Folding scale2 into
+    // Q instead would save that multiply but round Q's elements a second time (11 bits in f16, 8 in bf16), an error that
+    // grows in proportion to the scores.  The S^T accumulators and m are in units of 1 / rr.
+    // bf16 at the kernel's own head dims: Q takes the power of two in scale2 (pw), which is exact down to bf16's smallest
+    // normal value and keeps dot products of very large elements inside f32's range.  f16 takes none of it: elements below
+    // 2^-14 / pw would become subnormal and lose bits, and the products of f16 elements cannot leave f32's range.
+    constexpr bool FOLD = std::is_same<T, bf16_t>::value && !PAD;
+    const float pw = FOLD ? __uint_as_float(__float_as_uint(scale2) & 0x7F800000u) : 1.0f;
+    const float rr = FOLD ? scale2 / pw : scale2;
     vec8 qreg[QD / 16];
     {
         const uint16_t *qp = (const uint16_t *)p.q + b * p.qs[0] + h * p.qs[1] + (int64_t)qrow * p.qs[2];
@@ -567,8 +564,10 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnPara
         } else {
             issue_tile(0);
         }
+        if constexpr (FOLD) {
 #pragma unroll
-        for (int kb = 0; kb < QD / 16; kb++) qreg[kb] = Mma<T>::scaled(qreg[kb], pw);
+            for (int kb = 0; kb < QD / 16; kb++) qreg[kb] = Mma<T>::scaled(qreg[kb], pw);
+        }
         wait_tiles(integral_constant<int, 0>{});
         lds_barrier();
         if (group == 0) {

@@ -20,7 +20,7 @@
 // of four LDS stages each, loaded straight into LDS (no staging registers) two iterations ahead of their first
 // reader; one workgroup barrier per iteration publishes what has landed.
 //
-// Softmax as in the 256-row kernel: Q carries the power-of-two part of scale * log2(e), the rest (rr in [1, 2))
+// Softmax as in the 256-row kernel, with the power-of-two part of scale * log2(e) in Q; the rest (rr in [1, 2))
 // multiplies the scores in f32; a probability is exp2(fma(s, rr, -m * rr)) against the reference m the row already
 // has, and m moves only when a lane's probabilities of a tile sum to more than 2^15.
 // Masking is by interval (attn_bounds.h): analytic descriptors, key counts, the interval form of a mask tensor.

@@ -70,3 +70,22 @@ def test_forms_and_edges(device, form, D, dtype):
         err = np.linalg.norm(got[..., :D] - ref) / np.linalg.norm(ref)
         assert err <= tol, f"{form} D{D}: relative L2 {err:.2e}"
         assert (got[..., D:] == 7.0).all(), f"{form} D{D}: written behind head_dim"
+
+
+@pytest.mark.parametrize("dtype", [fa.F16, fa.BF16])
+@pytest.mark.parametrize("form,D", [("blocks_of_128", 80), ("blocks_of_256", 80), ("blocks_of_256", 40), ("keys_split", 120),
+                                    ("blocks_of_128", 64), ("blocks_of_256", 128)])
+@pytest.mark.parametrize("q_std,k_std,scale", [(1e-4, 1e4, None), (1.0, 1e4, 1e-5), (1.0, 1e4, 1e-6), (1e-5, 1e4, 0.5)])
+def test_small_scales_and_elements(device, form, D, dtype, q_std, k_std, scale):
+    """The scale is applied to the f32 scores: elements of Q times a power of two of it would leave f16's normal range, and
+    with it lose bits, for some of these.  (scores of a few units at most, so that every probability has weight)"""
+    B, H, Hkv, Sq, Skv, causal, window = FORMS[form]
+    scale = float(np.float32(D ** -0.5 if scale is None else scale))
+    rng = np.random.default_rng(D + 1)
+    stds, shapes = (q_std, k_std, 1.0), [(B, H, Sq, D), (B, Hkv, Skv, D), (B, Hkv, Skv, D)]
+    tq, tk, tv = (fa.Tensor.from_numpy(device, rng.normal(0, sd, sh).astype(np.float32), dtype) for sd, sh in zip(stds, shapes))
+    analytic = (True, Skv - Sq, window) if causal else None
+    out = tq.flash_attention(tk, tv, scale, analytic=analytic, out_dtype=fa.F32, force_kernel=fa.KERNEL_PREFILL_MFMA).to_numpy()
+    ref = in_64_bits(*(t.to_numpy().astype(np.float64) for t in (tq, tk, tv)), scale, causal, window)
+    err = np.linalg.norm(out - ref) / np.linalg.norm(ref)
+    assert err <= 3 * (2.0 ** -12 if dtype == fa.F16 else 2.0 ** -9), f"{form} D{D}: relative L2 {err:.2e}"
