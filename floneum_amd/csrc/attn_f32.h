@@ -17,6 +17,24 @@ constexpr float PF32_LOG2E = 1.4426950408889634f;
 //                   launch behind the tiled kernel; head_dim <= 64 (the register budget of both forms in one kernel).
 constexpr int PF32_INTERVALS = 0, PF32_BIAS = 1, PF32_EITHER = 2;
 
+// Probabilities are formed against a row's reference m, the maximum its scores had when it was last set: exp2(s * unit -
+// m * unit) in one fused multiply-add and one exponential, `unit` being 1 where scores are exponents of two and log2(e)
+// where a mask has been added to them.  (The score itself takes no log2(e): a sum of a score and a mask value that is rounded
+// again at its own size has lost another bit of it.)  m * unit is the rounded product everywhere.  It overflows for references
+// below -2.36e38, rows of which every score so far holds a padding value like f32's or bf16's lowest: neighbours are
+// 2e31 apart there, so a score that equals m has probability 1 and every other 0.
+__device__ __forceinline__ float probability(float s, float m, float unit) {
+    const float m2 = m * unit;
+    if (m2 == -INFINITY) return s == m && m > -INFINITY ? 1.0f : s != s ? s : 0.0f;
+    return __builtin_amdgcn_exp2f(__builtin_fmaf(s, unit, -m2));
+}
+// what probabilities formed against m are to be multiplied by when the reference is m_new >= m
+__device__ __forceinline__ float moved_reference(float m, float m_new, float unit) {
+#pragma clang fp contract(off)
+    const float m2 = m * unit, m2_new = m_new * unit;  // both rounded, as where probabilities are formed
+    return m == m_new ? 1.0f : m2 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m2 - m2_new);
+}
+
 // four consecutive elements of a row as f32 (16-bit storage types are widened exactly)
 __device__ __forceinline__ float4_t load4(const float *p) { return *(const float4_t *)p; }
 __device__ __forceinline__ float4_t load4(const half_t *p) {

@@ -291,8 +291,9 @@ __global__ __launch_bounds__(64 * PF32_WAVES, 2) void prefill_f32_kernel(AttnPar
     }
 }
 
-// Merge of the key shares: one wavefront per (batch, head, query row), log-sum-exp over the shares (the state is
-// in the base-2 domain), then the division the single-pass form does in its epilogue.
+// Merge of the key shares: one wavefront per (batch, head, query row), log-sum-exp over the shares, then the division the
+// single-pass form does in its epilogue.  A row's references m are exponents of two, or, where a mask is added to the
+// scores, in the scores' own units: those rows' sums l are parked with their sign set (-0.0 included).
 template <typename T>
 __global__ __launch_bounds__(256) void prefill_f32_merge_kernel(AttnParams p) {
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -322,17 +323,25 @@ __global__ __launch_bounds__(256) void prefill_f32_merge_kernel(AttnParams p) {
         float Mn = M;
 #pragma unroll
         for (int u = 0; u < 8; u++) Mn = fmaxf(Mn, ms[u]);
-        const float Ms = (Mn == -INFINITY) ? 0.0f : Mn;
-        const float c = __builtin_amdgcn_exp2f(M - Ms);
+        float c, w[8];
+        if (__builtin_amdgcn_readfirstlane(__float_as_int(ls[0])) >= 0) {
+            const float Ms = (Mn == -INFINITY) ? 0.0f : Mn;
+            c = __builtin_amdgcn_exp2f(M - Ms);
+#pragma unroll
+            for (int u = 0; u < 8; u++) w[u] = __builtin_amdgcn_exp2f(ms[u] - Ms);
+        } else {
+            c = moved_reference(M, Mn, PF32_LOG2E);
+#pragma unroll
+            for (int u = 0; u < 8; u++) w[u] = moved_reference(ms[u], Mn, PF32_LOG2E), ls[u] = fabsf(ls[u]);
+        }
         L *= c;
 #pragma unroll
         for (int k = 0; k < 4; k++) A[k] *= c;
 #pragma unroll
         for (int u = 0; u < 8; u++) {
-            const float w = __builtin_amdgcn_exp2f(ms[u] - Ms);
-            L += w * ls[u];
+            L += w[u] * ls[u];
 #pragma unroll
-            for (int k = 0; k < 4; k++) A[k] += w * av[u][k];
+            for (int k = 0; k < 4; k++) A[k] += w[u] * av[u][k];
         }
         M = Mn;
     }

@@ -147,20 +147,18 @@ __device__ __forceinline__ PlainRow plain_row(const AttnParams &p, __attribute__
     for (int d = lane; d < p.D; d += 64) q_lds[d] = to_float(q[d]);
     wave_lds_sync();
     PlainRow r = {-INFINITY, 0.0f, {0.0f, 0.0f}};
+    const float log2_unit = mrow ? PF32_LOG2E : 1.0f;  // as in the kernel
     for (int j0 = lo; j0 < hi; j0 += 64) {
         float s = -INFINITY;
         if (j0 + lane < hi) {
             const T *kr = k + (j0 + lane) * p.ks[2];
             float dot = 0.0f;
             for (int d = 0; d < p.D; d++) dot = __builtin_fmaf(q_lds[d], to_float(kr[d]), dot);
-            s = dot * p.scale;
-            if (mrow) s += to_float(mrow[(j0 + lane) * p.ms1]);
-            s *= PF32_LOG2E;
+            s = mrow ? __builtin_fmaf(dot, p.scale, to_float(mrow[(j0 + lane) * p.ms1])) : dot * (p.scale * PF32_LOG2E);
         }
-        // fmaxf passes NaN by: a score that is NaN leaves the exponent alone and makes the sums NaN; with no other score than
-        // -inf and NaN the exponent stays -inf and -inf - 0 gives 0, NaN gives NaN
-        const float m_new = fmaxf(r.m, wave_max(s)), base = m_new == -INFINITY ? 0.0f : m_new;
-        const float pj = __builtin_amdgcn_exp2f(s - base), corr = __builtin_amdgcn_exp2f(r.m - base);
+        // fmaxf passes NaN by: a score that is NaN leaves the reference alone and makes the sums NaN
+        const float m_new = fmaxf(r.m, wave_max(s));
+        const float pj = probability(s, m_new, log2_unit), corr = moved_reference(r.m, m_new, log2_unit);
         r.m = m_new;
         r.l = r.l * corr + wave_sum(pj);
         const int n = min(64, hi - j0);
@@ -332,9 +330,10 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
 
     // Q operand: the terms of Q[query][16 kb + 8 h2 .. +8].  The rows are read in whole lines and dealt out to the lanes
     // that own them through LDS, half of the dims at a time.
-    // An f32 Q takes the scale (and, unless a mask is added to the scores in between, log2(e)), so that the scores of S^T
-    // are exponents of two; 16-bit rows would need three terms for that, and their scores are multiplied instead.  Either
-    // way the largest score of a row's first tile has probability 1 exactly.
+    // An f32 Q takes the scale and log2(e), so that the scores of S^T are exponents of two; 16-bit rows would need three
+    // terms for that, and their scores are multiplied instead.  Where a mask is added to the scores, log2(e) waits for the
+    // difference from the row's reference (see the probabilities).  Either way the largest score of a row's first tile has
+    // probability 1 exactly.
     constexpr bool SCALED_Q = sizeof(T) == 4;
     bf16x8_t qt[NKB][N];
     const float score_scale = bias_on ? p.scale : p.scale * PF32_LOG2E, q_scale = SCALED_Q ? score_scale : 1.0f;
@@ -388,8 +387,9 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
     for (int db = 0; db < NDB; db++)
 #pragma unroll
         for (int r = 0; r < 16; r++) o[db][r] = 0.0f;
-    // m: the row's reference exponent (base 2); nmr = -m, +inf while the row has seen no key
+    // m: the row's reference (see `probability` in attn_f32.h); nmr = -m in powers of two, +inf while the row has seen no key
     float m = -INFINITY, l = 0.0f, nmr = INFINITY;
+    const float log2_unit = bias_on ? PF32_LOG2E : 1.0f;
     const T *mrow = nullptr;
     if constexpr (BIAS)
         mrow = (const T *)p.mask + (int64_t)(p.mask_kind == FHIP_MASK_QK ? min(query, p.Sq - 1) : b) * p.ms0;
@@ -473,7 +473,7 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
         if constexpr (BIAS) {
             if (bias_on) {
 #pragma unroll
-                for (int r = 0; r < 16; r++) s[r] = (s[r] + bias[r]) * PF32_LOG2E;
+                for (int r = 0; r < 16; r++) s[r] += bias[r];
             }
         }
         float ts = 0.0f, pr[16];
@@ -481,7 +481,7 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
             float sum[2] = {0.0f, 0.0f};
 #pragma unroll
             for (int r = 0; r < 16; r++) {
-                pr[r] = __builtin_amdgcn_exp2f(s[r] + nm);
+                pr[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], log2_unit, nm));
                 sum[r & 1] += pr[r];
             }
             return sum[0] + sum[1];
@@ -494,7 +494,7 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
             for (int r = 1; r < 16; r++) mx = fmaxf(mx, s[r]);
             mx = half_swap_max32(mx);
             const float m_new = fmaxf(m, mx);
-            const float corr = (m == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(m - m_new);
+            const float corr = moved_reference(m, m_new, log2_unit);
             m = m_new;
             l *= corr;
 #pragma unroll
@@ -502,8 +502,21 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
 #pragma unroll
                 for (int r = 0; r < 16; r++) o[db][r] *= corr;
             // still no visible key: the tile's probabilities are exp2(-inf) = 0 and the row stays without a reference
-            nmr = (m == -INFINITY) ? INFINITY : -m;
-            ts = probabilities((m == -INFINITY) ? 0.0f : nmr);
+            nmr = -(m * log2_unit);
+            ts = probabilities(nmr == INFINITY ? 0.0f : nmr);
+            if constexpr (BIAS) {
+                // nothing but lowest values yet (see `probability`): those came out 0 as well, and the row comes here with every
+                // tile until a score is higher
+                if (bias_on) {
+                    const float lowest = nmr == INFINITY && m > -INFINITY ? m : __builtin_nanf("");
+                    ts = 0.0f;
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        pr[r] = s[r] == lowest ? 1.0f : pr[r];
+                        ts += pr[r];
+                    }
+                }
+            }
         }
         l += ts;
 #pragma unroll
@@ -606,14 +619,13 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
             ml[src] = *LDST_PTR(float4_t, ((src - 1) * U + wave) * SLOT + lane * 16 + (NQ - 1) * 1024);
             m_all = fmaxf(m_all, ml[src][0]);
         }
-        const float m_safe = (m_all == -INFINITY) ? 0.0f : m_all;
-        const float w0 = __builtin_amdgcn_exp2f(m - m_safe);
+        const float w0 = moved_reference(m, m_all, log2_unit);
         l *= w0;
 #pragma unroll
         for (int db = 0; db < NDB; db++) o[db] *= w0;
 #pragma unroll
         for (int src = 1; src < KG; src++) {
-            const float w = __builtin_amdgcn_exp2f(ml[src][0] - m_safe);
+            const float w = moved_reference(ml[src][0], m_all, log2_unit);
             const int at = ((src - 1) * U + wave) * SLOT + lane * 16;
             l += ml[src][1] * w;
 #pragma unroll
@@ -645,7 +657,7 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
     if (parked) {
         if (h2 == 0 && query < p.Sq) {
             part[query * part_row + p.D] = m;
-            part[query * part_row + p.D + 1] = l_tot;
+            part[query * part_row + p.D + 1] = bias_on ? -l_tot : l_tot;  // (the sign tells the merge kernel m's unit)
         }
     } else {
         // o / l by one reciprocal and a correction of each quotient; no visible key: 0 x inf = NaN like the reference's 0 / 0
@@ -706,7 +718,7 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
         const PlainRow x = plain_row<T>(p, lds_base + mine, (const T *)p.q + b * p.qs[0] + h * p.qs[1] + q * p.qs[2],
                                         (const T *)p.k + b * p.ks[0] + g * p.ks[1], (const T *)p.v + b * p.vs[0] + g * p.vs[1],
                                         bias_row, __builtin_amdgcn_readlane(rb.klo, row), __builtin_amdgcn_readlane(rb.khi, row), lane);
-        if (parked && lane == 0) part[q * part_row + p.D] = x.m, part[q * part_row + p.D + 1] = x.l;
+        if (parked && lane == 0) part[q * part_row + p.D] = x.m, part[q * part_row + p.D + 1] = bias_on ? -x.l : x.l;
 #pragma unroll
         for (int t = 0; t < 2; t++) {
             const int dim = lane + 64 * t;

@@ -61,3 +61,42 @@ def test_views_of_a_score_mask(device, dtype, D, first, Skv):
                              force_kernel=fa.KERNEL_PREFILL_F32).to_numpy()
     q, k, v, m = (t.to_numpy() for t in (tq, tk, tv, tm))
     close(out, in_64_bits(q, k, v, D ** -0.5, np.asarray(m, np.float64)[:, first:first + Skv]), f"D{D}")
+
+
+@pytest.mark.parametrize("dtype", [fa.F32, fa.BF16])
+@pytest.mark.parametrize("D", [64, 128, 40])
+@pytest.mark.parametrize("kind", ["rows", "keys"])
+@pytest.mark.parametrize("Sq,Skv", [(45, 131), (21, 2111)])  # the second: keys split over workgroups
+def test_lowest_finite_values(device, dtype, D, kind, Sq, Skv):
+    """Padding with the type's lowest finite value, which is no -inf: beside a zero it has no weight, but a row of nothing else
+    takes the mean of its keys (every score vanishes beside it), and of two such values the higher one takes all."""
+    low = np.float32(-3.4028235e38 if dtype == fa.F32 else -3.3895314e38)
+    B = 3 if kind == "keys" else 2
+    q, k, v = tensors(10, B, 4, 2, Sq, Skv, D)
+    m = np.zeros((B if kind == "keys" else Sq, Skv), np.float32)
+    m[0] = low
+    m[1, : Skv // 3] = low
+    m[2, ::3] = low
+    m[2, m[2] == 0] = low * np.float32(0.8125)
+    tq, tk, tv, tm = (fa.Tensor.from_numpy(device, a, dtype) for a in (q, k, v, m))
+    out = tq.flash_attention(tk, tv, D ** -0.5, (tm, fa.MaskKind.QKMask if kind == "rows" else fa.MaskKind.BatchKeyMask),
+                             out_dtype=fa.F32, force_kernel=fa.KERNEL_PREFILL_F32).to_numpy()
+    q, k, v, m = (np.asarray(t.to_numpy(), np.float64) for t in (tq, tk, tv, tm))
+    close(out, in_64_bits(q, k, v, D ** -0.5, m if kind == "rows" else m[:, None, None, :]), f"D{D} {kind}")
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Sq,Skv", [(300, 300), (21, 2111)])
+def test_one_rounding_at_the_size_of_the_mask(device, D, Sq, Skv):
+    """Scores with mask values about -1000 added lie between -1024 and -512, where neighbours are 2^-14 apart.  The sum rounds
+    once there, as the reference's does: an error uniform over 2^-14, deviation 2^-14 / sqrt(12) = 1.76e-5, which is the
+    relative error of each probability and, the keys' errors being independent, of the result.  A second rounding, of
+    the score times log2(e), would bring it to 3.0e-5; 2.2e-5 is allowed."""
+    q, k, v = tensors(14, 2, 4, 2, Sq, Skv, D)
+    m = (-1000 + np.random.default_rng(15).normal(0, 1, (2, Skv))).astype(np.float32)
+    tq, tk, tv, tm = (fa.Tensor.from_numpy(device, a, fa.F32) for a in (q, k, v, m))
+    out = np.asarray(tq.flash_attention(tk, tv, D ** -0.5, (tm, fa.MaskKind.BatchKeyMask),
+                                        force_kernel=fa.KERNEL_PREFILL_F32).to_numpy(), np.float64)
+    ref = in_64_bits(q, k, v, D ** -0.5, np.asarray(m, np.float64)[:, None, None, :])
+    err = np.linalg.norm(out - ref) / np.linalg.norm(ref)
+    assert err <= 2.2e-5, f"relative L2 {err:.2e}"
