@@ -1,5 +1,6 @@
 // Prefill attention in f32 precision on the gfx950 f32 matrix instruction (v_mfma_f32_32x32x2_f32): head dims above 128, and
-// below for K / V views whose rows attn_prefill_f32_terms.hip cannot address (overlapping rows, slices of 2 GiB and more).
+// below for calls that attn_prefill_f32_terms.hip cannot address (prefill_f32_terms_takes): K or V rows that overlap, a K, V
+// or Q slice of 2 GiB and more, or grids beyond its dimensions.
 //
 // A workgroup of 4 wavefronts owns 128 query rows of one (batch, head), a wavefront 32 of them; K/V tiles of 32 rows pass
 // through LDS.
@@ -115,8 +116,8 @@ __global__ __launch_bounds__(64 * PF32_WAVES, 2) void prefill_f32_kernel(AttnPar
         for (int r = 0; r < 16; r++) o[db][r] = 0.0f;
     float m = -INFINITY, l = 0.0f;
     // scores reach the softmax in the base-2 domain: raw dot products times scale * log2(e); with BIAS they are
-    // scaled, biased, and then only multiplied by log2(e)
-    const float scale2 = bias_on ? PF32_LOG2E : p.scale * PF32_LOG2E;
+    // scaled, biased, and multiplied by log2(e) where probabilities are formed (see `probability` in attn_f32.h)
+    const float scale2 = bias_on ? PF32_LOG2E : p.scale * PF32_LOG2E, log2_unit = bias_on ? PF32_LOG2E : 1.0f;
     const T *mrow = nullptr;
     if constexpr (BIAS)
         mrow = (const T *)p.mask + (int64_t)(p.mask_kind == FHIP_MASK_QK ? min(query, p.Sq - 1) : b) * p.ms0;
@@ -172,14 +173,17 @@ __global__ __launch_bounds__(64 * PF32_WAVES, 2) void prefill_f32_kernel(AttnPar
 #pragma unroll
         for (int r = 1; r < 16; r++) mx = fmaxf(mx, s[r]);
         mx = half_swap_max32(mx);
-        const float m_new = fmaxf(m, mx * scale2);
-        const float m_safe = (m_new == -INFINITY) ? 0.0f : m_new;
-        const float corr = __builtin_amdgcn_exp2f(m - m_safe);
+        const float m_new = fmaxf(m, bias_on ? mx : mx * scale2);
+        const float corr = moved_reference(m, m_new, log2_unit);
         m = m_new;
+        const float m2 = m * log2_unit, m_safe = (m2 == -INFINITY) ? 0.0f : m2;
+        // rows that have seen nothing but lowest values: those equal to the reference count
+        const float lowest = bias_on && m2 == -INFINITY && m > -INFINITY ? m : __builtin_nanf("");
         float psum = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; r++) {
-            s[r] = __builtin_amdgcn_exp2f(fmaf(s[r], scale2, -m_safe));
+            const float pr = __builtin_amdgcn_exp2f(fmaf(s[r], scale2, -m_safe));
+            s[r] = BIAS && s[r] == lowest ? 1.0f : pr;
             psum += s[r];
         }
         l = l * corr + psum;
@@ -274,7 +278,7 @@ __global__ __launch_bounds__(64 * PF32_WAVES, 2) void prefill_f32_kernel(AttnPar
                 }
             if (h2 == 0) {
                 ws[p.D] = m;
-                ws[p.D + 1] = l_tot;
+                ws[p.D + 1] = bias_on ? -l_tot : l_tot;  // (the sign tells the merge kernel m's unit)
             }
         }
         return;
