@@ -8,7 +8,7 @@
 // this kernel serves where their own one does not (finite mask values), have two terms (f16) or one (bf16); the
 // probabilities are f32 values and always have three.
 // Infinities: an element of Q, K or V that is +-inf (or beyond 3.39e38, bf16's largest) makes its products NaN.  Rows whose
-// sums are not finite at the end are formed once more without terms (plain_row).
+// sums are not finite at the end are formed once more without terms (unit_in_f32).
 //
 // A unit is 32 query rows of one head; a wavefront owns one.  A workgroup holds U units that share a KV head (the heads of
 // a GQA group first, then further rows) and walks the keys they see in tiles of 32 rows, which are split into terms on the
@@ -101,6 +101,12 @@ __device__ __forceinline__ float4_t buffer_load4(__amdgpu_buffer_rsrc_t rows, in
     }
 }
 
+template <typename T>
+__device__ __forceinline__ float buffer_load1(__amdgpu_buffer_rsrc_t rows, int at, int from) {
+    if constexpr (sizeof(T) == 4) return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rows, at, from, 0));
+    else return to_float(__builtin_bit_cast(T, (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rows, at, from, 0)));
+}
+
 // U: units per workgroup, KG: key groups (wavefronts = U * KG)
 template <typename T, int D, int U>
 struct PtCfg {
@@ -133,47 +139,115 @@ struct TermsLaunch {
     int32_t mask_rows; // an added mask is read four keys at a time through a buffer
 };
 
-// One row by plain f32 sums over its keys [lo, hi): exponent, sum and (in acc) the unnormalised result, whose dims lane and
-// lane + 64 a lane holds.  For rows that met an element without a finite bf16 term, so only its answer matters: lanes split
-// the keys for the scores and the dims for P.V.  q_at: LDS space for head_dim floats; mrow: mask values to add, or NULL.
-struct PlainRow {
-    float m, l, acc[2];
+// K, V and Q of a unit as buffers: bytes from row to row, and where this lane's row of Q begins
+struct RowBuffers {
+    __amdgpu_buffer_rsrc_t k, v, q;
+    int k_bytes, v_bytes, q_at;
 };
-template <typename T>
-__device__ __forceinline__ PlainRow plain_row(const AttnParams &p, __attribute__((address_space(3))) char *q_at, const T *q, const T *k,
-                                              const T *v, const T *mrow, int lo, int hi, int lane) {
-    auto q_lds = (__attribute__((address_space(3))) float *)q_at;
-    wave_lds_sync();
-    for (int d = lane; d < p.D; d += 64) q_lds[d] = to_float(q[d]);
-    wave_lds_sync();
-    PlainRow r = {-INFINITY, 0.0f, {0.0f, 0.0f}};
-    const float log2_unit = mrow ? PF32_LOG2E : 1.0f;  // as in the kernel
-    for (int j0 = lo; j0 < hi; j0 += 64) {
-        float s = -INFINITY;
-        if (j0 + lane < hi) {
-            const T *kr = k + (j0 + lane) * p.ks[2];
-            float dot = 0.0f;
-            for (int d = 0; d < p.D; d++) dot = __builtin_fmaf(q_lds[d], to_float(kr[d]), dot);
-            s = mrow ? __builtin_fmaf(dot, p.scale, to_float(mrow[(j0 + lane) * p.ms1])) : dot * (p.scale * PF32_LOG2E);
-        }
-        // fmaxf passes NaN by: a score that is NaN leaves the reference alone and makes the sums NaN
-        const float m_new = fmaxf(r.m, wave_max(s));
-        const float pj = probability(s, m_new, log2_unit), corr = moved_reference(r.m, m_new, log2_unit);
-        r.m = m_new;
-        r.l = r.l * corr + wave_sum(pj);
-        const int n = min(64, hi - j0);
+
+// A wavefront's unit in f32 arithmetic (v_mfma_f32_32x32x2_f32), for units with rows that met an element without finite bf16
+// terms: references, sums (this half's keys) and unnormalised results as the kernel holds them.  K and V come straight from
+// memory, a wavefront's tile at a time.  Keys that a row does not see must not reach it (0 x inf is NaN): where some row sees a
+// tile in part and V's 32 dims of it are not finite, they are taken key by key.  mine: 4 KiB of LDS of this wavefront's; mrow:
+// this lane's mask values to add, or NULL; rows: those that matter, and once they are all NaN nothing more is formed.
+// Bound: the f32 matrix instruction, and memory latency where few wavefronts are left.  An infinity in V at the first key, so
+// that every unit comes here (us, without it in brackets; one row at a time before): 4096 causal rows of 32/8 heads, D = 128
+// 2250 (740; 86800), 512 rows at D = 64 81 (21.5; 4230), 129 rows on 8003 keys 418 (131; 22000).
+template <typename T, int D>
+__device__ __forceinline__ void unit_in_f32(const AttnParams &p, __attribute__((address_space(3))) char *mine, const RowBuffers &rows_of,
+                                            const T *mrow, const RowBounds &rb, uint32_t rows, int lane, float16_t (&o)[D / 32], float &m,
+                                            float &l) {
+    constexpr int NDB = D / 32, ES = sizeof(T);
+    const int ln = lane & 31, h2 = lane >> 5;
+    auto uniform = [](int x) __attribute__((always_inline)) { return __builtin_amdgcn_readfirstlane(x); };
+    const int lo_w = uniform(rb.lo_w), hi_w = uniform(rb.hi_w), full_lo_w = uniform(rb.full_lo_w), full_hi_w = uniform(rb.full_hi_w);
+    const float log2_unit = mrow ? PF32_LOG2E : 1.0f, score_scale = mrow ? p.scale : p.scale * PF32_LOG2E;
+    auto p_lds = (__attribute__((address_space(3))) float *)mine;  // [key][query] of a tile seen in part
+    m = -INFINITY, l = 0.0f;
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
-            const int d = lane + 64 * t;
-            float a = r.acc[t] * corr;
-            for (int jj = 0; jj < n; jj++) {
-                const float w = read_lane(pj, jj);
-                if (d < p.D) a = __builtin_fmaf(w, to_float(v[(j0 + jj) * p.vs[2] + d]), a);
+    for (int db = 0; db < NDB; db++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) o[db][r] = 0.0f;
+#pragma unroll 1
+    for (int tile = lo_w / PT_BN; tile * PT_BN < hi_w; tile++) {
+        int j0 = tile * PT_BN;
+        asm volatile("" : "+s"(j0));  // (no address of the body is carried from tile to tile: they would not fit the registers)
+        float16_t s;
+#pragma unroll
+        for (int r = 0; r < 16; r++) s[r] = 0.0f;
+#pragma unroll 1
+        for (int d0 = 0; d0 < D; d0 += 32) {
+            float4_t kr[4], qr[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int dim = d0 + 8 * i + 4 * h2, none = dim < p.D ? 0 : (int)0x80000000;
+                kr[i] = buffer_load4<T>(rows_of.k, (ln * rows_of.k_bytes + dim * ES) | none, j0 * rows_of.k_bytes);
+                qr[i] = buffer_load4<T>(rows_of.q, (rows_of.q_at + dim * ES) | none, 0);
             }
-            r.acc[t] = a;
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[i][e], qr[i][e], s, 0, 0, 0);
         }
+        float mx = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int key = j0 + 8 * (r >> 2) + 4 * h2 + (r & 3);
+            const bool seen = key >= rb.klo && key < rb.khi;
+            const float x = mrow ? __builtin_fmaf(s[r], score_scale, seen ? to_float(mrow[key * p.ms1]) : 0.0f) : s[r] * score_scale;
+            s[r] = seen ? x : -INFINITY;
+            mx = fmaxf(mx, s[r]);  // (passes NaN by: such a score leaves the reference alone and makes the sums NaN)
+        }
+        const float m_new = fmaxf(m, half_swap_max32(mx)), corr = moved_reference(m, m_new, log2_unit);
+        m = m_new;
+        l *= corr;
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            s[r] = probability(s[r], m, log2_unit);
+            l += s[r];
+        }
+#pragma unroll
+        for (int db = 0; db < NDB; db++) o[db] *= corr;
+        // (dims behind head_dim hold whatever follows, and are not written)
+        const bool full = j0 >= full_lo_w && j0 + PT_BN <= full_hi_w;
+        if (!full) {
+            wave_lds_sync();
+#pragma unroll
+            for (int r = 0; r < 16; r++) p_lds[(8 * (r >> 2) + 4 * h2 + (r & 3)) * 32 + ln] = s[r];
+            wave_lds_sync();
+        }
+#pragma unroll
+        for (int db = 0; db < NDB; db++) {
+            float a[16], zero = 0.0f;
+            const int at = 4 * h2 * rows_of.v_bytes + (32 * db + ln) * ES;
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                a[r] = buffer_load1<T>(rows_of.v, at, (j0 + 8 * (r >> 2) + (r & 3)) * rows_of.v_bytes);
+                zero = __builtin_fmaf(a[r], 0.0f, zero);
+            }
+            if (full || __builtin_amdgcn_ballot_w64(!(zero == 0.0f)) == 0) {
+#pragma unroll
+                for (int r = 0; r < 16; r++) o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[r], s[r], o[db], 0, 0, 0);
+            } else {
+                const int end = min(j0 + PT_BN, hi_w);
+#pragma unroll 1
+                for (int key = max(j0, lo_w); key < end; key++) {
+                    const float w = p_lds[(key - j0) * 32 + ln];
+                    const bool seen = key >= rb.klo && key < rb.khi;
+#pragma unroll
+                    for (int rq = 0; rq < 4; rq++) {
+                        const float4_t x = buffer_load4<T>(rows_of.v, (32 * db + 8 * rq + 4 * h2) * ES, key * rows_of.v_bytes);
+#pragma unroll
+                        for (int e = 0; e < 4; e++)
+                            o[db][4 * rq + e] = seen ? __builtin_fmaf(w, x[e], o[db][4 * rq + e]) : o[db][4 * rq + e];
+                    }
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);  // (16 loads at a time)
+        }
+        const uint64_t nan = __builtin_amdgcn_ballot_w64(l != l);
+        if ((((uint32_t)nan | (uint32_t)(nan >> 32)) & rows) == rows) return;
     }
-    return r;
 }
 
 template <typename T, int D, int U, int KG, int MODE>
@@ -337,9 +411,8 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
     constexpr bool SCALED_Q = sizeof(T) == 4;
     bf16x8_t qt[NKB][N];
     const float score_scale = bias_on ? p.scale : p.scale * PF32_LOG2E, q_scale = SCALED_Q ? score_scale : 1.0f;
+    const auto q_rows = __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)p.q + b * p.qs[0] + h * p.qs[1]), 0, 0x7fffffff, 0x00020000);
     {
-        const auto q_rows = __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)p.q + b * p.qs[0] + h * p.qs[1]), 0, 0x7fffffff,
-                                                              0x00020000);
         constexpr int CPH = D / 8, NQ = CPH / 2;  // 16-byte pieces per half row; loads per half
         float4_t x[2][NQ], v0[C::NCH];
 #pragma unroll
@@ -650,7 +723,7 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
 #pragma unroll
         for (int r = 0; r < 16; r++) zero[r & 3] = __builtin_fmaf(o[db][r], 0.0f, zero[r & 3]);
     const uint64_t odd = __builtin_amdgcn_ballot_w64(!(zero[0] + zero[1] + (zero[2] + zero[3]) == 0.0f));
-    uint32_t odd_rows = (uint32_t)odd | (uint32_t)(odd >> 32);
+    const uint32_t odd_rows = wave_has_rows ? (uint32_t)odd | (uint32_t)(odd >> 32) : 0;
     const bool parked = nks > 1;
     float *const part = p.partials + (((int64_t)b * p.H + h) * p.Sq * nks + ksplit) * p.pf_pitch;
     const int64_t part_row = (int64_t)nks * p.pf_pitch;
@@ -711,22 +784,22 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
     }
     if (odd_rows == 0) return;
     __threadfence();  // the stores above come first
-    for (; odd_rows; odd_rows &= odd_rows - 1) {
-        const int row = __builtin_ctz(odd_rows), q = qw0 + row;
-        if (q >= p.Sq) return;
-        const T *bias_row = bias_on ? (const T *)p.mask + (int64_t)(p.mask_kind == FHIP_MASK_QK ? q : b) * p.ms0 : nullptr;
-        const PlainRow x = plain_row<T>(p, lds_base + mine, (const T *)p.q + b * p.qs[0] + h * p.qs[1] + q * p.qs[2],
-                                        (const T *)p.k + b * p.ks[0] + g * p.ks[1], (const T *)p.v + b * p.vs[0] + g * p.vs[1],
-                                        bias_row, __builtin_amdgcn_readlane(rb.klo, row), __builtin_amdgcn_readlane(rb.khi, row), lane);
-        if (parked && lane == 0) part[q * part_row + p.D] = x.m, part[q * part_row + p.D + 1] = bias_on ? -x.l : x.l;
+    rb.lo_w = lo_w, rb.hi_w = hi_w, rb.full_lo_w = full_lo_w, rb.full_hi_w = full_hi_w;  // (the scalar copies)
+    const RowBuffers buffers = {k_rows, v_rows, q_rows, k_row, v_row, min(query, p.Sq - 1) * ((int)p.qs[2] * ES)};
+    wave_lds_sync();
+    unit_in_f32<T, D>(p, lds_base + mine, buffers, bias_on ? mrow : nullptr, rb, odd_rows, lane, o, m, l);
+    const float l_odd = half_swap_sum32(l);
+    if (query >= p.Sq || !(odd_rows >> ln & 1)) return;
+    if (parked && h2 == 0) part[query * part_row + p.D] = m, part[query * part_row + p.D + 1] = bias_on ? -l_odd : l_odd;
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
-            const int dim = lane + 64 * t;
+    for (int db = 0; db < NDB; db++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int dim = 32 * db + 8 * (r >> 2) + 4 * h2 + (r & 3);
             if (dim >= p.D) continue;
-            if (parked) part[q * part_row + dim] = x.acc[t];
-            else store_out<T>(p, ob + (int64_t)q * p.os[2] + dim * p.os[3], x.acc[t] / x.l);
+            if (parked) part[query * part_row + dim] = o[db][r];
+            else store_out<T>(p, ob + (int64_t)query * p.os[2] + dim * p.os[3], o[db][r] / l_odd);
         }
-    }
 }
 
 // workgroups of the form with U units each

@@ -6,6 +6,8 @@ Tolerance: a dot product of 128 f32 terms in a chain has a relative error of 128
 2e-7 in the mean, the result's sum over keys the same; 2e-6 relative L2 over all rows.
 Reference semantics: fusor-ml/fusor/src/composite/flash_attention.rs:141-199.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -84,3 +86,28 @@ def test_with_added_masks(device, dtype, D, kind):
     q, k, v, m = (t.to_numpy() for t in (tq, tk, tv, tm))
     m = np.asarray(m, np.float64)
     check(out, expect(q, k, v, D ** -0.5, np.broadcast_to(m[None] if kind == "rows" else m[:, None, :], (B, Sq, Skv))))
+
+
+@pytest.mark.parametrize("Sq,Skv,D,what", [(2048, 2048, 128, "V"), (512, 512, 64, "V"), (129, 8003, 128, "V"), (2048, 2048, 128, "K")])
+def test_one_infinite_element_does_not_multiply_the_time(device, Sq, Skv, D, what):
+    """An infinity in the first key's row reaches every row of its group; all of them in f32 arithmetic take some 3 times (V) to 4
+    times (512 rows) the time of a call without it.  One row at a time they took more than 100 times as long; 10 is allowed."""
+    q, k, v = tensors(14, 1, 32, 8, Sq, Skv, D)
+    q[..., 0] = np.abs(q[..., 0]) + 0.1
+
+    def best_of_three():
+        tq, tk, tv = (fa.Tensor.from_numpy(device, a, fa.F32) for a in (q, k, v))
+        times = []
+        for _ in range(4):
+            device.synchronize()
+            start = time.perf_counter()
+            for _ in range(5):
+                tq.flash_attention(tk, tv, D ** -0.5, analytic=(True, Skv - Sq, 0), force_kernel=fa.KERNEL_PREFILL_F32)
+            device.synchronize()
+            times.append(time.perf_counter() - start)
+        return min(times[1:])
+
+    usual = best_of_three()
+    (v if what == "V" else k)[:, :, 0, 0] = np.inf if what == "V" else -np.inf
+    odd = best_of_three()
+    assert odd <= 10 * usual, f"{odd / usual:.1f} times as long"
