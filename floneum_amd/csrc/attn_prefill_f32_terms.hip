@@ -7,8 +7,12 @@
 // the f32 accumulation; the other six are formed: 6 / 16 of the f32 instruction's matrix time.  16-bit tensors, which
 // this kernel serves where their own one does not (finite mask values), have two terms (f16) or one (bf16); the
 // probabilities are f32 values and always have three.
-// Infinities: an element of Q, K or V that is +-inf (or beyond 3.39e38, bf16's largest) makes its products NaN.  Rows whose
-// sums are not finite at the end are formed once more without terms (unit_in_f32).
+// Infinities: an element of Q, K or V that is +-inf (or beyond 3.39e38, bf16's largest) makes its products NaN.
+// Small elements: below 2^-110 the last bits of a value fall below bf16's smallest number, 2^-133, and its terms are off by up to
+// 2^-134.  That is nothing beside a result of 2^-110 and more, and nothing in a score unless the other factor is beyond 2^100.
+// Rows whose sums are not finite or smaller than that at the end, and rows with elements of (scaled) Q beyond either limit,
+// are formed once more without terms (unit_in_f32).  What is left: a probability below 2^-110 counts to 2^-134 only, which
+// shows where V's elements are 2^110 times the result, and results of elements below 2^-134 are zero.
 //
 // A unit is 32 query rows of one head; a wavefront owns one.  A workgroup holds U units that share a KV head (the heads of
 // a GQA group first, then further rows) and walks the keys they see in tiles of 32 rows, which are split into terms on the
@@ -89,6 +93,10 @@ __device__ __forceinline__ void split4(float4_t x, uint32_t (&lo)[N], uint32_t (
         }
     }
 }
+
+constexpr float SMALLEST_IN_TERMS = 0x1p-110f, LARGEST_Q = 0x1p100f;
+// orders values by their magnitude, with zero above all
+__device__ __forceinline__ uint32_t magnitude(float x) { return (__float_as_uint(x) << 1) - 1; }
 
 // four elements at a byte offset of a buffer, as f32
 template <typename T>
@@ -226,8 +234,13 @@ __device__ __forceinline__ void unit_in_f32(const AttnParams &p, __attribute__((
                 zero = __builtin_fmaf(a[r], 0.0f, zero);
             }
             if (full || __builtin_amdgcn_ballot_w64(!(zero == 0.0f)) == 0) {
+                // this tile's share on its own, then one addition at the size of the sum
+                float16_t sum;
 #pragma unroll
-                for (int r = 0; r < 16; r++) o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[r], s[r], o[db], 0, 0, 0);
+                for (int r = 0; r < 16; r++) sum[r] = 0.0f;
+#pragma unroll
+                for (int r = 0; r < 16; r++) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(a[r], s[r], sum, 0, 0, 0);
+                o[db] += sum;
             } else {
                 const int end = min(j0 + PT_BN, hi_w);
 #pragma unroll 1
@@ -410,6 +423,7 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
     // probability 1 exactly.
     constexpr bool SCALED_Q = sizeof(T) == 4;
     bf16x8_t qt[NKB][N];
+    uint32_t odd_rows = 0;  // rows that unit_in_f32 is to form
     const float score_scale = bias_on ? p.scale : p.scale * PF32_LOG2E, q_scale = SCALED_Q ? score_scale : 1.0f;
     const auto q_rows = __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)p.q + b * p.qs[0] + h * p.qs[1]), 0, 0x7fffffff, 0x00020000);
     {
@@ -426,6 +440,8 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
         // the first V tile is requested with K and Q, so that a short call waits for memory once
         if (ntiles > 0) load_rows(v0, v_rows, v_row, j_begin + grp * PT_BN);
         const int mine = wave * C::ROWS_BYTES;
+        uint32_t least = 0xffffffffu;
+        float most = 0.0f;
 #pragma unroll
         for (int hf = 0; hf < 2; hf++) {
             if (hf) wave_lds_sync();
@@ -441,12 +457,20 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
 #pragma unroll
                 for (int e = 0; e < 2; e++) {
                     const float4_t y = *LDST_PTR(float4_t, mine + ln * C::HALF_PITCH + (16 * kk + 8 * h2 + 4 * e) * 4) * q_scale;
+                    if constexpr (SCALED_Q) {
+#pragma unroll
+                        for (int i = 0; i < 4; i++) least = min(least, magnitude(y[i])), most = fmaxf(most, fabsf(y[i]));
+                    }
                     split4<N>(y, w[2 * e], w[2 * e + 1]);
                 }
 #pragma unroll
                 for (int i = 0; i < N; i++)
                     qt[hf * (NKB / 2) + kk][i] = __builtin_bit_cast(bf16x8_t, uint4_t{w[0][i], w[1][i], w[2][i], w[3][i]});
             }
+        }
+        if constexpr (SCALED_Q) {
+            const uint64_t odd = __builtin_amdgcn_ballot_w64(least < magnitude(SMALLEST_IN_TERMS) || most > LARGEST_Q);
+            odd_rows = (uint32_t)odd | (uint32_t)(odd >> 32);
         }
         lds_barrier();  // the tiles take the space over
         if (ntiles > 0) {
@@ -716,14 +740,19 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
     // ---- out[query][dim] = O^T[dim][query] / l; with the keys split over workgroups this share's state is parked and
     // the merge kernel normalises
     const float l_tot = half_swap_sum32(l);
-    // rows with a sum that is not finite: 0 x inf and 0 x NaN are NaN
+    // rows with a sum that is not finite (0 x inf and 0 x NaN are NaN), or with one so small that V's terms may lack bits of it
     float zero[4] = {l * 0.0f, 0.0f, 0.0f, 0.0f};
+    uint32_t least = 0xffffffffu;
 #pragma unroll
     for (int db = 0; db < NDB; db++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) zero[r & 3] = __builtin_fmaf(o[db][r], 0.0f, zero[r & 3]);
-    const uint64_t odd = __builtin_amdgcn_ballot_w64(!(zero[0] + zero[1] + (zero[2] + zero[3]) == 0.0f));
-    const uint32_t odd_rows = wave_has_rows ? (uint32_t)odd | (uint32_t)(odd >> 32) : 0;
+        for (int r = 0; r < 16; r++) {
+            zero[r & 3] = __builtin_fmaf(o[db][r], 0.0f, zero[r & 3]);
+            if constexpr (N == 3) least = min(least, magnitude(o[db][r]));
+        }
+    const uint64_t odd = __builtin_amdgcn_ballot_w64(!(zero[0] + zero[1] + (zero[2] + zero[3]) == 0.0f) ||
+                                                     least < magnitude(l_tot * SMALLEST_IN_TERMS));
+    odd_rows = wave_has_rows ? odd_rows | (uint32_t)odd | (uint32_t)(odd >> 32) : 0;
     const bool parked = nks > 1;
     float *const part = p.partials + (((int64_t)b * p.H + h) * p.Sq * nks + ksplit) * p.pf_pitch;
     const int64_t part_row = (int64_t)nks * p.pf_pitch;

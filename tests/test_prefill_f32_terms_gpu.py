@@ -74,6 +74,25 @@ def test_magnitudes(device, stds):
     close(tq.flash_attention(tk, tv, 128 ** -0.5).to_numpy(), in_64_bits(q, k, v, 128 ** -0.5), f"{stds}")
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("form", ["two_units_four_key_groups", "two_units_two_key_groups", "few_rows_keys_split"])
+@pytest.mark.parametrize("of", ["V", "Q", "K", "a dim of V"])
+def test_elements_whose_last_term_bf16_cannot_hold(device, of, form, D):
+    """Magnitudes down to f32's smallest normal one: results as small as V, and products of small elements with large ones.  (A
+    result of 2^-120 is rounded at 2^-144.)"""
+    B, H, Hkv, Sq, Skv, causal = FORMS[form]
+    small, large = 2.0 ** -120, 2.0 ** 120
+    q, k, v = tensors(16, B, H, Hkv, Sq, Skv, D, {"V": (1, 1, small), "Q": (small, large, 1), "K": (large, small, 1)}.get(of, (1, 1, 1)))
+    if of == "a dim of V":
+        v[..., 5] *= np.float32(small)
+    tq, tk, tv = (fa.Tensor.from_numpy(device, a, fa.F32) for a in (q, k, v))
+    out = tq.flash_attention(tk, tv, D ** -0.5, analytic=(True, Skv - Sq, 0) if causal else None,
+                             force_kernel=fa.KERNEL_PREFILL_F32).to_numpy()
+    ref = in_64_bits(q, k, v, D ** -0.5, causal_mask(Sq, Skv, Skv - Sq) if causal else None)
+    close(out, ref, of)
+    close(out[..., 5], ref[..., 5], of)
+
+
 @pytest.mark.parametrize("dtype", [fa.F32, fa.F16, fa.BF16])
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("rows", ["some", "many"])
