@@ -327,16 +327,19 @@ __global__ __launch_bounds__(256) void prefill_f32_merge_kernel(AttnParams p) {
         float Mn = M;
 #pragma unroll
         for (int u = 0; u < 8; u++) Mn = fmaxf(Mn, ms[u]);
+        // as moved_reference (attn_f32.h) does it; nothing here waits for a single load of the round
+        const float unit = __float_as_int(ls[0]) < 0 ? PF32_LOG2E : 1.0f, M2 = Mn * unit, Ms = M2 == -INFINITY ? 0.0f : M2;
         float c, w[8];
-        if (__builtin_amdgcn_readfirstlane(__float_as_int(ls[0])) >= 0) {
-            const float Ms = (Mn == -INFINITY) ? 0.0f : Mn;
-            c = __builtin_amdgcn_exp2f(M - Ms);
+        {
+#pragma clang fp contract(off)
+            c = __builtin_amdgcn_exp2f(M * unit - Ms);
 #pragma unroll
-            for (int u = 0; u < 8; u++) w[u] = __builtin_amdgcn_exp2f(ms[u] - Ms);
-        } else {
-            c = moved_reference(M, Mn, PF32_LOG2E);
+            for (int u = 0; u < 8; u++) w[u] = __builtin_amdgcn_exp2f(ms[u] * unit - Ms);
+        }
+        if (M2 == -INFINITY && Mn > -INFINITY) {
+            c = M == Mn ? 1.0f : 0.0f;
 #pragma unroll
-            for (int u = 0; u < 8; u++) w[u] = moved_reference(ms[u], Mn, PF32_LOG2E), ls[u] = fabsf(ls[u]);
+            for (int u = 0; u < 8; u++) w[u] = ms[u] == Mn ? 1.0f : 0.0f;
         }
         L *= c;
 #pragma unroll
@@ -349,6 +352,7 @@ __global__ __launch_bounds__(256) void prefill_f32_merge_kernel(AttnParams p) {
         }
         M = Mn;
     }
+    L = fabsf(L);
     const int64_t ob = b * p.os[0] + h * p.os[1] + (int64_t)query * p.os[2];
 #pragma unroll
     for (int k = 0; k < 4; k++)
