@@ -663,9 +663,24 @@ void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_s
             const long want = compute_units / wgs;
             return want < most ? want : most;
         };
+        // Workgroups of two units, or above head_dim 64 of four, whose shares are twice as many: for few rows, and from 768 keys
+        // on (causal, D = 128: 832 rows of 16/4 heads 50 us in two shares, 55 unsplit; 704 rows 45 and 48; 768 rows of 8/2 heads 33
+        // in three, 38 in two shares for two units each).  Shorter prompts if they come to three shares of 160 keys, or of 128
+        // where there is room for four: 640 rows of 16/4 heads 44.7 -> 39.1, 512 rows 33.7 -> 32.3, 384 rows of 8/2 heads 29.1 ->
+        // 22.0; but two batches of 12 heads at D = 96 take 27.8 in three shares of 128 keys against 25.0 unsplit (384 rows), and
+        // 41 in two shares against 37 (640 rows).
         long ns = shares(D > 64 && (few_rows || Skv >= 768) ? 4 : 2);
-        // Partials beyond 16 MiB: half the shares for workgroups of half the units, so that a call's workspace stays within
-        // about what its caller may have set aside for it (32/8 heads, 128 rows on 8192 keys: 4 shares 125 us, 8 shares 97).
+        if (D > 64 && !few_rows && Skv < 768) {
+            const long most_before = most, wgs = kv_heads * ((units + 3) / 4);
+            most = Skv / (4 * wgs <= compute_units ? 128 : 160);
+            const long of_four = shares(4);
+            if (of_four >= 3) ns = of_four;
+            most = most_before;
+        }
+        // A call asks for at most 16 MiB of partials.  Only full grids of four-unit workgroups (256 x 128 rows) are beyond that:
+        // 32, 64, 128, 256 or 512 rows of 32/8 heads at D = 128, and up to seven rows fewer.  They take half the shares on workgroups
+        // of half the units, the workspace that such calls have always had, and more time for it: on 8192 keys 32 rows 49 us (40 in
+        // twice the shares), 64 rows 79 (56), 128 rows 128 (96), 256 rows 244 (172), 512 rows 463 (327).
         constexpr size_t MOST_PARTIALS = (size_t)16 << 20;
         if (few_rows && D > 64 && prefill_f32_workspace_bytes(B, H, Sq, D, (int)ns) > MOST_PARTIALS) ns = shares(2);
         if (ns < 2) return;

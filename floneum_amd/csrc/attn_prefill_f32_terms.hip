@@ -884,9 +884,12 @@ static int launch_terms(const AttnParams &p, hipStream_t stream) {
     //   (4, 2)  eight wavefronts, one workgroup per CU: D = 128 1500 rows 115 against 142 for (4, 1), 4000 rows of 8 heads
     //           262 against 348, 129 rows on 8003 keys (keys split over workgroups) 111 against 133
     //   (2, 2)  D > 64: one wavefront per SIMD with 512 registers, half the units per workgroup, for short prompts (700 rows
-    //           48 against 55 for (4, 2), 200 rows 21 against 24).  D <= 64: two workgroups per CU; square causal prompts, whose
-    //           later rows see more keys, are spread more evenly by half the units (1024 rows 38 against 47 for (4, 2), 2048
-    //           rows 114 against 119 for (4, 1); 4096 rows 391 against 357)
+    //           48 against 55 for (4, 2), 200 rows 21 against 24) and others that fit the CUs once.  With the keys split there is no
+    //           short workgroup beside a long one unless the prompt is causal (768 rows of 8/2 heads, 288 workgroups: 33 against 36
+    //           with causality, 51 against 39 without; 16/4 heads, 384 workgroups: 58 against 47).  D <= 64: two workgroups per CU;
+    //           square causal prompts, whose later rows see more keys, are spread more evenly by half the units (1024 rows 38
+    //           against 47 for (4, 2), 2048 rows 111 and 2560 rows 159 against 118 and 165 for (4, 1); 3072 rows 224 against 216,
+    //           4096 rows 388 against 336)
     //   (2, 4)  D <= 64, eight wavefronts: 512 rows 18 against 21.5 for (2, 2), 1000 rows of 16 heads without a mask 31
     //           against 38
     // 16-bit storage takes (4, 1) always.
@@ -899,7 +902,8 @@ static int launch_terms(const AttnParams &p, hipStream_t stream) {
             if (uneven && 2 * w4 <= 5L * cus) return launch_form<T, 2, 2, MODE>(p, stream);
             if (!uneven && w4 <= cus) return launch_form<T, 4, 2, MODE>(p, stream);
         } else {
-            if (2 * w2 <= (few_rows ? 2L : 3L) * cus) return launch_form<T, 2, 2, MODE>(p, stream);
+            const bool fits = w2 <= cus || (p.pf_nsplit > 1 ? uneven && 4 * w2 <= 5L * cus : !few_rows && 2 * w2 <= 3L * cus);
+            if (fits) return launch_form<T, 2, 2, MODE>(p, stream);
             if (w4 < 2L * cus) return launch_form<T, 4, 2, MODE>(p, stream);
         }
     }

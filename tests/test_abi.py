@@ -279,6 +279,21 @@ def test_prefill_key_split_planning_on_256_cus():
     assert shares(64, 8192, fa.F16, 260, D=256, H=16, Hkv=4) == 8    # 64-row workgroups, two per CU
 
 
+@pytest.mark.parametrize("H,Hkv,S,D,shares", [
+    (16, 4, 384, 128, 3), (16, 4, 511, 128, 3), (16, 4, 512, 128, 4), (16, 4, 576, 128, 3), (16, 4, 640, 128, 3), (16, 4, 704, 128, 0),
+    (16, 4, 767, 128, 0), (16, 4, 768, 128, 2), (8, 2, 383, 128, 0), (8, 2, 384, 128, 3), (24, 24, 384, 96, 0), (24, 24, 640, 96, 0),
+    (32, 8, 512, 128, 0), (32, 8, 640, 128, 0), (16, 4, 512, 64, 2)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_key_shares_of_short_f32_prompts(H, Hkv, S, D, shares, causal):
+    """Three shares and more of four-unit workgroups below 768 keys, the former rule elsewhere; masked or not alike."""
+    need = ctypes.c_size_t()
+    a = make_args(B=1, H=H, Hkv=Hkv, Sq=S, Skv=S, D=D, dtype=fa.F32)
+    if causal:
+        a.analytic.enabled, a.analytic.causal = 1, 1
+    assert fa.lib().fhip_flash_attention_workspace_bytes(ctypes.byref(a), 256, ctypes.byref(need)) == fa.OK
+    assert need.value == H * S * (D + 2) * 4 * shares
+
+
 # ---- masks: bit-exact against the checker and the reference's vectors -----------------------------------
 
 NEG_BITS = {fa.F32: 0xFF800000, fa.F16: 0xFC00, fa.BF16: 0xFF80}

@@ -50,6 +50,8 @@ FORMS = {
     "four_units_two_key_groups": (2, 16, 16, 515, 545, False),
     "four_units": (34, 16, 16, 40, 65, False),
     "few_rows_keys_split": (1, 8, 2, 21, 2111, True),
+    "short_prompt_keys_split": (1, 16, 4, 545, 545, True),      # above 64: four units, two key groups, three shares
+    "shorter_prompt_keys_split": (1, 8, 2, 385, 385, True),     # above 64: two units, two key groups, three shares
     "one_tile": (1, 4, 4, 32, 32, True),
     "one_key": (3, 4, 1, 40, 1, False),
 }
