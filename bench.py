@@ -770,7 +770,7 @@ def record_traffic(name, fetch_csv, write_csv):
         main = {k: v for k, v in counts.items() if any(t in k for t in ("decode_mfma", "decode_vec", "prefill_mfma_kernel",
                                                                        "prefill_mfma_wide_kernel", "prefill_mfma_wide_rows32_kernel",
                                                                        "prefill_mfma_rows64_kernel",
-                                                                       "prefill_f32_kernel",
+                                                                       "prefill_f32_kernel", "prefill_f32_terms_kernel",
                                                                        "prefill_f32_wide", "attn_generic"))}
         assert len(main) == 1, f"{path}: expected one main kernel, found {sorted(main)}"
         kname, (count, _) = next(iter(main.items()))
@@ -783,7 +783,9 @@ def record_traffic(name, fetch_csv, write_csv):
     # the file the kernel lives in (the wide-head 16-bit prefill kernels have files of their own)
     out["source"] = "attn_prefill_mfma_rows32.hip" if "prefill_mfma_wide_rows32" in out["kernel_symbol"] else \
         "attn_prefill_mfma_rows64.hip" if "prefill_mfma_rows64" in out["kernel_symbol"] else \
-        "attn_prefill_mfma_wide.hip" if "prefill_mfma_wide" in out["kernel_symbol"] else KERNEL_SOURCES[kernel]
+        "attn_prefill_mfma_wide.hip" if "prefill_mfma_wide" in out["kernel_symbol"] else \
+        "attn_prefill_f32.hip" if "prefill_f32" in out["kernel_symbol"] and "terms" not in out["kernel_symbol"] else \
+        KERNEL_SOURCES[kernel]
     out["source_sha256"] = source_hash(kernel, out["source"])
     try:
         rec = json.load(open(TRAFFIC_RECORD))

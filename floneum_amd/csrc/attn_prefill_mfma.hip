@@ -716,12 +716,13 @@ static bool use_key_split_form(const AttnParams &p) {
     return p.Sq <= PF_BM / 2 || 2 * wgs <= cus || (wgs <= cus && nqb >= 8);
 }
 
-// Head dims 64, 96 and 128 are this kernel's own.  The other multiples of 8 above 64 run on it padded, quicker than on
-// the wide-head kernel, whose wavefronts read every LDS operand for half as many matrix instructions (f16, 16 heads, 4096 x 4096 keys without a mask: head_dim
-// 72 149 -> 118 us, 80 150 -> 118, 88 162 -> 120, 104 198 -> 132, 112 199 -> 133, 120 201 -> 139; causal, 80: 163 -> 68;
-// 512-token causal prompt, 32/8 heads, 80: 16.0 -> 15.4).  Below 64 the padding costs what the kernel gains unless the grid
-// fills the chip (head_dim 40: 4096 keys 131 -> 98 us, 512-token prompt 13.9 -> 14.2; head_dim 32: 112 -> 96 and 12.4 ->
-// 14.0), and to 32, where it is half of the work or more, also in short row blocks (300 rows of four sequences 60 -> 64).
+// Head dims 64, 96 and 128 are this kernel's own.  The other multiples of 8 above 64 run on it padded, quicker than on the
+// wide-head kernel, whose wavefronts read every LDS operand for half as many matrix instructions (both in turn on one box, us a
+// call; f16, 16 heads, 4096 x 4096 keys without a mask: head_dim 72 147 -> 120, 80 150 -> 124, 88 163 -> 130, 104 196 -> 136, 112
+// 202 -> 144, 120 201 -> 147; causal, 80: 157 -> 75 (two of that kernel's 128-row blocks per CU wait for the longest); 512-token
+// causal prompt, 32/8 heads, 80: 17.0 -> 15.9).  Below 64 the padding costs what the kernel gains unless the grid fills the
+// chip (head_dim 40: 4096 keys 134 -> 104; head_dim 32: 116 -> 102), and to 32, where it is half of the work or more, also in
+// short row blocks (300 rows of four sequences 60 -> 64).
 bool prefill_mfma_rows256_takes(int D, float scale, int B, int H, int Sq, int compute_units) {
     if (!(D % 8 == 0 && D >= 8 && D <= 128 && scale > 0.0f && scale * PF_LOG2E < 2.0f)) return false;
     if (D >= 64) return true;
