@@ -20,7 +20,7 @@
 // of four LDS stages each, loaded straight into LDS (no staging registers) two iterations ahead of their first
 // reader; one workgroup barrier per iteration publishes what has landed.
 //
-// Softmax as in the 256-row kernel, with the power-of-two part of scale * log2(e) in Q; the rest (rr in [1, 2))
+// Softmax as in the 256-row kernel: scale * log2(e) (rr; in bf16 its power of two is in Q and rr is the rest, in [1, 2))
 // multiplies the scores in f32; a probability is exp2(fma(s, rr, -m * rr)) against the reference m the row already
 // has, and m moves only when a lane's probabilities of a tile sum to more than 2^15.
 // Masking is by interval (attn_bounds.h): analytic descriptors, key counts, the interval form of a mask tensor.
@@ -67,11 +67,6 @@ struct R32Mma<half_t> {
     static __device__ __forceinline__ uint32_t pack2(float x, float y) {
         half2_t h = {(half_t)x, (half_t)y};
         return __builtin_bit_cast(uint32_t, h);
-    }
-    static __device__ __forceinline__ vec8 scaled(vec8 q, float c) {
-#pragma unroll
-        for (int e = 0; e < 8; e++) q[e] = (half_t)((float)q[e] * c);
-        return q;
     }
 };
 template <>
@@ -149,9 +144,11 @@ __global__ __launch_bounds__(256, 1) void prefill_mfma_wide_rows32_kernel(AttnPa
     const int qrow = min(query, p.Sq - 1);
 
     const float scale2 = p.scale * R32_LOG2E;
-    // scale2 = pw * rr with pw a power of two and rr in [1, 2): Q takes pw (exact), rr multiplies every score in f32
-    const float pw = __uint_as_float(__float_as_uint(scale2) & 0x7F800000u);
-    const float rr = scale2 / pw;
+    // bf16: scale2 = pw * rr with pw a power of two and rr in [1, 2), Q takes pw (exact) and rr multiplies every score in f32.
+    // f16: rr is all of it (elements below 2^-14 / pw would become subnormal and lose bits).
+    constexpr bool FOLD = std::is_same<T, bf16_t>::value;
+    const float pw = FOLD ? __uint_as_float(__float_as_uint(scale2) & 0x7F800000u) : 1.0f;
+    const float rr = FOLD ? scale2 / pw : scale2;
 
     const int j_begin = (lo_wg / R32_KEYS) * R32_KEYS;
     const int ntiles = hi_wg > j_begin ? (hi_wg - j_begin + R32_KEYS - 1) / R32_KEYS : 0;
@@ -370,8 +367,10 @@ __global__ __launch_bounds__(256, 1) void prefill_mfma_wide_rows32_kernel(AttnPa
     };
 
     if (ntiles > 0) {
+        if constexpr (FOLD) {
 #pragma unroll
-        for (int kb = 0; kb < D / 16; kb++) qreg[kb] = R32Mma<T>::scaled(qreg[kb], pw);
+            for (int kb = 0; kb < D / 16; kb++) qreg[kb] = R32Mma<T>::scaled(qreg[kb], pw);
+        }
         // "Tile -1", whose P . V the first iteration runs like any other: probabilities and V operands of zero (the
         // V stage of tile 3, which nothing has been loaded into yet, is cleared for its second contraction slice).
 #pragma unroll

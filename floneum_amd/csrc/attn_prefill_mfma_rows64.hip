@@ -21,7 +21,7 @@
 // one V tile in its second, each a whole iteration and a barrier ahead of its first reader; the one workgroup barrier
 // per iteration publishes what has landed.
 //
-// Softmax as in the 256-row kernel, with the power-of-two part of scale * log2(e) in Q; the rest (rr in [1, 2))
+// Softmax as in the 256-row kernel: scale * log2(e) (rr; in bf16 its power of two is in Q and rr is the rest, in [1, 2))
 // multiplies the scores in f32; a probability is exp2(fma(s, rr, -m * rr)) against the reference m the row already
 // has, and m moves only when a lane's probabilities of a tile sum to more than 2^15.
 // Masking is by interval (attn_bounds.h): analytic descriptors, key counts, the interval form of a mask tensor; the
@@ -83,11 +83,6 @@ struct R64Mma<half_t> {
     static __device__ __forceinline__ uint32_t pack2(float x, float y) {
         half2_t h = {(half_t)x, (half_t)y};
         return __builtin_bit_cast(uint32_t, h);
-    }
-    static __device__ __forceinline__ vec8 scaled(vec8 q, float c) {
-#pragma unroll
-        for (int e = 0; e < 8; e++) q[e] = (half_t)((float)q[e] * c);
-        return q;
     }
 };
 template <>
@@ -173,9 +168,11 @@ __global__ __launch_bounds__(256, 1) void prefill_mfma_rows64_kernel(AttnParams 
     for (int rb = 0; rb < RB; rb++) query[rb] = qw0 + 32 * rb + ln, qrow[rb] = min(query[rb], p.Sq - 1);
 
     const float scale2 = p.scale * R64_LOG2E;
-    // scale2 = pw * rr with pw a power of two and rr in [1, 2): Q takes pw (exact), rr multiplies every score in f32
-    const float pw = __uint_as_float(__float_as_uint(scale2) & 0x7F800000u);
-    const float rr = scale2 / pw;
+    // bf16: scale2 = pw * rr with pw a power of two and rr in [1, 2), Q takes pw (exact) and rr multiplies every score in f32.
+    // f16: rr is all of it (elements below 2^-14 / pw would become subnormal and lose bits).
+    constexpr bool FOLD = std::is_same<T, bf16_t>::value;
+    const float pw = FOLD ? __uint_as_float(__float_as_uint(scale2) & 0x7F800000u) : 1.0f;
+    const float rr = FOLD ? scale2 / pw : scale2;
 
     const int j_begin = (lo_wg / R64_TILE) * R64_TILE;
     const int ntiles = hi_wg > j_begin ? (hi_wg - j_begin + R64_KEYS - 1) / R64_KEYS : 0;  // sub-tiles
@@ -463,10 +460,12 @@ __global__ __launch_bounds__(256, 1) void prefill_mfma_rows64_kernel(AttnParams 
     using c1 = std::integral_constant<int, 1>;
 
     if (ntiles > 0) {
+        if constexpr (FOLD) {
 #pragma unroll
-        for (int rb = 0; rb < RB; rb++)
+            for (int rb = 0; rb < RB; rb++)
 #pragma unroll
-            for (int kb = 0; kb < KB; kb++) qreg[rb][kb] = R64Mma<T>::scaled(qreg[rb][kb], pw);
+                for (int kb = 0; kb < KB; kb++) qreg[rb][kb] = R64Mma<T>::scaled(qreg[rb][kb], pw);
+        }
         // "Sub-tile -1", whose P . V the first iteration runs like any other: probabilities and V operands of zero (the
         // V stage of tile 3, which nothing has been loaded into yet, is cleared for its second contraction slice).
 #pragma unroll

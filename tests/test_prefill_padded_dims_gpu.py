@@ -89,3 +89,20 @@ def test_small_scales_and_elements(device, form, D, dtype, q_std, k_std, scale):
     ref = in_64_bits(*(t.to_numpy().astype(np.float64) for t in (tq, tk, tv)), scale, causal, window)
     err = np.linalg.norm(out - ref) / np.linalg.norm(ref)
     assert err <= 3 * (2.0 ** -12 if dtype == fa.F16 else 2.0 ** -9), f"{form} D{D}: relative L2 {err:.2e}"
+
+
+@pytest.mark.parametrize("dtype", [fa.F16, fa.BF16])
+@pytest.mark.parametrize("D,kernel", [(256, fa.KERNEL_PREFILL_MFMA), (200, fa.KERNEL_PREFILL_MFMA),
+                                      (128, fa.KERNEL_PREFILL_MFMA_ROWS64)])
+@pytest.mark.parametrize("q_std,k_std,scale", [(1e-4, 1e4, None), (1e-5, 1e4, 0.5), (1.0, 1.0, None)])
+def test_small_elements_in_the_kernels_of_32_and_64_rows_per_wavefront(device, D, kernel, dtype, q_std, k_std, scale):
+    """The same for head dims above 192, and for the form of 64 rows per wavefront."""
+    B, H, Hkv, Sq, Skv, causal, window = 2, 4, 2, 300, 300, True, 0
+    scale = float(np.float32(D ** -0.5 if scale is None else scale))
+    rng = np.random.default_rng(D + 2)
+    stds, shapes = (q_std, k_std, 1.0), [(B, H, Sq, D), (B, Hkv, Skv, D), (B, Hkv, Skv, D)]
+    tq, tk, tv = (fa.Tensor.from_numpy(device, rng.normal(0, sd, sh).astype(np.float32), dtype) for sd, sh in zip(stds, shapes))
+    out = tq.flash_attention(tk, tv, scale, analytic=(True, 0, 0), out_dtype=fa.F32, force_kernel=kernel).to_numpy()
+    ref = in_64_bits(*(t.to_numpy().astype(np.float64) for t in (tq, tk, tv)), scale, causal, window)
+    err = np.linalg.norm(out - ref) / np.linalg.norm(ref)
+    assert err <= 3 * (2.0 ** -12 if dtype == fa.F16 else 2.0 ** -9), f"D{D}: relative L2 {err:.2e}"
