@@ -47,7 +47,7 @@ FORMS = {
     # the workgroups of 256 compute units decide: (B, H, Hkv, Sq, Skv, causal)
     "two_units_four_key_groups": (1, 6, 2, 33, 61, True),       # head_dim <= 64; above: two units, two key groups
     "two_units_two_key_groups": (2, 32, 8, 510, 510, True),     # 64; above: four units, two key groups
-    "four_units_two_key_groups": (2, 16, 16, 515, 545, False),
+    "four_units_two_key_groups": (2, 16, 16, 515, 545, False),  # 64; above: two units, two key groups
     "four_units": (34, 16, 16, 40, 65, False),
     "few_rows_keys_split": (1, 8, 2, 21, 2111, True),
     "short_prompt_keys_split": (1, 16, 4, 545, 545, True),      # above 64: four units, two key groups, three shares
