@@ -40,7 +40,7 @@ def build(verbose=True):
     if os.path.exists(STATIC):
         os.remove(STATIC)
     subprocess.check_call(["ar", "rcs", STATIC] + objs)
-    # the C++ host mirror's test program (runs on the GPU box, started by tests/test_host_mirror_gpu.py)
+    # the C++ host mirror's test program (needs a GPU, started by tests/test_host_mirror_gpu.py)
     root = os.path.dirname(HERE)
     cpp = os.path.join(root, "tests", "cpp", "test_host_mirror.cpp")
     if os.path.exists(cpp):

@@ -717,7 +717,7 @@ static bool use_key_split_form(const AttnParams &p) {
 }
 
 // Head dims 64, 96 and 128 are this kernel's own.  The other multiples of 8 above 64 run on it padded, quicker than on the
-// wide-head kernel, whose wavefronts read every LDS operand for half as many matrix instructions (both in turn on one box, us a
+// wide-head kernel, whose wavefronts read every LDS operand for half as many matrix instructions (both in turn on one card, us a
 // call; f16, 16 heads, 4096 x 4096 keys without a mask: head_dim 72 147 -> 120, 80 150 -> 124, 88 163 -> 130, 104 196 -> 136, 112
 // 202 -> 144, 120 201 -> 147; causal, 80: 157 -> 75 (two of that kernel's 128-row blocks per CU wait for the longest); 512-token
 // causal prompt, 32/8 heads, 80: 17.0 -> 15.9).  Below 64 the padding costs what the kernel gains unless the grid fills the
