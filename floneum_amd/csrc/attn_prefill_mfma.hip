@@ -706,14 +706,19 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnPara
 // cache), and a causal prompt's last blocks are several times longer than its first.  The key-split form (128
 // rows, twice the workgroups, the longest one half as long) costs about 7 % per tile and a longer prologue and
 // epilogue; measured, it wins (1.1-1.35 x) while the 256-row grid fills at most half the CUs, for up to 128
-// query rows (where the second wavefront group would have no rows at all), and for one workgroup per CU when a
-// head has 8 or more query blocks; it loses with fewer than three key tiles.
+// query rows (where the second wavefront group would have no rows at all), and, where later rows see more keys
+// than earlier ones, for one workgroup per CU when a head has 8 or more query blocks; it loses with fewer than
+// three key tiles.  Rows that all see the same keys keep the 256-row form there: its one workgroup per CU ends with
+// the others, and a CU would take two of the key-split form one after the other (f16, 16 heads without a mask, us a call,
+// both forms on one card: head_dim 80, 4096 x 4096 keys 113 -> 101, 3000 81 -> 68; 64, 2500 64 -> 57; 128, 2500 80 -> 59, 4096
+// 139 -> 123; causal, 4000 rows: 66 for the key-split form, 84 for the other).
 static bool use_key_split_form(const AttnParams &p) {
     const int cus = p.cus > 0 ? p.cus : 256;
     const int nqb = (p.Sq + PF_BM - 1) / PF_BM;
     const long wgs = (long)nqb * p.B * p.H * (p.pf_nsplit > 1 ? p.pf_nsplit : 1);
+    const bool uneven = 2L * p.Sq > p.Skv && ((p.analytic && p.causal) || p.mask_kind == FHIP_MASK_QK);
     if (p.Skv <= 2 * PF_BN) return false;
-    return p.Sq <= PF_BM / 2 || 2 * wgs <= cus || (wgs <= cus && nqb >= 8);
+    return p.Sq <= PF_BM / 2 || 2 * wgs <= cus || (wgs <= cus && nqb >= 8 && uneven);
 }
 
 // Head dims 64, 96 and 128 are this kernel's own.  The other multiples of 8 above 64 run on it padded, quicker than on the
