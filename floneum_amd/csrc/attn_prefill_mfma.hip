@@ -1,7 +1,7 @@
 // Prefill attention for f16 / bf16 on the gfx950 matrix cores.
 //
 // Workgroup = 8 wavefronts = 256 query rows of one (batch, head); each wavefront owns 32 rows.
-// Keys/values are walked in tiles of 64 rows that go from global memory straight into a three-stage
+// Keys/values are walked in tiles of 64 rows that go from global memory straight into a four-stage
 // LDS ring (direct-to-LDS buffer loads, no staging registers).  Per tile and wavefront:
 //   S^T (64 keys x 32 queries)  = K_tile . Q^T      v_mfma_f32_32x32x16  (A = K from LDS, B = Q in registers)
 //   scale * log2(e) (rr) multiplies the scores in f32: a probability is exp2(fma(s, rr, -m * rr)), one fused
@@ -15,11 +15,18 @@
 //   transposing LDS load ds_read_b64_tr_b16, B = P^T taken straight from the S^T accumulator
 //   registers (the contraction index is permuted identically on both operands)
 // The two wavefronts that share a SIMD (w and w + 4) run half a tile out of phase: while one is in
-// its matrix phase (S^T of the current tile, then P.V of the previous one) the other is in its
-// vector phase (softmax, tile loads), so the MFMA pipe and the VALU are busy at the same time.
+// its matrix phase (S^T of the current tile, P.V of the previous one, tile loads) the other is in its
+// vector phase (softmax), so the MFMA pipe and the VALU are busy at the same time.
 // Phases are separated by workgroup barriers; the tile loads ride on the same barriers.  The vector
 // phase uses no dot-product instructions: on this chip they queue behind the MFMAs of the other
 // wavefront instead of running beside them.
+// Bound: power at head_dim 128 (4096 x 4096 keys, 16 heads, no mask, f16: 123 us = 1.12 PFLOP/s); below, a vector phase
+// takes as long as a matrix phase or longer: its 111 vector instructions take a lone wavefront 617 cycles and beside the
+// matrix instructions of the other 785, the 16 / 20 / 24 matrix instructions of head_dim 64 / 80 / 96 take 512 / 704 / 768.
+// So everything but the softmax itself is done in the matrix phase, in the shadow of its instructions: tile loads, addresses,
+// the mask test (an instruction on the scalar unit costs a lone wavefront as much as one on the vector unit).  f16, the
+// call above at head_dim 64 / 80 / 96: 89 -> 75, 102 -> 92, 109 -> 100 us (loads, their addresses and an LDS wait in the
+// vector phase before: 1350 cycles, now about 950); causal, 32/8 heads, 4000 rows at 64: 97 -> 81.
 // All accumulation is f32; P is rounded to the input type for the second product.
 // Key-split form (template parameter KS): the workgroup owns 128 query rows and its two wavefront groups
 // take alternate key tiles of the same rows, each through the same matrix / vector phases, and merge their
@@ -79,27 +86,28 @@ struct Mma<bf16_t> {
     }
 };
 
-// LDS image of a 64-row tile.  Rows are kept in 16 groups of 4: row r sits in group r % 16 at
-// position r / 16.  A group is exactly what one wavefront-wide direct-to-LDS load writes (4 rows of
-// head_dim 16-bit values, contiguous), and groups are padded apart so that
-//   - the 16 rows a quarter-wavefront reads for the S^T operand (rows r .. r+15, same 16-byte
-//     column) fall 16 bytes apart modulo the 256-byte bank period            (K: pitch 8 D + 16)
-//   - the 4 rows x 64 bytes a half-wavefront reads with the transposing load fall 64 bytes apart
-//                                                                            (V: pitch 8 D + 64)
+// LDS image of a 64-row tile.  Rows are kept in NG groups: row r sits in group r % NG at position r / NG.  A group is what
+// one wavefront-wide direct-to-LDS load writes (D = 128: 4 rows, D = 64: 8), or three of them (D = 96: 16 rows), whole
+// kilobytes either way, so that every lane of every load moves 16 bytes.  Groups are padded apart so that
+//   - rows r .. r + 3 at one column fall 16 bytes apart modulo the 256-byte bank period, and the sixteen rows that the LDS
+//     serves at once in a 128-bit read (four such runs) fall into sixteen different places  (K: pitch of a group + 16)
+//   - the 4 rows x 64 bytes a half-wavefront reads with the transposing load fall 64 bytes apart  (V: pitch + 64)
 template <int D, bool KS>
 struct PfCfg {
     static constexpr int ROWB = D * 2;                               // bytes per tile row
-    static constexpr int KG = 4 * ROWB + 16;                         // K group pitch, bytes
-    static constexpr int VG = 4 * ROWB + 64;                         // V group pitch, bytes
-    static constexpr int K_BYTES = 16 * KG;
-    static constexpr int V_BYTES = 16 * VG;
+    static constexpr int NG = D == 128 ? 16 : D == 96 ? 4 : 8;       // groups of a tile
+    static constexpr int KG = PF_BN / NG * ROWB + 16;                // K group pitch, bytes
+    static constexpr int VG = PF_BN / NG * ROWB + 64;                // V group pitch, bytes
+    static constexpr int K_BYTES = NG * KG;
+    static constexpr int V_BYTES = NG * VG;
     static constexpr int CPR = D / 8;                                // 16-byte chunks per row
-    static constexpr int LOAD_LANES = 4 * CPR;                       // lanes of a wavefront-wide tile load (<= 64)
-    // tile buffers.  Unsplit form: three stages of (K tile, V tile), tile t in stage t % 3.  Key-split form
+    static constexpr int LOADS = PF_BN * ROWB / 4096;                // loads of each of the four wavefronts that move a tile
+    static constexpr int OFFSETS = NG == 4 ? LOADS : 1;              // (their lanes' offsets differ by a uniform value otherwise)
+    // tile buffers.  Unsplit form: four stages of (K tile, V tile), tile t in stage t % 4.  Key-split form
     // (KS): a ring of five K tiles followed by a ring of four V tiles (see the slot schedule in the kernel).
     static constexpr int STAGE = K_BYTES + V_BYTES;
-    static constexpr int NK = KS ? 5 : 3, NV = KS ? 4 : 3;
-    static constexpr int LDS_BYTES = KS ? NK * K_BYTES + NV * V_BYTES : 3 * STAGE;
+    static constexpr int NK = KS ? 5 : 4, NV = 4;
+    static constexpr int LDS_BYTES = KS ? NK * K_BYTES + NV * V_BYTES : 4 * STAGE;
     static constexpr int BM = KS ? PF_BM / 2 : PF_BM;                // query rows per workgroup
 };
 
@@ -223,10 +231,9 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnPara
 
     using std::integral_constant;
     // ---- tile movement: global -> LDS directly (no registers) --------------------------------------
-    // The four wavefronts of a group move one whole tile with four loads each.  Load j of wavefront w
-    // writes LDS group w + 4 j; lane i of it fetches row 16 (i / CPR) + w + 4 j, 16-byte column i % CPR, so
-    // the lanes of one load land contiguously (which is what the hardware does with a direct load) and the
-    // four loads of a wavefront differ by a uniform offset only.
+    // The four wavefronts of a group move one whole tile with LOADS loads each.  Load j of wavefront w writes LDS group
+    // w + 4 j (D = 96: the j-th kilobyte of group w); its lanes fetch that group's 16-byte chunks in order (which is how
+    // the hardware lays out a direct load).
     // Unsplit form: group 1 moves the K tiles, group 0 the V tiles.  Key-split form: the group that is in
     // its vector phase moves one K and one V tile.
     // The tensors as raw buffer descriptors (base, no stride, size in bytes, 32-bit raw format): a row beyond
@@ -239,58 +246,67 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnPara
                        0x00020000u};
     };
     const uint4_t krs = descriptor(kg, krow_bytes), vrs = descriptor(vg, vrow_bytes);
-    const bool padding = PAD && (lane % C::CPR) * 8 >= hd;
-    const int gofs_k = padding ? 0x7ffffff0 : (16 * (lane / C::CPR) + wv) * krow_bytes + (lane % C::CPR) * 16;
-    const int gofs_v = padding ? 0x7ffffff0 : (16 * (lane / C::CPR) + wv) * vrow_bytes + (lane % C::CPR) * 16;
+    int gofs_k[C::OFFSETS], gofs_v[C::OFFSETS];
+#pragma unroll
+    for (int j = 0; j < C::OFFSETS; j++) {
+        const int chunk = lane + 64 * j, row = C::NG * (chunk / C::CPR) + wv, col = chunk % C::CPR;
+        const bool padding = PAD && col * 8 >= hd;
+        gofs_k[j] = padding ? 0x7ffffff0 : row * krow_bytes + col * 16;
+        gofs_v[j] = padding ? 0x7ffffff0 : row * vrow_bytes + col * 16;
+    }
     // where tile t lives in LDS
-    auto k_stage = [&](int t) __attribute__((always_inline)) { return KS ? (t % C::NK) * C::K_BYTES : (t % 3) * STAGE; };
+    auto k_stage = [&](int t) __attribute__((always_inline)) { return KS ? (int)((uint32_t)t % C::NK) * C::K_BYTES : (t & 3) * STAGE; };
     auto v_stage = [&](int t) __attribute__((always_inline)) {
-        return KS ? C::NK * C::K_BYTES + (t % C::NV) * C::V_BYTES : (t % 3) * STAGE + C::K_BYTES;
+        return KS ? C::NK * C::K_BYTES + (t & 3) * C::V_BYTES : (t & 3) * STAGE + C::K_BYTES;
     };
     // a tile that starts beyond the key axis is never used: clamp the (uniform) offset so it stays
     // inside 32 bits; rows past Skv inside a used tile are out of range of the buffer and read 0
-    auto issue_loads = [&](const uint4_t rs, int gofs, int row_bytes, int tile, int lbase, int lstep)
-                           __attribute__((always_inline)) {
-        // (uniform values; pinned to scalar registers, which is what the instruction takes)
-        const int soff = __builtin_amdgcn_readfirstlane(min(j_begin + tile * PF_BN, p.Skv) * row_bytes);
-        // M0 takes an LDS address, not an offset into the tile buffers (they are the kernel's only LDS variable and
-        // start at 0, which the compiler folds in)
-        lbase = __builtin_amdgcn_readfirstlane(lbase + (int)(uint32_t)(uintptr_t)lds_base);
-        if (C::LOAD_LANES == 64 || lane < C::LOAD_LANES) {
-            // written as assembly on purpose: the compiler would otherwise make every later LDS read
-            // of this wavefront wait for these loads, whose data is not due before the next barrier
+    // (uniform values, pinned to scalar registers, which is what the instruction takes.  M0 takes an LDS address, not an
+    // offset into the tile buffers: they are the kernel's only LDS variable and start at 0, which the compiler folds in.
+    // Written as assembly on purpose: the compiler would otherwise make every later LDS read of this wavefront wait for
+    // these loads, whose data is not due before a later barrier.)
+    auto issue = [&](const uint4_t rs, const int (&gofs)[C::OFFSETS], int row_bytes, int soff, int lbase, int pitch, int j)
+                     __attribute__((always_inline)) {
+        const int lds = lbase + (C::NG == 4 ? 1024 * j : 4 * j * pitch), from = soff + (C::NG == 4 ? 0 : 4 * j * row_bytes);
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                     :
+                     : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(gofs[C::OFFSETS > 1 ? j : 0]), "s"(rs),
+                       "s"(__builtin_amdgcn_readfirstlane(from))
+                     : "m0");
+    };
+    auto row_offset = [&](int tile, int row_bytes) __attribute__((always_inline)) { return min(j_begin + tile * PF_BN, p.Skv) * row_bytes; };
+    const int lds0 = (int)(uint32_t)(uintptr_t)lds_base;
+    auto issue_k = [&](int tile, int j) __attribute__((always_inline)) {
+        issue(krs, gofs_k, krow_bytes, row_offset(tile, krow_bytes), lds0 + k_stage(tile) + wv * C::KG, C::KG, j);
+    };
+    auto issue_v = [&](int tile, int j) __attribute__((always_inline)) {
+        issue(vrs, gofs_v, vrow_bytes, row_offset(tile, vrow_bytes), lds0 + v_stage(tile) + wv * C::VG, C::VG, j);
+    };
+    // Load n of those that a matrix phase issues.  Unsplit form: of one tile of this group's tensor (K: group 1, V: group 0).
+    // Key-split form, slot s: of K(s + 4) and V(s + 1).
+    constexpr int PHASE_LOADS = KS ? 2 * C::LOADS : C::LOADS;
+    const uint4_t mrs = moves_k ? krs : vrs;
+    const int mrow_bytes = moves_k ? krow_bytes : vrow_bytes, mpitch = moves_k ? C::KG : C::VG;
+    const int mbase = lds0 + (moves_k ? 0 : C::K_BYTES) + wv * mpitch;
+    int mgofs[C::OFFSETS];
 #pragma unroll
-            for (int j = 0; j < 4; j++)
-                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                             :
-                             : "s"(lbase + j * lstep), "v"(gofs), "s"(rs), "s"(soff + 4 * j * row_bytes)
-                             : "memory", "m0");
+    for (int j = 0; j < C::OFFSETS; j++) mgofs[j] = moves_k ? gofs_k[j] : gofs_v[j];
+    auto load = [&](int at, int n) __attribute__((always_inline)) {
+        if (n >= PHASE_LOADS) return;
+        if constexpr (KS) {
+            if (n & 1) issue_v(at + 1, n >> 1);
+            else issue_k(at + 4, n >> 1);
+        } else {
+            issue(mrs, mgofs, mrow_bytes, row_offset(at, mrow_bytes), mbase + (at & 3) * STAGE, mpitch, n);
         }
     };
-    auto issue_k = [&](int tile) __attribute__((always_inline)) {
-        issue_loads(krs, gofs_k, krow_bytes, tile, k_stage(tile) + wv * C::KG, 4 * C::KG);
+    auto load_all = [&](int at) __attribute__((always_inline)) {
+#pragma unroll
+        for (int n = 0; n < PHASE_LOADS; n++) load(at, n);
     };
-    auto issue_v = [&](int tile) __attribute__((always_inline)) {
-        issue_loads(vrs, gofs_v, vrow_bytes, tile, v_stage(tile) + wv * C::VG, 4 * C::VG);
-    };
-    // unsplit form: this group's tensor, tile `tile`
-    const uint4_t mrs = moves_k ? krs : vrs;
-    const int mgofs = moves_k ? gofs_k : gofs_v, mrow_bytes = moves_k ? krow_bytes : vrow_bytes;
-    const int lds_move_base = (moves_k ? 0 : C::K_BYTES) + wv * (moves_k ? C::KG : C::VG);
-    const int lds_move_step = 4 * (moves_k ? C::KG : C::VG);
-    auto issue_tile = [&](int tile) __attribute__((always_inline)) {
-        issue_loads(mrs, mgofs, mrow_bytes, tile, (tile % 3) * STAGE + lds_move_base, lds_move_step);
-    };
-    // key-split form, slot s: K(s + 4) and V(s + 1)
-    auto issue_slot = [&](int slot) __attribute__((always_inline)) {
-        issue_k(slot + 4);
-        issue_v(slot + 1);
-    };
-    // all but the loads of this wavefront's most recent `newer` vector phases have landed
-    auto wait_tiles = [&](auto newer) __attribute__((always_inline)) {
-        if constexpr (decltype(newer)::value == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        else if constexpr (KS) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+    // all but the most recent N loads of this wavefront have landed
+    auto wait_loads = [&](auto n) __attribute__((always_inline)) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"i"(decltype(n)::value) : "memory");
     };
     // local tile index -> tile: in the key-split form group g owns the tiles t with t % 2 == g
     auto tile_of = [&](int i) __attribute__((always_inline)) { return KS ? 2 * i + group : i; };
@@ -298,130 +314,84 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnPara
     float16_t s[2];     // S^T of the tile in flight
     uint32_t pk[2][8];  // its probabilities, packed pairs in the MFMA operand order
 
-    // S^T = K . Q^T for this group's tile i (local index; see tile_of)
-    auto qk = [&](int i) __attribute__((always_inline)) {
-        const int kbase = k_stage(tile_of(i)) + (ln & 15) * C::KG + (ln >> 4) * C::ROWB + h2 * 16;
-#pragma unroll
-        for (int kb = 0; kb < QD / 16; kb++) {
-#pragma unroll
-            for (int t = 0; t < 2; t++) {
-                uint4_t raw = *LDS_PTR(uint4_t, kbase + t * 2 * C::ROWB + kb * 32);
-                s[t] = Mma<T>::mfma(__builtin_bit_cast(vec8, raw), qreg[kb], kb == 0 ? zero16 : s[t]);
-            }
-        }
-    };
-    // O^T += V^T . P^T for tile i: contraction slice (t, kk) holds this half-wave's keys
-    // 32 t + 16 kk + 4 h2 + {0..3} and + 8
-    auto pv = [&](int i) __attribute__((always_inline)) {
-        const int i16 = lane & 15;
-        const int bl = (lane & 31) >> 4;
-        const int vbase = v_stage(tile_of(i)) + (4 * h2 + (i16 >> 2)) * C::VG + (16 * bl + 4 * (i16 & 3)) * 2;
-#pragma unroll
-        for (int gq = 0; gq < 4; gq++) {  // gq = 2 t + kk: rows 16 gq + 4 h2 + {0..3} and + 8
-            const int t = gq >> 1, kk = gq & 1;
-            const uint4_t braw = {pk[t][4 * kk], pk[t][4 * kk + 1], pk[t][4 * kk + 2], pk[t][4 * kk + 3]};
-            const vec8 bop = __builtin_bit_cast(vec8, braw);
-#pragma unroll
-            for (int db = 0; db < D / 32; db++) {
-                const int addr = vbase + gq * C::ROWB + db * 64;
-                short4_t a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(short4_t, addr));
-                short4_t a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(short4_t, addr + 8 * C::VG));
-                const uint2_t u0 = __builtin_bit_cast(uint2_t, a0), u1 = __builtin_bit_cast(uint2_t, a1);
-                uint4_t araw = {u0[0], u0[1], u1[0], u1[1]};
-                o[db] = Mma<T>::mfma(__builtin_bit_cast(vec8, araw), bop, o[db]);
-            }
-        }
-    };
-    // Matrix phase in one basic block: S^T of tile ik, then P.V of tile ip.  The first four K operand
-    // slices are already in `ka` (read before the barrier that opens the phase, see prefetch_k), so the
-    // matrix pipe starts at once; the remaining LDS reads are issued several MFMAs ahead of their use
-    // (the order is pinned by the scheduling groups at the end; without them the reads sit right in
-    // front of their MFMAs and the pipe waits out the LDS latency every few instructions).
+    // A matrix phase: S^T of tile i (QK) and P.V of tile i - 1 (PV), and the tile loads of the slot.  S^T's K operands of the
+    // first PRE contraction slices have been read in the vector phase before (PREFETCHED), the others leave the LDS several
+    // matrix instructions ahead of their use, and V's likewise; each step is fenced, so that neither the reads nor the
+    // loads gather in front of the matrix instructions.
+    // O^T += V^T . P^T: contraction slice (t, kk) holds this half-wave's keys 32 t + 16 kk + 4 h2 + {0..3} and + 8
+    constexpr int NDB = D / 32, NKB = QD / 16;
     constexpr int PFK = (D == 128) ? 2 : 4;  // K operand slices in flight (register budget)
+    // Contraction slices read in the vector phase.  None where that phase is much the longer one: head_dim 64, 4096 x 4096 keys
+    // 76.8 -> 75.4 us; at 80 and 96 no difference, at 128 reading none costs 1 % (499 -> 504 us for an 8192-token prompt).
+    constexpr int PRE = D == 64 ? 0 : 2;
     uint4_t ka[PFK][2];
-    auto prefetch_k = [&](int ik) __attribute__((always_inline)) {
-        const int kbase = k_stage(tile_of(ik)) + (ln & 15) * C::KG + (ln >> 4) * C::ROWB + h2 * 16;
+    const int i16 = lane & 15, bl = (lane & 31) >> 4;
+    const int k_at = (ln % C::NG) * C::KG + (ln / C::NG) * C::ROWB + h2 * 16;
+    const int v_at = (C::NG == 4 ? (i16 >> 2) * C::VG + h2 * C::ROWB : (4 * h2 + (i16 >> 2)) * C::VG) + (16 * bl + 4 * (i16 & 3)) * 2;
+    constexpr int V_SLICE = 16 / C::NG * C::ROWB, V_PLUS8 = C::NG == 16 ? 8 * C::VG : 8 / C::NG * C::ROWB;
+    auto read_k = [&](int kbase, int kb) __attribute__((always_inline)) {
 #pragma unroll
-        for (int kb = 0; kb < PFK; kb++)
-#pragma unroll
-            for (int t = 0; t < 2; t++) ka[kb][t] = *LDS_PTR(uint4_t, kbase + t * 2 * C::ROWB + kb * 32);
+        for (int t = 0; t < 2; t++) ka[kb % PFK][t] = *LDS_PTR(uint4_t, kbase + t * (32 / C::NG) * C::ROWB + kb * 32);
     };
-    auto qk_pv = [&](int ip, int ik, auto do_pv, auto prefetched) __attribute__((always_inline)) {
-        constexpr bool PV = decltype(do_pv)::value;
-        constexpr bool PRE = decltype(prefetched)::value;
-        constexpr int NDB = D / 32, NKB = QD / 16;
-        const int vstage = v_stage(tile_of(ip)), kstage = k_stage(tile_of(ik));
-        const int i16 = lane & 15;
-        const int bl = (lane & 31) >> 4;
-        const int vbase = vstage + (4 * h2 + (i16 >> 2)) * C::VG + (16 * bl + 4 * (i16 & 3)) * 2;
-        const int kbase = kstage + (ln & 15) * C::KG + (ln >> 4) * C::ROWB + h2 * 16;
+    auto prefetch_k = [&](int i) __attribute__((always_inline)) {
+        const int kbase = k_stage(tile_of(i)) + k_at;
+#pragma unroll
+        for (int kb = 0; kb < PRE; kb++) read_k(kbase, kb);
+    };
+    bool masked = false;  // the tile whose S^T was formed last is not wholly visible to this wavefront
+    auto qk_pv = [&](int i, int at, auto do_qk, auto do_pv, auto prefetched) __attribute__((always_inline)) {
+        constexpr bool QK = decltype(do_qk)::value, PV = decltype(do_pv)::value, PREFETCHED = decltype(prefetched)::value;
+        const int kbase = k_stage(tile_of(i)) + k_at, vbase = v_stage(tile_of(i - 1)) + v_at;
         uint4_t va[2][NDB];
-        auto read_v = [&](int gq, uint4_t (&a)[NDB]) {  // gq = 2 t + kk: rows 32 t + 16 kk (+8)
+        auto read_v = [&](int gq) __attribute__((always_inline)) {  // gq = 2 t + kk: rows 16 gq + 4 h2 + {0..3} and + 8
 #pragma unroll
             for (int db = 0; db < NDB; db++) {
-                const int addr = vbase + gq * C::ROWB + db * 64;
+                const int addr = vbase + gq * V_SLICE + db * 64;
                 short4_t a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(short4_t, addr));
-                short4_t a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(short4_t, addr + 8 * C::VG));
+                short4_t a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(short4_t, addr + V_PLUS8));
                 const uint2_t u0 = __builtin_bit_cast(uint2_t, a0), u1 = __builtin_bit_cast(uint2_t, a1);
-                a[db] = uint4_t{u0[0], u0[1], u1[0], u1[1]};
+                va[gq & 1][db] = uint4_t{u0[0], u0[1], u1[0], u1[1]};
             }
         };
-        auto mfma_v = [&](int gq, const uint4_t (&a)[NDB]) {
-            const int t = gq >> 1, kk = gq & 1;
-            const uint4_t braw = {pk[t][4 * kk], pk[t][4 * kk + 1], pk[t][4 * kk + 2], pk[t][4 * kk + 3]};
-            const vec8 bop = __builtin_bit_cast(vec8, braw);
+        if constexpr (QK) {
 #pragma unroll
-            for (int db = 0; db < NDB; db++) o[db] = Mma<T>::mfma(__builtin_bit_cast(vec8, a[db]), bop, o[db]);
-        };
-        auto read_k = [&](int kb, uint4_t (&a)[2]) {
+            for (int kb = PREFETCHED ? PRE : 0; kb < PFK; kb++) read_k(kbase, kb);
 #pragma unroll
-            for (int t = 0; t < 2; t++) a[t] = *LDS_PTR(uint4_t, kbase + t * 2 * C::ROWB + kb * 32);
-        };
-        if constexpr (!PRE) {
+            for (int kb = 0; kb < NKB; kb++) {
 #pragma unroll
-            for (int kb = 0; kb < PFK; kb++) read_k(kb, ka[kb]);
-        }
-#pragma unroll
-        for (int kb = 0; kb < NKB; kb++) {
-#pragma unroll
-            for (int t = 0; t < 2; t++)
-                s[t] = Mma<T>::mfma(__builtin_bit_cast(vec8, ka[kb % PFK][t]), qreg[kb], kb == 0 ? zero16 : s[t]);
-            if (kb + PFK < NKB) read_k(kb + PFK, ka[kb % PFK]);
-            if (PV && kb >= NKB - 4 && kb < NKB - 2) read_v(kb + 4 - NKB, va[kb + 4 - NKB]);
+                for (int t = 0; t < 2; t++)
+                    s[t] = Mma<T>::mfma(__builtin_bit_cast(vec8, ka[kb % PFK][t]), qreg[kb], kb == 0 ? zero16 : s[t]);
+                if (kb + PFK < NKB) read_k(kbase, kb + PFK);
+                if (PV && kb >= NKB - 4 && kb < NKB - 2) read_v(kb + 4 - NKB);
+                load(at, kb);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            const int j0 = j_begin + tile_of(i) * PF_BN;
+            masked = !(j0 >= full_lo_w && j0 + PF_BN <= full_hi_w);
+        } else {
+            read_v(0);
+            read_v(1);
         }
         if constexpr (PV) {
-            mfma_v(0, va[0]);
-            read_v(2, va[0]);
-            mfma_v(1, va[1]);
-            read_v(3, va[1]);
-            mfma_v(2, va[0]);
-            mfma_v(3, va[1]);
-        }
-        // scheduling groups: 0x100 = LDS read, 0x008 = MFMA
-        auto constexpr_reads = [&](int kb) __attribute__((always_inline)) {
-            const bool rk = kb + PFK < NKB, rv = PV && kb >= NKB - 4 && kb < NKB - 2;
-            if (rk && rv) __builtin_amdgcn_sched_group_barrier(0x100, 2 + 2 * NDB, 0);
-            else if (rk) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-            else if (rv) __builtin_amdgcn_sched_group_barrier(0x100, 2 * NDB, 0);
-        };
-        if constexpr (!PRE) __builtin_amdgcn_sched_group_barrier(0x100, 2 * PFK, 0);
 #pragma unroll
-        for (int kb = 0; kb < NKB; kb++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-            constexpr_reads(kb);
+            for (int gq = 0; gq < 4; gq++) {
+                const int t = gq >> 1, kk = gq & 1;
+                const uint4_t braw = {pk[t][4 * kk], pk[t][4 * kk + 1], pk[t][4 * kk + 2], pk[t][4 * kk + 3]};
+#pragma unroll
+                for (int db = 0; db < NDB; db++)
+                    o[db] = Mma<T>::mfma(__builtin_bit_cast(vec8, va[gq & 1][db]), __builtin_bit_cast(vec8, braw), o[db]);
+                if (gq < 2) read_v(gq + 2);
+                load(at, (QK ? NKB : 0) + gq);
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
-        if constexpr (PV) {
-            __builtin_amdgcn_sched_group_barrier(0x008, NDB, 0);
-            __builtin_amdgcn_sched_group_barrier(0x100, 2 * NDB, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, NDB, 0);
-            __builtin_amdgcn_sched_group_barrier(0x100, 2 * NDB, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 2 * NDB, 0);
-        }
+#pragma unroll
+        for (int n = (QK ? NKB : 0) + (PV ? 4 : 0); n < PHASE_LOADS; n++) load(at, n);
     };
     // mask + online softmax (log2 domain, lazily rescaled) of tile i: s -> pk
     auto softmax = [&](int i) __attribute__((always_inline)) {
-        const int j0 = j_begin + tile_of(i) * PF_BN;
-        if (!(j0 >= full_lo_w && j0 + PF_BN <= full_hi_w)) {
+        if (masked) {
+            const int j0 = j_begin + tile_of(i) * PF_BN;
             // element r of block t is key j0 + 32 t + 8 (r / 4) + 4 h2 + r % 4
 #pragma unroll
             for (int t = 0; t < 2; t++)
@@ -436,23 +406,29 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnPara
         // type's range (P is rounded to it for the second product; l and O are f32), and that is what the check below
         // guarantees: a lane's 32 probabilities are positive, so while their sum is at most 2^15 each of them is.
         auto probabilities = [&](float nm) __attribute__((always_inline)) {
-            float ts = 0.0f;
+            // four products ahead of the exponentials and two exponentials ahead of their uses: a lone wavefront has nothing
+            // else to issue while one waits for the other
+            constexpr int AHEAD = 4, LAG = 2;
+            float x[32], sum[2] = {0.0f, 0.0f};
+            auto scaled = [&](int r) __attribute__((always_inline)) { x[r] = __builtin_fmaf(s[r >> 4][r & 15], rr, nm); };
 #pragma unroll
-            for (int t = 0; t < 2; t++)
+            for (int r = 0; r < AHEAD; r++) scaled(r);
 #pragma unroll
-                for (int r = 0; r < 16; r += 2) {
-                    const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][r], rr, nm));
-                    const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][r + 1], rr, nm));
-                    pk[t][r >> 1] = Mma<T>::pack2(p0, p1);
-                    ts += p0 + p1;  // plain f32 adds: a dot-product instruction here would queue behind the MFMAs
-                }
-            return ts;
+            for (int r = 0; r < 32 + LAG; r++) {
+                if (r < 32) x[r] = __builtin_amdgcn_exp2f(x[r]);
+                if (r + AHEAD < 32) scaled(r + AHEAD);
+                const int d = r - LAG;
+                if (d >= 0) sum[d & 1] = d < 2 ? x[d] : sum[d & 1] + x[d];  // (a dot-product instruction would queue behind the MFMAs)
+                if (d >= 0 && (d & 1)) pk[d >> 4][(d & 15) >> 1] = Mma<T>::pack2(x[d - 1], x[d]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            return sum[0] + sum[1];
         };
         float ts = probabilities(nmr);
         // Not at most 2^15 (which also catches the +inf and NaN a row without a reference produces): some row of the
         // wavefront needs its reference moved.  Take the tile's maximum, move every row's reference to at least that,
         // rescale what the row has accumulated, and form the tile's probabilities again.
-        if (__builtin_amdgcn_ballot_w64(!(ts <= 32768.0f)) != 0) {
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(ts <= 32768.0f)) != 0, 0)) {
             float mx = s[0][0];
 #pragma unroll
             for (int t = 0; t < 2; t++)
@@ -477,13 +453,13 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnPara
     // ---- slot schedule ---------------------------------------------------------------------------------
     // Slots are separated by workgroup barriers.  Group 0 is in its matrix phase in even slots and in
     // its vector phase in odd slots; group 1 the other way round, one slot later.  Matrix phase of
-    // tile i: S^T of tile i (reads K(i)), then P.V of tile i-1 (reads V(i-1)); K(i) is read in slots 2i
-    // and 2i+1, V(i) in slots 2i+2 and 2i+3.  Vector phase: issue a tile load, softmax, read the first
-    // K operands of the next matrix phase, wait for the tile load issued one vector phase earlier.
-    // Tile t lives in stage t % 3.  In even slot 2j group 1 issues K(j+2) (its stage was last read for
-    // K(j-1) in slot 2j-1) and makes sure K(j+1) has landed; in odd slot 2j+1 group 0 issues V(j+1)
-    // (stage last read for V(j-2) in slot 2j-1) and makes sure V(j) has landed.  Every tile is thus
-    // complete, and published by a barrier, before the slot of its first reader, and has had two
+    // tile i: S^T of tile i (reads K(i)), then P.V of tile i-1 (reads V(i-1)); K(i) is read in slots 2i - 1 (ahead, by
+    // group 0) to 2i+1, V(i) in slots 2i+2 and 2i+3.  Vector phase: read the first K operands of the next matrix phase,
+    // softmax, wait for a tile issued two matrix phases ago.
+    // Tile t lives in stage t % 4.  In odd slot 2j+1 group 1 issues K(j+3) (its stage was last read for
+    // K(j-1) in slot 2j-1) and makes sure in slot 2j+2 that K(j+2) has landed; in even slot 2j group 0 issues V(j+2)
+    // (stage last read for V(j-2) in slot 2j-1) and makes sure in slot 2j+1 that V(j) has landed.  Every tile is thus
+    // complete, and published by a barrier, before the slot of its first reader, and has had at least three
     // slots to arrive.
     // The tiles visible to a wavefront form one contiguous range [ia, ib).  Each group walks the slot
     // sequence in five static segments (nothing / first tile / steady state / last tile / nothing) so
@@ -491,11 +467,11 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnPara
     //
     // Key-split form (KS): both groups own the same 128 rows and group g takes the tiles t with t % 2 == g,
     // so a slot is the matrix phase of tile s for one group and the vector phase of tile s-1 for the other;
-    // the groups' (m, l, O) are merged at the end.  K(t) is read in slot t (its first operands at the end of
-    // slot t-1), V(t) in slot t+2.  The group in its vector phase in slot s issues K(s+4) into the stage K(s-1)
+    // the groups' (m, l, O) are merged at the end.  K(t) is read in slot t (its first operands in
+    // slot t-1), V(t) in slot t+2.  The group in its matrix phase in slot s issues K(s+4) into the stage K(s-1)
     // has just left (ring of 5) and V(s+1) into the stage of V(s-3), last read in slot s-1 (ring of 4), and
-    // makes sure its loads of slot s-2, K(s+2) and V(s-1), have landed: each is published by a barrier one
-    // slot before its first reader and has had two slots to arrive.  The segments below then run on the
+    // makes sure its loads of slot s-2, K(s+2) and V(s-1), have landed: each is published by a barrier
+    // before the slot of its first reader and has had two slots to arrive.  The segments below then run on the
     // group's own tile count: local tile i of group g is tile 2 i + g.
     int ia = 0, ib = 0;
     if (wave_has_rows && hi_w > lo_w) {
@@ -510,65 +486,65 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnPara
         n_iter = (ntiles + 3) >> 1;
     }
     // MODE bit 0: S^T of tile i; bit 1: P.V of tile i-1; bit 2: softmax of tile i (group 0) / i-1 (group 1);
-    // bit 3: the K operands of tile i were prefetched by the preceding vector phase
-    auto matrix_phase = [&](int i, auto mode) __attribute__((always_inline)) {
+    // bit 3: the K operands of tile i were prefetched by the preceding vector phase;
+    // bit 4: prefetch the K operands for the next matrix phase in the vector phase
+    auto matrix_phase = [&](int i, int at, auto mode) __attribute__((always_inline)) {
         constexpr int MODE = decltype(mode)::value;
         __builtin_amdgcn_s_setprio(1);
-        if constexpr ((MODE & 11) == 11) qk_pv(i - 1, i, std::true_type{}, std::true_type{});
-        else if constexpr ((MODE & 11) == 9) qk_pv(i - 1, i, std::false_type{}, std::true_type{});
-        else {
-            if constexpr ((MODE & 2) != 0) pv(i - 1);
-            if constexpr ((MODE & 1) != 0) qk(i);
-        }
+        if constexpr ((MODE & 3) != 0)
+            qk_pv(i, at, integral_constant<bool, (MODE & 1) != 0>{}, integral_constant<bool, (MODE & 2) != 0>{},
+                  integral_constant<bool, (MODE & 8) != 0>{});
+        else load_all(at);
         __builtin_amdgcn_s_setprio(0);
+        if constexpr (KS) wait_loads(integral_constant<int, PHASE_LOADS>{});  // those of the matrix phase before have landed
     };
     // next_k: the tile whose S^T this wavefront computes in its next matrix phase
-    auto vector_phase = [&](int i, int tile_to_load, int slot, int next_k, auto mode) __attribute__((always_inline)) {
+    auto vector_phase = [&](int i, int next_k, auto newer, auto mode) __attribute__((always_inline)) {
         constexpr int MODE = decltype(mode)::value;
-        if constexpr (KS) issue_slot(slot);
-        else issue_tile(tile_to_load);
-        if constexpr ((MODE & 4) != 0) softmax(i);
         if constexpr ((MODE & 16) != 0) prefetch_k(next_k);
-        wait_tiles(integral_constant<int, 1>{});  // the tile issued one vector phase ago has landed
+        if constexpr ((MODE & 4) != 0) softmax(i);
+        if constexpr (!KS) wait_loads(newer);
     };
-    // MODE bit 4: prefetch the K operands for the next matrix phase at the end of the vector phase
-    auto segment0 = [&](int i0, int i1, auto mode) __attribute__((always_inline)) {  // group 0: slot 2i matrix, slot 2i+1 vector + V(i)
+    // Between slots nothing but the barrier itself: no wavefront writes to LDS in the loop, and the K operands read ahead may
+    // still be on their way (their stage is written two slots later at the earliest).
+    auto slot_end = [&]() __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto segment0 = [&](int i0, int i1, auto mode) __attribute__((always_inline)) {  // group 0: slot 2i matrix + V(i+2), slot 2i+1 vector
         for (int i = i0; i < i1; i++) {
-            matrix_phase(i, mode);
-            lds_barrier();
-            vector_phase(i, i + 1, 2 * i + 1, i + 1, mode);
-            lds_barrier();
+            matrix_phase(i, KS ? 2 * i : i + 2, mode);
+            slot_end();
+            vector_phase(i, i + 1, integral_constant<int, 2 * C::LOADS>{}, mode);
+            slot_end();
         }
     };
-    auto segment1 = [&](int i0, int i1, auto mode) __attribute__((always_inline)) {  // group 1: slot 2i vector (tile i-1) + K(i+1), slot 2i+1 matrix
+    auto segment1 = [&](int i0, int i1, auto mode) __attribute__((always_inline)) {  // group 1: slot 2i vector (tile i-1), slot 2i+1 matrix + K(i+3)
         for (int i = i0; i < i1; i++) {
-            vector_phase(i - 1, i + 2, 2 * i, i, mode);
-            lds_barrier();
-            matrix_phase(i, mode);
-            lds_barrier();
+            vector_phase(i - 1, i, integral_constant<int, C::LOADS>{}, mode);
+            slot_end();
+            matrix_phase(i, KS ? 2 * i + 1 : i + 3, mode);
+            slot_end();
         }
     };
     if (ntiles > 0) {
         if constexpr (KS) {  // what slots -4 .. -1 would have issued
-            if (group == 0) {
-                issue_k(0);
-                issue_k(2);
-                issue_v(0);
-            } else {
-                issue_k(1);
-                issue_k(3);
+#pragma unroll
+            for (int j = 0; j < C::LOADS; j++) {
+                if (group == 0) issue_k(0, j), issue_k(2, j), issue_v(0, j);
+                else issue_k(1, j), issue_k(3, j);
             }
-        } else if (moves_k) {
-            issue_tile(0);
-            issue_tile(1);
         } else {
-            issue_tile(0);
+            load_all(0);
+            load_all(1);
+            if (moves_k) load_all(2);
         }
         if constexpr (FOLD) {
 #pragma unroll
             for (int kb = 0; kb < QD / 16; kb++) qreg[kb] = Mma<T>::scaled(qreg[kb], pw);
         }
-        wait_tiles(integral_constant<int, 0>{});
+        wait_loads(integral_constant<int, 0>{});
         lds_barrier();
         if (group == 0) {
             // iteration i: S^T(i), softmax(i), P.V(i-1)
@@ -596,7 +572,7 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnPara
     }
 
     // the epilogue reuses the tile buffers: no tile load may still be on its way into them
-    wait_tiles(integral_constant<int, 0>{});
+    wait_loads(integral_constant<int, 0>{});
     lds_barrier();
     constexpr int SLICE = 32 * (D * 2 + 16);  // bytes per wavefront of the output transposition below
     if constexpr (KS) {

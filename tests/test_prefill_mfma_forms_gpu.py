@@ -37,3 +37,14 @@ def run(device, dtype, B, H, Hkv, Sq, Skv, D, causal=False):
 def test_grids_of_even_rows_keep_the_256_row_form(device, dtype, D):
     """Eight query blocks per head on more than half of the compute units, every row with the same keys."""
     run(device, dtype, 1, 18, 6, 1801, 333, D)
+
+
+@pytest.mark.parametrize("D", [64, 72, 96, 128])
+@pytest.mark.parametrize("Skv", [1, 63, 65, 128, 129, 192, 193, 257, 320, 321, 449])
+def test_key_counts_around_the_rings_of_tiles(device, D, Skv):
+    """One tile to more than either ring holds (four; five of K in the key-split form), the last one whole, short by a key or a
+    single key.  130 heads give 129 rows to the 256-row form, four heads to the key-split form (from three tiles on)."""
+    run(device, fa.F16, 1, 130, 130, 129, Skv, D)
+    run(device, fa.BF16, 1, 4, 2, 130, Skv, D)
+    if Skv >= 130:
+        run(device, fa.F16, 1, 4, 2, 130, Skv, D, causal=True)
