@@ -19,6 +19,7 @@ missing the import of :func:`lib` raises.
 import ctypes
 import enum
 import os
+import struct
 
 import numpy as np
 
@@ -69,6 +70,14 @@ class CAttnArgs(ctypes.Structure):
                 ("kv_lens", ctypes.c_void_p), ("workspace", ctypes.c_void_p), ("workspace_bytes", ctypes.c_size_t),
                 ("force_kernel", ctypes.c_int32), ("main_kernel_done", ctypes.c_void_p),
                 ("main_kernel_start", ctypes.c_void_p), ("mask_intervals", ctypes.c_void_p)]
+
+
+# The same structures as one pack of their values: a decode step's two calls describe fifteen tensors, and filled field by
+# field through ctypes these descriptors cost the host more than the step costs the GPU (f32, 32/8 heads, 4096 keys: 25.5 us a
+# step, 20.1 packed; a 346-key step in f16 20.0 and 16.1).
+_TENSOR4 = struct.Struct("=QQ4I4q")
+_ATTN_ARGS = struct.Struct("=" + 4 * "QQ4I4q" + "iifi" + "QQ2I2q" + "iiqq" + "QQQ" + "i4x" + "QQQ")
+assert _TENSOR4.size == ctypes.sizeof(CTensor4) and _ATTN_ARGS.size == ctypes.sizeof(CAttnArgs)
 
 
 class CDecodePlanInfo(ctypes.Structure):
@@ -431,8 +440,8 @@ class Tensor:
     def __init__(self, buffer, dtype, shape, strides=None, offset=0):
         self.buffer = buffer
         self.dtype = dtype
-        self.shape = tuple(int(x) for x in shape)
-        self.strides = tuple(int(x) for x in (strides if strides is not None else _contig_strides(self.shape)))
+        self.shape = tuple(map(int, shape))
+        self.strides = tuple(map(int, strides)) if strides is not None else _contig_strides(self.shape)
         self.offset = int(offset)
 
     # -- construction / readback ------------------------------------------------------------------
@@ -442,7 +451,9 @@ class Tensor:
 
     @classmethod
     def empty(cls, device, shape, dtype):
-        n = int(np.prod(shape)) if len(shape) else 1
+        n = 1
+        for x in shape:
+            n *= int(x)
         return cls(Buffer(device, n * _DTYPE_BYTES[dtype]), dtype, shape)
 
     @classmethod
@@ -520,6 +531,10 @@ class Tensor:
 
     def _c4(self):
         assert len(self.shape) == 4
+        try:
+            return CTensor4.from_buffer_copy(_TENSOR4.pack(self.buffer.ptr, self.offset, *self.shape, *self.strides))
+        except (struct.error, TypeError):  # a value beyond its field: reduced to its width below, as ctypes does
+            pass
         t = CTensor4()
         t.ptr = self.buffer.ptr
         t.offset = self.offset
@@ -576,37 +591,46 @@ class Tensor:
         odt = self.dtype if out_dtype is None else out_dtype
         if out is None:
             out = Tensor.empty(self.device, self.shape, odt)  # fresh, contiguous, Q's shape (core :505-507)
-        args = CAttnArgs()
-        args.q, args.k, args.v, args.out = self._c4(), k._c4(), v._c4(), out._c4()
-        args.dtype, args.out_dtype = self.dtype, odt
-        args.scale = float(np.float32(scale))
-        keep = [out]
+        keep, mask_kind, mask_fields, table_ptr = [out], 0, (0, 0, 0, 0, 0, 0), None
         if mask is not None:
             m, kind, *table = mask  # (tensor, kind) or (tensor, kind, MaskIntervals of that tensor)
             if table:
-                args.mask_intervals = table[0].buffer.ptr
+                table_ptr = table[0].buffer.ptr
                 keep.append(table[0])
             if m.device is not self.device:
                 raise AssertionError("Mask must be on the same device as other tensors")  # fusor :64
             if m.dtype != self.dtype:
                 raise InvalidArgument(ERR_INVALID_ARG, "mask must have the element type of q")
-            args.mask = m._c2()
-            args.mask_kind = int(kind)
+            assert len(m.shape) == 2
+            mask_fields, mask_kind = (m.buffer.ptr, m.offset, *m.shape, *m.strides), int(kind)
             keep.append(m)
-        if analytic is not None:
-            if isinstance(analytic, CAnalyticMask):
-                args.analytic = analytic
-            else:
-                causal, off, window = analytic
-                args.analytic.enabled = 1
-                args.analytic.causal = 1 if causal else 0
-                args.analytic.q_pos_offset = int(off)
-                args.analytic.window = int(window or 0)
+        rows_of_mask = (0, 0, 0, 0)
+        if isinstance(analytic, CAnalyticMask):
+            rows_of_mask = (analytic.enabled, analytic.causal, analytic.q_pos_offset, analytic.window)
+        elif analytic is not None:
+            causal, off, window = analytic
+            rows_of_mask = (1, 1 if causal else 0, int(off), int(window or 0))
+        lens_ptr = None
         if kv_lens is not None:
             assert kv_lens.dtype == "i32" and kv_lens.shape == (self.shape[0],)
-            args.kv_lens = kv_lens.buffer.ptr + kv_lens.offset * 4
+            lens_ptr = kv_lens.buffer.ptr + kv_lens.offset * 4
             keep.append(kv_lens)
-        args.force_kernel = int(force_kernel)
+        try:
+            args = CAttnArgs.from_buffer_copy(_ATTN_ARGS.pack(
+                self.buffer.ptr, self.offset, *self.shape, *self.strides, k.buffer.ptr, k.offset, *k.shape, *k.strides,
+                v.buffer.ptr, v.offset, *v.shape, *v.strides, out.buffer.ptr, out.offset, *out.shape, *out.strides,
+                self.dtype, odt, scale, mask_kind, *mask_fields, *rows_of_mask, lens_ptr or 0, 0, 0, int(force_kernel), 0, 0,
+                table_ptr or 0))
+        except (struct.error, TypeError, OverflowError):  # a value beyond its field: see _c4
+            args = CAttnArgs()
+            args.q, args.k, args.v, args.out = self._c4(), k._c4(), v._c4(), out._c4()
+            args.dtype, args.out_dtype = self.dtype, odt
+            args.scale = float(np.float32(scale))
+            if mask is not None:
+                args.mask, args.mask_kind, args.mask_intervals = m._c2(), mask_kind, table_ptr
+            args.analytic = CAnalyticMask(*rows_of_mask)
+            args.kv_lens = lens_ptr
+            args.force_kernel = int(force_kernel)
         args._out_tensor = out
         args._keep = keep
         return args
@@ -739,6 +763,12 @@ class MaskCache:
 
 # ---- KV cache -----------------------------------------------------------------------------------------
 
+def _cache_view(cache, c):
+    """The tensor a CTensor4 that the library filled in describes: a view of `cache`'s memory."""
+    d = _TENSOR4.unpack_from(c)
+    return Tensor(_View(cache.device, d[0], cache), cache.dtype, d[2:6], d[6:10], d[1])
+
+
 class KvCache:
     """fusor::cache::KvCache over device memory (kv_cache.rs:13-68, tensor_cache.rs:9-124)."""
 
@@ -779,11 +809,7 @@ class KvCache:
         ka, va = CTensor4(), CTensor4()
         check(lib().fhip_kv_cache_append(self.handle, self.device.stream, ctypes.byref(ck), ctypes.byref(cv),
                                          ctypes.byref(ka), ctypes.byref(va)))
-
-        def wrap(c):
-            return Tensor(_View(self.device, c.ptr, self), self.dtype, tuple(c.shape), tuple(c.stride), c.offset)
-
-        return wrap(ka), wrap(va)
+        return _cache_view(self, ka), _cache_view(self, va)
 
     def append_rope(self, rope, k, v, start_pos, interleaved=False, k_norm=None):
         """append(rope(k), v) in one pass: the keys are rotated (RopeCache.forward semantics) and both
@@ -801,11 +827,7 @@ class KvCache:
             check(lib().fhip_kv_cache_norm_rope_append(self.handle, self.device.stream, ctypes.byref(cn),
                                                        ctypes.byref(tables), ctypes.byref(ck), ctypes.byref(cv), k.dtype,
                                                        ctypes.byref(ka), ctypes.byref(va)))
-
-        def wrap(c):
-            return Tensor(_View(self.device, c.ptr, self), self.dtype, tuple(c.shape), tuple(c.stride), c.offset)
-
-        return wrap(ka), wrap(va)
+        return _cache_view(self, ka), _cache_view(self, va)
 
 
 def _kv_step(self, rope, q, k, v, start_pos, interleaved=False, q_norm=None, k_norm=None, q_out_dtype=None):
@@ -821,11 +843,7 @@ def _kv_step(self, rope, q, k, v, start_pos, interleaved=False, q_norm=None, k_n
                                               ctypes.byref(kn) if kn is not None else None, ctypes.byref(tables),
                                               ctypes.byref(cq), q.dtype, ctypes.byref(co), q_out.dtype, ctypes.byref(ck),
                                               ctypes.byref(cv), k.dtype, ctypes.byref(ka), ctypes.byref(va)))
-
-    def wrap(c):
-        return Tensor(_View(self.device, c.ptr, self), self.dtype, tuple(c.shape), tuple(c.stride), c.offset)
-
-    return q_out, wrap(ka), wrap(va)
+    return q_out, _cache_view(self, ka), _cache_view(self, va)
 
 
 KvCache.qkv_rope_append = _kv_step
