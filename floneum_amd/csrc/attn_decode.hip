@@ -227,6 +227,7 @@ __device__ __forceinline__ float lpk_sum(float x) {
 
 template <typename T, int LPK, int GT>
 __global__ __launch_bounds__(64 * DEC_WAVES) void decode_vec_kernel(AttnParams p) {
+    request_arguments<AttnParams>();
     constexpr int KPI = 64 / LPK;   // key rows covered by one wavefront load
     constexpr int U = DEC_UNROLL;
     constexpr int DMAX = LPK * 8;
@@ -602,6 +603,7 @@ constexpr int DM_HEADS = 16; // query heads per workgroup (MFMA N dimension)
 // for each block, and each block keeps its own softmax state.
 template <typename T, int D, int WAVES, int CB>
 __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 8 / WAVES) void decode_mfma_kernel(AttnParams p) {
+    request_arguments<AttnParams>();
     typedef typename DecMma<T>::vec8 vec8;
     constexpr int KP = D * 2 + 16;          // K tile row pitch (bytes): rows 4 banks apart
     constexpr int VP = D * 2 + 32;          // V tile row pitch (bytes): rows 8 banks apart
@@ -617,7 +619,7 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 8 / WAVES) void decode_mf
     constexpr int LDS_BYTES = WAVES * WAVE_BYTES > MERGE_BYTES ? WAVES * WAVE_BYTES : MERGE_BYTES;
     __shared__ __attribute__((aligned(16))) char smem[LDS_BYTES];
 
-    const int wave = threadIdx.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // scalar: every loop below is uniform
     const int lane = threadIdx.x & 63;
     const int j = lane & 15;  // column of this lane inside each block
     const int q4 = lane >> 4; // key group
@@ -640,7 +642,8 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 8 / WAVES) void decode_mf
 #pragma unroll
     for (int cb = 0; cb < CB; cb++) {
         const int cj = c0 + min(j + DM_HEADS * cb, nh - 1);
-        hj[cb] = g * p.G + cj / rows, rj[cb] = cj % rows;
+        hj[cb] = g * p.G + cj, rj[cb] = 0;
+        if (rows > 1) hj[cb] = g * p.G + cj / rows, rj[cb] = cj % rows;
     }
 
     int kv_hi = p.Skv;
@@ -715,44 +718,54 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 8 / WAVES) void decode_mf
     using set0 = std::integral_constant<int, 0>;
     using set1 = std::integral_constant<int, DEPTH - 1>;
 
+    // Q^T operand: column j, dims 32 kb + 8 q4 .. +8 (zero for the padding columns)
+    vec8 qreg[CB][KB];
+    auto load_q = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int cb = 0; cb < CB; cb++) {
+            const uint16_t *qp = (const uint16_t *)p.q + b * p.qs[0] + (int64_t)hj[cb] * p.qs[1] + (int64_t)rj[cb] * p.qs[2];
+            const bool qvec = p.qs[3] == 1 && (((uintptr_t)qp) & 15) == 0;
+#pragma unroll
+            for (int kb = 0; kb < KB; kb++) {
+                uint4_t raw = {0, 0, 0, 0};
+                if (j + DM_HEADS * cb < nh) {
+                    if (qvec) {
+                        raw = *(const uint4_t *)(qp + 32 * kb + 8 * q4);
+                    } else {
+                        uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+                        for (int e = 0; e < 8; e++) {
+                            const uint32_t x = qp[(int64_t)(32 * kb + 8 * q4 + e) * p.qs[3]];
+                            w[e >> 1] |= x << ((e & 1) * 16);
+                        }
+                        raw = uint4_t{w[0], w[1], w[2], w[3]};
+                    }
+                }
+                qreg[cb][kb] = __builtin_bit_cast(vec8, raw);
+            }
+        }
+    };
+    // Q before the first tile where a workgroup has a step or two: behind the tile's loads, which wait for the memory of every
+    // other workgroup's, it holds the first products up (32/8 heads, 8000 keys, batch 1: 13.9 -> 13.2 us), and above head_dim
+    // 128, where the CU has no second workgroup to go on with (batch 16, 4001 keys, 256: 50.4 -> 49.9).  Otherwise behind it
+    // (batch 16, 4096 keys, 128: 45.6 -> 45.2).  The eight-wavefront form, whose chunks are long, does not ask (ragged to 32768
+    // keys, 96: 844 us, 855 with the question).
+    const bool q_first = D > 128 || (WAVES == DEC_WAVES && p.chunk <= 2 * WAVES * DM_KEYS);
+    if (q_first) load_q();
     int base = lo_al + wave * DM_KEYS;
-    if (base < hi) {  // issued first so the Q fetch below overlaps them
+    if (base < hi) {
         load_tile(base, set0{});
         if constexpr (DEPTH == 2) load_tile(base + step, set1{});
     }
+    if (!q_first) load_q();
 
-    // Q^T operand: column j, dims 32 kb + 8 q4 .. +8 (zero for the padding columns)
-    vec8 qreg[CB][KB];
-#pragma unroll
-    for (int cb = 0; cb < CB; cb++) {
-        const uint16_t *qp = (const uint16_t *)p.q + b * p.qs[0] + (int64_t)hj[cb] * p.qs[1] + (int64_t)rj[cb] * p.qs[2];
-        const bool qvec = p.qs[3] == 1 && (((uintptr_t)qp) & 15) == 0;
-#pragma unroll
-        for (int kb = 0; kb < KB; kb++) {
-            uint4_t raw = {0, 0, 0, 0};
-            if (j + DM_HEADS * cb < nh) {
-                if (qvec) {
-                    raw = *(const uint4_t *)(qp + 32 * kb + 8 * q4);
-                } else {
-                    uint32_t w[4] = {0, 0, 0, 0};
-#pragma unroll
-                    for (int e = 0; e < 8; e++) {
-                        const uint32_t x = qp[(int64_t)(32 * kb + 8 * q4 + e) * p.qs[3]];
-                        w[e >> 1] |= x << ((e & 1) * 16);
-                    }
-                    raw = uint4_t{w[0], w[1], w[2], w[3]};
-                }
-            }
-            qreg[cb][kb] = __builtin_bit_cast(vec8, raw);
-        }
-    }
 
     // one step: the staged tile `set` (keys base ..) goes to LDS, its registers take the tile DEPTH steps ahead, then the math
     auto one_step = [&](int base, auto set) __attribute__((always_inline)) {
         wave_lds_sync();  // the previous step's LDS reads precede these writes
         store_tile(set);
         wave_lds_sync();
-        load_tile(base + DEPTH * step, set);  // in flight during the math below (beyond the end: a row read again)
+        if (base + DEPTH * step < hi) load_tile(base + DEPTH * step, set);  // in flight during the math below
 
         // ---- S^T[key][col] = K . Q^T : two 16-key tiles, every K operand read serves all column blocks -------
         float4_t s[CB][2];
@@ -865,7 +878,8 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 8 / WAVES) void decode_mf
             L += wgt * src[D + 1];
             A += wgt * src[d];
         }
-        const int h = g * p.G + (c0 + hh) / rows, qr = (c0 + hh) % rows;
+        int h = g * p.G + c0 + hh, qr = 0;
+        if (rows > 1) h = g * p.G + (c0 + hh) / rows, qr = (c0 + hh) % rows;
         if (p.nsplit == 1) {
             const float val = A / L;  // no visible key: 0/0 = NaN like the reference
             const int64_t oi = b * p.os[0] + h * p.os[1] + qr * p.os[2] + d * p.os[3];
@@ -902,6 +916,7 @@ constexpr int DF_KEYS = 16;  // keys per wavefront step
 
 template <int D, int CB>  // CB: 16-column blocks per workgroup, see decode_mfma_kernel
 __global__ __launch_bounds__(64 * DEC_WAVES, D > 128 ? 1 : 2) void decode_mfma_f32_kernel(AttnParams p) {
+    request_arguments<AttnParams>();
     constexpr int KP = D * 4 + 16;             // tile row pitch (bytes): rows 4 banks apart
     constexpr int K_BYTES = DF_KEYS * KP;
     constexpr int WAVE_BYTES = 2 * K_BYTES;    // K tile, V tile
@@ -916,7 +931,7 @@ __global__ __launch_bounds__(64 * DEC_WAVES, D > 128 ? 1 : 2) void decode_mfma_f
     constexpr int LDS_BYTES = DEC_WAVES * WAVE_BYTES > MERGE_BYTES ? DEC_WAVES * WAVE_BYTES : MERGE_BYTES;
     __shared__ __attribute__((aligned(16))) char smem[LDS_BYTES];
 
-    const int wave = threadIdx.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // scalar: every loop below is uniform
     const int lane = threadIdx.x & 63;
     const int j = lane & 15;  // column of this lane inside each block
     const int q4 = lane >> 4; // key group
@@ -937,7 +952,8 @@ __global__ __launch_bounds__(64 * DEC_WAVES, D > 128 ? 1 : 2) void decode_mfma_f
 #pragma unroll
     for (int cb = 0; cb < CB; cb++) {
         const int cj = c0 + min(j + DM_HEADS * cb, nh - 1);
-        hj[cb] = g * p.G + cj / rows, rj[cb] = cj % rows;
+        hj[cb] = g * p.G + cj, rj[cb] = 0;
+        if (rows > 1) hj[cb] = g * p.G + cj / rows, rj[cb] = cj % rows;
     }
 
     int kv_hi = p.Skv;
@@ -1005,35 +1021,43 @@ __global__ __launch_bounds__(64 * DEC_WAVES, D > 128 ? 1 : 2) void decode_mfma_f
         }
     };
 
-    int base = lo_al + wave * DF_KEYS;
-    if (base < hi) load_tile(base);  // issued first so the Q fetch below overlaps it
-
     // Q^T operand: column j, dims 16 c + 4 q4 .. +4 (zero for the padding columns)
     float4_t qreg[CB][KC];
+    auto load_q = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int cb = 0; cb < CB; cb++) {
-        const float *qp = (const float *)p.q + b * p.qs[0] + (int64_t)hj[cb] * p.qs[1] + (int64_t)rj[cb] * p.qs[2];
-        const bool qvec = p.qs[3] == 1 && (((uintptr_t)qp) & 15) == 0;
+        for (int cb = 0; cb < CB; cb++) {
+            const float *qp = (const float *)p.q + b * p.qs[0] + (int64_t)hj[cb] * p.qs[1] + (int64_t)rj[cb] * p.qs[2];
+            const bool qvec = p.qs[3] == 1 && (((uintptr_t)qp) & 15) == 0;
 #pragma unroll
-        for (int c = 0; c < KC; c++) {
-            float4_t v = {0.f, 0.f, 0.f, 0.f};
-            if (j + DM_HEADS * cb < nh) {
-                if (qvec) {
-                    v = *(const float4_t *)(qp + 16 * c + 4 * q4);
-                } else {
+            for (int c = 0; c < KC; c++) {
+                float4_t v = {0.f, 0.f, 0.f, 0.f};
+                if (j + DM_HEADS * cb < nh) {
+                    if (qvec) {
+                        v = *(const float4_t *)(qp + 16 * c + 4 * q4);
+                    } else {
 #pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = qp[(int64_t)(16 * c + 4 * q4 + e) * p.qs[3]];
+                        for (int e = 0; e < 4; e++) v[e] = qp[(int64_t)(16 * c + 4 * q4 + e) * p.qs[3]];
+                    }
                 }
+                qreg[cb][c] = v;
             }
-            qreg[cb][c] = v;
         }
-    }
+    };
+    // Q before the first tile where a workgroup has a step or two: behind the tile's loads, which wait for the memory of every
+    // other workgroup's, it holds the first products up (32/8 heads, 4096 keys, batch 1: 16.1 -> 14.2 us).  Batch 8: 50.7 against
+    // 50.3 us the other way.
+    const bool q_first = p.chunk <= 2 * DEC_WAVES * DF_KEYS;
+    if (q_first) load_q();
+    int base = lo_al + wave * DF_KEYS;
+    if (base < hi) load_tile(base);
+    if (!q_first) load_q();
+
 
     for (; base < hi; base += step) {
         wave_lds_sync();  // the previous step's LDS reads precede these writes
         store_tile();
         wave_lds_sync();
-        load_tile(base + step);  // in flight during the math below (beyond the end: a row read again)
+        if (base + step < hi) load_tile(base + step);  // in flight during the math below
 
         // ---- S^T[key][col] = K . Q^T : every K operand read serves all column blocks ----------------------
         float4_t s[CB];
@@ -1143,7 +1167,8 @@ __global__ __launch_bounds__(64 * DEC_WAVES, D > 128 ? 1 : 2) void decode_mfma_f
             L += wgt * src[D + 1];
             A += wgt * src[d];
         }
-        const int h = g * p.G + (c0 + hh) / rows, qr = (c0 + hh) % rows;
+        int h = g * p.G + c0 + hh, qr = 0;
+        if (rows > 1) h = g * p.G + (c0 + hh) / rows, qr = (c0 + hh) % rows;
         if (p.nsplit == 1) {
             ((float *)p.out)[b * p.os[0] + h * p.os[1] + qr * p.os[2] + d * p.os[3]] = A / L;  // no visible key: 0/0 = NaN
         } else {
@@ -1166,6 +1191,7 @@ __global__ __launch_bounds__(64 * DEC_WAVES, D > 128 ? 1 : 2) void decode_mfma_f
 
 template <typename T, int U>
 __global__ __launch_bounds__(64) void decode_combine_kernel(AttnParams p) {
+    request_arguments<AttnParams>();
     const int qr = blockIdx.x % p.Sq, bh = blockIdx.x / p.Sq;  // one workgroup per (batch, head, query row)
     const int h = bh % p.H, b = bh / p.H;
     const int D = p.D;
@@ -1226,6 +1252,7 @@ __global__ __launch_bounds__(64) void decode_combine_kernel(AttnParams p) {
 // splits (U in flight per lane), and the first folds the four states through LDS.
 template <typename T, int U>
 __global__ __launch_bounds__(256) void decode_combine4_kernel(AttnParams p) {
+    request_arguments<AttnParams>();
     __shared__ float part[4][2 + 128];
     const int qr = blockIdx.x % p.Sq, bh = blockIdx.x / p.Sq;  // one workgroup per (batch, head, query row)
     const int h = bh % p.H, b = bh / p.H;

@@ -57,6 +57,20 @@ __device__ __forceinline__ void pin(V... v) {
     (pin_one(v), ...);
 }
 
+// Requests every 64-byte line of a kernel's arguments at once.  A kernel that reads its arguments where it uses them, between
+// branches, waits for one line after the other, a quarter of a microsecond each: a decode step of one sequence on 4096 keys,
+// two attention kernels of 16 us together, takes 0.7 us less with them requested at the start.
+template <typename... ARGS>
+__device__ __forceinline__ void request_arguments() {
+    constexpr int LINES = (int)((sizeof(ARGS) + ... + 0) + 63) / 64;
+    const auto words = (const __attribute__((address_space(4))) uint32_t *)__builtin_amdgcn_kernarg_segment_ptr();
+    uint32_t first[LINES];
+#pragma unroll
+    for (int i = 0; i < LINES; i++) first[i] = words[16 * i];
+#pragma unroll
+    for (int i = 0; i < LINES; i++) asm volatile("" ::"s"(first[i]));
+}
+
 // Orders this wavefront's LDS writes before its later LDS reads (no workgroup barrier).
 __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
