@@ -300,6 +300,7 @@ __global__ __launch_bounds__(64 * PF32_WAVES, 2) void prefill_f32_kernel(AttnPar
 // scores, in the scores' own units: those rows' sums l are parked with their sign set (-0.0 included).
 template <typename T>
 __global__ __launch_bounds__(256) void prefill_f32_merge_kernel(AttnParams p) {
+    request_arguments<AttnParams>();
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const int64_t rows = (int64_t)p.B * p.H * p.Sq;
@@ -369,6 +370,7 @@ constexpr int PFW_DP = 256, PFW_DH = 128;
 
 template <typename T>
 __global__ __launch_bounds__(64 * PF32_WAVES, 2) void prefill_f32_wide_kernel(AttnParams p, int nqb) {
+    request_arguments<AttnParams, int>();
     constexpr int BM = 64;
     constexpr int KP = PFW_DP * 4 + 16;
     constexpr int K_BYTES = PF32_BN * KP;

@@ -126,6 +126,7 @@ __device__ __forceinline__ float half_swap_sum(float x) {
 // the buffer) and are not written.
 template <typename T, int D, int QD, bool PAD, bool KS>
 __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnParams p, int nqb, int out_vec) {
+    request_arguments<AttnParams, int, int>();
     typedef PfCfg<D, KS> C;
     typedef typename Mma<T>::vec8 vec8;
     constexpr int STAGE = C::STAGE;

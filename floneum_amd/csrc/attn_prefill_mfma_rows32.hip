@@ -100,6 +100,7 @@ __device__ __forceinline__ float r32_half_swap_sum(float x) {
 // file, and the code of the split form costs the unsplit one spills inside its loop).
 template <typename T, bool SPLIT>
 __global__ __launch_bounds__(256, 1) void prefill_mfma_wide_rows32_kernel(AttnParams p, int nqb, int out_vec) {
+    request_arguments<AttnParams, int, int>();
     typedef typename R32Mma<T>::vec8 vec8;
     constexpr int D = R32_D, ROWB = R32_ROWB, KG = R32_KG, VG = R32_VG;
     __shared__ __attribute__((aligned(16))) char smem[R32_LDS_BYTES];

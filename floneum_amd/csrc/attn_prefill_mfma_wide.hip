@@ -81,6 +81,7 @@ __device__ __forceinline__ float pw_quad_sum(float x) {
 // grids that would leave CUs idle; <4, 2> (four wavefronts with the whole register file each) is not launched any more.
 template <typename T, int D, int PW_WAVES, int CB>
 __global__ __launch_bounds__(64 * PW_WAVES, PW_WAVES * CB >= 8 ? 1 : 2) void prefill_mfma_wide_kernel(AttnParams p, int nqb) {
+    request_arguments<AttnParams, int>();
     typedef typename WideMma<T>::vec8 vec8;
     constexpr int KP = D * 2 + 16;           // K tile row pitch (bytes): rows 4 banks apart
     constexpr int VP = D * 2 + 32;           // V tile row pitch (bytes): rows 8 banks apart
