@@ -185,7 +185,9 @@ struct RopeRows {
     int32_t norm_dtype;
     float eps;
     int32_t vec;  // rows and pointers allow the 16-byte forms (set by fill_row_job)
-    int32_t few;  // the wide normalised form with its rows per wavefront block divided by 1 or 4 (set by fill_row_job)
+    int32_t few;  // the wide normalised form with 32 / 16 / 8 rows per wavefront block divided by 2 or 4 (set by fill_row_job)
+    int32_t small;  // rows (and steps of the wide form without a norm) are fewer than 2^31: divided by multiplication
+    uint32_t mul[3], shift[3];  // by shape[2], shape[1] and the wide form's steps per row (mul 0: by 1)
 };
 struct RowJobs {
     RopeRows job[3];

@@ -20,6 +20,8 @@
 //   ss = fold(+, 0, x[i] * x[i]) left to right;  rms = sqrt(ss / D + eps);  n[i] = (x[i] / rms) * w[i] (+ bias[i])
 // and n is rounded to the tensor's element type before the rotation, because the reference's norm returns a
 // tensor of that type.
+#include <stddef.h>
+
 #include "common.h"
 #include "device_utils.h"
 
@@ -47,17 +49,28 @@ __device__ __forceinline__ float round_through(float v, int dtype) {
 // elements on both sides, and a head_dim that is a multiple of 8 (fill_row_job checks; `vec`).
 typedef uint32_t uint2r_t __attribute__((ext_vector_type(2)));
 
-__device__ __forceinline__ float4_t load4_as_f32(const void *p, int64_t idx, int dtype) {
-    if (dtype == FHIP_F32) return *(const float4_t *)((const float *)p + idx);
-    const uint2r_t raw = *(const uint2r_t *)((const uint16_t *)p + idx);
-    float4_t v;
+// Four elements as they lie in memory, and widened: apart, so that a lane's loads are all on their way before it waits for
+// the first.
+template <bool SRC16>
+struct Raw4 {
+    uint4_t w;
+    __device__ __forceinline__ void load(const void *p, int64_t idx) { w = *(const uint4_t *)((const float *)p + idx); }
+    __device__ __forceinline__ float4_t widened(int) const { return __builtin_bit_cast(float4_t, w); }
+};
+template <>
+struct Raw4<true> {
+    uint2r_t w;
+    __device__ __forceinline__ void load(const void *p, int64_t idx) { w = *(const uint2r_t *)((const uint16_t *)p + idx); }
+    __device__ __forceinline__ float4_t widened(int dtype) const {
+        float4_t v;
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const uint16_t bits = (uint16_t)(raw[e >> 1] >> (16 * (e & 1)));
-        v[e] = dtype == FHIP_F16 ? (float)__builtin_bit_cast(half_t, bits) : __uint_as_float((uint32_t)bits << 16);
+        for (int e = 0; e < 4; e++) {
+            const uint16_t bits = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
+            v[e] = dtype == FHIP_F16 ? (float)__builtin_bit_cast(half_t, bits) : __uint_as_float((uint32_t)bits << 16);
+        }
+        return v;
     }
-    return v;
-}
+};
 __device__ __forceinline__ void store4_from_f32(void *p, int64_t idx, int dtype, float4_t v) {
     if (dtype == FHIP_F32) {
         *(float4_t *)((float *)p + idx) = v;
@@ -79,37 +92,55 @@ __device__ __forceinline__ void row_bases(const RopeRows &a, int64_t t, int64_t 
     *db = b * a.ds[0] + h * a.ds[1] + *r * a.ds[2];
 }
 
+// t / d for the divisor whose (mul, shift) the host worked out (fill_row_job): exact for t < 2^31
+__device__ __forceinline__ uint32_t divided(uint32_t t, uint32_t mul, uint32_t shift) { return mul ? __umulhi(t, mul) >> shift : t; }
+__device__ __forceinline__ void row_bases_small(const RopeRows &a, uint32_t t, int64_t *sb, int64_t *db, uint32_t *r) {
+    const uint32_t bh = divided(t, a.mul[0], a.shift[0]), b = divided(bh, a.mul[1], a.shift[1]);
+    const uint32_t h = bh - b * a.shape[1];
+    *r = t - bh * a.shape[2];
+    *sb = b * a.ss[0] + h * a.ss[1] + *r * a.ss[2];
+    *db = b * a.ds[0] + h * a.ds[1] + *r * a.ds[2];
+}
+
 // Rotation / conversion without the norm, four pairs (or four elements) per lane and step: every load and store is
 // 16 bytes of f32 or 8 bytes of a 16-bit type, consecutive lanes take consecutive pieces of a row.
+template <bool SMALL, bool SRC16>
 __device__ __forceinline__ void rope_rows_vec_body(const RopeRows &a) {
     const uint32_t D = a.shape[3], half = D / 2;
     const uint32_t upr = a.mode == 2 ? D / 4 : half / 4;  // steps per row
     const int64_t total = (int64_t)a.shape[0] * a.shape[1] * a.shape[2] * upr;
     for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += (int64_t)gridDim.x * blockDim.x) {
-        const uint32_t j = (uint32_t)(idx % upr);
         int64_t sb, db;
-        uint32_t r;
-        row_bases(a, idx / upr, &sb, &db, &r);
+        uint32_t r, j;
+        if constexpr (SMALL) {
+            const uint32_t row = divided((uint32_t)idx, a.mul[2], a.shift[2]);
+            j = (uint32_t)idx - row * upr;
+            row_bases_small(a, row, &sb, &db, &r);
+        } else {
+            j = (uint32_t)(idx % upr);
+            row_bases(a, idx / upr, &sb, &db, &r);
+        }
+        Raw4<SRC16> p0, p1;
         if (a.mode == 2) {
-            store4_from_f32(a.dst, db + 4 * j, a.dst_dtype, load4_as_f32(a.src, sb + 4 * j, a.src_dtype));
+            p0.load(a.src, sb + 4 * j);
+            store4_from_f32(a.dst, db + 4 * j, a.dst_dtype, p0.widened(a.src_dtype));
             continue;
         }
+        // the pieces of a step: (4j, half + 4j) or, interleaved, (8j, 8j + 4)
+        const uint32_t d0 = a.mode == 0 ? 4 * j : 8 * j, d1 = a.mode == 0 ? half + 4 * j : 8 * j + 4;
+        p0.load(a.src, sb + d0);
+        p1.load(a.src, sb + d1);
         const float4_t c = *(const float4_t *)(a.cos + (a.pos0 + r) * half + 4 * j);
         const float4_t s = *(const float4_t *)(a.sin + (a.pos0 + r) * half + 4 * j);
+        const float4_t xa = p0.widened(a.src_dtype), xb = p1.widened(a.src_dtype);
         float4_t ya, yb;
         if (a.mode == 0) {  // pairs (4j + e, half + 4j + e)
-            const float4_t x0 = load4_as_f32(a.src, sb + 4 * j, a.src_dtype);
-            const float4_t x1 = load4_as_f32(a.src, sb + half + 4 * j, a.src_dtype);
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                ya[e] = __fsub_rn(__fmul_rn(x0[e], c[e]), __fmul_rn(x1[e], s[e]));
-                yb[e] = __fadd_rn(__fmul_rn(x1[e], c[e]), __fmul_rn(x0[e], s[e]));
+                ya[e] = __fsub_rn(__fmul_rn(xa[e], c[e]), __fmul_rn(xb[e], s[e]));
+                yb[e] = __fadd_rn(__fmul_rn(xb[e], c[e]), __fmul_rn(xa[e], s[e]));
             }
-            store4_from_f32(a.dst, db + 4 * j, a.dst_dtype, ya);
-            store4_from_f32(a.dst, db + half + 4 * j, a.dst_dtype, yb);
         } else {  // pairs (8j + 2e, 8j + 2e + 1)
-            const float4_t xa = load4_as_f32(a.src, sb + 8 * j, a.src_dtype);
-            const float4_t xb = load4_as_f32(a.src, sb + 8 * j + 4, a.src_dtype);
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const float x0 = e < 2 ? xa[2 * e] : xb[2 * e - 4], x1 = e < 2 ? xa[2 * e + 1] : xb[2 * e - 3];
@@ -118,165 +149,179 @@ __device__ __forceinline__ void rope_rows_vec_body(const RopeRows &a) {
                 if (e < 2) ya[2 * e] = y0, ya[2 * e + 1] = y1;
                 else yb[2 * e - 4] = y0, yb[2 * e - 3] = y1;
             }
-            store4_from_f32(a.dst, db + 8 * j, a.dst_dtype, ya);
-            store4_from_f32(a.dst, db + 8 * j + 4, a.dst_dtype, yb);
         }
+        store4_from_f32(a.dst, db + d0, a.dst_dtype, ya);
+        store4_from_f32(a.dst, db + d1, a.dst_dtype, yb);
+    }
+}
+__device__ __forceinline__ void rope_rows_vec_any(const RopeRows &a) {
+    const bool src16 = a.src_dtype != FHIP_F32;
+    if (!a.small) {
+        if (src16) rope_rows_vec_body<false, true>(a);
+        else rope_rows_vec_body<false, false>(a);
+    } else {
+        if (src16) rope_rows_vec_body<true, true>(a);
+        else rope_rows_vec_body<true, false>(a);
     }
 }
 
-// The normalised variant on whole row blocks.  The sum of squares of a row is one lane's left-to-right fold (the
-// order fixes the rounding), so a wavefront parks a block of rows in its own LDS tile with wide, consecutive loads
-// (pitch head_dim + 1 floats: the lanes then fold their rows without bank conflicts), every lane that has a row
-// folds it, all lanes normalise and rotate the pairs in place, and the tile leaves with wide stores.  The rows of a
-// block are all read before any is written, so the destination may be the source.
-constexpr int NORM_TILE_FLOATS = 2112;  // per wavefront: 16 rows of head_dim 128, 32 of 64, 8 of 256
+// The normalised variant on whole row blocks.  A lane holds four consecutive elements of a row; the sum of squares of a row
+// is one lane's left-to-right fold (the order fixes the rounding), so the rows also pass through the wavefront's own LDS tile
+// (pitch head_dim + 4 floats: the lanes then fold their rows without bank conflicts, four elements per read).  Every lane that
+// has a row folds it, all lanes normalise what they hold, fetch the other halves of their pairs from the lanes that hold
+// those, rotate and store.  The rows of a block are all read before any is written, so the destination may be the source.
+// Bound: where blocks are few, one block's chain (fetch, fold, divide, store): so everything a block reads, the tables and
+// weights included, is requested before it waits, and row numbers are divided by multiplication.  Where they are many,
+// wavefronts per SIMD: with 32 / 16 / 8 rows per block a wavefront holds 200 registers, two to a SIMD, and 1500 rows of 32/8
+// heads at 128 take 29.9 us; with half of them 128 registers, four to a SIMD, 22.5 (25.0 with a quarter and 80 registers).
+// The launch of q, k and v (f32, or 16-bit where said), this form and one that rotated pairs through the tile with twice the
+// rows per block: 31 rows of 16/4 heads at 64 6.7 -> 5.3 us, 512 rows of 32/8 at 64 8.2 -> 7.6, 300 of 16/4 at 128 8.6 -> 7.2,
+// 700 of 32/8 at 64 in f16 12.7 -> 8.9, 1500 of 32/8 at 128 29.4 -> 22.5.  Quotients by the row's reciprocal and two corrections
+// instead of divisions gave nothing.
+constexpr int NORM_TILE_FLOATS = 1088;  // per wavefront: 16 rows of head_dim 64, 8 of 128, 4 of 256
 struct NormWaveLds {
     float tile[NORM_TILE_FLOATS];
-    int64_t sb[64], db[64];  // element offsets of the block's rows in the source and the destination
-    uint32_t pos[64];        // their positions (rows of the cos / sin tables, before pos0)
-    float rms[64];
+    int64_t sb[32], db[32];  // element offsets of the block's rows in the source and the destination
+    uint32_t pos[32];        // their positions (rows of the cos / sin tables, before pos0)
+    float rms[32];
 };
-// FEW: the block's rows divided by FEW (1 or 4: down to 8 / 4 / 2 rows at head_dim 64 / 128 / 256), for inputs whose
-// blocks of the full size would leave most SIMDs with one wavefront or none: a block's stages (fetch, fold, normalise,
-// store) run one after the other, so a prompt of a few hundred rows is bound by one block's latencies, not by the
-// arithmetic.
-template <int D, int FEW>
+// value of x in the lane that holds the other half of this lane's pairs: CPR / 2 lanes away within the row's CPR lanes
+template <int CPR>
+__device__ __forceinline__ float other_half(float x) {
+    const uint32_t u = __float_as_uint(x);
+    if constexpr (CPR == 16) {
+        return __uint_as_float(__builtin_amdgcn_update_dpp(0u, u, 0x128, 0xf, 0xf, true));  // row_ror:8
+    } else if constexpr (CPR == 32) {
+        const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+        return __uint_as_float((threadIdx.x & 16) ? r[0] : r[1]);
+    } else {
+        const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        return __uint_as_float((threadIdx.x & 32) ? r[0] : r[1]);
+    }
+}
+// FEW: 32 / 16 / 8 rows at head_dim 64 / 128 / 256 divided by 2, or by 4 for inputs whose larger blocks would leave most SIMDs
+// with one wavefront or none.
+template <int D, int FEW, bool SRC16>
 __device__ __forceinline__ void norm_rope_rows_vec_body(const RopeRows &a, NormWaveLds *w) {
-    constexpr int HALF = D / 2, CPR = D / 4, P = D + 1;
+    constexpr int HALF = D / 2, CPR = D / 4, P = D + 4;
     static_assert(CPR <= 64 && 64 % CPR == 0 && D % 64 == 0, "head_dim 64, 128 or 256");
-    // A wavefront step moves RS rows: lane -> (row SUB of the step, 16-byte piece C4 of the row).  The pairs of a row
-    // likewise: lane -> (row psub of the step, pair pi), PP steps per row beyond 64 pairs.  A block is LSTEPS load
-    // steps = PSTEPS pair steps, all requested before the first is parked.
+    // A wavefront step moves RS rows: lane -> (row SUB of the step, 16-byte piece C4 of the row).  A block is STEPS steps.
     constexpr int RS = 64 / CPR;
-    constexpr int PRS = HALF <= 64 ? 64 / HALF : 1, PP = HALF <= 64 ? 1 : HALF / 64;
     constexpr int RPW = (D == 64 ? 32 : D == 128 ? 16 : 8) / FEW;  // rows per block
-    constexpr int LSTEPS = RPW / RS, PSTEPS = RPW * PP / PRS;
+    constexpr int STEPS = RPW / RS;
     static_assert(RPW * P <= NORM_TILE_FLOATS, "tile");
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwave = blockDim.x >> 6;
     float *tile = w->tile;
     const int sub = lane / CPR, c4 = lane % CPR;
-    const int psub = HALF <= 64 ? lane / HALF : 0, pi = HALF <= 64 ? lane % HALF : lane;
     const int64_t rows = (int64_t)a.shape[0] * a.shape[1] * a.shape[2];
     const int64_t nblk = (rows + RPW - 1) / RPW;
-    // weights (and bias) of this lane's pairs: the same for every row
-    float w0[PP], w1[PP], b0[PP], b1[PP];
-#pragma unroll
-    for (int k = 0; k < PP; k++) {
-        const int i = pi + 64 * k;
-        const int d0 = a.mode == 0 ? i : 2 * i, d1 = a.mode == 0 ? i + HALF : 2 * i + 1;
-        w0[k] = load_as_f32(a.norm_w, d0, a.norm_dtype), w1[k] = load_as_f32(a.norm_w, d1, a.norm_dtype);
-        b0[k] = a.norm_b ? load_as_f32(a.norm_b, d0, a.norm_dtype) : 0.0f;
-        b1[k] = a.norm_b ? load_as_f32(a.norm_b, d1, a.norm_dtype) : 0.0f;
-    }
-    const bool small = rows < (int64_t)0x7fffffff;
+    // cos and sin of this lane's elements: of pairs 4 c4 .. + 3 (halves: of the piece's place in its half), or of its two pairs
+    const int ti = a.mode == 0 ? 4 * (c4 % (CPR / 2)) : 2 * c4;
     for (int64_t blk = (int64_t)blockIdx.x * nwave + wave; blk < nblk; blk += (int64_t)gridDim.x * nwave) {
         const int64_t row0 = blk * RPW;
         const int nrow = (int)min((int64_t)RPW, rows - row0);
-        if (lane < nrow) {
+        if (lane < RPW) {
+            const int64_t row = row0 + min(lane, nrow - 1);  // (lanes beyond the last row repeat it; nothing of theirs is stored)
             int64_t sb, db;
             uint32_t r;
-            if (small) {  // 32-bit divisions
-                uint32_t t = (uint32_t)(row0 + lane);
-                r = t % a.shape[2];
-                t /= a.shape[2];
-                const uint32_t h = t % a.shape[1], b = t / a.shape[1];
-                sb = b * a.ss[0] + h * a.ss[1] + r * a.ss[2];
-                db = b * a.ds[0] + h * a.ds[1] + r * a.ds[2];
-            } else {
-                row_bases(a, row0 + lane, &sb, &db, &r);
-            }
+            if (a.small) row_bases_small(a, (uint32_t)row, &sb, &db, &r);
+            else row_bases(a, row, &sb, &db, &r);
             w->sb[lane] = sb, w->db[lane] = db, w->pos[lane] = r;
         }
         wave_lds_sync();
-        float4_t x[LSTEPS];
+        Raw4<SRC16> raw[STEPS];
+        float4_t tc[STEPS], ts[STEPS];
 #pragma unroll
-        for (int u = 0; u < LSTEPS; u++) {
+        for (int u = 0; u < STEPS; u++) {
             const int lr = u * RS + sub;
-            if (lr < nrow) x[u] = load4_as_f32(a.src, w->sb[lr] + 4 * c4, a.src_dtype);
-        }
-        float tc[PSTEPS], ts[PSTEPS];
-#pragma unroll
-        for (int q = 0; q < PSTEPS; q++) {
-            const int lr = PP == 1 ? q * PRS + psub : q / PP;
-            const int i = pi + 64 * (q % PP);
-            tc[q] = 1.0f, ts[q] = 0.0f;
-            if (a.mode != 2 && lr < nrow) {
-                const int64_t ti = (a.pos0 + w->pos[lr]) * HALF + i;
-                tc[q] = a.cos[ti], ts[q] = a.sin[ti];
+            raw[u].load(a.src, w->sb[lr] + 4 * c4);
+            tc[u] = float4_t{1.0f, 1.0f, 1.0f, 1.0f}, ts[u] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            const int64_t at = (a.pos0 + w->pos[lr]) * HALF + ti;
+            if (a.mode == 0) {
+                tc[u] = *(const float4_t *)(a.cos + at), ts[u] = *(const float4_t *)(a.sin + at);
+            } else if (a.mode == 1) {
+                tc[u][0] = a.cos[at], tc[u][1] = a.cos[at + 1], ts[u][0] = a.sin[at], ts[u][1] = a.sin[at + 1];
             }
         }
+        // weights (and bias) of this lane's elements: the same for every row
+        float4_t wt, bias = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int u = 0; u < LSTEPS; u++) {
-            const int lr = u * RS + sub;
-            if (lr < nrow) {
+        for (int e = 0; e < 4; e++) wt[e] = load_as_f32(a.norm_w, 4 * c4 + e, a.norm_dtype);
+        if (a.norm_b) {
 #pragma unroll
-                for (int e = 0; e < 4; e++) tile[lr * P + 4 * c4 + e] = x[u][e];
-            }
+            for (int e = 0; e < 4; e++) bias[e] = load_as_f32(a.norm_b, 4 * c4 + e, a.norm_dtype);
+        }
+        float4_t x[STEPS];
+#pragma unroll
+        for (int u = 0; u < STEPS; u++) {
+            x[u] = raw[u].widened(a.src_dtype);
+            *(float4_t *)(tile + (u * RS + sub) * P + 4 * c4) = x[u];
         }
         wave_lds_sync();
-        if (lane < nrow) {
+        if (lane < RPW) {
             float ss = 0.0f;
 #pragma unroll 2
-            for (int i = 0; i < D; i += 8) {  // eight values requested before the dependent chain consumes them
-                float v[8];
+            for (int i = 0; i < D; i += 16) {  // sixteen values requested before the dependent chain consumes them
+                float4_t v[4];
 #pragma unroll
-                for (int e = 0; e < 8; e++) v[e] = tile[lane * P + i + e];
+                for (int e = 0; e < 4; e++) v[e] = *(const float4_t *)(tile + lane * P + i + 4 * e);
 #pragma unroll
-                for (int e = 0; e < 8; e++) ss = __fadd_rn(ss, __fmul_rn(v[e], v[e]));
+                for (int e = 0; e < 16; e++) ss = __fadd_rn(ss, __fmul_rn(v[e >> 2][e & 3], v[e >> 2][e & 3]));
             }
             // sqrtf is the correctly rounded root (the __fsqrt_rn intrinsic is the 1-ulp hardware approximation here)
             w->rms[lane] = sqrtf(__fadd_rn(__fdiv_rn(ss, (float)D), a.eps));
         }
         wave_lds_sync();
-        // a pair: normalise both elements, round to the tensor's type as the reference's norm does, rotate
+        // normalise, round to the tensor's type as the reference's norm does, rotate
 #pragma unroll
-        for (int q = 0; q < PSTEPS; q++) {
-            const int lr = PP == 1 ? q * PRS + psub : q / PP;
-            const int k = q % PP, i = pi + 64 * k;
-            if (lr >= nrow) continue;
-            const int d0 = a.mode == 0 ? i : 2 * i, d1 = a.mode == 0 ? i + HALF : 2 * i + 1;
-            const float rms = w->rms[lr];
-            float x0 = __fmul_rn(__fdiv_rn(tile[lr * P + d0], rms), w0[k]);
-            float x1 = __fmul_rn(__fdiv_rn(tile[lr * P + d1], rms), w1[k]);
-            if (a.norm_b) {
-                x0 = __fadd_rn(x0, b0[k]);
-                x1 = __fadd_rn(x1, b1[k]);
-            }
-            x0 = round_through(x0, a.src_dtype);
-            x1 = round_through(x1, a.src_dtype);
-            float y0 = x0, y1 = x1;
-            if (a.mode != 2) {
-                y0 = __fsub_rn(__fmul_rn(x0, tc[q]), __fmul_rn(x1, ts[q]));
-                y1 = a.mode == 0 ? __fadd_rn(__fmul_rn(x1, tc[q]), __fmul_rn(x0, ts[q]))
-                                 : __fadd_rn(__fmul_rn(x0, ts[q]), __fmul_rn(x1, tc[q]));
-            }
-            tile[lr * P + d0] = y0;
-            tile[lr * P + d1] = y1;
-        }
-        wave_lds_sync();
-#pragma unroll
-        for (int u = 0; u < LSTEPS; u++) {
+        for (int u = 0; u < STEPS; u++) {
             const int lr = u * RS + sub;
-            if (lr < nrow) {
-                float4_t y;
+            const float rms = w->rms[lr];
+            float4_t n, y;
 #pragma unroll
-                for (int e = 0; e < 4; e++) y[e] = tile[lr * P + 4 * c4 + e];
-                store4_from_f32(a.dst, w->db[lr] + 4 * c4, a.dst_dtype, y);
+            for (int e = 0; e < 4; e++) {
+                n[e] = __fmul_rn(__fdiv_rn(x[u][e], rms), wt[e]);
+                if (a.norm_b) n[e] = __fadd_rn(n[e], bias[e]);
+                n[e] = round_through(n[e], a.src_dtype);
             }
+            if (a.mode == 2) {
+                y = n;
+            } else if (a.mode == 0) {
+                const bool upper = c4 >= CPR / 2;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float o = other_half<CPR>(n[e]);
+                    const float own = __fmul_rn(n[e], tc[u][e]), cross = __fmul_rn(o, ts[u][e]);
+                    y[e] = upper ? __fadd_rn(own, cross) : __fsub_rn(own, cross);
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 2; e++) {
+                    const float x0 = n[2 * e], x1 = n[2 * e + 1];
+                    y[2 * e] = __fsub_rn(__fmul_rn(x0, tc[u][e]), __fmul_rn(x1, ts[u][e]));
+                    y[2 * e + 1] = __fadd_rn(__fmul_rn(x0, ts[u][e]), __fmul_rn(x1, tc[u][e]));
+                }
+            }
+            if (lr < nrow) store4_from_f32(a.dst, w->db[lr] + 4 * c4, a.dst_dtype, y);
         }
-        wave_lds_sync();  // the tile and the row tables are rewritten by the next block
+        wave_lds_sync();  // the tile is rewritten by the next block
     }
 }
+template <int FEW, bool SRC16>
+__device__ __forceinline__ void norm_rope_rows_vec_dims(const RopeRows &a, NormWaveLds *w) {
+    if (a.shape[3] == 128) norm_rope_rows_vec_body<128, FEW, SRC16>(a, w);
+    else if (a.shape[3] == 256) norm_rope_rows_vec_body<256, FEW, SRC16>(a, w);
+    else norm_rope_rows_vec_body<64, FEW, SRC16>(a, w);
+}
 __device__ __forceinline__ void norm_rope_rows_vec_any(const RopeRows &a, NormWaveLds *w) {
+    const bool src16 = a.src_dtype != FHIP_F32;
     if (a.few == 4) {
-        if (a.shape[3] == 128) norm_rope_rows_vec_body<128, 4>(a, w);
-        else if (a.shape[3] == 256) norm_rope_rows_vec_body<256, 4>(a, w);
-        else norm_rope_rows_vec_body<64, 4>(a, w);
-        return;
+        if (src16) norm_rope_rows_vec_dims<4, true>(a, w);
+        else norm_rope_rows_vec_dims<4, false>(a, w);
+    } else {
+        if (src16) norm_rope_rows_vec_dims<2, true>(a, w);
+        else norm_rope_rows_vec_dims<2, false>(a, w);
     }
-    if (a.shape[3] == 128) norm_rope_rows_vec_body<128, 1>(a, w);
-    else if (a.shape[3] == 256) norm_rope_rows_vec_body<256, 1>(a, w);
-    else norm_rope_rows_vec_body<64, 1>(a, w);
 }
 
 // The general form of the normalised variant (any strides): a workgroup takes groups of rows; one lane per row folds the squares in the
@@ -338,7 +383,7 @@ __device__ __forceinline__ void norm_rope_rows_body(const RopeRows &a, float *rm
     }
 }
 
-__global__ __launch_bounds__(256, 2) void norm_rope_rows_kernel(RopeRows a) {
+__global__ __launch_bounds__(256, 4) void norm_rope_rows_kernel(RopeRows a) {
     __shared__ NormWaveLds lds[4];
     __shared__ float rms_of[NORM_ROPE_MAX_ROWS];
     if (a.vec) norm_rope_rows_vec_any(a, &lds[threadIdx.x >> 6]);
@@ -376,21 +421,23 @@ __device__ __forceinline__ void rope_rows_body(const RopeRows &a) {
 }
 
 __global__ __launch_bounds__(256) void rope_rows_kernel(RopeRows a) {
-    if (a.vec) rope_rows_vec_body(a);
+    if (a.vec) rope_rows_vec_any(a);
     else rope_rows_body(a);
 }
 
 // Several row jobs in one launch (blockIdx.y picks the job): the rotation of q, the rotated keys and the values of
 // one decode step are three tiny jobs whose launch cost exceeds their run time.
-__global__ __launch_bounds__(256, 2) void row_jobs_kernel(RowJobs js) {
+__global__ __launch_bounds__(256, 4) void row_jobs_kernel(RowJobs js) {
     __shared__ NormWaveLds lds[4];
     __shared__ float rms_of[NORM_ROPE_MAX_ROWS];
-    const RopeRows &a = js.job[blockIdx.y];
+    // (by way of the arguments' own address: the compiler would copy a struct that it indexes to the stack)
+    static_assert(offsetof(RowJobs, job) == 0, "the jobs come first");
+    const RopeRows &a = *(const RopeRows *)((const __attribute__((address_space(4))) RopeRows *)__builtin_amdgcn_kernarg_segment_ptr() + blockIdx.y);
     if (a.norm_w) {
         if (a.vec) norm_rope_rows_vec_any(a, &lds[threadIdx.x >> 6]);
         else norm_rope_rows_body(a, rms_of);
     } else {
-        if (a.vec) rope_rows_vec_body(a);
+        if (a.vec) rope_rows_vec_any(a);
         else rope_rows_body(a);
     }
 }
@@ -430,12 +477,23 @@ void fill_row_job(RopeRows *out, const void *src, const int64_t ss[4], fhip_dtyp
     a.vec = D % 8 == 0 && D >= 8 && wide(src, ss, src_dtype) && wide(dst, ds, dst_dtype) &&
             (mode == 2 || (((uintptr_t)cos % 16) == 0 && ((uintptr_t)sin % 16) == 0));
     if (a.norm_w && !(D == 64 || D == 128 || D == 256)) a.vec = 0;  // the head dims the wide normalised form is built for
-    // fewer than two full-size blocks per SIMD of a 256-CU chip: a quarter of the rows per block, four times the blocks
+    // Division by multiplication: with 2^(l - 1) < d <= 2^l and mul = floor(2^(31 + l) / d) + 1 (below 2^32), mul d is 2^(31 + l)
+    // and at most d <= 2^l more, so t mul / 2^(31 + l) is t / d and less than 1 / d more for t < 2^31.
+    const uint32_t divisors[3] = {shape[2], shape[1], mode == 2 ? D / 4 : D / 8};
+    for (int i = 0; i < 3; i++) {
+        const uint32_t d = divisors[i];
+        int l = 0;
+        while (l < 32 && ((uint64_t)1 << l) < d) l++;
+        a.mul[i] = d > 1 && l < 32 ? (uint32_t)(((uint64_t)1 << (31 + l)) / d + 1) : 0;
+        a.shift[i] = l > 0 ? l - 1 : 0;
+    }
+    const unsigned __int128 steps = (unsigned __int128)shape[0] * shape[1] * shape[2] * (norm ? 1 : divisors[2] ? divisors[2] : 1);
+    a.small = steps < (1u << 31);
+    // Rows per block (see norm_rope_rows_vec_body): a quarter of 32 / 16 / 8 below four of the larger blocks per SIMD of a 256-CU
+    // chip, where the launch ends with the last block's chain.
     const int64_t rows = (int64_t)shape[0] * shape[1] * shape[2];
     const int64_t full = D == 64 ? 32 : D == 128 ? 16 : 8;
-    // a quarter of the rows per block below 2048 full blocks (an eighth measured slower: 33.8 against 31.9 us on a
-    // 512-token prompt step whose full blocks took 35.9 us)
-    a.few = a.norm_w && a.vec && rows < 2048 * full ? 4 : 1;
+    a.few = a.norm_w && a.vec && rows < 2048 * full ? 4 : 2;
 }
 
 // rows per wavefront block of the wide normalised form (RPW in norm_rope_rows_vec_body)
