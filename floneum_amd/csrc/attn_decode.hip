@@ -50,6 +50,9 @@ static int decode_gt(int G, int D, bool f32) {
     return G <= 1 ? 1 : G <= 2 ? 2 : G <= 4 ? 4 : 8;
 }
 
+// whether the f32 matrix-core variant sums a step's keys on their own, see there
+static constexpr bool df_shares(int D, int column_blocks) { return column_blocks == 1 && D <= 192; }
+
 void decode_plan(int B, int Hkv, int G, int Skv, int D, int compute_units, bool ragged, bool f32, int *chunk,
                  int *nsplit, int *waves) {
     const int gt = decode_gt(G, D, f32);
@@ -104,8 +107,32 @@ void decode_plan(int B, int Hkv, int G, int Skv, int D, int compute_units, bool 
     if (ns < 1 || (Skv <= 256 && decode_use_mfma(D, f32, G))) ns = 1;
     long c = (Skv + ns - 1) / ns;
     c = (c + step_keys - 1) / step_keys * step_keys;  // whole workgroup steps
+    long n = (Skv + c - 1) / c;
+    // Fewer, longer chunks where the workgroups would need a further round for the last few of them: the chip runs rounds of
+    // `target` workgroups that all take as long as their chunk and about 100 keys more.  Taken where that is shorter by a
+    // twelfth and the call's workspace does not grow (us a step, before and after: f16, 16 sequences of 32/8 heads at 128, 4104
+    // keys 56.5 -> 47.3, 6000 72.4 -> 64.9, 8200 91 -> 88; bf16, 20 of 16/4 at 256, 4001 keys 81 -> 60; f16, 14 of 16/4 at 256,
+    // two rows on 4647 keys 71 -> 56; f32, 20 of 32/8 at 128, 4500 keys 135 -> 120).  Not for calls with per-sequence lengths,
+    // whose workgroups are uneven anyway (f32, 16 sequences of up to 13172 keys 254 -> 332), nor where two workgroups share a CU
+    // and the chunks are as long as they were asked to be: such calls share their plan with those.  Nor for f32 calls on the
+    // kernels that round once per four keys, where longer sums lose precision (9 sequences at 128: 2.36e-7 -> 2.53e-7 against
+    // 64 bits; 1.50e-7 as it is).
+    const bool asked = wgs_per_cu > 1 && ns_min <= (target + units - 1) / units;
+    if (!ragged && !asked && (!f32 || (decode_use_mfma(D, true, G) && df_shares(D, gt / 16)))) {
+        auto rounds_time = [&](long splits, long keys) { return (units * splits + target - 1) / target * (keys + 100); };
+        const size_t bytes = decode_workspace_bytes(B, Hkv * G, Hkv, D, (int)n);
+        const long time = rounds_time(n, c);
+        long best = time;
+        for (long k = n - 1; k >= 2; k--) {
+            const long kc = ((Skv + k - 1) / k + step_keys - 1) / step_keys * step_keys, kn = (Skv + kc - 1) / kc;
+            if (kc > 4 * max_chunk) break;
+            const long t = rounds_time(kn, kc);
+            if (kn >= 2 && 12 * t < 11 * time && t < best && decode_workspace_bytes(B, Hkv * G, Hkv, D, (int)kn) <= bytes)
+                best = t, n = kn, c = kc;
+        }
+    }
     *chunk = (int)c;
-    *nsplit = (int)((Skv + c - 1) / c);
+    *nsplit = (int)n;
 }
 
 // Workspace: the partials, B * H * nsplit * (D + 2) floats (H counts (head, row) pairs), plus what the fused merge adds:
@@ -1105,29 +1132,36 @@ __global__ __launch_bounds__(64 * DEC_WAVES, D > 128 ? 1 : 2) void decode_mfma_f
                     for (int r = 0; r < 4; r++) o[cb][nb][e][r] *= corr;
         }
 
-        // ---- O^T[dim][col] += V^T . P^T : step ks contracts the keys 4 q4 + ks ----------------------------
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++) {
+        // ---- O^T[dim][col] += V^T . P^T : step ks contracts the keys 4 q4 + ks.  The 16 keys' share forms on its own and is
+        // added once: one rounding at the size of the sum instead of four (4096 keys at 128 against 64 bits 2.4e-7 -> 1.5e-7;
+        // no slower, but for 1 % above head_dim 192 and 70 spilled registers with two column blocks).
+        typedef float vrow_t __attribute__((ext_vector_type(VW)));
+        if constexpr (df_shares(D, CB)) {
 #pragma unroll
             for (int nb = 0; nb < NBLK; nb++) {
-                const int voff = K_BYTES + (4 * q4 + ks) * KP + (16 * VW * nb + VW * j) * 4;
-                if constexpr (VW == 4) {
-                    const float4_t a = *DLDS_PTR(float4_t, voff);
+                vrow_t a[4];
 #pragma unroll
-                    for (int cb = 0; cb < CB; cb++)
+                for (int ks = 0; ks < 4; ks++) a[ks] = *DLDS_PTR(vrow_t, K_BYTES + (4 * q4 + ks) * KP + (16 * VW * nb + VW * j) * 4);
 #pragma unroll
-                        for (int e = 0; e < 4; e++)
-                            o[cb][nb][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], pe[cb][ks], o[cb][nb][e], 0, 0, 0);
-                } else {
-                    typedef float float2v_t __attribute__((ext_vector_type(2)));
-                    const float2v_t a = *DLDS_PTR(float2v_t, voff);
+                for (int e = 0; e < VW; e++) {
+                    float4_t share = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                    for (int cb = 0; cb < CB; cb++)
-#pragma unroll
-                        for (int e = 0; e < 2; e++)
-                            o[cb][nb][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], pe[cb][ks], o[cb][nb][e], 0, 0, 0);
+                    for (int ks = 0; ks < 4; ks++) share = __builtin_amdgcn_mfma_f32_16x16x4f32(a[ks][e], pe[0][ks], share, 0, 0, 0);
+                    o[0][nb][e] += share;
                 }
             }
+        } else {
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++)
+#pragma unroll
+                for (int nb = 0; nb < NBLK; nb++) {
+                    const vrow_t a = *DLDS_PTR(vrow_t, K_BYTES + (4 * q4 + ks) * KP + (16 * VW * nb + VW * j) * 4);
+#pragma unroll
+                    for (int cb = 0; cb < CB; cb++)
+#pragma unroll
+                        for (int e = 0; e < VW; e++)
+                            o[cb][nb][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], pe[cb][ks], o[cb][nb][e], 0, 0, 0);
+                }
         }
     }
 
