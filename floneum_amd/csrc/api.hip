@@ -770,6 +770,18 @@ int fhip_flash_attention_select(const fhip_attn_args *args, int32_t *kernel_id) 
     return rc;
 }
 
+// Workspace of a split-KV decode call: what it reports, and what it writes to (no more than that).
+static void decode_call_bytes(const fhip_attn_args *args, int32_t compute_units, size_t *reported, size_t *used) {
+    const int B = (int)args->q.shape[0], H = (int)args->q.shape[1], rows = (int)args->q.shape[2], D = (int)args->q.shape[3];
+    const int Hkv = (int)args->k.shape[1];
+    int chunk, nsplit, waves, workspace_splits, lo0, len;
+    decode_visible_range(args, &lo0, &len);
+    decode_plan(B, Hkv, H / Hkv * rows, len, D, compute_units > 0 ? compute_units : 256, args->kv_lens != nullptr,
+                args->dtype == FHIP_F32, &chunk, &nsplit, &waves, &workspace_splits);
+    if (reported) *reported = decode_workspace_bytes(B, H * rows, Hkv, D, workspace_splits);
+    if (used) *used = decode_workspace_bytes(B, H * rows, Hkv, D, nsplit);
+}
+
 int fhip_flash_attention_workspace_bytes(const fhip_attn_args *args, int32_t compute_units, size_t *bytes) {
     if (!bytes) {
         set_error("bytes is NULL");
@@ -797,17 +809,7 @@ int fhip_flash_attention_workspace_bytes(const fhip_attn_args *args, int32_t com
                                                          (int)args->q.shape[3], ns);
         if (part) *bytes = f32_partials_offset(args) + part;
     }
-    if (id == FHIP_KERNEL_DECODE_SPLITKV) {
-        int chunk, nsplit, waves;
-        const int B = (int)args->q.shape[0], H = (int)args->q.shape[1], D = (int)args->q.shape[3];
-        const int Hkv = (int)args->k.shape[1], Skv = (int)args->k.shape[2], rows = (int)args->q.shape[2];
-        int lo0, len;
-        decode_visible_range(args, &lo0, &len);
-        (void)Skv;
-        decode_plan(B, Hkv, H / Hkv * rows, len, D, compute_units > 0 ? compute_units : 256, args->kv_lens != nullptr,
-                    args->dtype == FHIP_F32, &chunk, &nsplit, &waves);
-        *bytes = decode_workspace_bytes(B, H * rows, Hkv, D, nsplit);
-    }
+    if (id == FHIP_KERNEL_DECODE_SPLITKV) decode_call_bytes(args, compute_units, bytes, nullptr);
     return FHIP_OK;
 }
 
@@ -823,8 +825,9 @@ static void plan_decode_call(fhip_device *dev, const fhip_attn_args *args, AttnP
         p->Skv = vis_len;
         p->q_pos_offset -= lo0;
     }
+    int workspace_splits;
     decode_plan(p->B, p->Hkv, p->G * p->Sq, p->Skv, p->D, dev->prop.multiProcessorCount, p->kv_lens != nullptr,
-                args->dtype == FHIP_F32, &p->chunk, &p->nsplit, &p->dec_waves);
+                args->dtype == FHIP_F32, &p->chunk, &p->nsplit, &p->dec_waves, &workspace_splits);
     int stride;
     size_t ctr_off;
     p->dec_fused = 0;
@@ -1113,6 +1116,7 @@ int fhip_flash_attention_noalloc(fhip_stream *s, const fhip_attn_args *args) {
     if (rc) return rc;
     if ((id == FHIP_KERNEL_PREFILL_MFMA || id == FHIP_KERNEL_PREFILL_F32) && !output_is_empty(args) && !no_keys(args))
         need = mask_scratch_bytes(args);
+    if (id == FHIP_KERNEL_DECODE_SPLITKV && need > 0) decode_call_bytes(args, s->dev->prop.multiProcessorCount, nullptr, &need);
     if (need > STATIC_WORKSPACE_BYTES) {
         set_error("this call needs a workspace of %zu bytes; fhip_flash_attention_noalloc holds %zu (use "
                   "fhip_flash_attention with a workspace of your own)", need, STATIC_WORKSPACE_BYTES);

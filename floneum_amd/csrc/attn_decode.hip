@@ -54,7 +54,7 @@ static int decode_gt(int G, int D, bool f32) {
 static constexpr bool df_shares(int D, int column_blocks) { return column_blocks == 1 && D <= 192; }
 
 void decode_plan(int B, int Hkv, int G, int Skv, int D, int compute_units, bool ragged, bool f32, int *chunk,
-                 int *nsplit, int *waves) {
+                 int *nsplit, int *waves, int *workspace_splits) {
     const int gt = decode_gt(G, D, f32);
     const int hb = (G + gt - 1) / gt;
     const long units = (long)B * Hkv * hb;
@@ -67,7 +67,7 @@ void decode_plan(int B, int Hkv, int G, int Skv, int D, int compute_units, bool 
         if (units >= compute_units) {
             *waves = 8;
             *chunk = 2048;
-            *nsplit = (Skv + 2047) / 2048;
+            *nsplit = *workspace_splits = (Skv + 2047) / 2048;
             return;
         }
         const long ns = compute_units / units;  // >= 1
@@ -75,7 +75,7 @@ void decode_plan(int B, int Hkv, int G, int Skv, int D, int compute_units, bool 
         if (G > 8 && c >= 2048) {
             *waves = 8;
             *chunk = (int)c;
-            *nsplit = (int)((Skv + c - 1) / c);
+            *nsplit = *workspace_splits = (int)((Skv + c - 1) / c);
             return;
         }
     }
@@ -108,6 +108,9 @@ void decode_plan(int B, int Hkv, int G, int Skv, int D, int compute_units, bool 
     long c = (Skv + ns - 1) / ns;
     c = (c + step_keys - 1) / step_keys * step_keys;  // whole workgroup steps
     long n = (Skv + c - 1) / c;
+    // The workspace is reported for these splits, also where fewer are run below: calls that one workspace served (a cache
+    // that grows, the same batch with and without per-sequence lengths) still share it.
+    *workspace_splits = (int)n;
     // Fewer, longer chunks where the workgroups would need a further round for the last few of them: the chip runs rounds of
     // `target` workgroups that all take as long as their chunk and about 100 keys more.  Taken where that is shorter by a
     // twelfth and the call's workspace does not grow (us a step, before and after: f16, 16 sequences of 32/8 heads at 128, 4104

@@ -139,9 +139,10 @@ bool prefill_f32_terms_scans(const AttnParams &p, fhip_dtype dtype);  // no scan
 int launch_prefill_f32_terms(const AttnParams &p, fhip_dtype dtype, int mode, hipStream_t stream);
 
 // decode planning (host): keys per split and number of splits; `ragged`: per-batch key counts are given;
-// `f32`: the tensors are f32 (vector variant) rather than 16-bit
+// `f32`: the tensors are f32 rather than 16-bit.  *workspace_splits, at least *nsplit: the splits that the call's reported
+// workspace is sized for
 void decode_plan(int B, int Hkv, int G, int Skv, int D, int compute_units, bool ragged, bool f32, int *chunk,
-                 int *nsplit, int *waves);
+                 int *nsplit, int *waves, int *workspace_splits);
 size_t decode_workspace_bytes(int B, int H, int Hkv, int D, int nsplit);
 
 // calibration (calibration.hip): the register-only matrix-core loop and the scratch it reports into

@@ -240,7 +240,8 @@ int fhip_flash_attention_validate(const fhip_attn_args *args);
 int fhip_flash_attention_select(const fhip_attn_args *args, int32_t *kernel_id);
 
 /* Bytes of device workspace the call needs (0 for the single-pass kernels).  `compute_units`
- * is fhip_device_info.compute_units (split count depends on it). */
+ * is fhip_device_info.compute_units (split count depends on it).  A split-KV decode call that runs with fewer, longer
+ * splits than usual still reports what the usual ones take. */
 int fhip_flash_attention_workspace_bytes(const fhip_attn_args *args, int32_t compute_units, size_t *bytes);
 
 /* out = softmax(q k^T * scale + mask) v with GQA head mapping kv_head = head / (H / Hkv).

@@ -1,5 +1,6 @@
 """How a split-KV decode call's keys are divided: where chunks of the ordinary length would leave the last few workgroups a
-round of their own, fewer and longer ones are taken, never with more workspace; and such calls against the formula in 64 bits.
+round of their own, fewer and longer ones are taken, and the workspace stays that of the ordinary ones; and such calls against
+the formula in 64 bits.
 
 Tolerance: as tests/test_prefill_mfma_forms_gpu.py for 16-bit tensors.  In f32 a score rounds D / 4 times, once per step of the
 matrix instruction, and twice more before the exponential, a result once per 16 keys of a wavefront (24) and a dozen times
@@ -13,15 +14,26 @@ import numpy as np
 import pytest
 
 import floneum_amd as fa
-from test_abi import make_args
+from test_abi import FAKE, make_args
 
 CUS = 256
 
 
-def workspace(B, H, Hkv, rows, Skv, D, dtype):
+def workspace(B, H, Hkv, rows, Skv, D, dtype, lens=False):
     a, need = make_args(B=B, H=H, Hkv=Hkv, Sq=rows, Skv=Skv, D=D, dtype=dtype), ctypes.c_size_t()
+    if lens:
+        a.kv_lens = FAKE
     assert fa.lib().fhip_flash_attention_workspace_bytes(ctypes.byref(a), CUS, ctypes.byref(need)) == fa.OK
     return need.value
+
+
+def planned_splits(B, H, Hkv, rows, Skv, D, dtype, lens=False):
+    """The library's own plan, through its planning function (the C ABI's query of it asks for a GPU's stream)."""
+    plan = fa.lib()._ZN4fhip11decode_planEiiiiiibbPiS0_S0_S0_
+    chunk, n, waves, reported = (ctypes.c_int() for _ in range(4))
+    plan(B, Hkv, H // Hkv * rows, Skv, D, CUS, ctypes.c_bool(lens), ctypes.c_bool(dtype == fa.F32), *map(ctypes.byref, (chunk, n, waves, reported)))
+    assert (n.value - 1) * chunk.value < Skv <= n.value * chunk.value and n.value <= reported.value
+    return n.value
 
 
 def bytes_of(B, H, Hkv, D, n):
@@ -35,8 +47,9 @@ def bytes_of(B, H, Hkv, D, n):
     return partials if n > 8 else partials + B * Hkv * ((cols + 15) // 16) * (n * 128 + 4) + 256
 
 
-def ordinary_splits(B, Hkv, cols, Skv, D, f32):
-    """Of chunks of at most 1024 keys, for as many workgroups as the chip holds (None: the eight-wavefront form's own rule)."""
+def ordinary_splits(B, Hkv, cols, Skv, D, f32, lens=False):
+    """Of chunks of at most 1024 keys (512 for many sequences of lengths of their own), for as many workgroups as the chip holds
+    (None: the eight-wavefront form's own rule)."""
     mfma = D % 32 == 0 and 32 <= D <= 256 and not (f32 and D > 192 and cols <= 4)
     gt = (32 if cols > 16 and D <= (192 if f32 else 128) else 16) if mfma else 1 if cols <= 1 else 2 if cols <= 2 else 4 if cols <= 4 else 8
     units = B * Hkv * ((cols + gt - 1) // gt)
@@ -46,27 +59,39 @@ def ordinary_splits(B, Hkv, cols, Skv, D, f32):
     step = 64 if f32 else 128
     if not mfma:
         step = min(128, 16 * (64 // (4 if D <= 32 else 8 if D <= 64 else 16 if D <= 128 else 32)))
-    n = max(min(-(-target // units), -(-Skv // step)), -(-Skv // 1024), 1)
+    n = max(min(-(-target // units), -(-Skv // step)), -(-Skv // (512 if lens and units >= target else 1024)), 1)
     if Skv <= 256 and mfma:
         n = 1
     chunk = -(-(-(-Skv // n)) // step) * step
     return -(-Skv // chunk)
 
 
-def test_the_workspace_never_grows():
+def test_the_workspace_is_that_of_the_ordinary_splits():
+    """Reported for them also where fewer are run, and what those write fits into it."""
     rng = random.Random(3)
     fewer = 0
     for _ in range(3000):
         B, (H, Hkv) = rng.randint(1, 40), rng.choice([(32, 8), (16, 4), (16, 16), (8, 4), (32, 32), (7, 7), (40, 2)])
         D, rows, dtype = rng.choice([32, 64, 80, 96, 128, 192, 256]), rng.choice([1, 1, 2, 4]), rng.choice([fa.F32, fa.F16, fa.BF16])
-        Skv = int(2 ** rng.uniform(7, 15))
-        n = ordinary_splits(B, Hkv, H // Hkv * rows, Skv, D, dtype == fa.F32)
+        Skv, lens = int(2 ** rng.uniform(7, 15)), rng.random() < 0.3
+        n = ordinary_splits(B, Hkv, H // Hkv * rows, Skv, D, dtype == fa.F32, lens)
         if n is None or B * H * Skv * D > 2 ** 33:
             continue
-        need, most = workspace(B, H, Hkv, rows, Skv, D, dtype), bytes_of(B, H * rows, Hkv, D, n)
-        assert need <= most, (B, H, Hkv, rows, Skv, D, dtype)
-        fewer += need < most
+        call = (B, H, Hkv, rows, Skv, D, dtype, lens)
+        need, run = workspace(*call), planned_splits(*call)
+        assert need == bytes_of(B, H * rows, Hkv, D, n), call
+        assert bytes_of(B, H * rows, Hkv, D, run) <= need, call
+        assert run == n or not lens, call
+        fewer += run < n
     assert fewer > 50
+
+
+@pytest.mark.parametrize("B, H, Hkv, Skv, D, dtype", [(20, 16, 4, 4001, 256, fa.BF16), (20, 32, 8, 4500, 128, fa.F32)])
+def test_calls_share_a_workspace(B, H, Hkv, Skv, D, dtype):
+    """With and without per-sequence lengths, and at the lengths that a growing cache has been through."""
+    need = workspace(B, H, Hkv, 1, Skv, D, dtype)
+    assert workspace(B, H, Hkv, 1, Skv, D, dtype, lens=True) == need
+    assert all(workspace(B, H, Hkv, 1, n, D, dtype) <= need for n in range(1, Skv))
 
 
 @pytest.mark.parametrize("B, H, Hkv, Skv, D, dtype, splits", [
@@ -74,7 +99,7 @@ def test_the_workspace_never_grows():
     (20, 16, 4, 4001, 256, fa.BF16, 3), (20, 32, 8, 4500, 128, fa.F32, 3), (9, 32, 8, 4096, 128, fa.F32, 8), (12, 32, 8, 3000, 128, fa.F16, 6),
 ])
 def test_splits(B, H, Hkv, Skv, D, dtype, splits):
-    assert workspace(B, H, Hkv, 1, Skv, D, dtype) == bytes_of(B, H, Hkv, D, splits)
+    assert planned_splits(B, H, Hkv, 1, Skv, D, dtype) == splits
 
 
 @pytest.mark.gpu
