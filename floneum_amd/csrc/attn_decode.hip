@@ -112,25 +112,38 @@ void decode_plan(int B, int Hkv, int G, int Skv, int D, int compute_units, bool 
     // that grows, the same batch with and without per-sequence lengths) still share it.
     *workspace_splits = (int)n;
     // Fewer, longer chunks where the workgroups would need a further round for the last few of them: the chip runs rounds of
-    // `target` workgroups that all take as long as their chunk and about 100 keys more.  Taken where that is shorter by a
-    // twelfth and the call's workspace does not grow (us a step, before and after: f16, 16 sequences of 32/8 heads at 128, 4104
-    // keys 56.5 -> 47.3, 6000 72.4 -> 64.9, 8200 91 -> 88; bf16, 20 of 16/4 at 256, 4001 keys 81 -> 60; f16, 14 of 16/4 at 256,
-    // two rows on 4647 keys 71 -> 56; f32, 20 of 32/8 at 128, 4500 keys 135 -> 120).  Not for calls with per-sequence lengths,
-    // whose workgroups are uneven anyway (f32, 16 sequences of up to 13172 keys 254 -> 332), nor where two workgroups share a CU
-    // and the chunks are as long as they were asked to be: such calls share their plan with those.  Nor for f32 calls on the
-    // kernels that round once per four keys, where longer sums lose precision (9 sequences at 128: 2.36e-7 -> 2.53e-7 against
-    // 64 bits; 1.50e-7 as it is).
+    // `target` workgroups that all take as long as their chunk and about 100 keys more; merged inside the kernel (to 8 splits) a
+    // unit's splits share an XCD, and the fullest XCD counts.  Taken where that is shorter by an eighth and the call's workspace does
+    // not grow (us a step, before and after: f16, 16 sequences of 32/8 heads at 128, 4104 keys 56.1 -> 45.9, 6000 71.9 -> 64.0; bf16,
+    // 20 of 16/4 at 256, 4001 keys 81.5 -> 59.5; f16, 14 of 16/4 at 256, two rows on 4647 keys 69.6 -> 55.2; f32, 20 of 32/8 at 128,
+    // 4500 keys 134 -> 120, 9 of 16/4 at 192, 1435 keys 38.5 -> 25.7).  Of 300 random calls whose plan it changes
+    // one is slower by more than 1 % (3 %, head_dim 32); above head_dim 128 they take 0.78 of their time in the mean, to 128 0.91.
+    // Where it is not taken:
+    //  - beyond four workgroups per CU in all: they have drifted apart by then, and the last round costs little (f32, 26 sequences of
+    //    16/16 at 64, 9663 keys: 314 -> 340);
+    //  - where the fullest XCD takes a round more than the chip as a whole would (bf16, 21 of 8/4 at 256, 4701 keys: 80 -> 96);
+    //  - on the vector variant (f16, 13 of 32/8 at 48, four rows on 6032 keys: 214 -> 236);
+    //  - from more than 8 splits to 8 or fewer with two workgroups per CU: merged inside the kernel, many splits of small rows
+    //    take longer than with a second launch (f16, 8 of 32/8 at 32, 8946 keys: 17.7 -> 23.4);
+    //  - calls with per-sequence lengths, whose workgroups are uneven anyway (f32, 16 sequences of up to 13172 keys: 254 -> 332), and
+    //    where two workgroups share a CU and the chunks are as long as they were asked to be: such calls share their plan with those;
+    //  - f32 calls on the kernels that round once per four keys, where longer sums lose precision (9 sequences at 128: 2.36e-7 ->
+    //    2.53e-7 against 64 bits; 1.50e-7 as it is).
     const bool asked = wgs_per_cu > 1 && ns_min <= (target + units - 1) / units;
-    if (!ragged && !asked && (!f32 || (decode_use_mfma(D, true, G) && df_shares(D, gt / 16)))) {
-        auto rounds_time = [&](long splits, long keys) { return (units * splits + target - 1) / target * (keys + 100); };
+    if (!ragged && !asked && decode_use_mfma(D, f32, G) && (!f32 || df_shares(D, gt / 16)) && units * n <= 4L * compute_units) {
+        auto rounds_time = [&](long splits, long keys) {
+            const long xcd = target >= 8 ? target / 8 : 1;
+            const long rounds = splits <= 8 ? ((units + 7) / 8 * splits + xcd - 1) / xcd : (units * splits + target - 1) / target;
+            return rounds * (keys + 100);
+        };
         const size_t bytes = decode_workspace_bytes(B, Hkv * G, Hkv, D, (int)n);
-        const long time = rounds_time(n, c);
+        const long time = rounds_time(n, c), n0 = n;
         long best = time;
         for (long k = n - 1; k >= 2; k--) {
             const long kc = ((Skv + k - 1) / k + step_keys - 1) / step_keys * step_keys, kn = (Skv + kc - 1) / kc;
-            if (kc > 4 * max_chunk) break;
+            if (kc > 4 * max_chunk || (wgs_per_cu > 1 && n0 > 8 && kn <= 8)) break;
             const long t = rounds_time(kn, kc);
-            if (kn >= 2 && 12 * t < 11 * time && t < best && decode_workspace_bytes(B, Hkv * G, Hkv, D, (int)kn) <= bytes)
+            if (kn >= 2 && 8 * t < 7 * time && t < best && decode_workspace_bytes(B, Hkv * G, Hkv, D, (int)kn) <= bytes)
                 best = t, n = kn, c = kc;
         }
     }

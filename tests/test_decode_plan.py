@@ -102,6 +102,16 @@ def test_splits(B, H, Hkv, Skv, D, dtype, splits):
     assert planned_splits(B, H, Hkv, 1, Skv, D, dtype) == splits
 
 
+@pytest.mark.parametrize("B, H, Hkv, rows, Skv, D, dtype", [
+    (26, 16, 16, 1, 9663, 64, fa.F32), (16, 32, 8, 1, 8200, 128, fa.F16),  # more than four workgroups per CU
+    (21, 8, 4, 1, 4701, 256, fa.BF16), (21, 8, 4, 1, 1512, 160, fa.F32),   # eleven units of three splits on an XCD of 32 CUs
+    (8, 32, 8, 1, 8946, 32, fa.F16), (17, 16, 4, 1, 9008, 128, fa.F16),    # from nine splits to seven
+    (13, 32, 8, 4, 6032, 48, fa.F16), (11, 32, 8, 1, 15870, 80, fa.BF16),  # the vector variant
+])
+def test_calls_that_keep_their_ordinary_splits(B, H, Hkv, rows, Skv, D, dtype):
+    assert planned_splits(B, H, Hkv, rows, Skv, D, dtype) == ordinary_splits(B, Hkv, H // Hkv * rows, Skv, D, dtype == fa.F32)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [fa.F32, fa.F16, fa.BF16])
 @pytest.mark.parametrize("B, H, Hkv, rows, Skv, D", [(16, 8, 8, 1, 4104, 32), (17, 16, 8, 2, 4500, 32), (20, 8, 4, 1, 3000, 160)])
