@@ -31,7 +31,7 @@
 // Key-split form (template parameter KS): the workgroup owns 128 query rows and its two wavefront groups
 // take alternate key tiles of the same rows, each through the same matrix / vector phases, and merge their
 // (m, l, O) through LDS at the end: twice the workgroups, half the longest one, for grids that do not fill
-// the chip (see use_key_split_form).
+// the chip (see prefill_mfma_block_rows).
 // Masking is by interval: every query row sees one range of keys, known analytically (causal with
 // offset, sliding window, per-batch kv length, tail of the key axis) or read from the interval form
 // of a dense mask tensor (attn_bounds.h, mask_intervals.hip); key tiles that are invisible to the
@@ -681,21 +681,30 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnPara
 
 // Query blocks of 256 rows leave CUs idle when there are few of them (short prompts, a few new rows on a long
 // cache), and a causal prompt's last blocks are several times longer than its first.  The key-split form (128
-// rows, twice the workgroups, the longest one half as long) costs about 7 % per tile and a longer prologue and
-// epilogue; measured, it wins (1.1-1.35 x) while the 256-row grid fills at most half the CUs, for up to 128
-// query rows (where the second wavefront group would have no rows at all), and, where later rows see more keys
-// than earlier ones, for one workgroup per CU when a head has 8 or more query blocks; it loses with fewer than
-// three key tiles.  Rows that all see the same keys keep the 256-row form there: its one workgroup per CU ends with
-// the others, and a CU would take two of the key-split form one after the other (f16, 16 heads without a mask, us a call,
-// both forms on one card: head_dim 80, 4096 x 4096 keys 113 -> 101, 3000 81 -> 68; 64, 2500 64 -> 57; 128, 2500 80 -> 59, 4096
-// 139 -> 123; causal, 4000 rows: 66 for the key-split form, 84 for the other).
-static bool use_key_split_form(const AttnParams &p) {
-    const int cus = p.cus > 0 ? p.cus : 256;
-    const int nqb = (p.Sq + PF_BM - 1) / PF_BM;
-    const long wgs = (long)nqb * p.B * p.H * (p.pf_nsplit > 1 ? p.pf_nsplit : 1);
-    const bool uneven = 2L * p.Sq > p.Skv && ((p.analytic && p.causal) || p.mask_kind == FHIP_MASK_QK);
-    if (p.Skv <= 2 * PF_BN) return false;
-    return p.Sq <= PF_BM / 2 || 2 * wgs <= cus || (wgs <= cus && nqb >= 8 && uneven);
+// rows, twice the workgroups, the longest one half as long) costs about 11 % per tile (f16, 32/8 heads at 128, 8192-token
+// prompt: 535 us against 481) and a longer prologue and epilogue; measured, it wins while the 256-row grid fills at most half the CUs (8 to 32
+// heads, 1024 to 2049 rows: 1.25 - 1.5 x), for up to 128 query rows (where the second wavefront group would have no
+// rows at all; 1.07 x at 128, 1.15 at 64), and, where later rows see more keys than earlier ones, for one workgroup per CU
+// when a head has 8 or more query blocks; it loses with fewer than three key tiles.
+// For one workgroup per CU the 256-row form takes as long as its longest block, the key-split form about a quarter more than the
+// mean one (two of its workgroups follow each other on a CU).  f16, us a call, 256-row and key-split form on one card: without a
+// mask, 16 heads, head_dim 80, 4096 x 4096 keys 89 and 99, 3000 57 and 66; 64, 2500 40 and 49; 128, 2500 58 and 76, 4096 122 and 136;
+// causal, 128, 32/8 heads, 2048 rows on 2048 keys 50 and 47, 4096 106.1 and 105.5, 5120 133.8 and 136.2, 8192 218 and 227; 24/8
+// heads 46 and 39, on 4096 keys 91 and 88, 5120 113.2 and 112.9, 6144 136 and 138; 16/8 heads, 3000 rows on 3000 keys 61 and 48, 6000 125
+// and 121, 7500 158.2 and 157.4, 9000 190 and 193.  So rows that all see the same keys keep the 256-row form, and where they see
+// the keys up to their own position the line is 2.5 keys per row.  Under a window narrower than that it stays at 2, beyond which
+// the 256-row form wins by more (2048 rows on 4096 keys under a window of 2048: 68 and 78).  Sequences of different lengths in
+// a batch are even grids in this sense (2 to 8 of them, 500 to 2048 keys long: 0.80 to 0.85 of the key-split form's time).
+// later_rows_see: the keys up to the last row's own where rows see the keys up to their own position, 0 where all see the same.
+int prefill_mfma_block_rows(int B, int H, int Sq, int Skv, int key_shares, int64_t later_rows_see, int64_t window, int compute_units) {
+    const int nqb = (Sq + PF_BM - 1) / PF_BM;
+    const long wgs = (long)nqb * B * H * (key_shares > 1 ? key_shares : 1);
+    if (Skv <= 2 * PF_BN) return PF_BM;
+    if (Sq <= PF_BM / 2 || 2 * wgs <= compute_units) return PF_BM / 2;
+    if (wgs > compute_units || nqb < 8 || later_rows_see <= 0) return PF_BM;
+    const int64_t keys = later_rows_see < Skv ? later_rows_see : Skv;
+    const bool narrow = window > 0 && window < keys;
+    return 2L * Sq > Skv || (!narrow && 5L * Sq >= 2 * keys) ? PF_BM / 2 : PF_BM;
 }
 
 // Head dims 64, 96 and 128 are this kernel's own.  The other multiples of 8 above 64 run on it padded, quicker than on the
@@ -715,9 +724,11 @@ bool prefill_mfma_rows256_takes(int D, float scale, int B, int H, int Sq, int co
 template <typename T>
 static int launch_t(const AttnParams &p0, hipStream_t stream) {
     AttnParams p = p0;
-    const bool ks = use_key_split_form(p);
-    p.pf_pack = ks ? prefill_mfma_pack(p.B, p.H, p.G, p.Sq, p.Skv, p.cus > 0 ? p.cus : 256) : 0;
-    const int bm = ks ? PF_BM / 2 : PF_BM;
+    const int cus = p.cus > 0 ? p.cus : 256;
+    const int64_t later_rows_see = p.analytic && p.causal ? p.q_pos_offset + p.Sq : p.mask_kind == FHIP_MASK_QK ? p.Skv : 0;
+    const int bm = prefill_mfma_block_rows(p.B, p.H, p.Sq, p.Skv, p.pf_nsplit, later_rows_see, p.analytic ? p.window : 0, cus);
+    const bool ks = bm == PF_BM / 2;
+    p.pf_pack = ks ? prefill_mfma_pack(p.B, p.H, p.G, p.Sq, p.Skv, cus) : 0;
     const int nqb = p.pf_pack ? 1 : (p.Sq + bm - 1) / bm;
     const long blocks = (long)nqb * p.B * (p.pf_pack ? p.H / 4 : p.H) * (p.pf_nsplit > 1 ? p.pf_nsplit : 1);
     if (blocks > 0x7fffffffL) {

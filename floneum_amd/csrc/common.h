@@ -73,6 +73,8 @@ void prefill_mfma_plan(int B, int H, int G, int Sq, int Skv, bool causal_square,
 // query heads that share one workgroup's K/V tiles (0: one head per workgroup)
 int prefill_mfma_pack(int B, int H, int G, int Sq, int Skv, int compute_units);
 size_t prefill_mfma_workspace_bytes(int B, int H, int Sq, int D, int nsplit);
+// its query rows per workgroup: 256, or 128 in the key-split form
+int prefill_mfma_block_rows(int B, int H, int Sq, int Skv, int key_shares, int64_t later_rows_see, int64_t window, int compute_units);
 // merges the key shares parked in p.partials (p.pf_nsplit, p.pf_pitch) into p.out
 int launch_prefill_merge(const AttnParams &p, fhip_dtype dtype, hipStream_t stream);
 
