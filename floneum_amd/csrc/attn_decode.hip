@@ -957,8 +957,10 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 8 / WAVES) void decode_mf
 // the softmax of a column is computed once, by the four lanes that hold its 16 scores.
 constexpr int DF_KEYS = 16;  // keys per wavefront step
 
+// Head_dim 96 keeps the registers of three wavefronts per SIMD, as many as its LDS allows: 20 sequences of 32/8 heads on 600 keys 27.9 us
+// with two, 21.3 with three, two rows on 1099 keys 40 and 33 (at 128 and above the LDS holds two and one).
 template <int D, int CB>  // CB: 16-column blocks per workgroup, see decode_mfma_kernel
-__global__ __launch_bounds__(64 * DEC_WAVES, D > 128 ? 1 : 2) void decode_mfma_f32_kernel(AttnParams p) {
+__global__ __launch_bounds__(64 * DEC_WAVES, D > 128 ? 1 : D == 96 && CB == 1 ? 3 : 2) void decode_mfma_f32_kernel(AttnParams p) {
     request_arguments<AttnParams>();
     constexpr int KP = D * 4 + 16;             // tile row pitch (bytes): rows 4 banks apart
     constexpr int K_BYTES = DF_KEYS * KP;
@@ -1164,6 +1166,8 @@ __global__ __launch_bounds__(64 * DEC_WAVES, D > 128 ? 1 : 2) void decode_mfma_f
 #pragma unroll
                     for (int ks = 0; ks < 4; ks++) share = __builtin_amdgcn_mfma_f32_16x16x4f32(a[ks][e], pe[0][ks], share, 0, 0, 0);
                     o[0][nb][e] += share;
+                    // (the compiler would keep an element of the sum in the share's registers, and those with it: 188 instead of 165)
+                    if constexpr (D == 96) asm volatile("" : "+v"(o[0][nb][e]), "+v"(share));
                 }
             }
         } else {
