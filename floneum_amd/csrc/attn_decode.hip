@@ -1088,15 +1088,15 @@ __global__ __launch_bounds__(64 * DEC_WAVES, D > 128 ? 1 : D == 96 && CB == 1 ? 
             }
         }
     };
-    // Q before the first tile where a workgroup has a step or two: behind the tile's loads, which wait for the memory of every
-    // other workgroup's, it holds the first products up (32/8 heads, 4096 keys, batch 1: 16.1 -> 14.2 us).  Batch 8: 50.7 against
-    // 50.3 us the other way.
-    const bool q_first = p.chunk <= 2 * DEC_WAVES * DF_KEYS;
+    // Q before the first tile: behind the tile's loads, which wait for the memory of every other workgroup's, it holds the first
+    // products up (32/8 heads at 128, us a step, behind and before: 4096 keys, batch 1 15.6 and 13.8; 32768 keys 50.5 and 49; 20
+    // sequences of 1099 keys 44.2 and 42).  At 32, whose tiles are small, only where a workgroup has a step or two (16 of 4096
+    // keys 26.2, 27.4 the other way; a question that every head_dim asks costs 128 4 % of those 20 sequences' step).
+    const bool q_first = D > 32 || p.chunk <= 2 * DEC_WAVES * DF_KEYS;
     if (q_first) load_q();
     int base = lo_al + wave * DF_KEYS;
     if (base < hi) load_tile(base);
     if (!q_first) load_q();
-
 
     for (; base < hi; base += step) {
         wave_lds_sync();  // the previous step's LDS reads precede these writes
