@@ -34,6 +34,7 @@ def kernels(tmp_path_factory):
 
 @pytest.mark.parametrize("kernel, wavefronts", [
     ("decode_mfma_f32_kernelILi96ELi1EE", 3), ("decode_mfma_f32_kernelILi128ELi1EE", 2), ("decode_mfma_f32_kernelILi64ELi1EE", 4),
+    ("16rope_rows_kernel", 8), ("15row_jobs_kernel", 4),
 ])
 def test_wavefronts_per_simd(kernels, kernel, wavefronts):
     """512 vector registers per SIMD lane, in steps of 8, and 800 scalar ones in steps of 16."""
@@ -41,4 +42,5 @@ def test_wavefronts_per_simd(kernels, kernel, wavefronts):
     assert found
     for k in found:
         assert (k["vgpr_count"] + 7) // 8 * 8 * wavefronts <= 512, k
+        assert (k["sgpr_count"] + 15) // 16 * 16 * wavefronts <= 800, k
         assert k["vgpr_spill_count"] == 0, k
