@@ -179,12 +179,14 @@ __device__ __forceinline__ void rope_rows_vec_any(const RopeRows &a) {
 // 700 of 32/8 at 64 in f16 12.7 -> 8.9, 1500 of 32/8 at 128 29.4 -> 22.5.  Quotients by the row's reciprocal and two corrections
 // instead of divisions gave nothing.
 constexpr int NORM_TILE_FLOATS = 1088;  // per wavefront: 16 rows of head_dim 64, 8 of 128, 4 of 256
-struct NormWaveLds {
-    float tile[NORM_TILE_FLOATS];
-    int64_t sb[32], db[32];  // element offsets of the block's rows in the source and the destination
-    uint32_t pos[32];        // their positions (rows of the cos / sin tables, before pos0)
-    float rms[32];
+constexpr int NORM_BLOCK_ROWS = 16;     // of a block at most
+struct alignas(16) NormWaveLds {
+    float tile[NORM_TILE_FLOATS];  // read and written in pieces of 16 bytes
+    int64_t sb[NORM_BLOCK_ROWS], db[NORM_BLOCK_ROWS];  // element offsets of the block's rows in the source and the destination
+    uint32_t pos[NORM_BLOCK_ROWS];                     // their positions (rows of the cos / sin tables, before pos0)
+    float rms[NORM_BLOCK_ROWS];
 };
+static_assert(offsetof(NormWaveLds, tile) % 16 == 0 && sizeof(NormWaveLds) % 16 == 0, "16-byte pieces of every wavefront's tile");
 // value of x in the lane that holds the other half of this lane's pairs: CPR / 2 lanes away within the row's CPR lanes
 template <int CPR>
 __device__ __forceinline__ float other_half(float x) {
@@ -209,7 +211,7 @@ __device__ __forceinline__ void norm_rope_rows_vec_body(const RopeRows &a, NormW
     constexpr int RS = 64 / CPR;
     constexpr int RPW = (D == 64 ? 32 : D == 128 ? 16 : 8) / FEW;  // rows per block
     constexpr int STEPS = RPW / RS;
-    static_assert(RPW * P <= NORM_TILE_FLOATS, "tile");
+    static_assert(RPW <= NORM_BLOCK_ROWS && RPW * P <= NORM_TILE_FLOATS && P % 4 == 0, "tile");
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwave = blockDim.x >> 6;
     float *tile = w->tile;
     const int sub = lane / CPR, c4 = lane % CPR;
@@ -501,7 +503,7 @@ void fill_row_job(RopeRows *out, const void *src, const int64_t ss[4], fhip_dtyp
 // rows per wavefront block of the wide normalised form (RPW in norm_rope_rows_vec_body)
 static int norm_rows_per_wave(const RopeRows &a) {
     const int D = (int)a.shape[3];
-    return (D == 64 ? 32 : D == 128 ? 16 : 8) / (a.few > 1 ? a.few : 1);
+    return (D == 64 ? 32 : D == 128 ? 16 : 8) / a.few;
 }
 
 static int64_t job_blocks(const RopeRows &a) {
