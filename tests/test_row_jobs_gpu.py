@@ -2,6 +2,8 @@
 blocks, over views and odd head and row counts, bit for bit against the CPU restatements; and, on the host, the division by
 multiplication that numbers their rows.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -45,18 +47,62 @@ def test_blocks_of_rows(device, dtype, D, heads, rows):
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
 
 
+class RopeRows(ctypes.Structure):
+    """fhip::RopeRows (floneum_amd/csrc/common.h)."""
+    _fields_ = [("src", ctypes.c_void_p), ("dst", ctypes.c_void_p), ("ss", ctypes.c_int64 * 4), ("ds", ctypes.c_int64 * 4),
+                ("shape", ctypes.c_uint32 * 4), ("src_dtype", ctypes.c_int32), ("dst_dtype", ctypes.c_int32),
+                ("cos", ctypes.c_void_p), ("sin", ctypes.c_void_p), ("pos0", ctypes.c_int64), ("mode", ctypes.c_int32),
+                ("norm_w", ctypes.c_void_p), ("norm_b", ctypes.c_void_p), ("norm_dtype", ctypes.c_int32), ("eps", ctypes.c_float),
+                ("vec", ctypes.c_int32), ("few", ctypes.c_int32), ("small", ctypes.c_int32), ("mul", ctypes.c_uint32 * 3),
+                ("shift", ctypes.c_uint32 * 3)]
+
+
+class RowNorm(ctypes.Structure):
+    _fields_ = [("weight", ctypes.c_void_p), ("bias", ctypes.c_void_p), ("dtype", ctypes.c_int32), ("eps", ctypes.c_float)]
+
+
+FILL = "_ZN4fhip12fill_row_jobEPNS_8RopeRowsEPKvPKl10fhip_dtypePvS5_S6_PKjPKfSB_liPKNS_7RowNormE"
+
+
+def filled(shape, mode=0, norm=False):
+    """What the library's launcher passes to its kernels for contiguous rows of this shape (nothing is launched)."""
+    out, at, strides = RopeRows(), ctypes.c_void_p(0x10000), (ctypes.c_int64 * 4)(*fa._contig_strides(shape))
+    row_norm = RowNorm(0x10000, None, fa.F32, 1e-6)
+    getattr(fa.lib(), FILL)(ctypes.byref(out), at, strides, fa.F32, at, strides, fa.F32, (ctypes.c_uint32 * 4)(*shape), at, at,
+                            ctypes.c_int64(7), mode, ctypes.byref(row_norm) if norm else None)
+    assert (tuple(out.shape), out.pos0, out.mode, bool(out.norm_w)) == (shape, 7, mode, norm)
+    return out
+
+
+def quotient(t, mul, shift):  # as the kernels divide: the upper half of a product of 32 bits, shifted
+    return ((t * mul) >> 32) >> shift if mul else t
+
+
 def test_division_by_multiplication():
-    """The multiplier and shift of fill_row_job, for every divisor to 5000 and others to 2^31, at the quotients' edges."""
+    """The multipliers and shifts that rows and heads are numbered with, for every divisor to 5000 and others to 2^31, at the
+    quotients' edges."""
     rng = np.random.default_rng(1)
-    ds = np.concatenate([np.arange(2, 5001), rng.integers(5001, 2 ** 31, 4000), 2 ** np.arange(1, 31), 2 ** np.arange(2, 31) + 1,
+    ds = np.concatenate([np.arange(1, 5001), rng.integers(5001, 2 ** 31, 4000), 2 ** np.arange(1, 31), 2 ** np.arange(2, 31) + 1,
                          2 ** np.arange(2, 31) - 1]).astype(object)
-    for d in ds:
-        d = int(d)
-        log = (d - 1).bit_length()
-        mul, shift = (1 << (31 + log)) // d + 1, log - 1
-        assert mul < 2 ** 32
+    for d in map(int, ds):
+        job = filled((1, d, 1, 64))
+        assert (job.mul[0], job.shift[0]) == (0, 0)
+        assert tuple(filled((1, 1, d, 64)).mul)[:2] == (job.mul[1], 0)
         top = (2 ** 31 - 1) // d
         for q in {0, 1, top // 2, top}:
             for t in (q * d - 1, q * d, q * d + d - 1):
                 if 0 <= t < 2 ** 31:
-                    assert ((t * mul) >> 32) >> shift == t // d, (t, d)
+                    assert quotient(t, job.mul[1], job.shift[1]) == t // d, (t, d)
+
+
+@pytest.mark.parametrize("mode, norm", [(0, False), (1, False), (2, False), (0, True), (1, True), (2, True)])
+def test_steps_of_a_row(mode, norm):
+    """Steps per row: four pairs each, or four elements where nothing is rotated; and which inputs are numbered in 32 bits."""
+    for D in (8, 64, 96, 128, 200, 256):
+        job, per_row = filled((2, 3, 5, D), mode, norm), D // 4 if mode == 2 else D // 8
+        assert job.small
+        for t in (0, per_row - 1, per_row, 7 * per_row + per_row - 1, 30 * per_row - 1):
+            assert quotient(t, job.mul[2], job.shift[2]) == t // per_row
+        rows = (2 ** 31 - 1) // (1 if norm else per_row)
+        assert filled((1, 1, rows, D), mode, norm).small and not filled((1, 1, rows + 1, D), mode, norm).small
+        assert not filled((2 ** 20, 2 ** 20, 2 ** 25, D), mode, norm).small  # 2^65 rows
