@@ -452,8 +452,8 @@ class Tensor:
     @classmethod
     def empty(cls, device, shape, dtype):
         n = 1
-        for x in shape:
-            n *= int(x)
+        for i in range(len(shape)):
+            n *= int(shape[i])
         return cls(Buffer(device, n * _DTYPE_BYTES[dtype]), dtype, shape)
 
     @classmethod
@@ -616,12 +616,15 @@ class Tensor:
             lens_ptr = kv_lens.buffer.ptr + kv_lens.offset * 4
             keep.append(kv_lens)
         try:
+            # (shapes and strides of other lengths could make up for each other in the pack; one by one they are refused)
+            if not 4 == len(self.strides) == len(k.strides) == len(v.strides) == len(out.strides) == len(out.shape) or len(mask_fields) != 6:
+                raise struct.error
             args = CAttnArgs.from_buffer_copy(_ATTN_ARGS.pack(
                 self.buffer.ptr, self.offset, *self.shape, *self.strides, k.buffer.ptr, k.offset, *k.shape, *k.strides,
                 v.buffer.ptr, v.offset, *v.shape, *v.strides, out.buffer.ptr, out.offset, *out.shape, *out.strides,
                 self.dtype, odt, scale, mask_kind, *mask_fields, *rows_of_mask, lens_ptr or 0, 0, 0, int(force_kernel), 0, 0,
                 table_ptr or 0))
-        except (struct.error, TypeError, OverflowError):  # a value beyond its field: see _c4
+        except (struct.error, TypeError, OverflowError):  # a value beyond its field, or not of rank 4: see _c4
             args = CAttnArgs()
             args.q, args.k, args.v, args.out = self._c4(), k._c4(), v._c4(), out._c4()
             args.dtype, args.out_dtype = self.dtype, odt

@@ -66,3 +66,35 @@ def test_packed_arguments_are_the_fields(analytic, with_mask, rows, ptr, scale):
     assert bytes(got) == bytes(want)
     view = fa._cache_view(type("C", (), dict(device=dev, dtype=fa.F16)), v._c4())
     assert (view.buffer.ptr, view.offset, view.shape, view.strides) == (v.buffer.ptr, v.offset, v.shape, v.strides)
+
+
+@pytest.mark.parametrize("which, shape, strides, other, other_strides", [
+    ("k", (1, 2, 9, 64), (1, 2, 3), "v", (1, 2, 3, 4, 5)),  # strides that make up for each other's number
+    ("q", (1, 2, 3, 64), (1, 2, 3, 4, 5), "out", (1, 2, 3)),
+    ("out", (1, 2, 3), (6, 3, 1), "v", (1, 2, 3, 4, 5, 6)),
+    ("out", (1, 2, 3), (1, 2, 3, 4, 5), None, None),
+    ("out", (1, 2, 3, 4, 5), (1, 2, 3), None, None),
+])
+def test_ranks_and_strides_of_other_lengths_are_refused(which, shape, strides, other, other_strides):
+    dev = _Device()
+    t = {n: fa.Tensor(_Memory(0x1000, dev), fa.F16, (1, 2, 9 if n in "kv" else 3, 64)) for n in ("q", "k", "v", "out")}
+    t[which].shape, t[which].strides = shape, strides
+    if other:
+        t[other].strides = other_strides
+    with pytest.raises((AssertionError, ValueError, IndexError)):
+        t["q"]._attn_args(t["k"], t["v"], 0.1, None, None, None, None, fa.KERNEL_AUTO, t["out"])
+
+
+@pytest.mark.parametrize("shape, strides", [((3, 9), (9, 1, 1)), ((3, 9), (9,))])
+def test_masks_of_other_ranks_are_refused(shape, strides):
+    dev = _Device()
+    q, k = (fa.Tensor(_Memory(0x1000, dev), fa.F16, (1, 2, n, 64)) for n in (3, 9))
+    mask = fa.Tensor(_Memory(0x2000, dev), fa.F16, shape, strides)
+    k.strides = (k.strides + (1, 1))[:8 - len(shape) - len(strides)]  # as many values in all as well-formed tensors have
+    with pytest.raises((AssertionError, ValueError, IndexError)):
+        q._attn_args(k, q, 0.1, (mask, fa.MaskKind.QKMask), None, None, None, fa.KERNEL_AUTO, q)
+
+
+def test_a_shape_has_a_length():
+    with pytest.raises(TypeError):
+        fa.Tensor.empty(_Device(), (n for n in (2, 3)), fa.F16)
