@@ -788,20 +788,19 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 8 / WAVES) void decode_mf
             }
         }
     };
-    // Q before the first tile where a workgroup has a step or two: behind the tile's loads, which wait for the memory of every
-    // other workgroup's, it holds the first products up (32/8 heads, 8000 keys, batch 1: 13.9 -> 13.2 us), and above head_dim
-    // 128, where the CU has no second workgroup to go on with (batch 16, 4001 keys, 256: 50.4 -> 49.9).  Otherwise behind it
-    // (batch 16, 4096 keys, 128: 45.6 -> 45.2).  The eight-wavefront form, whose chunks are long, does not ask (ragged to 32768
-    // keys, 96: 844 us, 855 with the question).
-    const bool q_first = D > 128 || (WAVES == DEC_WAVES && p.chunk <= 2 * WAVES * DM_KEYS);
-    if (q_first) load_q();
+    // Q before the first tile: behind the tile's loads, which wait for the memory of every other workgroup's, it holds the first
+    // products up (us a step, behind and before: 32/8 heads at 128, batch 1, 8000 keys 13.9 and 13.2; 24/8 heads at 96, 24 sequences of
+    // 1654 keys 27.3 and 26.0; 16/4 at 256, 16 of 4001 50.4 and 49.9).  Known at compile time: asked of a call's chunk length, the
+    // question alone cost 18 of 110 random calls at 64 to 128 more than 1 %, up to 5.  The eight-wavefront form, whose chunks are
+    // long, has it behind the tile (ragged to 32768 keys, 96: 844 us, 855 otherwise).
+    constexpr bool q_first = D > 128 || WAVES == DEC_WAVES;
+    if constexpr (q_first) load_q();
     int base = lo_al + wave * DM_KEYS;
     if (base < hi) {
         load_tile(base, set0{});
         if constexpr (DEPTH == 2) load_tile(base + step, set1{});
     }
-    if (!q_first) load_q();
-
+    if constexpr (!q_first) load_q();
 
     // one step: the staged tile `set` (keys base ..) goes to LDS, its registers take the tile DEPTH steps ahead, then the math
     auto one_step = [&](int base, auto set) __attribute__((always_inline)) {
