@@ -537,9 +537,10 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnPara
                 else issue_k(1, j), issue_k(3, j);
             }
         } else {
+            // (tiles that are there: three of 64 keys at head_dim 128 cost a prompt of 18 rows 0.4 us of 8.5)
             load_all(0);
-            load_all(1);
-            if (moves_k) load_all(2);
+            if (ntiles > 1) load_all(1);
+            if (moves_k && ntiles > 2) load_all(2);
         }
         if constexpr (FOLD) {
 #pragma unroll
