@@ -732,9 +732,10 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 8 / WAVES) void decode_mf
     const int lo_al = lo - (lo % DM_KEYS);
     const int step = WAVES * DM_KEYS;
     // Staging registers of the tiles in flight: DEPTH tiles per wavefront.
-    // Every lane always loads: a row outside [lo, hi) is replaced by the nearest one inside (its score is set to
-    // -inf below, so what it holds never counts).  Without branches around the loads the compiler can count them,
-    // and the wait in front of an LDS store is for that tile's loads only, not for everything in flight.
+    // Every lane of a tile loads: a row outside [lo, hi) is replaced by the nearest one inside (its score is set to
+    // -inf below, so what it holds never counts).  Whether a next tile is loaded is the same for the whole wavefront and
+    // asked once in front of its loads; they are waited for before the LDS stores of the next step.  No tile is read behind the
+    // last one (110 random calls at 64 to 128: 2 % less in the mean than with its rows read again).
     constexpr int DEPTH = DM_DEPTH;
     uint4_t kst[DEPTH][NLD], vst[DEPTH][NLD];
     auto load_tile = [&](int base, auto set) __attribute__((always_inline)) {
@@ -1040,8 +1041,9 @@ __global__ __launch_bounds__(64 * DEC_WAVES, D > 128 ? 1 : D == 96 && CB == 1 ? 
         m[cb] = -INFINITY, l[cb] = 0.0f;
     }
 
-    // one wavefront step = 16 consecutive keys; the four wavefronts interleave their steps.  Every lane always loads
-    // (rows outside [lo, hi) are replaced by the nearest one inside; their scores are masked below).
+    // one wavefront step = 16 consecutive keys; the four wavefronts interleave their steps.  Every lane of a tile loads
+    // (rows outside [lo, hi) are replaced by the nearest one inside; their scores are masked below); behind the last tile
+    // nothing is loaded.
     const int lo_al = lo - (lo % DF_KEYS);
     const int step = DEC_WAVES * DF_KEYS;
     float4_t kst[NLD], vst[NLD];

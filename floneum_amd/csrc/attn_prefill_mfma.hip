@@ -20,13 +20,13 @@
 // Phases are separated by workgroup barriers; the tile loads ride on the same barriers.  The vector
 // phase uses no dot-product instructions: on this chip they queue behind the MFMAs of the other
 // wavefront instead of running beside them.
-// Bound: power at head_dim 128 (4096 x 4096 keys, 16 heads, no mask, f16: 123 us = 1.12 PFLOP/s); below, a vector phase
+// Bound: power at head_dim 128 (4096 x 4096 keys, 16 heads, no mask, f16: 121 us = 1.13 PFLOP/s); below, a vector phase
 // takes as long as a matrix phase or longer: its 111 vector instructions take a lone wavefront 617 cycles and beside the
-// matrix instructions of the other 785, the 16 / 20 / 24 matrix instructions of head_dim 64 / 80 / 96 take 512 / 704 / 768.
+// matrix instructions of the other 785, the 16 / 22 / 24 matrix instructions of head_dim 64 / 80 / 96 take 512 / 704 / 768.
 // So everything but the softmax itself is done in the matrix phase, in the shadow of its instructions: tile loads, addresses,
 // the mask test (an instruction on the scalar unit costs a lone wavefront as much as one on the vector unit).  f16, the
-// call above at head_dim 64 / 80 / 96: 89 -> 75, 102 -> 92, 109 -> 100 us (loads, their addresses and an LDS wait in the
-// vector phase before: 1350 cycles, now about 950); causal, 32/8 heads, 4000 rows at 64: 97 -> 81.
+// call above at head_dim 64 / 80 / 96: 88 -> 74, 100 -> 90, 107 -> 97 us (loads, their addresses and an LDS wait in the
+// vector phase before: 1350 cycles, now about 950); causal, 32/8 heads, 4000 rows at 64: 97 -> 80.
 // All accumulation is f32; P is rounded to the input type for the second product.
 // Key-split form (template parameter KS): the workgroup owns 128 query rows and its two wavefront groups
 // take alternate key tiles of the same rows, each through the same matrix / vector phases, and merge their
@@ -689,7 +689,7 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnPara
 // when a head has 8 or more query blocks; it loses with fewer than three key tiles.
 // For one workgroup per CU the 256-row form takes as long as its longest block, the key-split form about a quarter more than the
 // mean one (two of its workgroups follow each other on a CU).  f16, us a call, 256-row and key-split form on one card: without a
-// mask, 16 heads, head_dim 80, 4096 x 4096 keys 89 and 99, 3000 57 and 66; 64, 2500 40 and 49; 128, 2500 58 and 76, 4096 122 and 136;
+// mask, 16 heads, head_dim 80, 4096 x 4096 keys 90 and 99, 3000 57 and 66; 64, 2500 40 and 49; 128, 2500 58 and 76, 4096 122 and 136;
 // causal, 128, 32/8 heads, 2048 rows on 2048 keys 50 and 47, 4096 106.1 and 105.5, 5120 133.8 and 136.2, 8192 218 and 227; 24/8
 // heads 46 and 39, on 4096 keys 91 and 88, 5120 113.2 and 112.9, 6144 136 and 138; 16/8 heads, 3000 rows on 3000 keys 61 and 48, 6000 125
 // and 121, 7500 158.2 and 157.4, 9000 190 and 193.  So rows that all see the same keys keep the 256-row form, and where they see

@@ -173,11 +173,13 @@ __device__ __forceinline__ void rope_rows_vec_any(const RopeRows &a) {
 // Bound: where blocks are few, one block's chain (fetch, fold, divide, store): so everything a block reads, the tables and
 // weights included, is requested before it waits, and row numbers are divided by multiplication.  Where they are many,
 // wavefronts per SIMD: with 32 / 16 / 8 rows per block a wavefront holds 200 registers, two to a SIMD, and 1500 rows of 32/8
-// heads at 128 take 29.9 us; with half of them 128 registers, four to a SIMD, 22.5 (25.0 with a quarter and 80 registers).
-// The launch of q, k and v (f32, or 16-bit where said), this form and one that rotated pairs through the tile with twice the
-// rows per block: 31 rows of 16/4 heads at 64 6.7 -> 5.3 us, 512 rows of 32/8 at 64 8.2 -> 7.6, 300 of 16/4 at 128 8.6 -> 7.2,
-// 700 of 32/8 at 64 in f16 12.7 -> 8.9, 1500 of 32/8 at 128 29.4 -> 22.5.  Quotients by the row's reciprocal and two corrections
-// instead of divisions gave nothing.
+// heads at 128, launched one by one, take 29.9 us; with half of them 128 registers, four to a SIMD, 22.5 (25.0 with a quarter
+// and 80 registers).
+// A form that rotated pairs through the tile with twice the rows per block, and this one, us a launch of a recorded graph (f32, or
+// 16-bit where said): q, k and v of 31 rows of 16/4 heads at 64 6.0 -> 5.0, 512 of 32/8 at 64 7.0 -> 6.0, 300 of 16/4 at 128
+// 6.6 -> 5.7, 700 of 32/8 at 64 in f16 10.6 -> 7.1, 1500 of 32/8 at 128 27.2 -> 21.0, 4096 61.6 -> 47.7, 16384 248 -> 221; q alone,
+// 32 heads at 128, 4096 rows 41.7 -> 30.6, 16384 133 -> 125 (f16 148 -> 106).  Quotients by the row's reciprocal and two
+// corrections instead of divisions gave nothing.
 constexpr int NORM_TILE_FLOATS = 1088;  // per wavefront: 16 rows of head_dim 64, 8 of 128, 4 of 256
 constexpr int NORM_BLOCK_ROWS = 16;     // of a block at most
 struct alignas(16) NormWaveLds {
