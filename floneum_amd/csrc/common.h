@@ -188,13 +188,14 @@ struct RopeRows {
     int32_t norm_dtype;
     float eps;
     int32_t vec;  // rows and pointers allow the 16-byte forms (set by fill_row_job)
-    int32_t few;  // the wide normalised form with 32 / 16 / 8 rows per wavefront block divided by 2 or 4 (set by fill_row_job)
+    int32_t few;  // the wide normalised form: rows per wavefront block and their order, see NORM_FEW (set by fill_row_job)
     int32_t small;  // rows (and steps of the wide form without a norm) are fewer than 2^31: divided by multiplication
     uint32_t mul[3], shift[3];  // by shape[2], shape[1] and the wide form's steps per row (mul 0: by 1)
 };
 struct RowJobs {
     RopeRows job[3];
     int32_t n;
+    uint32_t first[3];  // a job's first workgroup of the launch (set by launch_row_jobs)
 };
 void fill_row_job(RopeRows *out, const void *src, const int64_t sstride[4], fhip_dtype src_dtype, void *dst,
                   const int64_t dstride[4], fhip_dtype dst_dtype, const uint32_t shape[4], const float *cos, const float *sin,

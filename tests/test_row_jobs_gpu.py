@@ -106,3 +106,38 @@ def test_steps_of_a_row(mode, norm):
         rows = (2 ** 31 - 1) // (1 if norm else per_row)
         assert filled((1, 1, rows, D), mode, norm).small and not filled((1, 1, rows + 1, D), mode, norm).small
         assert not filled((2 ** 20, 2 ** 20, 2 ** 25, D), mode, norm).small  # 2^65 rows
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [fa.F32, fa.F16, fa.BF16])
+@pytest.mark.parametrize("D, heads, kv_heads, rows, turned", [
+    (64, 5, 1, 4779, True), (64, 5, 1, 4777, True), (64, 5, 1, 4779, False),  # 3584 blocks of eight rows and a few less
+    (128, 7, 2, 801, True), (256, 4, 2, 601, True), (256, 4, 2, 601, False), (128, 3, 1, 2, True),
+])
+def test_jobs_of_a_layer(device, dtype, D, heads, kv_heads, rows, turned):
+    """q, k and v of two sequences in one launch, each with blocks of its own, against the same jobs one by one; views of
+    [rows, heads, D] and of [heads, rows, D], around the sizes between which blocks change their rows and their order."""
+    rng = np.random.default_rng(D + rows)
+
+    def rows_of(h):
+        x = rng.normal(0, 1, (2, rows, h, D) if turned else (2, h, rows, D)).astype(np.float32)
+        t = fa.Tensor.from_numpy(device, x, dtype)
+        return t.transpose(1, 2) if turned else t
+
+    q, k, v = rows_of(heads), rows_of(kv_heads), rows_of(kv_heads)
+    rope = fa.RopeCache(D, rows + 5, 10000.0, device)
+    q_norm, k_norm = (fa.RmsNorm(rng.normal(1, 0.2, D).astype(np.float32), b, 1e-6, dtype, device)
+                      for b in (None, rng.normal(0, 0.2, D).astype(np.float32)))
+    cache = fa.KvCache(2, rows, dtype, device)
+    got = cache.qkv_rope_append(rope, q, k, v, 5, False, q_norm, k_norm)
+    want = [rope.apply(q, 5, norm=q_norm), rope.apply(k, 5, norm=k_norm), v]
+    for g, w in zip(got, want):
+        assert np.array_equal(g.to_numpy().view(np.uint32 if dtype != fa.F16 else np.uint16),
+                              np.ascontiguousarray(w.to_numpy()).view(np.uint32 if dtype != fa.F16 else np.uint16))
+    # the rows of one launch against the restatement: the first, the last and one between
+    host = q.to_numpy()
+    for r in {0, rows // 2, rows - 1}:
+        x = rounded(host, dtype)[:, :, r:r + 1]
+        n = rounded(oracle.rms_norm(np.ascontiguousarray(x), rounded(q_norm.weight.to_numpy()[0], dtype), None, 1e-6), dtype)
+        y = rounded(oracle.rope(n, rope.cos_host, rope.sin_host, 5 + r), dtype)
+        assert np.array_equal(rounded(got[0].to_numpy(), dtype)[:, :, r:r + 1].view(np.uint32), y.view(np.uint32))
