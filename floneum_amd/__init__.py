@@ -177,6 +177,7 @@ SYMBOLS = {
 }
 
 _LIB = None
+_native = None  # csrc/host_python.cpp, loaded with the library
 
 
 def lib():
@@ -191,8 +192,20 @@ def lib():
             fn = getattr(L, name)
             fn.restype = res
             fn.argtypes = args
+        _bind_native()
         _LIB = L
     return _LIB
+
+
+def _bind_native():
+    """Loads the calls of a decode step in native code (csrc/host_python.cpp), which is built with the library."""
+    global _native
+    try:
+        from . import _host
+    except ImportError as e:
+        raise ImportError(f"{_HERE}/_host.so: {e}: run `python -m floneum_amd.build` (or __graft_entry__.build()) first") from e
+    _host.bind(Tensor, _View, KvCache, RopeCache, RmsNorm, IntTensor)
+    _native = _host
 
 
 def check(code):
@@ -413,6 +426,8 @@ class Buffer:
 class _View:
     """Non-owning device memory (e.g. KV-cache storage owned by the C library)."""
 
+    __slots__ = ("device", "ptr", "keepalive", "__dict__", "__weakref__")
+
     def __init__(self, device, ptr, keepalive=None):
         self.device = device
         self.ptr = ptr
@@ -437,6 +452,8 @@ class Tensor:
     """A strided view of device memory: {buffer, offset, shape, strides} in element units, the
     layout contract of fusor tensors (fusor-ml/types/src/layout.rs:88-129)."""
 
+    __slots__ = ("buffer", "dtype", "shape", "strides", "offset", "__dict__", "__weakref__")
+
     def __init__(self, buffer, dtype, shape, strides=None, offset=0):
         self.buffer = buffer
         self.dtype = dtype
@@ -451,6 +468,10 @@ class Tensor:
 
     @classmethod
     def empty(cls, device, shape, dtype):
+        if cls is Tensor and _native is not None:
+            made = _native.contiguous(Buffer, device, _DTYPE_BYTES[dtype], dtype, shape)
+            if made is not None:
+                return made
         n = 1
         for i in range(len(shape)):
             n *= int(shape[i])
@@ -561,8 +582,15 @@ class Tensor:
         AnalyticMask from MaskCache.get_analytic; `kv_lens` = device int32 [B] tensor of valid key
         counts; `out_dtype` F32 for 16-bit inputs.  Raises InvalidArgument (an AssertionError)
         where the reference panics."""
+        L = _LIB or lib()
+        if out is None and len(self.shape) == 4:
+            out = Tensor.empty(self.buffer.device, self.shape, self.dtype if out_dtype is None else out_dtype)
+        rc = _native.attention(self, k, v, scale, mask, analytic, kv_lens, out_dtype, force_kernel, out)
+        if rc is not None:
+            if rc != OK:
+                check(rc)
+            return out
         args = self._attn_args(k, v, scale, mask, analytic, kv_lens, out_dtype, force_kernel, out)
-        L = lib()
         dev = self.device
         need = ctypes.c_size_t()
         check(L.fhip_flash_attention_workspace_bytes(ctypes.byref(args), dev.compute_units, ctypes.byref(need)))
@@ -837,6 +865,11 @@ def _kv_step(self, rope, q, k, v, start_pos, interleaved=False, q_norm=None, k_n
     """rope(norm(q)) and append(rope(norm(k)), v) in one launch; returns (q_rotated, k_all, v_all)."""
     assert k.dtype == v.dtype
     q_out = Tensor.empty(self.device, q.shape, q_out_dtype if q_out_dtype is not None else q.dtype)
+    done = _native.append(self, rope, q, q_out, k, v, start_pos, interleaved, q_norm, k_norm)
+    if done is not None:
+        if done[0] != OK:
+            check(done[0])
+        return q_out, done[1], done[2]
     cq, co, ck, cv = q._c4(), q_out._c4(), k._c4(), v._c4()
     ka, va = CTensor4(), CTensor4()
     tables = rope._tables(start_pos, interleaved)

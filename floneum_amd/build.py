@@ -1,7 +1,8 @@
-"""Builds libfusor_hip.so (and libfusor_hip.a) for gfx950 from floneum_amd/csrc with hipcc."""
+"""Builds libfusor_hip.so (and libfusor_hip.a) for gfx950 from floneum_amd/csrc with hipcc, and the Python mirror's _host.so."""
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -10,6 +11,7 @@ SOURCES = ["api.hip", "attn_generic.hip", "attn_decode.hip", "attn_prefill_mfma.
            "attn_prefill_f32.hip", "attn_prefill_f32_terms.hip",
            "kv_cache.hip", "mask_intervals.hip", "rope.hip", "calibration.hip"]
 LIB = os.path.join(HERE, "libfusor_hip.so")
+HOST = os.path.join(HERE, "_host.so")
 STATIC = os.path.join(HERE, "libfusor_hip.a")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fno-gpu-rdc", "-Wall", "-Wno-unused-function", "-Wno-inline-asm",
@@ -40,6 +42,10 @@ def build(verbose=True):
     if os.path.exists(STATIC):
         os.remove(STATIC)
     subprocess.check_call(["ar", "rcs", STATIC] + objs)
+    # the Python mirror's native half
+    subprocess.check_call(["g++", "-std=c++17", "-O2", "-Wall", "-Wno-missing-field-initializers", "-fPIC", "-shared", "-fvisibility=hidden",
+                           "-I", sysconfig.get_paths()["include"], os.path.join(CSRC, "host_python.cpp"), "-o", HOST, "-L", HERE,
+                           "-lfusor_hip", "-Wl,-rpath,$ORIGIN"])
     # the C++ host mirror's test program (needs a GPU, started by tests/test_host_mirror_gpu.py)
     root = os.path.dirname(HERE)
     cpp = os.path.join(root, "tests", "cpp", "test_host_mirror.cpp")

@@ -98,3 +98,109 @@ def test_masks_of_other_ranks_are_refused(shape, strides):
 def test_a_shape_has_a_length():
     with pytest.raises(TypeError):
         fa.Tensor.empty(_Device(), (n for n in (2, 3)), fa.F16)
+
+
+def native(dev):
+    """The native half, and tensors, a rotary cache and norms on made-up memory for it."""
+    fa.lib()
+
+    def tensor(p, shape, strides=None, offset=0, dtype=fa.F16):
+        return fa.Tensor(_Memory(p, dev), dtype, shape, strides, offset)
+
+    def norm(bias):
+        n = fa.RmsNorm.__new__(fa.RmsNorm)
+        n.device, n.dtype, n.eps = dev, fa.BF16, 1e-6
+        n.weight, n.bias = tensor(0x3330, (1, 64)), tensor(0x3440, (1, 64)) if bias else None
+        return n
+
+    rope = fa.RopeCache.__new__(fa.RopeCache)
+    rope.cos, rope.sin, rope.rows = tensor(0x6660, (9, 32)), tensor(0x6670, (9, 32)), 9
+    return fa._native, tensor, norm, rope
+
+
+@pytest.mark.parametrize("analytic", [None, (True, 5, 0), (False, -3, 2 ** 40)])
+@pytest.mark.parametrize("with_mask", [None, "mask", "mask and table"])
+@pytest.mark.parametrize("lens, out_dtype, scale", [(False, None, 0.1), (True, fa.F32, -1e-3), (True, None, float(np.float32(0.3)))])
+def test_native_arguments_are_the_packed_ones(analytic, with_mask, lens, out_dtype, scale):
+    dev = _Device()
+    host, tensor, _, _ = native(dev)
+    q = tensor(0x7f1234567000, (2, 3, 8, 64), offset=7).transpose(1, 2)
+    k, v = (tensor(0x2000 * i, (2, 4, 9, 64), (-4 * 16 * 64, 16 * 64, 64, 0), 2 ** 63 + i) for i in (1, 2))
+    out = tensor(0x9000, (2, 3, 8, 64), dtype=fa.F32).transpose(1, 2)
+    mask = None
+    if with_mask:
+        table = fa.MaskIntervals.__new__(fa.MaskIntervals)
+        table.buffer = _Memory(0x5550, dev)
+        mask = (tensor(0x4440, (3, 9)), fa.MaskKind.QKMask) + ((table,) if "table" in with_mask else ())
+    counts = None
+    if lens:
+        counts = fa.IntTensor.__new__(fa.IntTensor)
+        counts.buffer, counts.shape, counts.offset = _Memory(0x7770, dev), (2,), 3
+    a = (k, v, scale, mask, analytic, counts, out_dtype, fa.KERNEL_PREFILL_F32, out)
+    assert host.attention_descriptor(q, *a) == bytes(q._attn_args(*a))
+
+
+def test_calls_that_are_not_plain_are_left_to_the_general_way():
+    """Each of these the mirror still accepts or refuses by itself: the native half answers None and leaves no exception."""
+    dev, other = _Device(), _Device()
+    host, tensor, _, _ = native(dev)
+    plain = dict(q=tensor(0x1000, (1, 2, 3, 64)), k=tensor(0x2000, (1, 2, 9, 64)), v=tensor(0x3000, (1, 2, 9, 64)), scale=0.1, mask=None,
+                 analytic=None, lens=None, odt=None, force=0, out=tensor(0x4000, (1, 2, 3, 64)))
+    assert host.attention_descriptor(*plain.values()) is not None
+
+    class Odd(fa.Tensor):
+        pass
+
+    lens = fa.IntTensor.__new__(fa.IntTensor)
+    lens.buffer, lens.shape, lens.offset = _Memory(0x7770, dev), (2,), 0
+    m = tensor(0x4440, (3, 9))
+    foreign = fa.Tensor(_Memory(0x2000, other), fa.F16, (1, 2, 9, 64))
+    for change in [dict(k=foreign), dict(v=foreign), dict(q=tensor(0x1000, (2, 3, 64))), dict(k=tensor(0x2000, (1, 2, 9, 64), (1, 2, 3))),
+                   dict(k=tensor(0x2000, (1, 2, 9, 64), dtype=fa.F32)), dict(q=tensor(None, (1, 2, 3, 64))), dict(scale=1), dict(scale=1e39),
+                   dict(scale=float("nan")), dict(scale=np.float32(0.1)), dict(q=tensor(0x1000, (1, 2, 2 ** 33, 64))), dict(out=None),
+                   dict(k=tensor(0x2000, (1, 2, 9, 64), offset=-1)), dict(k=tensor(0x2000, (1, 2, 9, 64), (1, 2, 2 ** 70, 1))),
+                   dict(q=Odd(_Memory(0x1000, dev), fa.F16, (1, 2, 3, 64))), dict(lens=lens), dict(lens=[1]), dict(odt="f32"), dict(force=2 ** 40),
+                   dict(mask=m), dict(mask=(m,)), dict(mask=[m, fa.MaskKind.QKMask]), dict(mask=(m, None)), dict(mask=(m, 1, None)),
+                   dict(mask=(tensor(0x4440, (3, 9), dtype=fa.F32), 1)), dict(mask=(tensor(0x4440, (1, 3, 9)), 1)),
+                   dict(analytic=(1, 5, 0)), dict(analytic=(True, 5, None)), dict(analytic=[True, 5, 0]), dict(analytic=(True, 2 ** 70, 0)),
+                   dict(analytic=fa.CAnalyticMask(1, 1, 0, 0)), dict(analytic=(True, 5))]:
+        assert host.attention_descriptor(*dict(plain, **change).values()) is None, change
+
+
+@pytest.mark.parametrize("q_bias, k_bias, interleaved", [(None, None, False), (False, True, True), (True, None, False)])
+def test_native_append_describes_what_ctypes_does(q_bias, k_bias, interleaved):
+    dev = _Device()
+    host, tensor, norm, rope = native(dev)
+    cache = fa.KvCache.__new__(fa.KvCache)
+    cache.device, cache.dtype, cache.handle = dev, fa.F16, None
+    q, k, v = (tensor(0x1000 * i, (1, 2, h, 64), offset=i).transpose(1, 2) for i, h in ((1, 8), (2, 4), (3, 4)))
+    q_out = tensor(0x8000, q.shape, dtype=fa.F32)
+    norms = [norm(b) if b is not None else None for b in (q_bias, k_bias)]
+    got = host.append_descriptors(cache, rope, q, q_out, k, v, 5, interleaved, *norms)
+    want = b"".join(bytes(t._c4()) for t in (q, q_out, k, v)) + np.array([fa.F16, fa.F32, fa.F16, fa.F16], np.int32).tobytes()
+    want += bytes(rope._tables(5, interleaved)) + b"".join(bytes(n._c() if n else fa.CRmsNorm()) for n in norms)
+    assert got == want
+    for a in [(cache, rope, q, q_out, k, tensor(0x3000, k.shape, dtype=fa.F32), 5, False, None, None), (cache, rope, q, None, k, v, 5, False, None, None),
+              (cache, rope, q, q_out, k, v, -1, False, None, None), (cache, rope, q, q_out, k, v, 5, 0, None, None),
+              (cache, rope, q, q_out, k, v, 5, False, object(), None), (object(), rope, q, q_out, k, v, 5, False, None, None)]:
+        assert host.append_descriptors(*a) is None
+    cache.handle = None
+
+
+def test_native_tensors_are_the_mirror_s():
+    dev = _Device()
+    host, tensor, _, _ = native(dev)
+    blocks = []
+
+    def memory(device, nbytes):
+        blocks.append((device, nbytes))
+        return _Memory(0x1000, device)
+
+    for shape in [(2, 3, 4, 64), (5,), (), (2, 0, 3), (1, 1, 1, 1)]:
+        t, want = host.contiguous(memory, dev, 2, fa.F16, shape), tensor(0x1000, shape)
+        assert type(t) is fa.Tensor and (t.shape, t.strides, t.offset, t.dtype) == (want.shape, want.strides, want.offset, want.dtype)
+        assert blocks[-1] == (dev, 2 * int(np.prod(shape))) and t.device is dev
+    for shape in [[2, 3], (2, -1), (2.0, 3), (np.int64(2), 3), (2 ** 33, 1), (2 ** 31, 2 ** 31)]:
+        assert host.contiguous(memory, dev, 2, fa.F16, shape) is None
+    with pytest.raises(ZeroDivisionError):
+        host.contiguous(lambda *_: 1 // 0, dev, 2, fa.F16, (1,))
