@@ -295,35 +295,42 @@ __global__ __launch_bounds__(64 * PF32_WAVES, 2) void prefill_f32_kernel(AttnPar
     }
 }
 
-// Merge of the key shares: one wavefront per (batch, head, query row), log-sum-exp over the shares, then the division the
+// Merge of the key shares: a log-sum-exp over the shares of each (batch, head, query row), then the division the
 // single-pass form does in its epilogue.  A row's references m are exponents of two, or, where a mask is added to the
 // scores, in the scores' own units: those rows' sums l are parked with their sign set (-0.0 included).
-template <typename T>
-__global__ __launch_bounds__(256) void prefill_f32_merge_kernel(AttnParams p) {
+// LPR lanes share a row, four dims each: a share is one load of four values and one of (m, l).
+// Bound: the memory latency of a round of eight shares, and the partials' bytes where there are many.  One wavefront per row with six
+// loads per share before: 16-bit calls in two to eight shares take 0.92 to 0.96 of their time, f32 ones 0.97 (2 x 16 heads, 526 rows of 64 dims in
+// six shares 11.0 -> 7 us for this kernel).
+typedef float4_t __attribute__((aligned(8))) float4_at8_t;  // a row of the partials is D + 2 or D + 4 floats
+typedef float float2_at8_t __attribute__((ext_vector_type(2)));
+template <typename T, int LPR>
+__global__ __launch_bounds__(256) void prefill_f32_merge_kernel(AttnParams p, int out_vec) {
     request_arguments<AttnParams>();
-    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
+    const int64_t row = (int64_t)blockIdx.x * (256 / LPR) + threadIdx.x / LPR;
+    const int D = p.D, dim = 4 * (threadIdx.x % LPR);
     const int64_t rows = (int64_t)p.B * p.H * p.Sq;
-    if (row >= rows) return;
+    if (row >= rows || dim >= D) return;
     // the same hand-over between the interval form and the mask-adding form as in the main kernel (none when the
     // main kernel held both forms)
     if (!p.iv_either && ((p.iv_bad && *p.iv_bad == p.bad_tag) || (p.only_if_bad && *p.only_if_bad != p.bad_tag))) return;
-    const int query = (int)(row % p.Sq);
-    const int h = (int)((row / p.Sq) % p.H), b = (int)(row / p.Sq / p.H);
-    const int D = p.D, ns = p.pf_nsplit, pitch = p.pf_pitch;
+    const int ns = p.pf_nsplit, pitch = p.pf_pitch;
     const float *ws = p.partials + row * ns * pitch;
     // eight shares per round of loads (a round costs one memory latency)
-    float M = -INFINITY, L = 0.0f, A[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // dims lane, lane + 64, lane + 128, lane + 192
+    float M = -INFINITY, L = 0.0f;
+    float4_t A = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int s0 = 0; s0 < ns; s0 += 8) {
-        float ms[8], ls[8], av[8][4];
+        float ms[8], ls[8];
+        float4_t av[8];
 #pragma unroll
         for (int u = 0; u < 8; u++) {
             const bool ok = s0 + u < ns;
             const float *src = ws + (ok ? s0 + u : s0) * pitch;
-            ms[u] = ok ? src[D] : -INFINITY;
-            ls[u] = ok ? src[D + 1] : 0.0f;
-#pragma unroll
-            for (int k = 0; k < 4; k++) av[u][k] = (ok && lane + 64 * k < D) ? src[lane + 64 * k] : 0.0f;
+            const float2_at8_t ml = *(const float2_at8_t *)(src + D);
+            av[u] = *(const float4_at8_t *)(src + dim);
+            ms[u] = ok ? ml[0] : -INFINITY;
+            ls[u] = ok ? ml[1] : 0.0f;
+            if (!ok) av[u] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
         }
         float Mn = M;
 #pragma unroll
@@ -343,21 +350,37 @@ __global__ __launch_bounds__(256) void prefill_f32_merge_kernel(AttnParams p) {
             for (int u = 0; u < 8; u++) w[u] = ms[u] == Mn ? 1.0f : 0.0f;
         }
         L *= c;
-#pragma unroll
-        for (int k = 0; k < 4; k++) A[k] *= c;
+        A *= c;
 #pragma unroll
         for (int u = 0; u < 8; u++) {
             L += w[u] * ls[u];
 #pragma unroll
-            for (int k = 0; k < 4; k++) A[k] += w[u] * av[u][k];
+            for (int e = 0; e < 4; e++) A[e] += w[u] * av[u][e];
         }
         M = Mn;
     }
     L = fabsf(L);
-    const int64_t ob = b * p.os[0] + h * p.os[1] + (int64_t)query * p.os[2];
+    int64_t at;  // of the row in the result
+    if (rows <= 0x7fffffff) {
+        const uint32_t bh = (uint32_t)row / (uint32_t)p.Sq, b = bh / (uint32_t)p.H;
+        at = b * p.os[0] + (bh - b * p.H) * p.os[1] + ((uint32_t)row - bh * p.Sq) * p.os[2];
+    } else {
+        at = row / p.Sq / p.H * p.os[0] + row / p.Sq % p.H * p.os[1] + row % p.Sq * p.os[2];
+    }
+    at += dim * p.os[3];
 #pragma unroll
-    for (int k = 0; k < 4; k++)
-        if (lane + 64 * k < D) store_out<T>(p, ob + (lane + 64 * k) * p.os[3], A[k] / L);  // no visible key: 0/0 = NaN
+    for (int e = 0; e < 4; e++) A[e] /= L;  // no visible key: 0/0 = NaN
+    if (out_vec && sizeof(T) == 2 && !p.out_f32) {
+        T four[4] = {from_float<T>(A[0]), from_float<T>(A[1]), from_float<T>(A[2]), from_float<T>(A[3])};
+        uint2_t w;
+        __builtin_memcpy(&w, four, 8);
+        *(uint2_t *)((T *)p.out + at) = w;
+    } else if (out_vec) {
+        *(float4_t *)((float *)p.out + at) = A;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++) store_out<T>(p, at + e * p.os[3], A[e]);
+    }
 }
 
 // ---- head_dim 129 .. 256 (Gemma-3's key length is 256) -------------------------------------------------------
@@ -610,7 +633,16 @@ static int launch_wide(const AttnParams &p_in, hipStream_t stream) {
 template <typename T>
 static int launch_merge_t(const AttnParams &p, hipStream_t stream) {
     const int64_t rows = (int64_t)p.B * p.H * p.Sq;
-    hipLaunchKernelGGL(prefill_f32_merge_kernel<T>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, p);
+    const int lpr = p.D <= 64 ? 16 : p.D <= 128 ? 32 : 64, per = 256 / lpr;
+    // rows of the result written in pieces of four elements
+    const int oeb = sizeof(T) == 4 || p.out_f32 ? 4 : 2;
+    int out_vec = p.os[3] == 1 && (uintptr_t)p.out % (4 * oeb) == 0;
+    for (int i = 0; i < 3; i++)
+        if (p.os[i] % 4 != 0) out_vec = 0;
+    const dim3 grid((unsigned)((rows + per - 1) / per));
+    if (lpr == 16) hipLaunchKernelGGL((prefill_f32_merge_kernel<T, 16>), grid, dim3(256), 0, stream, p, out_vec);
+    else if (lpr == 32) hipLaunchKernelGGL((prefill_f32_merge_kernel<T, 32>), grid, dim3(256), 0, stream, p, out_vec);
+    else hipLaunchKernelGGL((prefill_f32_merge_kernel<T, 64>), grid, dim3(256), 0, stream, p, out_vec);
     FHIP_HIP_CHECK(hipGetLastError());
     return FHIP_OK;
 }
