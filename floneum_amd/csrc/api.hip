@@ -303,11 +303,12 @@ static bool f32_adds_masks(const fhip_attn_args *a) { return a->q.shape[3] <= 12
 // is queued behind it.
 static bool f32_serves_both_mask_forms(const fhip_attn_args *a) { return a->q.shape[3] <= 64; }
 
-// The keys a decode call can see at all, when the analytic descriptor alone says so (no mask tensor, no per-sequence key
+// The keys a call can see at all, when the analytic descriptor alone says so (no mask tensor, no per-sequence key
 // counts): [*lo0, *lo0 + *len) with *lo0 a multiple of 128.  The kernels are handed the tensors from key *lo0 on (and the
-// query position moved by as much), so the split-KV plan covers this range only: a window of 4096 keys at the end of a
-// 16384-key cache is spread over as many workgroups as a 4096-key cache would be.
-static void decode_visible_range(const fhip_attn_args *a, int *lo0, int *len) {
+// query position moved by as much), so a split of the keys covers this range only: a window of 4096 keys at the end of a
+// 16384-key cache is spread over as many workgroups as a 4096-key cache would be.  (128 keys are whole tiles of every tiled kernel,
+// so a call that is not split sums as it would from key 0 on.)
+static void visible_range(const fhip_attn_args *a, int *lo0, int *len) {
     const int64_t Skv = a->k.shape[2], rows = a->q.shape[2];
     int64_t lo = 0, hi = Skv;
     if (a->analytic.enabled && !a->kv_lens && a->mask_kind == FHIP_MASK_NONE) {
@@ -322,27 +323,31 @@ static void decode_visible_range(const fhip_attn_args *a, int *lo0, int *len) {
 // Key split of a call the f32-arithmetic tiled kernel serves (few query rows on a long cache), and where its
 // partial results go in the workspace: behind the mask scratch, 256-byte aligned.
 static void f32_split_plan(const fhip_attn_args *a, int cus, int *nsplit, int *chunk) {
-    const bool causal_square = a->analytic.enabled && a->analytic.causal && 2ull * a->q.shape[2] > a->k.shape[2];
+    int lo0, len;
+    visible_range(a, &lo0, &len);
+    const bool causal_square = a->analytic.enabled && a->analytic.causal && 2ll * a->q.shape[2] > len;
     const int Hkv = (int)a->k.shape[1];
     prefill_f32_plan((int)a->q.shape[0], (int)a->q.shape[1], Hkv ? (int)a->q.shape[1] / Hkv : 1, (int)a->q.shape[2],
-                     (int)a->k.shape[2], (int)a->q.shape[3], causal_square, cus > 0 ? cus : 256, nsplit, chunk);
+                     len, (int)a->q.shape[3], causal_square, cus > 0 ? cus : 256, nsplit, chunk);
 }
 static size_t f32_partials_offset(const fhip_attn_args *a) { return (mask_scratch_bytes(a) + 255) & ~(size_t)255; }
 static void mfma_split_plan(const fhip_attn_args *a, int cus, int *nsplit, int *chunk) {
+    int lo0, len;
+    visible_range(a, &lo0, &len);
     if (a->force_kernel == FHIP_KERNEL_PREFILL_MFMA_ROWS64) {  // that form never splits the keys
         *nsplit = 1;
-        *chunk = (int)a->k.shape[2];
+        *chunk = len;
         return;
     }
-    const bool causal_square = a->analytic.enabled && a->analytic.causal && 2ull * a->q.shape[2] > a->k.shape[2];
+    const bool causal_square = a->analytic.enabled && a->analytic.causal && 2ll * a->q.shape[2] > len;
     const int Hkv = (int)a->k.shape[1];
     if (!prefill_mfma_rows256_takes((int)a->q.shape[3], a->scale, (int)a->q.shape[0], (int)a->q.shape[1], (int)a->q.shape[2],
                                     cus > 0 ? cus : 256))  // the wide-head form: 128-row query blocks
         prefill_mfma_wide_plan((int)a->q.shape[0], (int)a->q.shape[1], Hkv ? (int)a->q.shape[1] / Hkv : 1, (int)a->q.shape[2],
-                               (int)a->k.shape[2], causal_square, cus > 0 ? cus : 256, nsplit, chunk);
+                               len, causal_square, cus > 0 ? cus : 256, nsplit, chunk);
     else
         prefill_mfma_plan((int)a->q.shape[0], (int)a->q.shape[1], Hkv ? (int)a->q.shape[1] / Hkv : 1, (int)a->q.shape[2],
-                          (int)a->k.shape[2], causal_square, cus > 0 ? cus : 256, nsplit, chunk);
+                          len, causal_square, cus > 0 ? cus : 256, nsplit, chunk);
 }
 
 // A workspace too small for the planned key split still takes the largest split that fits (shares stay multiples of 64
@@ -775,7 +780,7 @@ static void decode_call_bytes(const fhip_attn_args *args, int32_t compute_units,
     const int B = (int)args->q.shape[0], H = (int)args->q.shape[1], rows = (int)args->q.shape[2], D = (int)args->q.shape[3];
     const int Hkv = (int)args->k.shape[1];
     int chunk, nsplit, waves, workspace_splits, lo0, len;
-    decode_visible_range(args, &lo0, &len);
+    visible_range(args, &lo0, &len);
     decode_plan(B, Hkv, H / Hkv * rows, len, D, compute_units > 0 ? compute_units : 256, args->kv_lens != nullptr,
                 args->dtype == FHIP_F32, &chunk, &nsplit, &waves, &workspace_splits);
     if (reported) *reported = decode_workspace_bytes(B, H * rows, Hkv, D, workspace_splits);
@@ -813,18 +818,21 @@ int fhip_flash_attention_workspace_bytes(const fhip_attn_args *args, int32_t com
     return FHIP_OK;
 }
 
+// The tensors from the first key on that the call can see: the kernels see keys lo0 .. lo0 + len as keys 0 .. len.
+static void take_visible_range(const fhip_attn_args *args, AttnParams *p) {
+    int lo0, len;
+    visible_range(args, &lo0, &len);
+    const int64_t eb = elem_bytes(args->dtype);
+    p->k = (const char *)p->k + lo0 * p->ks[2] * eb;
+    p->v = (const char *)p->v + lo0 * p->vs[2] * eb;
+    p->Skv = len;
+    p->q_pos_offset -= lo0;
+}
+
 // The plan of a split-KV decode call: the visible stretch of the cache, the split, and whether the splits are merged
 // inside the main kernel (when the device's workgroups are grouped by XCD as that form needs, see probe_xcd_grouping).
 static void plan_decode_call(fhip_device *dev, const fhip_attn_args *args, AttnParams *p) {
-    int lo0, vis_len;
-    decode_visible_range(args, &lo0, &vis_len);
-    if (lo0 > 0 || vis_len < p->Skv) {  // the kernels see keys lo0 .. lo0 + vis_len as keys 0 .. vis_len
-        const int64_t eb = elem_bytes(args->dtype);
-        p->k = (const char *)p->k + lo0 * p->ks[2] * eb;
-        p->v = (const char *)p->v + lo0 * p->vs[2] * eb;
-        p->Skv = vis_len;
-        p->q_pos_offset -= lo0;
-    }
+    take_visible_range(args, p);
     int workspace_splits;
     decode_plan(p->B, p->Hkv, p->G * p->Sq, p->Skv, p->D, dev->prop.multiProcessorCount, p->kv_lens != nullptr,
                 args->dtype == FHIP_F32, &p->chunk, &p->nsplit, &p->dec_waves, &workspace_splits);
@@ -907,6 +915,7 @@ int fhip_flash_attention(fhip_stream *s, const fhip_attn_args *args) {
         }
     }
     p.cus = s->dev->prop.multiProcessorCount;
+    if (id == FHIP_KERNEL_PREFILL_F32 || id == FHIP_KERNEL_PREFILL_MFMA) take_visible_range(args, &p);
     if (id == FHIP_KERNEL_PREFILL_F32) {
         // few query rows on a long cache: split the keys over workgroups if the caller brought the scratch for it
         int ns, chunk;
