@@ -326,9 +326,10 @@ static void f32_split_plan(const fhip_attn_args *a, int cus, int *nsplit, int *c
     int lo0, len;
     visible_range(a, &lo0, &len);
     const bool causal_square = a->analytic.enabled && a->analytic.causal && 2ll * a->q.shape[2] > len;
+    const bool uneven = causal_square || (a->mask_kind == FHIP_MASK_QK && 2ll * a->q.shape[2] > len);
     const int Hkv = (int)a->k.shape[1];
     prefill_f32_plan((int)a->q.shape[0], (int)a->q.shape[1], Hkv ? (int)a->q.shape[1] / Hkv : 1, (int)a->q.shape[2],
-                     len, (int)a->q.shape[3], causal_square, cus > 0 ? cus : 256, nsplit, chunk);
+                     len, (int)a->q.shape[3], causal_square, uneven, cus > 0 ? cus : 256, nsplit, chunk);
 }
 static size_t f32_partials_offset(const fhip_attn_args *a) { return (mask_scratch_bytes(a) + 255) & ~(size_t)255; }
 static void mfma_split_plan(const fhip_attn_args *a, int cus, int *nsplit, int *chunk) {
@@ -341,13 +342,17 @@ static void mfma_split_plan(const fhip_attn_args *a, int cus, int *nsplit, int *
     }
     const bool causal_square = a->analytic.enabled && a->analytic.causal && 2ll * a->q.shape[2] > len;
     const int Hkv = (int)a->k.shape[1];
+    const bool uneven = causal_square || (a->mask_kind == FHIP_MASK_QK && 2ll * a->q.shape[2] > len);
+    const int64_t later_rows_see = a->analytic.enabled && a->analytic.causal ? a->analytic.q_pos_offset - lo0 + a->q.shape[2]
+                                   : a->mask_kind == FHIP_MASK_QK          ? len : 0;
     if (!prefill_mfma_rows256_takes((int)a->q.shape[3], a->scale, (int)a->q.shape[0], (int)a->q.shape[1], (int)a->q.shape[2],
                                     cus > 0 ? cus : 256))  // the wide-head form: 128-row query blocks
         prefill_mfma_wide_plan((int)a->q.shape[0], (int)a->q.shape[1], Hkv ? (int)a->q.shape[1] / Hkv : 1, (int)a->q.shape[2],
                                len, causal_square, cus > 0 ? cus : 256, nsplit, chunk);
     else
-        prefill_mfma_plan((int)a->q.shape[0], (int)a->q.shape[1], Hkv ? (int)a->q.shape[1] / Hkv : 1, (int)a->q.shape[2],
-                          len, causal_square, cus > 0 ? cus : 256, nsplit, chunk);
+        prefill_mfma_plan((int)a->q.shape[0], (int)a->q.shape[1], Hkv ? (int)a->q.shape[1] / Hkv : 1, (int)a->q.shape[2], len,
+                          (int)a->q.shape[3], causal_square, uneven, later_rows_see, a->analytic.enabled ? a->analytic.window : 0, cus > 0 ? cus : 256,
+                          nsplit, chunk);
 }
 
 // A workspace too small for the planned key split still takes the largest split that fits (shares stay multiples of 64

@@ -299,9 +299,8 @@ __global__ __launch_bounds__(64 * PF32_WAVES, 2) void prefill_f32_kernel(AttnPar
 // single-pass form does in its epilogue.  A row's references m are exponents of two, or, where a mask is added to the
 // scores, in the scores' own units: those rows' sums l are parked with their sign set (-0.0 included).
 // LPR lanes share a row, four dims each: a share is one load of four values and one of (m, l).
-// Bound: the memory latency of a round of eight shares, and the partials' bytes where there are many.  One wavefront per row with six
-// loads per share before: 16-bit calls in two to eight shares take 0.92 to 0.96 of their time, f32 ones 0.97 (2 x 16 heads, 526 rows of 64 dims in
-// six shares 11.0 -> 7 us for this kernel).
+// Bound: the memory latency of a round of eight shares, and the partials' bytes where there are many.  With one wavefront per row and
+// six loads per share 16-bit calls in two to eight shares took 1.04 to 1.09 times as long in all, f32 ones 1.03.
 typedef float4_t __attribute__((aligned(8))) float4_at8_t;  // a row of the partials is D + 2 or D + 4 floats
 typedef float float2_at8_t __attribute__((ext_vector_type(2)));
 template <typename T, int LPR>
@@ -680,7 +679,7 @@ static int launch_rows(const AttnParams &p, hipStream_t stream) {
 
 // Few query rows on a long cache (a new chat turn, a prompt fed in pieces): the grid of query blocks alone leaves
 // most CUs idle, so the keys are split over workgroups as well.
-void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_square, int compute_units, int *nsplit, int *chunk) {
+void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_square, bool uneven, int compute_units, int *nsplit, int *chunk) {
     *nsplit = 1;
     *chunk = Skv;
     if (D <= 128) {
@@ -711,12 +710,37 @@ void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_s
             if (of_four >= 3) ns = of_four;
             most = most_before;
         }
-        // A call asks for at most 16 MiB of partials.  Only full grids of four-unit workgroups (256 x 128 rows) are beyond that:
+        // By this rule a call asks for at most 16 MiB of partials.  Only full grids of four-unit workgroups (256 x 128 rows) are beyond that:
         // 32, 64, 128, 256 or 512 rows of 32/8 heads at D = 128, and up to seven rows fewer.  They take half the shares on workgroups
         // of half the units, the workspace that such calls have always had, and more time for it: on 8192 keys 32 rows 49 us (40 in
         // twice the shares), 64 rows 79 (56), 128 rows 128 (96), 256 rows 244 (172), 512 rows 463 (327).
         constexpr size_t MOST_PARTIALS = (size_t)16 << 20;
         if (few_rows && D > 64 && prefill_f32_workspace_bytes(B, H, Sq, D, (int)ns) > MOST_PARTIALS) ns = shares(2);
+        // More than 128 rows that see about the same keys (chunks, images): the shares of least time, the fewest within 2 % of
+        // it, where that is 5 % less than the rule's; at most 64 MiB of partials (us a call: two sequences of 275 rows of 32/8
+        // heads at 64 on 2911 keys 116 -> 92; 16 heads without a mask, 1156 rows at 128 148 -> 80, 2506 366 -> 285, 1147 at 80 109 -> 59; over 90
+        // random calls the time is 0.91, the worst 1.03 of the rule's).  Square prompts to 768 keys keep the rule, masked or not.
+        if (!uneven && Sq > 128 && (few_rows || Skv > 768)) {
+            const TermsCall call = {B, H / G, G, Sq, Skv, D, compute_units, false};
+            constexpr int SHARES[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48};
+            double times[sizeof(SHARES) / sizeof(SHARES[0])], least = 0.0;
+            int tried = 0;
+            for (const int n : SHARES) {
+                // (shares that make three rounds of the smallest workgroups gain nothing more)
+                if (n > 1 && (Skv / n < 64 || prefill_f32_workspace_bytes(B, H, Sq, D, n) > ((size_t)64 << 20) ||
+                              (n - 1) * kv_heads * units > 6L * compute_units))
+                    break;
+                times[tried] = prefill_f32_terms_time(call, prefill_f32_terms_quickest(call, n), n);
+                if (tried == 0 || times[tried] < least) least = times[tried];
+                tried++;
+            }
+            const long ordinary = ns < 2 ? 1 : ns;
+            for (int i = 0; i < tried; i++) {
+                if (times[i] > 1.02 * least) continue;
+                if (times[i] < 0.95 * prefill_f32_terms_time(call, prefill_f32_terms_form(call, (int)ordinary), (int)ordinary)) ns = SHARES[i];
+                break;
+            }
+        }
         if (ns < 2) return;
         const long c = ((Skv + ns - 1) / ns + 31) / 32 * 32;
         *chunk = (int)c;

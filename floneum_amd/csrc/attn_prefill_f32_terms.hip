@@ -831,17 +831,99 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
         }
 }
 
-// workgroups of the form with U units each
-static long terms_workgroups(const AttnParams &p, int U) {
-    const long units = (long)p.G * ((p.Sq + 31) / 32);
-    return (units + U - 1) / U * p.B * p.Hkv * (p.pf_nsplit > 1 ? p.pf_nsplit : 1);
+// ---- which form a call takes ------------------------------------------------------------------------------------------------
+
+static long units_of(const TermsCall &c) { return (long)c.G * ((c.Sq + 31) / 32); }
+
+// workgroups of the form with U units each, in ns shares of the keys
+static long terms_workgroups(const TermsCall &c, int U, int ns) {
+    return (units_of(c) + U - 1) / U * c.B * c.Hkv * (ns > 1 ? ns : 1);
+}
+
+// The form by the numbers of its workgroups (measured on f32 calls, time per call in us; w2, w4: workgroups with 2 or 4 units):
+//   (4, 1)  two workgroups per CU, least splitting per tile: grids that fill the chip twice
+//   (4, 2)  eight wavefronts, one workgroup per CU: D = 128 1500 rows 115 against 142 for (4, 1), 4000 rows of 8 heads
+//           262 against 348, 129 rows on 8003 keys (keys split over workgroups) 111 against 133
+//   (2, 2)  D > 64: one wavefront per SIMD with 512 registers, half the units per workgroup, for short prompts (700 rows
+//           48 against 55 for (4, 2), 200 rows 21 against 24) and others that fit the CUs once.  With the keys split there is no
+//           short workgroup beside a long one unless the prompt is causal (768 rows of 8/2 heads, 288 workgroups: 33 against 36
+//           with causality, 51 against 39 without; 16/4 heads, 384 workgroups: 58 against 47).  D <= 64: two workgroups per CU;
+//           square causal prompts, whose later rows see more keys, are spread more evenly by half the units (1024 rows 38
+//           against 47 for (4, 2), 2048 rows 111 and 2560 rows 159 against 118 and 165 for (4, 1); 3072 rows 224 against 216,
+//           4096 rows 388 against 336), and up to two tiles have nothing for more than two groups (55 rows of 16/4 heads 9.4 in
+//           (2, 4), 8.0)
+//   (2, 4)  D <= 64, eight wavefronts: 512 rows 18 against 21.5 for (2, 2), 1000 rows of 16 heads without a mask 31
+//           against 38
+static TermsForm form_by_workgroups(const TermsCall &c, int ns) {
+    const int cus = c.cus;
+    const long w2 = terms_workgroups(c, 2, ns), w4 = terms_workgroups(c, 4, ns);
+    const bool few_rows = 2L * c.Sq <= c.Skv;
+    if (c.D <= 64) {
+        if (c.Skv <= 2 * PT_BN) return {2, 2};
+        if (2 * w2 <= (c.uneven ? 3L : 2L) * cus) return {2, 4};
+        if (c.uneven && 2 * w4 <= 5L * cus) return {2, 2};
+        if (!c.uneven && w4 <= cus) return {4, 2};
+    } else {
+        const bool fits = w2 <= cus || (ns > 1 ? c.uneven && 4 * w2 <= 5L * cus : !few_rows && 2 * w2 <= 3L * cus);
+        if (fits) return {2, 2};
+        if (w4 < 2L * cus) return {4, 2};
+    }
+    return {4, 1};
+}
+
+// Time of a call whose rows all see about the same keys, in us: rounds of workgroups that walk their tiles, and parking and
+// merging the shares.  Constants fitted to 210 random calls (chunks, turns, images and encoders of 8 to 32 heads at 64 to 128
+// dims, each in every form and up to 48 shares): 6 % off in the mean square.
+double prefill_f32_terms_time(const TermsCall &c, TermsForm f, int ns) {
+    const double dims = (c.D <= 64 ? 64 : c.D <= 96 ? 96 : 128) / 64.0;
+    double tile, ends, alone = 1.0;  // per tile of a group, per workgroup, and a tile's time where a CU has one of two workgroups
+    bool two_per_cu = false;
+    if (f.U == 2 && f.KG == 2 && c.D <= 64) tile = 2.65, ends = 1.4, alone = 0.71, two_per_cu = true;
+    else if (f.U == 2 && f.KG == 2) tile = 0.38 + 1.494 * dims, ends = 3.9;
+    else if (f.KG == 2) tile = 0.306 + 1.945 * dims, ends = 3.45;
+    else if (f.KG == 4) tile = 2.65, ends = 3.87;
+    else tile = 0.374 + 1.78 * dims, ends = 0.8, alone = 0.74, two_per_cu = true;
+    const int chunk = ((c.Skv + ns - 1) / ns + PT_BN - 1) / PT_BN * PT_BN, n = (c.Skv + chunk - 1) / chunk;
+    const double walk = tile * ((chunk / PT_BN + f.KG - 1) / f.KG);
+    const long wgs = terms_workgroups(c, f.U, n), slots = (two_per_cu ? 2L : 1L) * c.cus, rest = wgs % slots;
+    double us = 4.9 + wgs / slots * (ends + walk);
+    if (rest) us += ends + walk * (rest <= c.cus ? alone : 1.0);
+    if (n > 1) us += 3.24 + 0.456e-6 * prefill_f32_workspace_bytes(c.B, c.Hkv * c.G, c.Sq, c.D, n);
+    return us;
+}
+
+TermsForm prefill_f32_terms_quickest(const TermsCall &c, int ns) {
+    TermsForm best = {4, 1};
+    double least = prefill_f32_terms_time(c, best, ns);
+    for (const TermsForm f : {TermsForm{4, 2}, TermsForm{2, 2}, TermsForm{2, 4}}) {
+        if (f.KG == 4 && c.D > 64) continue;
+        const double us = prefill_f32_terms_time(c, f, ns);
+        if (us < least) least = us, best = f;
+    }
+    return best;
+}
+
+// Where all rows see about the same keys the rule above leaves much to gain, and the form is the quickest by the time above if that
+// is 7 % better (us a call: 16 heads without a mask, 1356 rows at 128 169 -> 99; 6 encoder sequences of 436 tokens 41.5 -> 30.6, 11
+// of 169 23.2 -> 18.4).  Up to 128 rows the rule is as good.
+TermsForm prefill_f32_terms_form(const TermsCall &c, int ns) {
+    const TermsForm ordinary = form_by_workgroups(c, ns);
+    if (c.uneven || c.Sq <= 128 || c.Skv <= 2 * PT_BN) return ordinary;
+    const TermsForm other = prefill_f32_terms_quickest(c, ns);
+    return prefill_f32_terms_time(c, other, ns) < 0.93 * prefill_f32_terms_time(c, ordinary, ns) ? other : ordinary;
+}
+
+// (rows of a square prompt under a causal mask, for which a mask tensor is taken, see from one to all of the keys)
+static TermsCall terms_call(const AttnParams &p) {
+    const bool uneven = 2L * p.Sq > p.Skv && (p.causal || p.mask_kind == FHIP_MASK_QK);
+    return {p.B, p.Hkv, p.G, p.Sq, p.Skv, p.D, p.cus > 0 ? p.cus : 256, uneven};
 }
 
 template <typename T, int U, int KG, int MODE>
 static int launch_form(const AttnParams &p_in, hipStream_t stream) {
     AttnParams p = p_in;
     const int cus = p.cus > 0 ? p.cus : 256;
-    const long blocks = terms_workgroups(p, U);
+    const long blocks = terms_workgroups(terms_call(p), U, p.pf_nsplit);
     if (blocks > 0x7fffffffL) {
         set_error("prefill f32: too many workgroups (%ld)", blocks);
         return FHIP_ERR_UNSUPPORTED;
@@ -878,34 +960,12 @@ static int launch_form(const AttnParams &p_in, hipStream_t stream) {
 
 template <typename T, int MODE>
 static int launch_terms(const AttnParams &p, hipStream_t stream) {
-    const int cus = p.cus > 0 ? p.cus : 256;
-    // Which form (measured on f32 calls, time per call in us; w2, w4: workgroups with 2 or 4 units):
-    //   (4, 1)  two workgroups per CU, least splitting per tile: grids that fill the chip twice
-    //   (4, 2)  eight wavefronts, one workgroup per CU: D = 128 1500 rows 115 against 142 for (4, 1), 4000 rows of 8 heads
-    //           262 against 348, 129 rows on 8003 keys (keys split over workgroups) 111 against 133
-    //   (2, 2)  D > 64: one wavefront per SIMD with 512 registers, half the units per workgroup, for short prompts (700 rows
-    //           48 against 55 for (4, 2), 200 rows 21 against 24) and others that fit the CUs once.  With the keys split there is no
-    //           short workgroup beside a long one unless the prompt is causal (768 rows of 8/2 heads, 288 workgroups: 33 against 36
-    //           with causality, 51 against 39 without; 16/4 heads, 384 workgroups: 58 against 47).  D <= 64: two workgroups per CU;
-    //           square causal prompts, whose later rows see more keys, are spread more evenly by half the units (1024 rows 38
-    //           against 47 for (4, 2), 2048 rows 111 and 2560 rows 159 against 118 and 165 for (4, 1); 3072 rows 224 against 216,
-    //           4096 rows 388 against 336)
-    //   (2, 4)  D <= 64, eight wavefronts: 512 rows 18 against 21.5 for (2, 2), 1000 rows of 16 heads without a mask 31
-    //           against 38
-    // 16-bit storage takes (4, 1) always.
+    // 16-bit storage takes (4, 1) always
     if constexpr (sizeof(T) == 4) {
-        const long w2 = terms_workgroups(p, 2), w4 = terms_workgroups(p, 4);
-        // rows of a square prompt under a causal mask (a mask tensor is taken for one) see from one to all of the keys
-        const bool few_rows = 2L * p.Sq <= p.Skv, uneven = !few_rows && (p.causal || p.mask_kind == FHIP_MASK_QK);
-        if (p.D <= 64) {
-            if (2 * w2 <= (uneven ? 3L : 2L) * cus) return launch_form<T, 2, 4, MODE>(p, stream);
-            if (uneven && 2 * w4 <= 5L * cus) return launch_form<T, 2, 2, MODE>(p, stream);
-            if (!uneven && w4 <= cus) return launch_form<T, 4, 2, MODE>(p, stream);
-        } else {
-            const bool fits = w2 <= cus || (p.pf_nsplit > 1 ? uneven && 4 * w2 <= 5L * cus : !few_rows && 2 * w2 <= 3L * cus);
-            if (fits) return launch_form<T, 2, 2, MODE>(p, stream);
-            if (w4 < 2L * cus) return launch_form<T, 4, 2, MODE>(p, stream);
-        }
+        const TermsForm f = prefill_f32_terms_form(terms_call(p), p.pf_nsplit > 1 ? p.pf_nsplit : 1);
+        if (f.U == 2 && f.KG == 4) return launch_form<T, 2, 4, MODE>(p, stream);
+        if (f.U == 2) return launch_form<T, 2, 2, MODE>(p, stream);
+        if (f.KG == 2) return launch_form<T, 4, 2, MODE>(p, stream);
     }
     return launch_form<T, 4, 1, MODE>(p, stream);
 }

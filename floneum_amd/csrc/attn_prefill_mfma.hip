@@ -775,13 +775,30 @@ int prefill_mfma_pack(int B, int H, int G, int Sq, int Skv, int compute_units) {
     return 2 * (long)B * (H / 4) * shares >= compute_units ? 4 : 0;
 }
 
-void prefill_mfma_plan(int B, int H, int G, int Sq, int Skv, bool causal_square, int compute_units, int *nsplit, int *chunk) {
+// Time of a call in us, by the form it takes in that many shares: rounds of workgroups that walk their tiles, and parking and
+// merging the shares.  Constants fitted to 140 random calls (chunks, turns and images of 8 to 32 heads at 64 to 128 dims, each in both
+// forms and up to 48 shares): 10 % off in the mean square.
+static double prefill_mfma_time(int B, int H, int G, int Sq, int Skv, int D, int64_t later_rows_see, int64_t window, int compute_units, int ns) {
+    const int c = ((Skv + ns - 1) / ns + PF_BN - 1) / PF_BN * PF_BN, n = (Skv + c - 1) / c;
+    const int bm = prefill_mfma_block_rows(B, H, Sq, Skv, n, later_rows_see, window, compute_units);
+    const bool ks = bm == PF_BM / 2, packed = ks && prefill_mfma_pack(B, H, G, Sq, Skv, compute_units);
+    const long wgs = (long)B * (packed ? H / 4 : H) * ((Sq + bm - 1) / bm) * n, rounds = (wgs + compute_units - 1) / compute_units;
+    const double dims = D <= 64 ? 1.0 : D <= 96 ? 1.43 : 1.86;
+    double us = 4.6 + rounds * (ks ? 5.3 + 0.356 * dims * (c / PF_BN) : 3.9 + 0.579 * dims * (c / PF_BN));
+    if (n > 1) us += 3.0 + 0.488e-6 * prefill_mfma_workspace_bytes(B, H, Sq, D, n);
+    return us;
+}
+
+// uneven: a square call whose rows see the keys up to their own position (a mask tensor is taken for one): by the rules alone.
+// later_rows_see, window: as for prefill_mfma_block_rows.
+void prefill_mfma_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_square, bool uneven, int64_t later_rows_see, int64_t window,
+                       int compute_units, int *nsplit, int *chunk) {
     *nsplit = 1;
     *chunk = Skv;
     if (causal_square) return;
     const long wgs = (long)B * (prefill_mfma_pack(B, H, G, Sq, Skv, compute_units) ? H / 4 : H) * ((Sq + PF_BM - 1) / PF_BM);
-    if (2 * wgs > compute_units) return;  // the query blocks alone keep at least half the chip busy: parking and
-                                          // merging partial results would cost more than it gains (measured)
+    if (wgs == 0) return;
+    // While the query blocks alone keep at least half the chip busy, parking and merging partial results costs more than it gains.
     const long want = (2L * compute_units + wgs - 1) / wgs;
     long most = Skv / 1024;
     // A few rows on a short cache: shares down to 512 keys, and for up to 64 rows to 256, while CUs would stay without a
@@ -790,7 +807,27 @@ void prefill_mfma_plan(int B, int H, int G, int Sq, int Skv, bool causal_square,
     const bool few_rows = 2L * Sq <= Skv && (Sq <= 64 || Skv >= 2048);
     if (few_rows && (want < most ? want : most) * wgs < compute_units) most = Skv / 512;
     if (few_rows && Sq <= 64 && (want < most ? want : most) * wgs < compute_units) most = Skv / 256;
-    long ns = want < most ? want : most;
+    long ns = 2 * wgs > compute_units ? 1 : want < most ? want : most;
+    if (ns < 1) ns = 1;
+    // These rules count workgroups and not their rounds, nor the bytes of the partials: the shares of least time by the function
+    // above, the fewest within 1 % of it, are taken where that is 5 % less than the rules' (us a call: four sequences of 207 rows of
+    // 32/8 heads at 96 under a window of 4096 84 -> 56 in none; 189 rows of 8/4 heads at 80 on 1993 keys 23.5 -> 19, 231 of 32/8 at 64 on 14900
+    // 59 -> 48, 49 of 32/32 at 128 on 3032 36 -> 22; over 140 random calls 0.93 of the rules' time, the worst 1.06).
+    constexpr int SHARES[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48};
+    double times[sizeof(SHARES) / sizeof(SHARES[0])], least = 0.0;
+    int tried = 0;
+    for (const int n : SHARES) {
+        if (uneven) break;
+        if (n > 1 && (Skv / n < 128 || (n - 1) * wgs > 3L * compute_units)) break;  // (three rounds gain nothing more)
+        times[tried] = prefill_mfma_time(B, H, G, Sq, Skv, D, later_rows_see, window, compute_units, n);
+        if (tried == 0 || times[tried] < least) least = times[tried];
+        tried++;
+    }
+    for (int i = 0; i < tried; i++) {
+        if (times[i] > 1.01 * least) continue;
+        if (times[i] < 0.95 * prefill_mfma_time(B, H, G, Sq, Skv, D, later_rows_see, window, compute_units, (int)ns)) ns = SHARES[i];
+        break;
+    }
     if (ns < 2) return;
     long c = (Skv + ns - 1) / ns;
     c = (c + PF_BN - 1) / PF_BN * PF_BN;

@@ -488,7 +488,8 @@ void prefill_mfma_wide_plan(int B, int H, int G, int Sq, int Skv, bool causal_sq
     if (wgs >= places) return;
     // The share count that needs the fewest tile steps: rounds of `places` workgroups, each walking its share of the
     // keys tile by tile, plus a few steps for parking and merging the partial results of a split.
-    const long most = Skv / 1024 < 64 ? Skv / 1024 : 64;
+    // Shares of at least 1024 keys, or up to four of 512.
+    const long most = Skv / 1024 > 64 ? 64 : Skv / 1024 > 4 ? Skv / 1024 : Skv / 512 < 4 ? Skv / 512 : 4;
     long best_ns = 1, best_cost = (Skv + PW_KEYS - 1) / PW_KEYS;
     for (long ns = 2; ns <= most; ns++) {
         const long rounds = (wgs * ns + places - 1) / places;

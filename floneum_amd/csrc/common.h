@@ -66,10 +66,23 @@ struct AttnParams {
 };
 
 // the key split of a tiled f32 prefill call (1 = none) and the scratch it needs
-void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_square, int compute_units, int *nsplit, int *chunk);
+// uneven: a square call whose rows see the keys up to their own position (a mask tensor is taken for one)
+void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_square, bool uneven, int compute_units, int *nsplit, int *chunk);
+// The forms of the f32 terms kernel (attn_prefill_f32_terms.hip): units and key groups per workgroup, and what a call takes in them
+struct TermsCall {
+    int B, Hkv, G, Sq, Skv, D, cus;
+    bool uneven;
+};
+struct TermsForm {
+    int U, KG;
+};
+double prefill_f32_terms_time(const TermsCall &call, TermsForm form, int key_shares);  // us, of calls that are not uneven
+TermsForm prefill_f32_terms_quickest(const TermsCall &call, int key_shares);           // by that time
+TermsForm prefill_f32_terms_form(const TermsCall &call, int key_shares);               // the one that runs
 size_t prefill_f32_workspace_bytes(int B, int H, int Sq, int D, int nsplit);
 // the same for the 16-bit matrix-core prefill kernel (256-row query blocks, one workgroup per CU)
-void prefill_mfma_plan(int B, int H, int G, int Sq, int Skv, bool causal_square, int compute_units, int *nsplit, int *chunk);
+void prefill_mfma_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_square, bool uneven, int64_t later_rows_see,
+                       int64_t window, int compute_units, int *nsplit, int *chunk);
 // query heads that share one workgroup's K/V tiles (0: one head per workgroup)
 int prefill_mfma_pack(int B, int H, int G, int Sq, int Skv, int compute_units);
 size_t prefill_mfma_workspace_bytes(int B, int H, int Sq, int D, int nsplit);

@@ -1,0 +1,96 @@
+"""Calls whose rows all see about the same keys (chunks of a prompt, follow-up messages, images): into how many shares their keys go,
+by the workspace the library asks for, and such calls against the formula in 64 bits, into outputs of any stride and type.
+
+Tolerance: 16-bit results as in tests/test_prefill_mfma_forms_gpu.py.  In f32 a score sums D products in terms of which each is
+exact, 2^-24 and less of its size apart from a rounding per slice of 16, the probabilities and the shares' sums round a dozen times each:
+40 roundings of 2^-24 and either sign bound the relative L2 by 40^0.5 2^-24 = 3.8e-7; twice that.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+import floneum_amd as fa
+from test_abi import make_args
+
+CUS = 256
+
+
+def shares(B, H, Hkv, Sq, Skv, D, dtype, causal=True, window=0):
+    a, need = make_args(B=B, H=H, Hkv=Hkv, Sq=Sq, Skv=Skv, D=D, dtype=dtype), ctypes.c_size_t()
+    if causal:
+        a.analytic.enabled, a.analytic.causal, a.analytic.q_pos_offset, a.analytic.window = 1, 1, Skv - Sq, window
+    assert fa.lib().fhip_flash_attention_workspace_bytes(ctypes.byref(a), CUS, ctypes.byref(need)) == fa.OK
+    per = B * H * Sq * (D + (2 if dtype == fa.F32 else 4)) * 4
+    assert need.value % per == 0
+    return need.value // per
+
+
+@pytest.mark.parametrize("call, want", [
+    # 16-bit: short views of more than 64 rows, full rounds of workgroups, no split where one round is there already
+    ((1, 8, 4, 189, 1993, 80, fa.F16), 8), ((4, 32, 8, 207, 4303, 96, fa.F16), 0), ((1, 32, 32, 49, 3032, 128, fa.BF16), 8),
+    ((1, 32, 8, 231, 14900, 64, fa.F16), 8), ((1, 16, 16, 4096, 4096, 80, fa.F16, False), 0),
+    # f32: even rows in the shares of least time; up to 128 rows, squares and up to 768 keys by the former rule
+    ((2, 32, 8, 275, 2911, 64, fa.F32), 3), ((1, 16, 16, 1156, 1156, 128, fa.F32, False), 3), ((1, 16, 16, 1156, 1156, 128, fa.F32), 0),
+    ((1, 16, 16, 768, 768, 128, fa.F32, False), 2), ((1, 32, 8, 128, 8192, 128, fa.F32), 4), ((1, 32, 8, 129, 8003, 128, fa.F32), 6),
+    # above 128 dims: up to four shares of 512 keys
+    ((1, 16, 4, 141, 2659, 256, fa.BF16), 4), ((1, 16, 4, 141, 1000, 256, fa.BF16), 0),
+])
+def test_shares(call, want):
+    assert shares(*call) == want
+
+
+@pytest.mark.parametrize("D, dtype", [(64, fa.F32), (96, fa.F32), (256, fa.F32), (64, fa.F16), (128, fa.BF16), (256, fa.F16)])
+@pytest.mark.parametrize("before", [0, 1, 127, 128, 4000, 20000])
+def test_a_window_is_planned_on_its_keys(D, dtype, before):
+    """A view with more keys in front of the window asks for what the window's own keys ask for, to the next 128."""
+    rows, window = 300, 2048
+    seen = rows + window - 1
+    got = shares(2, 16, 4, rows, before + seen, D, dtype, window=window)
+    assert got in {shares(2, 16, 4, rows, n, D, dtype) for n in range(seen, seen + 128)}
+
+
+def tensor(device, rng, dtype, shape):
+    return fa.Tensor.from_numpy(device, rng.normal(0, 1, shape).astype(np.float32), dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype, B, H, Hkv, Sq, Skv, D, causal, window", [
+    (fa.F16, 1, 8, 4, 189, 1993, 80, True, 0), (fa.BF16, 1, 4, 4, 65, 1291, 128, True, 0), (fa.F16, 1, 4, 2, 201, 3333, 64, True, 700),
+    (fa.F16, 2, 4, 1, 33, 1409, 96, True, 0), (fa.BF16, 1, 4, 4, 300, 1000, 72, False, 0), (fa.F16, 1, 4, 2, 140, 1999, 256, True, 0),
+    (fa.F32, 1, 4, 2, 275, 2911, 64, True, 0), (fa.F32, 1, 4, 4, 1156, 1156, 128, False, 0), (fa.F32, 1, 8, 2, 131, 3000, 80, True, 900),
+    (fa.F32, 1, 2, 2, 129, 1025, 36, False, 0), (fa.F32, 2, 4, 2, 150, 900, 256, True, 0),
+])
+@pytest.mark.parametrize("out", ["contiguous", "turned", "odd rows", "every second"])
+def test_shared_keys(device, dtype, B, H, Hkv, Sq, Skv, D, causal, window, out):
+    """Every form of the merge's stores: rows of four, rows that are not aligned, elements apart; f32 results of 16-bit calls."""
+    rng = np.random.default_rng(Sq * 31 + Skv)
+    q, k, v = tensor(device, rng, dtype, (B, H, Sq, D)), tensor(device, rng, dtype, (B, Hkv, Skv, D)), tensor(device, rng, dtype, (B, Hkv, Skv, D))
+    analytic = (True, Skv - Sq, window) if causal else None
+    out_dtype = fa.F32 if out in ("turned", "every second") else dtype
+    if out == "odd rows":
+        o = fa.Tensor.from_numpy(device, np.full((B, H, Sq, D + 1), 7.0, np.float32), out_dtype)
+        view = fa.Tensor(o.buffer, out_dtype, (B, H, Sq, D), o.strides, 1)
+    elif out == "every second":
+        o = fa.Tensor.from_numpy(device, np.full((B, H, Sq, 2 * D), 7.0, np.float32), out_dtype)
+        view = fa.Tensor(o.buffer, out_dtype, (B, H, Sq, D), o.strides[:3] + (2,), 0)
+    else:
+        o = fa.Tensor.from_numpy(device, np.full((B, Sq, H, D) if out == "turned" else (B, H, Sq, D), 7.0, np.float32), out_dtype)
+        view = o.transpose(1, 2) if out == "turned" else o
+    q.flash_attention(k, v, D ** -0.5, analytic=analytic, out_dtype=out_dtype, out=view)
+    whole = np.asarray(o.to_numpy(), np.float64)
+    got = whole[..., 1:] if out == "odd rows" else whole[..., ::2] if out == "every second" else whole.transpose(0, 2, 1, 3) if out == "turned" else whole
+    if out == "odd rows":
+        assert np.all(whole[..., 0] == 7.0)
+    if out == "every second":
+        assert np.all(whole[..., 1::2] == 7.0)
+    a, b, c = (np.asarray(t.to_numpy(), np.float64) for t in (q, k, v))
+    b, c = (np.repeat(t, H // Hkv, axis=1) for t in (b, c))
+    s = a @ b.transpose(0, 1, 3, 2) * D ** -0.5
+    if causal:
+        i, j = np.arange(Sq)[:, None] + Skv - Sq, np.arange(Skv)[None, :]
+        s = np.where((j > i) | ((j + window <= i) if window else False), -np.inf, s)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    ref = (p / p.sum(-1, keepdims=True)) @ c
+    err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    assert err <= {fa.F32: 7.6e-7, fa.F16: 2.0 ** -10, fa.BF16: 2.0 ** -7}[dtype], f"relative L2 {err:.2e}"
