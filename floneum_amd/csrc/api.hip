@@ -842,12 +842,12 @@ static void plan_decode_call(fhip_device *dev, const fhip_attn_args *args, AttnP
     decode_plan(p->B, p->Hkv, p->G * p->Sq, p->Skv, p->D, dev->prop.multiProcessorCount, p->kv_lens != nullptr,
                 args->dtype == FHIP_F32, &p->chunk, &p->nsplit, &p->dec_waves, &workspace_splits);
     int stride;
-    size_t ctr_off;
+    size_t marks_off;
     p->dec_fused = 0;
-    if (dev->xcd_grouped.load() && decode_fused_layout(*p, args->dtype == FHIP_F32, &stride, &ctr_off)) {
+    if (dev->xcd_grouped.load() && decode_fused_layout(*p, args->dtype == FHIP_F32, &stride, &marks_off)) {
         p->dec_fused = 1;
         p->dec_unit_stride = stride;
-        p->dec_counters_offset = ctr_off;
+        p->dec_marks_offset = marks_off;
     }
 }
 
@@ -1036,7 +1036,7 @@ int fhip_flash_attention(fhip_stream *s, const fhip_attn_args *args) {
                     return FHIP_ERR_HIP;
                 }
                 if (p.dec_fused) {
-                    p.dec_counters = (uint32_t *)((char *)args->workspace + p.dec_counters_offset);
+                    p.dec_marks = (uint32_t *)((char *)args->workspace + p.dec_marks_offset);
                     p.dec_trip = dev->trip_dev;
                     do p.dec_tag = dev->next_tag.fetch_add(1, std::memory_order_relaxed) & 0xfffffu;
                     while (p.dec_tag == 0);

@@ -30,6 +30,8 @@ namespace fhip {
 constexpr int DEC_WAVES = 4;
 constexpr int DEC_UNROLL = 4;
 constexpr float LOG2E = 1.4426950408889634f;
+typedef float4_t __attribute__((aligned(8))) float4_at8_t;  // a row of the partials is D + 2 floats
+typedef float float2_at8_t __attribute__((ext_vector_type(2)));
 
 // the matrix-core variants: 16-bit tensors on the 16-bit instruction at every multiple of 32 up to 256, f32 tensors on
 // the f32 one likewise, except that at 224 and 256 a step of up to four columns per KV head (a plain decode step of a
@@ -152,7 +154,7 @@ void decode_plan(int B, int Hkv, int G, int Skv, int D, int compute_units, bool 
 }
 
 // Workspace: the partials, B * H * nsplit * (D + 2) floats (H counts (head, row) pairs), plus what the fused merge adds:
-// every split's partials start on a 128-byte line, and one arrival counter per unit behind them.
+// every split's partials start on a 128-byte line, and the marks of its units' arrivals behind them, a word per split.
 size_t decode_workspace_bytes(int B, int H, int Hkv, int D, int nsplit) {
     if (nsplit <= 1) return 0;
     // columns of a KV head, padded to whole column blocks of 16 or 32 where there is more than one block
@@ -167,9 +169,9 @@ size_t decode_workspace_bytes(int B, int H, int Hkv, int D, int nsplit) {
 }
 
 // The fused merge (the matrix-core variants with p.dec_fused): 2 to 8 splits, equal lengths.
-// *unit_stride: floats between the partials of consecutive units; *counters_offset: bytes from the workspace's start
-// to the arrival counters.
-bool decode_fused_layout(const AttnParams &p, bool f32, int *unit_stride, size_t *counters_offset) {
+// *unit_stride: floats between the partials of consecutive units; *marks_offset: bytes from the workspace's start
+// to the marks.
+bool decode_fused_layout(const AttnParams &p, bool f32, int *unit_stride, size_t *marks_offset) {
     const int cols = p.G * p.Sq;
     if (!decode_use_mfma(p.D, f32, cols) || p.nsplit < 2 || p.nsplit > 8 || p.kv_lens) return false;
     const int gt = decode_gt(cols, p.D, f32);
@@ -177,7 +179,7 @@ bool decode_fused_layout(const AttnParams &p, bool f32, int *unit_stride, size_t
     const long stride = p.nsplit * (((long)(cols < gt ? cols : gt) * (p.D + 2) + 31) / 32 * 32);
     if ((units + 7) / 8 * 8 * p.nsplit > 0x7fffffffL || stride > 0x7fffffffL) return false;
     *unit_stride = (int)stride;
-    *counters_offset = ((size_t)units * stride * sizeof(float) + 255) & ~(size_t)255;
+    *marks_offset = ((size_t)units * stride * sizeof(float) + 255) & ~(size_t)255;
     return true;
 }
 
@@ -532,10 +534,10 @@ __device__ __forceinline__ float quad_rows_sum(float x) {
 // before), so workgroups with the same L % 8 share an XCD whether the device has 8, 4, 2 or 1 of them (checked per
 // device before the form is ever chosen).  Their partials then meet in that XCD's L2 and the last workgroup of the unit
 // to arrive merges them: no second kernel, whose dependent launch costs a few microseconds (batch 16 x 4096 keys, f16:
-// 47.1 -> 46.3 us per step; head_dim 256: 54.3 -> 52.2).  The arrival counter itself is kept coherent over the whole
-// device (with partials AND counter device-coherent the form is slower than two kernels) and carries the XCC id of the
-// first workgroup to arrive: a workgroup that arrives from another XCD sets the host-visible word p.dec_trip, which
-// fails the device's next decode call and switches the form off.
+// 47.1 -> 46.3 us per step; head_dim 256: 54.3 -> 52.2).  Only the marks of the arrivals are kept coherent over the whole device
+// (with the partials device-coherent too the form is slower than two kernels), with the XCC id of the workgroup: one that
+// finds a mark from another XCD sets the host-visible word p.dec_trip, which fails the device's next decode call and switches the
+// form off.
 __device__ __forceinline__ uint32_t xcc_id() {
     uint32_t x;
     asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(x));
@@ -572,63 +574,102 @@ __device__ __forceinline__ float *fused_partial_row(const AttnParams &p, int uni
     return (float *)p.partials + (int64_t)unit * p.dec_unit_stride + split * (p.dec_unit_stride / p.nsplit) + hh * (D + 2);
 }
 
-// After every thread of the workgroup has stored its part of the unit's partials: count the arrival; the last
-// workgroup of the unit merges the splits in order with the arithmetic of decode_combine_kernel (same bits) and
-// writes the output rows.  Every access is served by this XCD's L2: the stores have been acknowledged by it before
-// the arrival is counted (an atomic in the same L2), and the last workgroup reads lines nobody on its CU has read in
-// this launch (every split's partials have whole lines to themselves, one writer and one reader).  Nothing spins: a workgroup that
-// is not the last leaves.  The counter holds (tag << 8) | arrivals with a tag unique to the call, so it needs no
-// clearing: whatever else it holds (another call's count, the finished count of a replay of this call) restarts it.
+// After every thread of the workgroup has stored its part of the unit's partials: mark the arrival; a workgroup that finds that the
+// whole unit has arrived merges the splits in order with the arithmetic of decode_combine_kernel (same bits) and writes the output
+// rows.  Partials are served by this XCD's L2: the stores have been acknowledged by it before the arrival is marked, and the merging
+// workgroup reads lines nobody on its CU has read in this launch (every split's partials have whole lines to themselves).  Nothing
+// spins: a workgroup that finds others missing leaves.  Marks are kept coherent over the whole device and carry the XCC id, so that
+// a unit whose workgroups are NOT on one XCD is seen, and a tag unique to the call, so that whatever else their words hold (another
+// call's data) is no mark.
+//  - Two or three splits count in one word, by compare-and-swap: one round trip, and hardly ever a second one.  The finished count of
+//    a replay of the recorded call restarts it.
+//  - More would retry each other (8 splits of 128 keys, f16, 16/16 heads at 128: 14.1 us a call; 7 of B4, 64: 15.3): every split has a
+//    word of its own, stored, acknowledged, and only then are the unit's words read, so that of any two workgroups at least one sees
+//    the other's mark, and the last one all (two may, and write the same results).  One that sees all clears them for a replay.  (8.2 us
+//    and 9.1; two kernels 8.9 and 9.8.)
 template <typename T, int THREADS>
-__device__ __forceinline__ void fused_merge_tail(const AttnParams &p, int unit, int nh, int D, int b, int g, int c0, int rows) {
-    __shared__ int is_last;
+__device__ __forceinline__ void fused_merge_tail(const AttnParams &p, int unit, int split, int nh, int D, int b, int g, int c0, int rows) {
+    __shared__ int all_here;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (threadIdx.x == 0) {
-        // word: tag (20 bits) | XCC id of the first workgroup to arrive (4) | arrivals (8)
-        uint32_t *ctr = p.dec_counters + unit;
-        const uint32_t tag = p.dec_tag & 0xfffffu, xcc = xcc_id();
-        const uint32_t fresh = (tag << 12) | (xcc << 8) | 1u;
-        uint32_t cur = (tag << 12) | (xcc << 8), want;
-        do {
-            want = ((cur >> 12) == tag && (cur & 255u) < (uint32_t)p.nsplit) ? cur + 1 : fresh;
-        } while (!__hip_atomic_compare_exchange_strong(ctr, &cur, want, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                       __HIP_MEMORY_SCOPE_AGENT));
-        // the count is kept coherent over the whole device, so a unit whose workgroups are NOT on one XCD is seen here
-        if (((want >> 8) & 15u) != xcc) __hip_atomic_store(p.dec_trip, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        is_last = (want & 255u) == (uint32_t)p.nsplit;
+    uint32_t *const marks = p.dec_marks + (int64_t)unit * p.nsplit;
+    const uint32_t tag = p.dec_tag << 12, xcc = xcc_id() << 8;
+    if (p.nsplit <= 3) {
+        if (threadIdx.x == 0) {
+            // word: tag (20 bits) | XCC id of the first workgroup to arrive (4) | arrivals (8)
+            uint32_t cur = tag | xcc, want;
+            do {
+                want = (cur & ~0xfffu) == tag && (cur & 255u) < (uint32_t)p.nsplit ? cur + 1 : tag | xcc | 1u;
+            } while (!__hip_atomic_compare_exchange_strong(marks, &cur, want, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+            if ((want & 0xf00u) != xcc) __hip_atomic_store(p.dec_trip, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            all_here = (want & 255u) == (uint32_t)p.nsplit;
+        }
+    } else if (threadIdx.x < 64) {
+        // a split's word: tag (20 bits) | XCC id of its workgroup (4) | 1
+        const int lane = threadIdx.x;
+        const bool mine = lane < p.nsplit;
+        if (lane == 0) __hip_atomic_store(marks + split, tag | xcc | 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        const uint32_t mark = mine ? __hip_atomic_load(marks + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : tag | xcc | 1u;
+        const bool there = (mark & ~0xf00u) == (tag | 1u), all = __builtin_amdgcn_ballot_w64(!there) == 0;
+        if (there && (mark & 0xf00u) != xcc) __hip_atomic_store(p.dec_trip, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (all && mine) __hip_atomic_store(marks + lane, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (lane == 0) all_here = all;
     }
     __syncthreads();
-    if (!is_last) return;
+    if (!all_here) return;
     const float *wu = (const float *)p.partials + (int64_t)unit * p.dec_unit_stride;
-    const int split_stride = p.dec_unit_stride / p.nsplit;
-    for (int idx = threadIdx.x; idx < nh * D; idx += THREADS) {
-        const int hh = idx / D, d = idx % D;
-        float ms[8], ls[8], as[8];
+    const int split_stride = p.dec_unit_stride / p.nsplit, pieces = D / 4;
+    for (int idx = threadIdx.x; idx < nh * pieces; idx += THREADS) {
+        const int hh = idx / pieces, d = 4 * (idx % pieces);
+        float ms[8], ls[8];
+        float4_t as[8];
 #pragma unroll
         for (int u = 0; u < 8; u++) {
             const bool ok = u < p.nsplit;
             const float *src = wu + (ok ? u : 0) * split_stride + hh * (D + 2);
-            ms[u] = ok ? src[D] : -INFINITY;
-            ls[u] = ok ? src[D + 1] : 0.0f;
-            as[u] = ok ? src[d] : 0.0f;
+            const float2_at8_t ml = *(const float2_at8_t *)(src + D);
+            as[u] = *(const float4_at8_t *)(src + d);
+            ms[u] = ok ? ml[0] : -INFINITY;
+            ls[u] = ok ? ml[1] : 0.0f;
+            if (!ok) as[u] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
         }
         float Mn = -INFINITY;
 #pragma unroll
         for (int u = 0; u < 8; u++) Mn = fmaxf(Mn, ms[u]);
         const float Ms = (Mn == -INFINITY) ? 0.0f : Mn;
-        float L = 0.0f, A = 0.0f;
+        float L = 0.0f;
+        float4_t A = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int u = 0; u < 8; u++) {
             const float w = __builtin_amdgcn_exp2f(ms[u] - Ms);
             L += w * ls[u];
-            A += w * as[u];
+#pragma unroll
+            for (int e = 0; e < 4; e++) A[e] += w * as[u][e];
         }
-        const int h = g * p.G + (c0 + hh) / rows, qr = (c0 + hh) % rows;
-        const float val = A / L;  // no visible key: 0/0 = NaN like the reference
+        int h = g * p.G + c0 + hh, qr = 0;
+        if (rows > 1) h = g * p.G + (c0 + hh) / rows, qr = (c0 + hh) % rows;
         const int64_t oi = b * p.os[0] + h * p.os[1] + qr * p.os[2] + d * p.os[3];
-        if (p.out_f32) ((float *)p.out)[oi] = val;
-        else ((T *)p.out)[oi] = from_float<T>(val);
+#pragma unroll
+        for (int e = 0; e < 4; e++) A[e] /= L;  // no visible key: 0/0 = NaN like the reference
+        const bool f32 = sizeof(T) == 4 || p.out_f32;
+        char *const at = (char *)p.out + oi * (f32 ? 4 : 2);
+        if (p.os[3] == 1 && ((uintptr_t)at & (f32 ? 15 : 7)) == 0) {
+            if (f32) {
+                *(float4_t *)at = A;
+            } else if constexpr (sizeof(T) == 2) {
+                const T four[4] = {from_float<T>(A[0]), from_float<T>(A[1]), from_float<T>(A[2]), from_float<T>(A[3])};
+                uint2_t w;
+                __builtin_memcpy(&w, four, 8);
+                *(uint2_t *)at = w;
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                if (f32) ((float *)p.out)[oi + e * p.os[3]] = A[e];
+                else ((T *)p.out)[oi + e * p.os[3]] = from_float<T>(A[e]);
+            }
+        }
     }
 }
 
@@ -939,7 +980,7 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 8 / WAVES) void decode_mf
             }
         }
     }
-    if (p.dec_fused && p.nsplit > 1) fused_merge_tail<T, 64 * WAVES>(p, unit, nh, D, b, g, c0, rows);
+    if (p.dec_fused && p.nsplit > 1) fused_merge_tail<T, 64 * WAVES>(p, unit, split, nh, D, b, g, c0, rows);
 }
 
 // ---- pass 1, matrix-core variant for f32 tensors -------------------------------------------------------
@@ -1237,7 +1278,7 @@ __global__ __launch_bounds__(64 * DEC_WAVES, D > 128 ? 1 : D == 96 && CB == 1 ? 
             }
         }
     }
-    if (p.dec_fused && p.nsplit > 1) fused_merge_tail<float, 64 * DEC_WAVES>(p, unit, nh, D, b, g, c0, rows);
+    if (p.dec_fused && p.nsplit > 1) fused_merge_tail<float, 64 * DEC_WAVES>(p, unit, split, nh, D, b, g, c0, rows);
 }
 
 // ---- pass 2 -------------------------------------------------------------------------------------

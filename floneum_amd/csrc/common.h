@@ -33,9 +33,9 @@ struct AttnParams {
     // unit run on one XCD, park their partials in that XCD's L2 and the last one to arrive merges them.
     int32_t dec_fused;        // 0: two kernels
     int32_t dec_unit_stride;  // floats between the partials of consecutive units (a multiple of 32: 128-byte lines)
-    uint32_t dec_tag;         // unique to the call (20 bits are used): arrival counters need no clearing
-    uint32_t *dec_counters;   // [units] arrival counters: tag | XCC id of the first arrival | arrivals
-    size_t dec_counters_offset;  // host side: bytes from the workspace's start to the counters
+    uint32_t dec_tag;         // unique to the call (20 bits are used): whatever else a mark's word holds is no mark
+    uint32_t *dec_marks;      // [units][splits] the marks of arrivals, see fused_merge_tail
+    size_t dec_marks_offset;  // host side: bytes from the workspace's start to the marks
     int32_t *dec_trip;        // host-visible word set when the workgroups of a unit turn out to run on different XCDs
     // host-side only (profiling hook).  Both set: the dispatch of the main kernel carries the two events, which then
     // hold its own begin and end timestamps.  Only main_done: recorded on the stream after the main kernel.
@@ -102,7 +102,7 @@ int launch_mask_build(void *out, fhip_dtype dtype, uint32_t rows, uint64_t cols,
                       uint64_t window, hipStream_t stream);
 
 // layout of the fused split-KV merge in the workspace (false: the call takes the two-kernel form)
-bool decode_fused_layout(const AttnParams &p, bool f32, int *unit_stride, size_t *counters_offset);
+bool decode_fused_layout(const AttnParams &p, bool f32, int *unit_stride, size_t *marks_offset);
 // writes the XCC id each of `workgroups` workgroups of a one-dimensional launch runs on
 int launch_xcd_probe(uint8_t *out, int workgroups, hipStream_t stream);
 
