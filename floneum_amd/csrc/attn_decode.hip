@@ -131,6 +131,13 @@ void decode_plan(int B, int Hkv, int G, int Skv, int D, int compute_units, bool 
     //    where two workgroups share a CU and the chunks are as long as they were asked to be: such calls share their plan with those;
     //  - f32 calls on the kernels that round once per four keys, where longer sums lose precision (9 sequences at 128: 2.36e-7 ->
     //    2.53e-7 against 64 bits; 1.50e-7 as it is).
+    // As many splits as were asked for fill one round, to the next whole one: a few workgroups more than the chip holds, which
+    // run a round of their own, are taken back while more than 8 splits are left (us a step: bf16, 3 sequences of 32/8 at 96, 13774 keys
+    // 30.0 -> 25.3; f16, 10 of 8/4 at 96, two rows on 10826 keys 37.2 -> 31.1).
+    if (!ragged && decode_use_mfma(D, f32, G) && (!f32 || df_shares(D, gt / 16)) && ns == (target + units - 1) / units && units * n > target) {
+        const long k = target / units, kc = k > 8 ? ((Skv + k - 1) / k + step_keys - 1) / step_keys * step_keys : 0;
+        if (kc > 0 && (Skv + kc - 1) / kc > 8) c = kc, n = (Skv + kc - 1) / kc;
+    }
     const bool asked = wgs_per_cu > 1 && ns_min <= (target + units - 1) / units;
     if (!ragged && !asked && decode_use_mfma(D, f32, G) && (!f32 || df_shares(D, gt / 16)) && units * n <= 4L * compute_units) {
         auto rounds_time = [&](long splits, long keys) {
