@@ -14,7 +14,7 @@
 //     products on v_dot2, DPP reductions; every group of LPK lanes keeps its own softmax state.
 // Both keep (m, l, acc) in the log2 domain, merge lanes -> wavefront -> workgroup at the end and
 // write one partial (acc[D], m, l) per (batch, head, split).
-// Pass 2 (decode_combine_kernel, decode_combine4_kernel): log-sum-exp merge of the partials of each (batch, head).
+// Pass 2 (decode_combine_kernel): log-sum-exp merge of the partials of each (batch, head).
 // With a single split pass 1 writes the final output and pass 2 is not launched.
 //
 // Reference semantics: fusor-ml/fusor/src/composite/flash_attention.rs:141-199 (f32 accumulation
@@ -1289,160 +1289,124 @@ __global__ __launch_bounds__(64 * DEC_WAVES, D > 128 ? 1 : D == 96 && CB == 1 ? 
 }
 
 // ---- pass 2 -------------------------------------------------------------------------------------
-// One 64-lane wavefront per (batch, head); up to U partials are fetched in one round of loads (a round costs
-// one memory latency, so calls with many splits take the wide form).
-
-template <typename T, int U>
-__global__ __launch_bounds__(64) void decode_combine_kernel(AttnParams p) {
-    request_arguments<AttnParams>();
-    const int qr = blockIdx.x % p.Sq, bh = blockIdx.x / p.Sq;  // one workgroup per (batch, head, query row)
-    const int h = bh % p.H, b = bh / p.H;
-    const int D = p.D;
+// LPR lanes take a row's dims, four each, so that a split is one load of four values and one of (m, l); U splits are fetched in one
+// round (a round costs a memory latency).  With few (batch, head, query row) rows of many splits (one chat stream) GROUPS groups of
+// lanes share a row, each merges its part of the splits, and the first folds the groups' states through LDS.
+// Bound: one round's memory latency behind the launch's own.  Us a call with 64 lanes of one or two dims per row (four loads a split;
+// four wavefronts per row where rows are few), and now: f32, 32/8 at 128, 5040 keys
+// (40 splits) 17.1 -> 16.2, 8/4 at 256, 1239 keys 11.4 -> 8.8, 16/4 at 64, 11739 keys 13.6 -> 11.0; bf16, 16/4 at 128, 4489 keys 9.4 -> 8.6; f16,
+// B6 32/8 at 256, up to 407 keys each 12.5 -> 11.3.  Over 60 random calls 0.95 of the time, the worst 1.02.  To 32 splits four
+// groups: sixteen of 16 lanes took longer to fold than they gained (1.02 to 1.06 at 64 dims).
+template <typename T, int LPR, int GROUPS, int U>
+__global__ __launch_bounds__(GROUPS > 1 ? LPR * GROUPS : 256) void decode_combine_kernel(AttnParams p, int out_vec) {
+    request_arguments<AttnParams, int>();
+    constexpr int ROWS = GROUPS > 1 ? 1 : 256 / LPR;  // of a workgroup
+    __shared__ float parts[GROUPS > 1 ? GROUPS : 1][GROUPS > 1 ? 4 * LPR : 1];
+    __shared__ float states[GROUPS > 1 ? GROUPS : 1][2];
+    const uint32_t row = GROUPS > 1 ? blockIdx.x : blockIdx.x * ROWS + threadIdx.x / LPR;
+    if (GROUPS == 1 && row >= (uint32_t)(p.B * p.H * p.Sq)) return;
+    const int group = GROUPS > 1 ? threadIdx.x / LPR : 0, D = p.D, lane_dim = 4 * (threadIdx.x % LPR), dim = lane_dim < D ? lane_dim : 0;
+    const uint32_t bh = row / (uint32_t)p.Sq, qr = row - bh * p.Sq, b = bh / (uint32_t)p.H, h = bh - b * p.H;
     int ns = p.nsplit;
     if (p.kv_lens) {
         const int len = min(p.Skv, max(p.kv_lens[b], 0));
         ns = max(1, min(ns, (len + p.chunk - 1) / p.chunk));  // split 0 is always written
     }
-    const float *ws = (const float *)p.partials + (int64_t)blockIdx.x * p.nsplit * (D + 2);
-    const int64_t ob = b * p.os[0] + h * p.os[1] + qr * p.os[2];
-    // 128 dims per round (one round up to head_dim 128, two at 256)
-    for (int dbase = 0; dbase < D; dbase += 128) {
-        const int d0 = dbase + threadIdx.x, d1 = dbase + threadIdx.x + 64;
-        float M = -INFINITY, L = 0.0f, A0 = 0.0f, A1 = 0.0f;
-        for (int s0 = 0; s0 < ns; s0 += U) {
-            float ms[U], ls[U], a0[U], a1[U];
+    const float *ws = (const float *)p.partials + (int64_t)row * p.nsplit * (D + 2);
+    const int per = (ns + GROUPS - 1) / GROUPS, s_lo = group * per, s_hi = min(ns, s_lo + per);
+    float M = -INFINITY, L = 0.0f;
+    float4_t A = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s0 = s_lo; s0 < s_hi; s0 += U) {
+        float ms[U], ls[U];
+        float4_t as[U];
 #pragma unroll
-            for (int u = 0; u < U; u++) {
-                const bool ok = s0 + u < ns;
-                const float *src = ws + (int64_t)(ok ? s0 + u : s0) * (D + 2);
-                ms[u] = ok ? src[D] : -INFINITY;
-                ls[u] = ok ? src[D + 1] : 0.0f;
-                a0[u] = (ok && d0 < D) ? src[d0] : 0.0f;
-                a1[u] = (ok && d1 < D) ? src[d1] : 0.0f;
-            }
-            float Mn = M;
+        for (int u = 0; u < U; u++) {
+            const bool ok = s0 + u < s_hi;
+            const float *src = ws + (int64_t)(ok ? s0 + u : s0) * (D + 2);
+            const float2_at8_t ml = *(const float2_at8_t *)(src + D);
+            as[u] = *(const float4_at8_t *)(src + dim);
+            ms[u] = ok ? ml[0] : -INFINITY;
+            ls[u] = ok ? ml[1] : 0.0f;
+            if (!ok) as[u] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+        float Mn = M;
 #pragma unroll
-            for (int u = 0; u < U; u++) Mn = fmaxf(Mn, ms[u]);
-            const float Ms = (Mn == -INFINITY) ? 0.0f : Mn;
-            const float c = __builtin_amdgcn_exp2f(M - Ms);
-            L *= c;
-            A0 *= c;
-            A1 *= c;
+        for (int u = 0; u < U; u++) Mn = fmaxf(Mn, ms[u]);
+        const float Ms = (Mn == -INFINITY) ? 0.0f : Mn;
+        const float c = __builtin_amdgcn_exp2f(M - Ms);
+        L *= c;
+        A *= c;
 #pragma unroll
-            for (int u = 0; u < U; u++) {
-                const float w = __builtin_amdgcn_exp2f(ms[u] - Ms);
-                L += w * ls[u];
-                A0 += w * a0[u];
-                A1 += w * a1[u];
-            }
-            M = Mn;
+        for (int u = 0; u < U; u++) {
+            const float w = __builtin_amdgcn_exp2f(ms[u] - Ms);
+            L += w * ls[u];
+#pragma unroll
+            for (int e = 0; e < 4; e++) A[e] += w * as[u][e];
         }
-        if (d0 < D) {
-            const float val = A0 / L;
-            if (p.out_f32) ((float *)p.out)[ob + d0 * p.os[3]] = val;
-            else ((T *)p.out)[ob + d0 * p.os[3]] = from_float<T>(val);
-        }
-        if (d1 < D) {
-            const float val = A1 / L;
-            if (p.out_f32) ((float *)p.out)[ob + d1 * p.os[3]] = val;
-            else ((T *)p.out)[ob + d1 * p.os[3]] = from_float<T>(val);
-        }
+        M = Mn;
     }
-}
-
-// Few (batch, head) rows with many splits (batch 1 on a long cache): one wavefront per row leaves the chip empty
-// and issues every load of a row from 64 lanes.  Here four wavefronts share a row, each merges a quarter of the
-// splits (U in flight per lane), and the first folds the four states through LDS.
-template <typename T, int U>
-__global__ __launch_bounds__(256) void decode_combine4_kernel(AttnParams p) {
-    request_arguments<AttnParams>();
-    __shared__ float part[4][2 + 128];
-    const int qr = blockIdx.x % p.Sq, bh = blockIdx.x / p.Sq;  // one workgroup per (batch, head, query row)
-    const int h = bh % p.H, b = bh / p.H;
-    const int D = p.D;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    int ns = p.nsplit;
-    if (p.kv_lens) {
-        const int len = min(p.Skv, max(p.kv_lens[b], 0));
-        ns = max(1, min(ns, (len + p.chunk - 1) / p.chunk));  // split 0 is always written
-    }
-    const float *ws = (const float *)p.partials + (int64_t)blockIdx.x * p.nsplit * (D + 2);
-    const int64_t ob = b * p.os[0] + h * p.os[1] + qr * p.os[2];
-    const int per = (ns + 3) / 4, s_lo = wave * per, s_hi = min(ns, s_lo + per);
-    for (int dbase = 0; dbase < D; dbase += 128) {
-        const int d0 = dbase + lane, d1 = dbase + lane + 64;
-        float M = -INFINITY, L = 0.0f, A0 = 0.0f, A1 = 0.0f;
-        for (int s0 = s_lo; s0 < s_hi; s0 += U) {
-            float ms[U], ls[U], a0[U], a1[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const bool ok = s0 + u < s_hi;
-                const float *src = ws + (int64_t)(ok ? s0 + u : s0) * (D + 2);
-                ms[u] = ok ? src[D] : -INFINITY;
-                ls[u] = ok ? src[D + 1] : 0.0f;
-                a0[u] = (ok && d0 < D) ? src[d0] : 0.0f;
-                a1[u] = (ok && d1 < D) ? src[d1] : 0.0f;
-            }
-            float Mn = M;
-#pragma unroll
-            for (int u = 0; u < U; u++) Mn = fmaxf(Mn, ms[u]);
-            const float Ms = (Mn == -INFINITY) ? 0.0f : Mn;
-            const float c = __builtin_amdgcn_exp2f(M - Ms);
-            L *= c;
-            A0 *= c;
-            A1 *= c;
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const float w = __builtin_amdgcn_exp2f(ms[u] - Ms);
-                L += w * ls[u];
-                A0 += w * a0[u];
-                A1 += w * a1[u];
-            }
-            M = Mn;
-        }
-        if (dbase > 0) __syncthreads();  // the previous round's states have been read
-        part[wave][2 + lane] = A0;
-        part[wave][2 + 64 + lane] = A1;
-        if (lane == 0) {
-            part[wave][0] = M;
-            part[wave][1] = L;
-        }
+    if constexpr (GROUPS > 1) {
+        *(float4_t *)&parts[group][lane_dim] = A;
+        if (lane_dim == 0) states[group][0] = M, states[group][1] = L;
         __syncthreads();
-        if (wave == 0) {
-            float Mn = -INFINITY;
+        if (group > 0) return;
 #pragma unroll
-            for (int w = 0; w < 4; w++) Mn = fmaxf(Mn, part[w][0]);
-            const float Ms = (Mn == -INFINITY) ? 0.0f : Mn;
-            float Lt = 0.0f, B0 = 0.0f, B1 = 0.0f;
+        for (int w = 1; w < GROUPS; w++) M = fmaxf(M, states[w][0]);
+        const float Ms = (M == -INFINITY) ? 0.0f : M;
+        L = 0.0f, A = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int w = 0; w < 4; w++) {
-                const float c = __builtin_amdgcn_exp2f(part[w][0] - Ms);
-                Lt += c * part[w][1];
-                B0 += c * part[w][2 + lane];
-                B1 += c * part[w][2 + 64 + lane];
-            }
-            if (d0 < D) {
-                const float val = B0 / Lt;  // no visible key: 0/0 = NaN like the reference
-                if (p.out_f32) ((float *)p.out)[ob + d0 * p.os[3]] = val;
-                else ((T *)p.out)[ob + d0 * p.os[3]] = from_float<T>(val);
-            }
-            if (d1 < D) {
-                const float val = B1 / Lt;
-                if (p.out_f32) ((float *)p.out)[ob + d1 * p.os[3]] = val;
-                else ((T *)p.out)[ob + d1 * p.os[3]] = from_float<T>(val);
-            }
+        for (int w = 0; w < GROUPS; w++) {
+            const float c = __builtin_amdgcn_exp2f(states[w][0] - Ms);
+            const float4_t a = *(const float4_t *)&parts[w][lane_dim];
+            L += c * states[w][1];
+#pragma unroll
+            for (int e = 0; e < 4; e++) A[e] += c * a[e];
+        }
+    }
+    if (lane_dim >= D) return;
+    const int64_t at = b * p.os[0] + h * p.os[1] + qr * p.os[2] + dim * p.os[3];
+#pragma unroll
+    for (int e = 0; e < 4; e++) A[e] /= L;  // no visible key: 0/0 = NaN like the reference
+    const bool f32 = sizeof(T) == 4 || p.out_f32;
+    if (out_vec && f32) {
+        *(float4_t *)((float *)p.out + at) = A;
+    } else if (out_vec) {
+        if constexpr (sizeof(T) == 2) {
+            const T four[4] = {from_float<T>(A[0]), from_float<T>(A[1]), from_float<T>(A[2]), from_float<T>(A[3])};
+            uint2_t w;
+            __builtin_memcpy(&w, four, 8);
+            *(uint2_t *)((T *)p.out + at) = w;
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            if (f32) ((float *)p.out)[at + e * p.os[3]] = A[e];
+            else ((T *)p.out)[at + e * p.os[3]] = from_float<T>(A[e]);
         }
     }
 }
 
+template <typename T, int LPR>
+static void launch_combine_dims(const AttnParams &p, hipStream_t stream) {
+    const int cus = p.cus > 0 ? p.cus : 256;
+    const long rows = (long)p.B * p.H * p.Sq;
+    // rows of the result written in pieces of four elements
+    const int oeb = sizeof(T) == 4 || p.out_f32 ? 4 : 2;
+    int out_vec = p.os[3] == 1 && (uintptr_t)p.out % (4 * oeb) == 0;
+    for (int i = 0; i < 3; i++)
+        if (p.os[i] % 4 != 0) out_vec = 0;
+    constexpr int ROWS = 256 / LPR;
+    const dim3 grid((unsigned)((rows + ROWS - 1) / ROWS)), block(256);
+    if (p.nsplit <= 8) hipLaunchKernelGGL((decode_combine_kernel<T, LPR, 1, 8>), grid, block, 0, stream, p, out_vec);
+    else if (rows > 2L * cus) hipLaunchKernelGGL((decode_combine_kernel<T, LPR, 1, 16>), grid, block, 0, stream, p, out_vec);
+    else if (p.nsplit <= 32) hipLaunchKernelGGL((decode_combine_kernel<T, LPR, 4, 8>), dim3((unsigned)rows), dim3(LPR * 4), 0, stream, p, out_vec);
+    else hipLaunchKernelGGL((decode_combine_kernel<T, LPR, 8, 8>), dim3((unsigned)rows), dim3(LPR * 8), 0, stream, p, out_vec);
+}
 template <typename T>
 static void launch_combine(const AttnParams &p, hipStream_t stream) {
-    const dim3 grid((unsigned)(p.B * p.H * p.Sq)), block(64);
-    const int cus = p.cus > 0 ? p.cus : 256;
-    if (p.nsplit <= 8) hipLaunchKernelGGL((decode_combine_kernel<T, 8>), grid, block, 0, stream, p);
-    else if ((long)p.B * p.H * p.Sq > 2L * cus) hipLaunchKernelGGL((decode_combine_kernel<T, 32>), grid, block, 0, stream, p);
-    else if (p.nsplit <= 32) hipLaunchKernelGGL((decode_combine4_kernel<T, 8>), grid, dim3(256), 0, stream, p);
-    else hipLaunchKernelGGL((decode_combine4_kernel<T, 16>), grid, dim3(256), 0, stream, p);
+    if (p.D <= 64) launch_combine_dims<T, 16>(p, stream);
+    else if (p.D <= 128) launch_combine_dims<T, 32>(p, stream);
+    else launch_combine_dims<T, 64>(p, stream);
 }
 
 template <typename T, int LPK>
