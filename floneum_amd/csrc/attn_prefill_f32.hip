@@ -1,6 +1,6 @@
-// Prefill attention in f32 precision on the gfx950 f32 matrix instruction (v_mfma_f32_32x32x2_f32): head dims above 128, and
-// below for calls that attn_prefill_f32_terms.hip cannot address (prefill_f32_terms_takes): K or V rows that overlap, a K, V
-// or Q slice of 2 GiB and more, or grids beyond its dimensions.
+// Prefill attention in f32 precision on the gfx950 f32 matrix instruction (v_mfma_f32_32x32x2_f32): calls that
+// attn_prefill_f32_terms.hip cannot address (prefill_f32_terms_takes): K or V rows that overlap, a K, V
+// or Q slice of 2 GiB and more, or grids beyond its dimensions; and of head dims above 128 short calls of few rows (wide_in_terms).
 //
 // A workgroup of 4 wavefronts owns 128 query rows of one (batch, head), a wavefront 32 of them; K/V tiles of 32 rows pass
 // through LDS.
@@ -609,12 +609,14 @@ static int launch_merge_t(const AttnParams &p, hipStream_t stream);
 // query heads that share one workgroup of the wide-head kernel (0: one head, up to 64 rows)
 static int prefill_f32_wide_pack(int G, int Sq, int D) { return (D > 128 && Sq <= 32 && G >= 2 && G % 2 == 0) ? 2 : 0; }
 
+static int no_wide_bias() {
+    set_error("prefill f32: a mask tensor without its interval form is not supported above head_dim 128");
+    return FHIP_ERR_UNSUPPORTED;
+}
+
 template <typename T>
 static int launch_wide(const AttnParams &p_in, hipStream_t stream) {
-    if (p_in.mask && !p_in.iv) {
-        set_error("prefill f32: a mask tensor without its interval form is not supported above head_dim 128");
-        return FHIP_ERR_UNSUPPORTED;
-    }
+    if (p_in.mask && !p_in.iv) return no_wide_bias();
     AttnParams p = p_in;
     p.pf_pack = prefill_f32_wide_pack(p.G, p.Sq, p.D);
     const int nqb = p.pf_pack ? 1 : (p.Sq + 63) / 64;
@@ -677,9 +679,31 @@ static int launch_rows(const AttnParams &p, hipStream_t stream) {
     return FHIP_OK;
 }
 
+// Shares of the keys: the fewest within 2 % of the least time, where that is 5 % less than the time of `ordinary` ones.
+static long shares_of_least_time(const TermsCall &c, long ordinary) {
+    constexpr int SHARES[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48};
+    const long units = (long)c.G * ((c.Sq + 31) / 32);
+    double times[sizeof(SHARES) / sizeof(SHARES[0])], least = 0.0;
+    int tried = 0;
+    for (const int n : SHARES) {
+        // (shares that make three rounds of the smallest workgroups gain nothing more)
+        if (n > 1 && (c.Skv / n < 64 || prefill_f32_workspace_bytes(c.B, c.Hkv * c.G, c.Sq, c.D, n) > ((size_t)64 << 20) ||
+                      (n - 1) * (long)c.B * c.Hkv * units > 6L * c.cus))
+            break;
+        times[tried] = prefill_f32_terms_time(c, prefill_f32_terms_quickest(c, n), n);
+        if (tried == 0 || times[tried] < least) least = times[tried];
+        tried++;
+    }
+    for (int i = 0; i < tried; i++) {
+        if (times[i] > 1.02 * least) continue;
+        return times[i] < 0.95 * prefill_f32_terms_time(c, prefill_f32_terms_form(c, (int)ordinary), (int)ordinary) ? SHARES[i] : ordinary;
+    }
+    return ordinary;
+}
+
 // Few query rows on a long cache (a new chat turn, a prompt fed in pieces): the grid of query blocks alone leaves
 // most CUs idle, so the keys are split over workgroups as well.
-void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_square, bool uneven, int compute_units, int *nsplit, int *chunk) {
+void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, bool causal_square, bool uneven, int compute_units, int *nsplit, int *chunk) {
     *nsplit = 1;
     *chunk = Skv;
     if (D <= 128) {
@@ -716,38 +740,28 @@ void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_s
         // twice the shares), 64 rows 79 (56), 128 rows 128 (96), 256 rows 244 (172), 512 rows 463 (327).
         constexpr size_t MOST_PARTIALS = (size_t)16 << 20;
         if (few_rows && D > 64 && prefill_f32_workspace_bytes(B, H, Sq, D, (int)ns) > MOST_PARTIALS) ns = shares(2);
-        // More than 128 rows that see about the same keys (chunks, images): the shares of least time, the fewest within 2 % of
-        // it, where that is 5 % less than the rule's; at most 64 MiB of partials (us a call: two sequences of 275 rows of 32/8
+        // More than 128 rows that see about the same keys (chunks, images): the shares of least time, where that is 5 % less than the
+        // rule's; at most 64 MiB of partials (us a call: two sequences of 275 rows of 32/8
         // heads at 64 on 2911 keys 116 -> 92; 16 heads without a mask, 1156 rows at 128 148 -> 80, 2506 366 -> 285, 1147 at 80 109 -> 59; over 90
         // random calls the time is 0.91, the worst 1.03 of the rule's).  Square prompts to 768 keys keep the rule, masked or not.
-        if (!uneven && Sq > 128 && (few_rows || Skv > 768)) {
-            const TermsCall call = {B, H / G, G, Sq, Skv, D, compute_units, false};
-            constexpr int SHARES[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48};
-            double times[sizeof(SHARES) / sizeof(SHARES[0])], least = 0.0;
-            int tried = 0;
-            for (const int n : SHARES) {
-                // (shares that make three rounds of the smallest workgroups gain nothing more)
-                if (n > 1 && (Skv / n < 64 || prefill_f32_workspace_bytes(B, H, Sq, D, n) > ((size_t)64 << 20) ||
-                              (n - 1) * kv_heads * units > 6L * compute_units))
-                    break;
-                times[tried] = prefill_f32_terms_time(call, prefill_f32_terms_quickest(call, n), n);
-                if (tried == 0 || times[tried] < least) least = times[tried];
-                tried++;
-            }
-            const long ordinary = ns < 2 ? 1 : ns;
-            for (int i = 0; i < tried; i++) {
-                if (times[i] > 1.02 * least) continue;
-                if (times[i] < 0.95 * prefill_f32_terms_time(call, prefill_f32_terms_form(call, (int)ordinary), (int)ordinary)) ns = SHARES[i];
-                break;
-            }
-        }
+        if (!uneven && Sq > 128 && (few_rows || Skv > 768)) ns = shares_of_least_time({B, H / G, G, Sq, Skv, D, compute_units, false}, ns < 2 ? 1 : ns);
         if (ns < 2) return;
         const long c = ((Skv + ns - 1) / ns + 31) / 32 * 32;
         *chunk = (int)c;
         *nsplit = (int)((Skv + c - 1) / c);
         return;
     }
-    // head dims above 128: down to 512 keys per share, until there are about two workgroups per CU.  Square causal calls are
+    if (f32 && Sq > 64) {
+        // Head dims above 128 in the terms kernel: the shares of least time (us, 16/4 heads at 256 causal, in one share and in
+        // the shares taken: 148 rows on 3510 keys 584 -> 80, 300 on 700 128 -> 49, 1024 on 1024 187 -> 119, 2048 on 2048 stays at 355).
+        const long ns = shares_of_least_time({B, H / G, G, Sq, Skv, D, compute_units, uneven}, 1);
+        if (ns < 2) return;
+        const long c = ((Skv + ns - 1) / ns + 31) / 32 * 32;
+        *chunk = (int)c;
+        *nsplit = (int)((Skv + c - 1) / c);
+        return;
+    }
+    // Up to 64 rows, and 16-bit rows that only the kernel of this file takes (head dims not a multiple of 8): down to 512 keys per share, until there are about two workgroups per CU.  Square causal calls are
     // left alone (their shares would be uneven, and they fill the chip from 1024 rows on).
     if (causal_square) return;
     const int pack = prefill_f32_wide_pack(G, Sq, D);
@@ -778,9 +792,21 @@ size_t prefill_f32_workspace_bytes(int B, int H, int Sq, int D, int nsplit) {
     return (size_t)B * H * Sq * nsplit * (size_t)(D + 2) * sizeof(float);
 }
 
+// Head dims above 128 in f32: the terms kernel, but for up to 64 rows on up to 2048 keys whose shares leave CUs without a workgroup of
+// launch_wide's: a workgroup alone on its CU takes longer to split its first tile and Q into terms than the f32 instruction takes for both
+// (us, head_dim 256, here and in terms: 9 rows of 16/4 heads on 2048 keys 34.7 and 37.3, 33 rows on 1000 39.6 and 43.0; 64 rows of 4 heads
+// on 4096 50.2 and 41.1, 17 rows of 32/8 heads on 8192 108 and 70).
+static bool wide_in_terms(const AttnParams &p) {
+    if (p.Sq > 64) return true;
+    const long ns = p.pf_nsplit > 1 ? p.pf_nsplit : 1, keys = ns > 1 ? ns * p.pf_chunk : p.Skv;
+    const long wgs = (long)p.B * (prefill_f32_wide_pack(p.G, p.Sq, p.D) ? p.H / 2 : p.H) * ns;
+    return keys > 2048 || wgs >= (p.cus > 0 ? p.cus : 256);
+}
+
 template <typename T>
 static int launch_prefill_f32_t(const AttnParams &p, hipStream_t stream) {
-    if (p.D > 128) return launch_wide<T>(p, stream);
+    if (p.D > 128 && !(sizeof(T) == 4 && wide_in_terms(p) && prefill_f32_terms_takes(p))) return launch_wide<T>(p, stream);
+    if (p.D > 128 && p.mask && !p.iv) return no_wide_bias();
     const int mode = !p.mask ? PF32_INTERVALS : !p.iv && !p.iv_either ? PF32_BIAS : p.iv_either ? PF32_EITHER : PF32_INTERVALS;
     if (mode == PF32_EITHER && p.D > 64) {
         set_error("internal: the two-form f32 kernel takes head_dim <= 64");

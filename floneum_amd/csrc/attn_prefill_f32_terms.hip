@@ -145,6 +145,7 @@ struct TermsLaunch {
     int32_t snake;     // workgroups from this one of the last grid dimension on are numbered backwards (0: none)
     int32_t out_vec;   // bytes per store of the result: 16 (f32), 8 (16-bit), or 0: element by element
     int32_t mask_rows; // an added mask is read four keys at a time through a buffer
+    uint32_t share_magic;  // z / shares = (z * share_magic) >> 32, where the shares' order turns with z (0: it does not)
 };
 
 // K, V and Q of a unit as buffers: bytes from row to row, and where this lane's row of Q begins
@@ -264,7 +265,7 @@ __device__ __forceinline__ void unit_in_f32(const AttnParams &p, __attribute__((
 }
 
 template <typename T, int D, int U, int KG, int MODE>
-__global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG == 1 && D == 64 && MODE == PF32_INTERVALS ? 3 : 2) void prefill_f32_terms_kernel(AttnParams p, TermsLaunch tl) {
+__global__ __launch_bounds__(64 * U * KG, D > 128 || (KG == 2 && U == 2 && D > 64) ? 1 : KG == 1 && D == 64 && MODE == PF32_INTERVALS ? 3 : 2) void prefill_f32_terms_kernel(AttnParams p, TermsLaunch tl) {
     typedef PtCfg<T, D, U> C;
     constexpr int N = C::N, NDB = D / 32, NKB = D / 16;
     constexpr bool BIAS = MODE != PF32_INTERVALS;
@@ -302,8 +303,17 @@ __global__ __launch_bounds__(64 * U * KG, KG == 2 && U == 2 && D > 64 ? 1 : KG =
     // Workgroup -> (units, batch, kv head): the units of a KV head are its row blocks times the query heads that share it,
     // numbered heads first, so that U consecutive ones read the same keys; those with the most keys first.
     // (grid: shares of the keys, kv heads of the batch, workgroups per kv head)
-    const int nks = gridDim.x, ksplit = blockIdx.x;
+    const int nks = gridDim.x;
     const int nwg = gridDim.z, wz = blockIdx.z;
+    int ksplit = blockIdx.x;
+    // Workgroups go to the XCDs in turn: an even number of shares would leave the first one, which all rows of a square prompt see, to
+    // some of them (head_dim 256, 2048 rows of 8/1 heads in four shares 215 us).
+    if constexpr (D > 128) {
+        if (tl.share_magic) {
+            ksplit += wz - (int)__umulhi((uint32_t)wz, tl.share_magic) * nks;
+            if (ksplit >= nks) ksplit -= nks;
+        }
+    }
     // with the whole grid resident at once (two workgroups per CU) a CU gets a long and a short one
     const int wg = tl.snake > 0 && wz >= tl.snake ? tl.snake + nwg - 1 - wz : wz;
     const int first_unit = (nwg - 1 - wg) * U;
@@ -841,7 +851,10 @@ static long terms_workgroups(const TermsCall &c, int U, int ns) {
 }
 
 // The form by the numbers of its workgroups (measured on f32 calls, time per call in us; w2, w4: workgroups with 2 or 4 units):
-//   (4, 1)  two workgroups per CU, least splitting per tile: grids that fill the chip twice
+//   (4, 1)  two workgroups per CU, least splitting per tile: grids that fill the chip twice.  Head dims above 128, one workgroup per CU
+//           (106 KiB of LDS, 512 registers): a wavefront per SIMD issues its matrix and vector work in turn, 5.3 us a tile at 256 of
+//           which 2.6 are matrix instructions (16/4 heads causal, us before, on the f32 matrix instruction: 148 rows on 3510 keys
+//           192 -> 80, 1024 x 1024 181 -> 119, 3191 x 3191 826 -> 555, 1500 x 6000 1577 -> 905)
 //   (4, 2)  eight wavefronts, one workgroup per CU: D = 128 1500 rows 115 against 142 for (4, 1), 4000 rows of 8 heads
 //           262 against 348, 129 rows on 8003 keys (keys split over workgroups) 111 against 133
 //   (2, 2)  D > 64: one wavefront per SIMD with 512 registers, half the units per workgroup, for short prompts (700 rows
@@ -874,7 +887,9 @@ static TermsForm form_by_workgroups(const TermsCall &c, int ns) {
 // Time of a call whose rows all see about the same keys, in us: rounds of workgroups that walk their tiles, and parking and
 // merging the shares.  Constants fitted to 210 random calls (chunks, turns, images and encoders of 8 to 32 heads at 64 to 128
 // dims, each in every form and up to 48 shares): 6 % off in the mean square.
+static double wide_terms_time(const TermsCall &c, int ns);
 double prefill_f32_terms_time(const TermsCall &c, TermsForm f, int ns) {
+    if (c.D > 128) return wide_terms_time(c, ns);
     const double dims = (c.D <= 64 ? 64 : c.D <= 96 ? 96 : 128) / 64.0;
     double tile, ends, alone = 1.0;  // per tile of a group, per workgroup, and a tile's time where a CU has one of two workgroups
     bool two_per_cu = false;
@@ -892,7 +907,35 @@ double prefill_f32_terms_time(const TermsCall &c, TermsForm f, int ns) {
     return us;
 }
 
+// The same above head_dim 128, where the form is (4, 1) with one workgroup per CU, of uneven calls too.  The hardware deals workgroups out
+// to the 32 shader engines in turn, so a CU gets a second one before all have their first: fitted to 330 calls, 2.7 % off in the mean
+// square with each engine's queue played through.  In closed form: workgroups whose rows see a key of their share go in one round up to
+// 0.85 of the CUs, in one and a half where they fit, and uneven calls with more take one share.
+static double wide_terms_time(const TermsCall &c, int ns) {
+    const double tile = 1.33 * (c.D <= 192 ? 3 : 4), ends = 6.9;
+    const int chunk = ((c.Skv + ns - 1) / ns + PT_BN - 1) / PT_BN * PT_BN, n = (c.Skv + chunk - 1) / chunk;
+    const double wgs = (double)terms_workgroups(c, 4, 1);
+    double rounds;
+    if (!c.uneven) {
+        rounds = (double)(((long)wgs * n + c.cus - 1) / c.cus);
+    } else if (n == 1) {
+        rounds = 1.0;
+    } else {
+        const double first = c.Skv > c.Sq ? c.Skv - c.Sq : 0.0;  // keys before the first row
+        double active = 0.0;
+        for (int i = 0; i < n; i++) {
+            const double rows = (c.Skv - (double)i * chunk) / (c.Skv - first);
+            active += rows < 0.0 ? 0.0 : rows > 1.0 ? 1.0 : rows;
+        }
+        rounds = wgs * active <= 0.85 * c.cus ? 1.0 : wgs * active <= 1.0 * c.cus ? 1.5 : 1e6;
+    }
+    double us = 4.9 + rounds * (ends + tile * (chunk / PT_BN));
+    if (n > 1) us += 3.24 + 0.456e-6 * prefill_f32_workspace_bytes(c.B, c.Hkv * c.G, c.Sq, c.D, n);
+    return us;
+}
+
 TermsForm prefill_f32_terms_quickest(const TermsCall &c, int ns) {
+    if (c.D > 128) return {4, 1};
     TermsForm best = {4, 1};
     double least = prefill_f32_terms_time(c, best, ns);
     for (const TermsForm f : {TermsForm{4, 2}, TermsForm{2, 2}, TermsForm{2, 4}}) {
@@ -907,6 +950,7 @@ TermsForm prefill_f32_terms_quickest(const TermsCall &c, int ns) {
 // is 7 % better (us a call: 16 heads without a mask, 1356 rows at 128 169 -> 99; 6 encoder sequences of 436 tokens 41.5 -> 30.6, 11
 // of 169 23.2 -> 18.4).  Up to 128 rows the rule is as good.
 TermsForm prefill_f32_terms_form(const TermsCall &c, int ns) {
+    if (c.D > 128) return {4, 1};
     const TermsForm ordinary = form_by_workgroups(c, ns);
     if (c.uneven || c.Sq <= 128 || c.Skv <= 2 * PT_BN) return ordinary;
     const TermsForm other = prefill_f32_terms_quickest(c, ns);
@@ -930,8 +974,9 @@ static int launch_form(const AttnParams &p_in, hipStream_t stream) {
     }
     TermsLaunch tl;
     const unsigned nks = p.pf_nsplit > 1 ? p.pf_nsplit : 1, groups = (unsigned)(p.B * p.Hkv), nwg = (unsigned)(blocks / nks / groups);
+    tl.share_magic = p.D > 128 && nks > 1 && terms_call(p).uneven ? (uint32_t)((0x100000000ull + nks - 1) / nks) : 0;
     tl.g_magic = p.G > 1 ? (uint32_t)((0x100000000ull + p.G - 1) / p.G) : 0;
-    const bool two_per_cu = KG == 1 || (U * KG == 4 && p.D <= 64);
+    const bool two_per_cu = (KG == 1 && p.D <= 128) || (U * KG == 4 && p.D <= 64);
     tl.snake = (two_per_cu && blocks > cus && blocks <= 2L * cus) ? (int)((cus + nks * groups - 1) / (nks * groups)) : 0;
     // rows of the result written in 16-byte (f32) or 8-byte pieces
     const int oeb = sizeof(T) == 4 || p.out_f32 ? 4 : 2;
@@ -952,7 +997,15 @@ static int launch_form(const AttnParams &p_in, hipStream_t stream) {
         case 128:
             if constexpr (MODE != PF32_EITHER && KG < 4) FHIP_LAUNCH_MAIN((prefill_f32_terms_kernel<T, 128, U, KG, MODE>), grid, block, stream, p, p, tl);
             break;
-        default: set_error("prefill f32 kernel: head_dim %d is not a multiple of 4 up to 128", p.D); return FHIP_ERR_UNSUPPORTED;
+        case 160:
+        case 192:
+            if constexpr (sizeof(T) == 4 && U == 4 && KG == 1 && MODE == PF32_INTERVALS) FHIP_LAUNCH_MAIN((prefill_f32_terms_kernel<T, 192, U, KG, MODE>), grid, block, stream, p, p, tl);
+            break;
+        case 224:
+        case 256:
+            if constexpr (sizeof(T) == 4 && U == 4 && KG == 1 && MODE == PF32_INTERVALS) FHIP_LAUNCH_MAIN((prefill_f32_terms_kernel<T, 256, U, KG, MODE>), grid, block, stream, p, p, tl);
+            break;
+        default: set_error("prefill f32 kernel: head_dim %d is not a multiple of 4 up to 256", p.D); return FHIP_ERR_UNSUPPORTED;
     }
     FHIP_HIP_CHECK(hipGetLastError());
     return FHIP_OK;
@@ -970,6 +1023,7 @@ static int launch_terms(const AttnParams &p, hipStream_t stream) {
     return launch_form<T, 4, 1, MODE>(p, stream);
 }
 
+// (16-bit storage above head_dim 128 is not asked for: attn_prefill_mfma_wide.hip has it.)
 // K and V rows are fetched through 32-bit buffer offsets: rows must not overlap, and one (batch, kv head) slice must span
 // less than 2 GiB, the tiles behind its end included.
 bool prefill_f32_terms_takes(const AttnParams &p) {
@@ -977,7 +1031,7 @@ bool prefill_f32_terms_takes(const AttnParams &p) {
     // (grid dimensions, and the exactness of unit / G by multiplication)
     if ((int64_t)p.B * p.Hkv > 65535 || units > 65535 || units * p.G > 0x7fffffffLL) return false;
     if (p.qs[2] < 0 || (int64_t)p.Sq * p.qs[2] * 4 >= 0x7fffffffLL) return false;
-    return p.D <= 128 && p.ks[2] >= p.D && p.vs[2] >= p.D && rows * p.ks[2] * 4 < 0x7fffffffLL && rows * p.vs[2] * 4 < 0x7fffffffLL;
+    return p.D <= 256 && p.ks[2] >= p.D && p.vs[2] >= p.D && rows * p.ks[2] * 4 < 0x7fffffffLL && rows * p.vs[2] * 4 < 0x7fffffffLL;
 }
 
 // A BatchKeyMask whose row every wavefront can look at for itself, four keys per load and all loads at once: no scan launch.

@@ -67,7 +67,7 @@ struct AttnParams {
 
 // the key split of a tiled f32 prefill call (1 = none) and the scratch it needs
 // uneven: a square call whose rows see the keys up to their own position (a mask tensor is taken for one)
-void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_square, bool uneven, int compute_units, int *nsplit, int *chunk);
+void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, bool causal_square, bool uneven, int compute_units, int *nsplit, int *chunk);
 // The forms of the f32 terms kernel (attn_prefill_f32_terms.hip): units and key groups per workgroup, and what a call takes in them
 struct TermsCall {
     int B, Hkv, G, Sq, Skv, D, cus;
@@ -76,7 +76,7 @@ struct TermsCall {
 struct TermsForm {
     int U, KG;
 };
-double prefill_f32_terms_time(const TermsCall &call, TermsForm form, int key_shares);  // us, of calls that are not uneven
+double prefill_f32_terms_time(const TermsCall &call, TermsForm form, int key_shares);  // us, of calls that are not uneven, or above head_dim 128
 TermsForm prefill_f32_terms_quickest(const TermsCall &call, int key_shares);           // by that time
 TermsForm prefill_f32_terms_form(const TermsCall &call, int key_shares);               // the one that runs
 size_t prefill_f32_workspace_bytes(int B, int H, int Sq, int D, int nsplit);
@@ -148,7 +148,7 @@ bool prefill_mfma_rows64_takes(int D, float scale);
 int launch_prefill_mfma_rows64(const AttnParams &p, fhip_dtype dtype, hipStream_t stream);
 // f32 precision; `dtype` is the tensors' storage type (16-bit rows are widened on load)
 int launch_prefill_f32(const AttnParams &p, fhip_dtype dtype, hipStream_t stream);
-// the same precision on the bf16 matrix cores, head dims to 128 (mode: a PF32_... of attn_f32.h); no merge of key shares
+// the same precision on the bf16 matrix cores (mode: a PF32_... of attn_f32.h); no merge of key shares
 bool prefill_f32_terms_takes(const AttnParams &p);
 bool prefill_f32_terms_scans(const AttnParams &p, fhip_dtype dtype);  // no scan launch is needed: iv_either may be 2
 int launch_prefill_f32_terms(const AttnParams &p, fhip_dtype dtype, int mode, hipStream_t stream);

@@ -68,6 +68,45 @@ def test_forms_and_edges(device, form, D):
     close(out, in_64_bits(q, k, v, D ** -0.5, causal_mask(Sq, Skv, Skv - Sq) if causal else None), f"{form} D{D}")
 
 
+WIDE = {
+    # above head_dim 128: (B, H, Hkv, Sq, Skv, causal)
+    "one_tile": (1, 4, 1, 65, 32, False), "unsplit": (2, 16, 4, 130, 65, False), "one_key": (3, 4, 1, 70, 1, False),
+    "even_shares": (1, 8, 4, 148, 1251, True), "uneven_shares": (1, 8, 4, 417, 417, True), "shares_some_rows_do_not_see": (1, 4, 4, 801, 801, True),
+    "few_rows": (1, 4, 2, 33, 2500, True), "few_rows_in_f32": (1, 4, 2, 33, 1500, True),
+}
+
+
+@pytest.mark.parametrize("D", [256, 192, 132, 160, 228])
+@pytest.mark.parametrize("form", list(WIDE))
+def test_wide_heads(device, form, D):
+    B, H, Hkv, Sq, Skv, causal = WIDE[form]
+    q, k, v = tensors(6, B, H, Hkv, Sq, Skv, D)
+    tq, tk, tv = (fa.Tensor.from_numpy(device, a, fa.F32) for a in (q, k, v))
+    out = tq.flash_attention(tk, tv, D ** -0.5, analytic=(True, Skv - Sq, 0) if causal else None,
+                             force_kernel=fa.KERNEL_PREFILL_F32).to_numpy()
+    close(out, in_64_bits(q, k, v, D ** -0.5, causal_mask(Sq, Skv, Skv - Sq) if causal else None), f"{form} D{D}")
+
+
+@pytest.mark.parametrize("D", [256, 160])
+@pytest.mark.parametrize("of", ["V", "Q"])
+@pytest.mark.parametrize("form", ["unsplit", "uneven_shares"])
+def test_wide_heads_beyond_bf16(device, form, of, D):
+    """Rows that are formed once more in f32: magnitudes at the bottom of f32's range, and an infinity that one key's V holds."""
+    B, H, Hkv, Sq, Skv, causal = WIDE[form]
+    q, k, v = tensors(7, B, H, Hkv, Sq, Skv, D, {"V": (1, 1, 2.0 ** -120), "Q": (2.0 ** -120, 2.0 ** 120, 1)}[of])
+    if of == "V":
+        v[0, 0, 3, 7] = np.inf
+    tq, tk, tv = (fa.Tensor.from_numpy(device, a, fa.F32) for a in (q, k, v))
+    out = tq.flash_attention(tk, tv, D ** -0.5, analytic=(True, Skv - Sq, 0) if causal else None, force_kernel=fa.KERNEL_PREFILL_F32).to_numpy()
+    ref = in_64_bits(q, k, np.where(np.isinf(v), 0.0, v), D ** -0.5, causal_mask(Sq, Skv, Skv - Sq) if causal else None)
+    if of == "V":
+        seen = np.arange(Sq) + (Skv - Sq) >= 3 if causal else np.full(Sq, True)
+        assert np.all(out[0, :H // Hkv, :, 7][:, seen] == np.inf)
+        out, ref = out.copy(), ref.copy()
+        out[0, :H // Hkv, :, 7][:, seen] = ref[0, :H // Hkv, :, 7][:, seen] = 0.0
+    close(out, ref, f"{form} {of}")
+
+
 @pytest.mark.parametrize("stds", [(1.0, 1.0, 1e30), (1e-12, 1e12, 1e-30), (1e4, 1e-4, 1.0)])
 def test_magnitudes(device, stds):
     """The terms keep f32's range."""

@@ -33,6 +33,9 @@ def shares(B, H, Hkv, Sq, Skv, D, dtype, causal=True, window=0):
     # f32: even rows in the shares of least time; up to 128 rows, squares and up to 768 keys by the former rule
     ((2, 32, 8, 275, 2911, 64, fa.F32), 3), ((1, 16, 16, 1156, 1156, 128, fa.F32, False), 3), ((1, 16, 16, 1156, 1156, 128, fa.F32), 0),
     ((1, 16, 16, 768, 768, 128, fa.F32, False), 2), ((1, 32, 8, 128, 8192, 128, fa.F32), 4), ((1, 32, 8, 129, 8003, 128, fa.F32), 6),
+    # above 128 dims in f32: one round of workgroups, of a square those whose rows see a key; up to 64 rows the former rule
+    ((1, 16, 4, 148, 3510, 256, fa.F32), 11), ((1, 16, 4, 300, 700, 256, fa.F32), 6), ((1, 8, 4, 1024, 1024, 256, fa.F32), 6),
+    ((1, 16, 4, 2048, 2048, 256, fa.F32), 0), ((1, 16, 4, 1024, 1024, 256, fa.F32, False), 2), ((1, 16, 4, 64, 4096, 256, fa.F32), 16),
     # above 128 dims: up to four shares of 512 keys
     ((1, 16, 4, 141, 2659, 256, fa.BF16), 4), ((1, 16, 4, 141, 1000, 256, fa.BF16), 0),
 ])
