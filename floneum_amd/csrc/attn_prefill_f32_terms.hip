@@ -947,14 +947,14 @@ TermsForm prefill_f32_terms_quickest(const TermsCall &c, int ns) {
 }
 
 // Where all rows see about the same keys the rule above leaves much to gain, and the form is the quickest by the time above if that
-// is 7 % better (us a call: 16 heads without a mask, 1356 rows at 128 169 -> 99; 6 encoder sequences of 436 tokens 41.5 -> 30.6, 11
+// is 10 % better (7 % moves ten encoder sequences of 154 tokens, 240 workgroups of five tiles, from 16.4 to 17.1; us a call: 16 heads without a mask, 1356 rows at 128 169 -> 99; 6 encoder sequences of 436 tokens 41.5 -> 30.6, 11
 // of 169 23.2 -> 18.4).  Up to 128 rows the rule is as good.
 TermsForm prefill_f32_terms_form(const TermsCall &c, int ns) {
     if (c.D > 128) return {4, 1};
     const TermsForm ordinary = form_by_workgroups(c, ns);
     if (c.uneven || c.Sq <= 128 || c.Skv <= 2 * PT_BN) return ordinary;
     const TermsForm other = prefill_f32_terms_quickest(c, ns);
-    return prefill_f32_terms_time(c, other, ns) < 0.93 * prefill_f32_terms_time(c, ordinary, ns) ? other : ordinary;
+    return prefill_f32_terms_time(c, other, ns) < 0.9 * prefill_f32_terms_time(c, ordinary, ns) ? other : ordinary;
 }
 
 // (rows of a square prompt under a causal mask, for which a mask tensor is taken, see from one to all of the keys)
