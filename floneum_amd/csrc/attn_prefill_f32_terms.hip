@@ -947,8 +947,8 @@ TermsForm prefill_f32_terms_quickest(const TermsCall &c, int ns) {
 }
 
 // Where all rows see about the same keys the rule above leaves much to gain, and the form is the quickest by the time above if that
-// is 10 % better (7 % moves ten encoder sequences of 154 tokens, 240 workgroups of five tiles, from 16.4 to 17.1; us a call: 16 heads without a mask, 1356 rows at 128 169 -> 99; 6 encoder sequences of 436 tokens 41.5 -> 30.6, 11
-// of 169 23.2 -> 18.4).  Up to 128 rows the rule is as good.
+// is 10 % better (us a call: 16 heads without a mask, 1356 rows at 128 169 -> 99; 6 encoder sequences of 436 tokens 41.5 -> 30.6, 11
+// of 169 23.2 -> 18.4; at 7 % ten sequences of 154, 240 workgroups of five tiles, 16.4 -> 17.1).  Up to 128 rows the rule is as good.
 TermsForm prefill_f32_terms_form(const TermsCall &c, int ns) {
     if (c.D > 128) return {4, 1};
     const TermsForm ordinary = form_by_workgroups(c, ns);
