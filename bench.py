@@ -31,8 +31,7 @@ sys.path.insert(0, ROOT)
 METRIC = "attn prefill TFLOP/s + decode KV GB/s, % of roofline, 1xMI355X"
 PEAK_HBM_GBS = 8000.0
 PEAK_MFMA_F16_TFLOPS = 2500.0
-PEAK_MFMA_F32_TFLOPS = 157.3
-# f32 prefill to head_dim 128 forms a product of two f32 values as six bf16 products of their terms
+# f32 prefill forms a product of two f32 values as six bf16 products of their terms
 PEAK_F32_FROM_BF16_TFLOPS = PEAK_MFMA_F16_TFLOPS / 6
 SEED = 0xF10E0000
 # HBM bytes per launch of the dominant kernel, from two rocprofv3 --pmc runs of this file (FETCH_SIZE, then
@@ -389,9 +388,7 @@ def run_config(name, steps, warmup, with_cpu=True):
         value, unit = byts / (wall_ms * 1e-3) / 1e9, "GB/s"
         roof = dict(bound="hbm", achieved=byts / (main_ms_mean * 1e-3) / 1e9, peak=PEAK_HBM_GBS, unit="GB/s")
     else:
-        peak = PEAK_MFMA_F16_TFLOPS
-        if c["dtype"] == "f32":
-            peak = PEAK_F32_FROM_BF16_TFLOPS if c["D"] <= 128 else PEAK_MFMA_F32_TFLOPS
+        peak = PEAK_F32_FROM_BF16_TFLOPS if c["dtype"] == "f32" else PEAK_MFMA_F16_TFLOPS
         value, unit = flops / (wall_ms * 1e-3) / 1e12, "TFLOP/s"
         roof = dict(bound="mfma", achieved=flops / (main_ms_mean * 1e-3) / 1e12, peak=peak, unit="TFLOP/s")
     roof["frac"] = roof["achieved"] / roof["peak"]

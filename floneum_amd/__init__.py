@@ -74,7 +74,8 @@ class CAttnArgs(ctypes.Structure):
 
 # The same structures as one pack of their values: a decode step's two calls describe fifteen tensors, and filled field by
 # field through ctypes these descriptors cost the host more than the step costs the GPU (f32, 32/8 heads, 4096 keys: 23.6 us a
-# step, 19.1 packed, with the same library; a 346-key step in f16 20.3 and 16.0).
+# step, 19.1 packed, with the same library; a 346-key step in f16 20.3 and 16.0.  Plain calls go through native code, csrc/host_python.cpp: a
+# 301-key step 16.1 packed and 8.8 there).
 _TENSOR4 = struct.Struct("=QQ4I4q")
 _ATTN_ARGS = struct.Struct("=" + 4 * "QQ4I4q" + "iifi" + "QQ2I2q" + "iiqq" + "QQQ" + "i4x" + "QQQ")
 assert _TENSOR4.size == ctypes.sizeof(CTensor4) and _ATTN_ARGS.size == ctypes.sizeof(CAttnArgs)
