@@ -753,7 +753,8 @@ void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, boo
     }
     if (f32 && Sq > 64) {
         // Head dims above 128 in the terms kernel: the shares of least time (us, 16/4 heads at 256 causal, in one share and in
-        // the shares taken: 148 rows on 3510 keys 584 -> 80, 300 on 700 128 -> 49, 1024 on 1024 187 -> 119, 2048 on 2048 stays at 355).
+        // the shares taken: 148 rows on 3510 keys 584 -> 80, 300 on 700 128 -> 49, 1000 on 1000 182 -> 93, 2000 on 2000 347 -> 235; 2048 on 2048 stays at 355, its two shares
+        // would be more than 64 MiB of partials).
         const long ns = shares_of_least_time({B, H / G, G, Sq, Skv, D, compute_units, uneven}, 1);
         if (ns < 2) return;
         const long c = ((Skv + ns - 1) / ns + 31) / 32 * 32;

@@ -37,6 +37,8 @@
 //
 // Reference semantics: fusor-ml/fusor/src/composite/flash_attention.rs:141-199; f32 is the data type kalosm-llama always
 // calls with (models/kalosm-llama/src/raw/attention_layer.rs:400-448).
+#include <algorithm>
+
 #include "attn_bounds.h"
 #include "attn_f32.h"
 #include "common.h"
@@ -145,7 +147,7 @@ struct TermsLaunch {
     int32_t snake;     // workgroups from this one of the last grid dimension on are numbered backwards (0: none)
     int32_t out_vec;   // bytes per store of the result: 16 (f32), 8 (16-bit), or 0: element by element
     int32_t mask_rows; // an added mask is read four keys at a time through a buffer
-    uint32_t share_magic;  // z / shares = (z * share_magic) >> 32, where the shares' order turns with z (0: it does not)
+    int32_t level_pitch;  // uneven shares: workgroups per KV head that a share's keys are ahead of the next one's (0: the grid's order)
 };
 
 // K, V and Q of a unit as buffers: bytes from row to row, and where this lane's row of Q begins
@@ -303,22 +305,37 @@ __global__ __launch_bounds__(64 * U * KG, D > 128 || (KG == 2 && U == 2 && D > 6
     // Workgroup -> (units, batch, kv head): the units of a KV head are its row blocks times the query heads that share it,
     // numbered heads first, so that U consecutive ones read the same keys; those with the most keys first.
     // (grid: shares of the keys, kv heads of the batch, workgroups per kv head)
-    const int nks = gridDim.x;
-    const int nwg = gridDim.z, wz = blockIdx.z;
-    int ksplit = blockIdx.x;
-    // Workgroups go to the XCDs in turn: an even number of shares would leave the first one, which all rows of a square prompt see, to
-    // some of them (head_dim 256, 2048 rows of 8/1 heads in four shares 215 us).
+    const int nks = gridDim.x, nwg = gridDim.z;
+    int ksplit = blockIdx.x, rem = blockIdx.y, wz = blockIdx.z;
+    // The shares of a square prompt differ in length: workgroup wz + P of a share sees as many keys of it as workgroup wz of the next
+    // one (P: level_pitch), so those with equal wz + share * P are a level, and the levels are numbered the longest first, without gaps.
+    // Workgroups are dealt to the shader engines in turn, which a descending order evens out.  us at head_dim 256, in the grid's order
+    // turned with wz and its plan, and now: 1300 rows of 12/12 heads 141 -> 111, 2000 of 16/4 347 -> 235, 800 of 32/8 151 -> 105.
     if constexpr (D > 128) {
-        if (tl.share_magic) {
-            ksplit += wz - (int)__umulhi((uint32_t)wz, tl.share_magic) * nks;
-            if (ksplit >= nks) ksplit -= nks;
+        if (tl.level_pitch) {
+            const int id = (wz * gridDim.y + rem) * nks + ksplit, pitch = tl.level_pitch;
+            int t = id / (int)gridDim.y, level = 0, first = 0, end = 1;  // shares first .. end - 1 have workgroups in this level
+            rem = id - t * (int)gridDim.y;
+            for (;;) {
+                const int start = end < nks ? end * pitch : 0x7fffffff, stop = first * pitch + nwg, next = min(start, stop);
+                const int shares = end - first, here = (next - level) * shares;
+                if (t < here) {
+                    level += t / shares;
+                    ksplit = first + t % shares;
+                    break;
+                }
+                t -= here;
+                level = next;
+                end += next == start;
+                first += next == stop;
+            }
+            wz = level - ksplit * pitch;
         }
     }
     // with the whole grid resident at once (two workgroups per CU) a CU gets a long and a short one
     const int wg = tl.snake > 0 && wz >= tl.snake ? tl.snake + nwg - 1 - wz : wz;
     const int first_unit = (nwg - 1 - wg) * U;
     auto over_g = [&](int u) __attribute__((always_inline)) { return tl.g_magic ? (int)__umulhi((uint32_t)u, tl.g_magic) : u; };
-    const int rem = blockIdx.y;
     const int b = p.B > 1 ? rem / p.Hkv : 0;
     int g = rem - b * p.Hkv;
     if ((p.Hkv & 7) == 0) g = (g & 7) * (p.Hkv >> 3) + (g >> 3);  // workgroups of one XCD share KV heads
@@ -908,28 +925,39 @@ double prefill_f32_terms_time(const TermsCall &c, TermsForm f, int ns) {
 }
 
 // The same above head_dim 128, where the form is (4, 1) with one workgroup per CU, of uneven calls too.  The hardware deals workgroups out
-// to the 32 shader engines in turn, so a CU gets a second one before all have their first: fitted to 330 calls, 2.7 % off in the mean
-// square with each engine's queue played through.  In closed form: workgroups whose rows see a key of their share go in one round up to
-// 0.85 of the CUs, in one and a half where they fit, and uneven calls with more take one share.
+// to the 32 shader engines in turn: with each engine's queue played through, 330 calls come out 2.7 % off in the mean square.  In
+// closed form: even shares in rounds; of uneven ones, dealt out the longest first, the longest, the mean load, or twice (three times) the
+// first workgroup of the second (third) round.
 static double wide_terms_time(const TermsCall &c, int ns) {
     const double tile = 1.33 * (c.D <= 192 ? 3 : 4), ends = 6.9;
     const int chunk = ((c.Skv + ns - 1) / ns + PT_BN - 1) / PT_BN * PT_BN, n = (c.Skv + chunk - 1) / chunk;
-    const double wgs = (double)terms_workgroups(c, 4, 1);
-    double rounds;
+    const long wgs = terms_workgroups(c, 4, 1);
+    const double longest = ends + tile * (chunk / PT_BN);
+    double us;
     if (!c.uneven) {
-        rounds = (double)(((long)wgs * n + c.cus - 1) / c.cus);
-    } else if (n == 1) {
-        rounds = 1.0;
+        us = (double)((wgs * n + c.cus - 1) / c.cus) * longest;
     } else {
         const double first = c.Skv > c.Sq ? c.Skv - c.Sq : 0.0;  // keys before the first row
-        double active = 0.0;
-        for (int i = 0; i < n; i++) {
-            const double rows = (c.Skv - (double)i * chunk) / (c.Skv - first);
-            active += rows < 0.0 ? 0.0 : rows > 1.0 ? 1.0 : rows;
-        }
-        rounds = wgs * active <= 0.85 * c.cus ? 1.0 : wgs * active <= 1.0 * c.cus ? 1.5 : 1e6;
+        // workgroups that see this many keys of their share
+        auto with_keys = [&](double keys) {
+            double sum = 0.0;
+            for (int i = 0; i < n; i++) {
+                const double rows = (c.Skv - (double)i * chunk - keys) / (c.Skv - first);
+                sum += rows < 0.0 ? 0.0 : rows > 1.0 ? 1.0 : rows;
+            }
+            return sum * wgs;
+        };
+        auto time_of = [&](double nth) {  // of the nth workgroup
+            if (with_keys(0.0) < nth) return 0.0;
+            double keys = 0.0;
+            for (double step = 0.5 * chunk; step >= 16.0; step *= 0.5)
+                if (with_keys(keys + step) >= nth) keys += step;
+            return ends + tile / PT_BN * keys;
+        };
+        const double load = (wgs * (n * ends + (first + c.Skv) * 0.5 / PT_BN * tile)) / c.cus;
+        us = std::max({longest, 1.08 * load, 2.0 * time_of(c.cus + 1.0), 3.0 * time_of(2.0 * c.cus + 1.0)});
     }
-    double us = 4.9 + rounds * (ends + tile * (chunk / PT_BN));
+    us += 4.9;
     if (n > 1) us += 3.24 + 0.456e-6 * prefill_f32_workspace_bytes(c.B, c.Hkv * c.G, c.Sq, c.D, n);
     return us;
 }
@@ -974,7 +1002,9 @@ static int launch_form(const AttnParams &p_in, hipStream_t stream) {
     }
     TermsLaunch tl;
     const unsigned nks = p.pf_nsplit > 1 ? p.pf_nsplit : 1, groups = (unsigned)(p.B * p.Hkv), nwg = (unsigned)(blocks / nks / groups);
-    tl.share_magic = p.D > 128 && nks > 1 && terms_call(p).uneven ? (uint32_t)((0x100000000ull + nks - 1) / nks) : 0;
+    tl.level_pitch = 0;
+    // (grids of one round too: without it calls of 500 rows take 2 to 5 % longer, those of 300 1 to 2 % less)
+    if (p.D > 128 && nks > 1 && terms_call(p).uneven) tl.level_pitch = std::max(1, (int)((int64_t)p.pf_chunk * p.G / (32 * U)));
     tl.g_magic = p.G > 1 ? (uint32_t)((0x100000000ull + p.G - 1) / p.G) : 0;
     const bool two_per_cu = (KG == 1 && p.D <= 128) || (U * KG == 4 && p.D <= 64);
     tl.snake = (two_per_cu && blocks > cus && blocks <= 2L * cus) ? (int)((cus + nks * groups - 1) / (nks * groups)) : 0;

@@ -72,6 +72,7 @@ WIDE = {
     # above head_dim 128: (B, H, Hkv, Sq, Skv, causal)
     "one_tile": (1, 4, 1, 65, 32, False), "unsplit": (2, 16, 4, 130, 65, False), "one_key": (3, 4, 1, 70, 1, False),
     "even_shares": (1, 8, 4, 148, 1251, True), "uneven_shares": (1, 8, 4, 417, 417, True), "shares_some_rows_do_not_see": (1, 4, 4, 801, 801, True),
+    "shares_behind_a_cache": (1, 8, 4, 500, 801, True), "shares_of_odd_heads": (2, 6, 3, 330, 330, True),
     "few_rows": (1, 4, 2, 33, 2500, True), "few_rows_in_f32": (1, 4, 2, 33, 1500, True),
 }
 
