@@ -9,6 +9,7 @@
 #include <new>
 
 #include "common.h"
+#include "decode_marks.h"
 
 // Workspace of fhip_flash_attention_noalloc: device memory the library itself holds, so that the call needs no
 // allocation by anyone.  Each GPU the library runs on has its own copy of the array at its own address, looked
@@ -23,9 +24,10 @@ struct fhip_device {
     int ordinal;
     hipDeviceProp_t prop;
     void *scratch_ptr;  // this device's address of `scratch`
-    // Source of the per-call marks of masked prefill calls (AttnParams::bad_tag): the one piece of state a device
-    // handle changes after its creation.
+    // Sources of the per-call marks of masked prefill calls (AttnParams::bad_tag) and of decode calls (dec_tag): the state a
+    // device handle changes after its creation.
     std::atomic<uint32_t> next_tag;
+    std::atomic<uint64_t> next_mark;
     // The fused split-KV merge needs workgroups L of a one-dimensional launch with the same L % 8 to share an XCD (and
     // with it an L2).  Probed once per handle.  `trip` is a word of pinned host memory the decode kernels set when the
     // workgroups of a unit find themselves on different XCDs all the same: the next decode call then fails once and the
@@ -489,6 +491,7 @@ int fhip_device_create(int32_t ordinal, fhip_device **out) {
     d->ordinal = ordinal;
     // handles of one device start their marks far apart, so that two of them sharing a workspace do not collide
     d->next_tag.store(0x5eed0001u + (uint32_t)((uintptr_t)d >> 4) * 2654435761u, std::memory_order_relaxed);
+    d->next_mark.store(0x5eed0001u + (uint64_t)((uintptr_t)d >> 4) * 0xd1342543de82ef95ull, std::memory_order_relaxed);
     hipError_t e = hipGetDeviceProperties(&d->prop, ordinal);
     if (e != hipSuccess) {
         delete d;
@@ -1036,9 +1039,9 @@ int fhip_flash_attention(fhip_stream *s, const fhip_attn_args *args) {
                     return FHIP_ERR_HIP;
                 }
                 if (p.dec_fused) {
-                    p.dec_marks = (uint32_t *)((char *)args->workspace + p.dec_marks_offset);
+                    p.dec_marks = (uint64_t *)((char *)args->workspace + p.dec_marks_offset);
                     p.dec_trip = dev->trip_dev;
-                    do p.dec_tag = dev->next_tag.fetch_add(1, std::memory_order_relaxed) & 0xfffffu;
+                    do p.dec_tag = mark_tag(dev->next_mark.fetch_add(1, std::memory_order_relaxed));
                     while (p.dec_tag == 0);
                 }
             }

@@ -23,6 +23,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "decode_marks.h"
 #include "device_utils.h"
 
 namespace fhip {
@@ -161,7 +162,9 @@ void decode_plan(int B, int Hkv, int G, int Skv, int D, int compute_units, bool 
 }
 
 // Workspace: the partials, B * H * nsplit * (D + 2) floats (H counts (head, row) pairs), plus what the fused merge adds:
-// every split's partials start on a 128-byte line, and the marks of its units' arrivals behind them, a word per split.
+// every split's partials start on a 128-byte line, and the marks of its units' arrivals behind them, eight bytes per split.  (These
+// need no room of their own: a split's rows are a multiple of eight bytes long, so the start of the next one on a line takes at most 120
+// of the 128 bytes counted for it.)
 size_t decode_workspace_bytes(int B, int H, int Hkv, int D, int nsplit) {
     if (nsplit <= 1) return 0;
     // columns of a KV head, padded to whole column blocks of 16 or 32 where there is more than one block
@@ -187,7 +190,7 @@ bool decode_fused_layout(const AttnParams &p, bool f32, int *unit_stride, size_t
     if ((units + 7) / 8 * 8 * p.nsplit > 0x7fffffffL || stride > 0x7fffffffL) return false;
     *unit_stride = (int)stride;
     *marks_offset = ((size_t)units * stride * sizeof(float) + 255) & ~(size_t)255;
-    return true;
+    return *marks_offset + (size_t)units * p.nsplit * sizeof(uint64_t) <= decode_workspace_bytes(p.B, p.H * p.Sq, p.Hkv, p.D, p.nsplit);
 }
 
 // ---- element helpers ---------------------------------------------------------------------------
@@ -586,8 +589,8 @@ __device__ __forceinline__ float *fused_partial_row(const AttnParams &p, int uni
 // rows.  Partials are served by this XCD's L2: the stores have been acknowledged by it before the arrival is marked, and the merging
 // workgroup reads lines nobody on its CU has read in this launch (every split's partials have whole lines to themselves).  Nothing
 // spins: a workgroup that finds others missing leaves.  Marks are kept coherent over the whole device and carry the XCC id, so that
-// a unit whose workgroups are NOT on one XCD is seen, and a tag unique to the call, so that whatever else their words hold (another
-// call's data) is no mark.
+// a unit whose workgroups are NOT on one XCD is seen, and the call's tag, which tells them from what else their words hold
+// (another call's data), see decode_marks.h.
 //  - Two or three splits count in one word, by compare-and-swap: one round trip, and hardly ever a second one.  The finished count of
 //    a replay of the recorded call restarts it.
 //  - More would retry each other (8 splits of 128 keys, f16, 16/16 heads at 128: 14.1 us a call; 7 of B4, 64: 15.3): every split has a
@@ -599,28 +602,28 @@ __device__ __forceinline__ void fused_merge_tail(const AttnParams &p, int unit, 
     __shared__ int all_here;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    uint32_t *const marks = p.dec_marks + (int64_t)unit * p.nsplit;
-    const uint32_t tag = p.dec_tag << 12, xcc = xcc_id() << 8;
+    uint64_t *const marks = p.dec_marks + (int64_t)unit * p.nsplit;
+    const uint64_t tag = p.dec_tag;
+    const uint32_t xcc = xcc_id(), splits = (uint32_t)p.nsplit;
     if (p.nsplit <= 3) {
         if (threadIdx.x == 0) {
-            // word: tag (20 bits) | XCC id of the first workgroup to arrive (4) | arrivals (8)
-            uint32_t cur = tag | xcc, want;
+            // (the XCC id is that of the first workgroup to arrive)
+            uint64_t cur = mark_of(tag, xcc, 0), want;
             do {
-                want = (cur & ~0xfffu) == tag && (cur & 255u) < (uint32_t)p.nsplit ? cur + 1 : tag | xcc | 1u;
+                want = mark_is_of(cur, tag) && mark_arrivals(cur) < splits ? cur + 1 : mark_of(tag, xcc, 1);
             } while (!__hip_atomic_compare_exchange_strong(marks, &cur, want, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-            if ((want & 0xf00u) != xcc) __hip_atomic_store(p.dec_trip, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            all_here = (want & 255u) == (uint32_t)p.nsplit;
+            if (!mark_same_xcc(want, xcc)) __hip_atomic_store(p.dec_trip, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            all_here = mark_arrivals(want) == splits;
         }
     } else if (threadIdx.x < 64) {
-        // a split's word: tag (20 bits) | XCC id of its workgroup (4) | 1
         const int lane = threadIdx.x;
         const bool mine = lane < p.nsplit;
-        if (lane == 0) __hip_atomic_store(marks + split, tag | xcc | 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (lane == 0) __hip_atomic_store(marks + split, mark_of(tag, xcc, 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        const uint32_t mark = mine ? __hip_atomic_load(marks + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : tag | xcc | 1u;
-        const bool there = (mark & ~0xf00u) == (tag | 1u), all = __builtin_amdgcn_ballot_w64(!there) == 0;
-        if (there && (mark & 0xf00u) != xcc) __hip_atomic_store(p.dec_trip, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        if (all && mine) __hip_atomic_store(marks + lane, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint64_t mark = mine ? __hip_atomic_load(marks + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : mark_of(tag, xcc, 1);
+        const bool there = mark_is(mark, tag, 1), all = __builtin_amdgcn_ballot_w64(!there) == 0;
+        if (there && !mark_same_xcc(mark, xcc)) __hip_atomic_store(p.dec_trip, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (all && mine) __hip_atomic_store(marks + lane, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (lane == 0) all_here = all;
     }
     __syncthreads();

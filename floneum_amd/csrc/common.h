@@ -33,8 +33,8 @@ struct AttnParams {
     // unit run on one XCD, park their partials in that XCD's L2 and the last one to arrive merges them.
     int32_t dec_fused;        // 0: two kernels
     int32_t dec_unit_stride;  // floats between the partials of consecutive units (a multiple of 32: 128-byte lines)
-    uint32_t dec_tag;         // unique to the call (20 bits are used): whatever else a mark's word holds is no mark
-    uint32_t *dec_marks;      // [units][splits] the marks of arrivals, see fused_merge_tail
+    uint64_t dec_tag;         // the call's own, see decode_marks.h
+    uint64_t *dec_marks;      // [units][splits] the marks of arrivals, see fused_merge_tail
     size_t dec_marks_offset;  // host side: bytes from the workspace's start to the marks
     int32_t *dec_trip;        // host-visible word set when the workgroups of a unit turn out to run on different XCDs
     // host-side only (profiling hook).  Both set: the dispatch of the main kernel carries the two events, which then
