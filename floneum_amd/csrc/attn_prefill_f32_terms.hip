@@ -916,7 +916,9 @@ double prefill_f32_terms_time(const TermsCall &c, TermsForm f, int ns) {
     else if (f.KG == 4) tile = 2.65, ends = 3.87;
     else tile = 0.374 + 1.78 * dims, ends = 0.8, alone = 0.74, two_per_cu = true;
     const int chunk = ((c.Skv + ns - 1) / ns + PT_BN - 1) / PT_BN * PT_BN, n = (c.Skv + chunk - 1) / chunk;
-    const double walk = tile * ((chunk / PT_BN + f.KG - 1) / f.KG);
+    int tiles = chunk / PT_BN;
+    if (c.window > 0 && c.window < c.Skv) tiles = std::min(tiles, ((int)c.window + 2 * PT_BN - 1) / PT_BN + 1);
+    const double walk = tile * ((tiles + f.KG - 1) / f.KG);
     const long wgs = terms_workgroups(c, f.U, n), slots = (two_per_cu ? 2L : 1L) * c.cus, rest = wgs % slots;
     double us = 4.9 + wgs / slots * (ends + walk);
     if (rest) us += ends + walk * (rest <= c.cus ? alone : 1.0);
@@ -924,15 +926,22 @@ double prefill_f32_terms_time(const TermsCall &c, TermsForm f, int ns) {
     return us;
 }
 
-// The same above head_dim 128, where the form is (4, 1) with one workgroup per CU, of uneven calls too.  The hardware deals workgroups out
-// to the 32 shader engines in turn: with each engine's queue played through, 330 calls come out 2.7 % off in the mean square.  In
-// closed form: even shares in rounds; of uneven ones, dealt out the longest first, the longest, the mean load, or twice (three times) the
-// first workgroup of the second (third) round.
+// The same above head_dim 128, where the form is (4, 1) with one workgroup per CU, of uneven calls too: even shares in rounds; of uneven
+// ones, dealt out the longest first, the longest, the mean load, or twice (three times) the first workgroup of the second (third) round.
+// Over 420 random calls at 160 to 256 dims in up to 48 shares it is 6 % off in the mean square, 9 % under a window.
+// Under a window a row block sees the window's keys and meets few of the shares; the
+// workgroups of the others still split Q, park a state and have it merged (us, planned without the window and with it: 16/8 heads at 256,
+// 786 rows under a window of 127 59 -> 47; 12/12 at 160, 1317 under 103 58 -> 46; 6/3 at 192, three sequences of 718 under 117 50 -> 38).
 static double wide_terms_time(const TermsCall &c, int ns) {
     const double tile = 1.33 * (c.D <= 192 ? 3 : 4), ends = 6.9;
     const int chunk = ((c.Skv + ns - 1) / ns + PT_BN - 1) / PT_BN * PT_BN, n = (c.Skv + chunk - 1) / chunk;
     const long wgs = terms_workgroups(c, 4, 1);
-    const double longest = ends + tile * (chunk / PT_BN);
+    const int rows = std::min(c.Sq, 32 * ((4 + c.G - 1) / c.G));  // of a workgroup
+    const bool narrow = c.window > 0 && c.window < c.Skv - rows;
+    const double sight = narrow ? (double)c.window + rows : c.Skv;  // keys from the first to the last that a workgroup's rows see
+    double most = chunk / PT_BN;
+    if (narrow && sight <= chunk) most = (int)(sight - 1 + PT_BN - 1) / PT_BN + 1;
+    const double longest = ends + tile * most;
     double us;
     if (!c.uneven) {
         us = (double)((wgs * n + c.cus - 1) / c.cus) * longest;
@@ -942,19 +951,23 @@ static double wide_terms_time(const TermsCall &c, int ns) {
         auto with_keys = [&](double keys) {
             double sum = 0.0;
             for (int i = 0; i < n; i++) {
-                const double rows = (c.Skv - (double)i * chunk - keys) / (c.Skv - first);
-                sum += rows < 0.0 ? 0.0 : rows > 1.0 ? 1.0 : rows;
+                const double from = std::max(first, (double)i * chunk + keys);
+                const double to = narrow ? std::min<double>(c.Skv, std::min<double>(c.Skv, (i + 1.0) * chunk) + sight - keys) : c.Skv;
+                const double part = (to - from) / (c.Skv - first);
+                sum += part < 0.0 ? 0.0 : part > 1.0 ? 1.0 : part;
             }
             return sum * wgs;
         };
         auto time_of = [&](double nth) {  // of the nth workgroup
-            if (with_keys(0.0) < nth) return 0.0;
+            if (with_keys(0.0) < nth) return narrow && wgs * n >= nth ? ends : 0.0;
             double keys = 0.0;
             for (double step = 0.5 * chunk; step >= 16.0; step *= 0.5)
-                if (with_keys(keys + step) >= nth) keys += step;
+                if (keys + step <= sight && with_keys(keys + step) >= nth) keys += step;
             return ends + tile / PT_BN * keys;
         };
-        const double load = (wgs * (n * ends + (first + c.Skv) * 0.5 / PT_BN * tile)) / c.cus;
+        double seen = (first + c.Skv) * 0.5;  // by a row in the mean
+        if (narrow) seen = first >= sight ? sight : (0.5 * (sight * sight - first * first) + sight * (c.Skv - sight)) / (c.Skv - first);
+        const double load = wgs * (n * ends + seen / PT_BN * tile) / c.cus;
         us = std::max({longest, 1.08 * load, 2.0 * time_of(c.cus + 1.0), 3.0 * time_of(2.0 * c.cus + 1.0)});
     }
     us += 4.9;
@@ -988,7 +1001,7 @@ TermsForm prefill_f32_terms_form(const TermsCall &c, int ns) {
 // (rows of a square prompt under a causal mask, for which a mask tensor is taken, see from one to all of the keys)
 static TermsCall terms_call(const AttnParams &p) {
     const bool uneven = 2L * p.Sq > p.Skv && (p.causal || p.mask_kind == FHIP_MASK_QK);
-    return {p.B, p.Hkv, p.G, p.Sq, p.Skv, p.D, p.cus > 0 ? p.cus : 256, uneven};
+    return {p.B, p.Hkv, p.G, p.Sq, p.Skv, p.D, p.cus > 0 ? p.cus : 256, uneven, p.analytic ? p.window : 0};
 }
 
 template <typename T, int U, int KG, int MODE>
@@ -1003,7 +1016,8 @@ static int launch_form(const AttnParams &p_in, hipStream_t stream) {
     TermsLaunch tl;
     const unsigned nks = p.pf_nsplit > 1 ? p.pf_nsplit : 1, groups = (unsigned)(p.B * p.Hkv), nwg = (unsigned)(blocks / nks / groups);
     tl.level_pitch = 0;
-    // (grids of one round too: without it calls of 500 rows take 2 to 5 % longer, those of 300 1 to 2 % less)
+    // (grids of one round too: without it calls of 500 rows take 2 to 5 % longer, those of 300 1 to 2 % less; under a window the same
+    // workgroups of a share still see alike: the grid's order takes 1.07 to 1.16 times as long in two to eight shares of 120 random prompts)
     if (p.D > 128 && nks > 1 && terms_call(p).uneven) tl.level_pitch = std::max(1, (int)((int64_t)p.pf_chunk * p.G / (32 * U)));
     tl.g_magic = p.G > 1 ? (uint32_t)((0x100000000ull + p.G - 1) / p.G) : 0;
     const bool two_per_cu = (KG == 1 && p.D <= 128) || (U * KG == 4 && p.D <= 64);

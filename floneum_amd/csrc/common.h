@@ -66,12 +66,15 @@ struct AttnParams {
 };
 
 // the key split of a tiled f32 prefill call (1 = none) and the scratch it needs
-// uneven: a square call whose rows see the keys up to their own position (a mask tensor is taken for one)
-void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, bool causal_square, bool uneven, int compute_units, int *nsplit, int *chunk);
+// uneven: a square call whose rows see the keys up to their own position (a mask tensor is taken for one); window: of those the last
+// so many (0: all)
+void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, bool causal_square, bool uneven, int64_t window, int compute_units,
+                      int *nsplit, int *chunk);
 // The forms of the f32 terms kernel (attn_prefill_f32_terms.hip): units and key groups per workgroup, and what a call takes in them
 struct TermsCall {
     int B, Hkv, G, Sq, Skv, D, cus;
     bool uneven;
+    int64_t window;
 };
 struct TermsForm {
     int U, KG;

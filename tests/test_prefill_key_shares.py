@@ -53,6 +53,58 @@ def test_a_window_is_planned_on_its_keys(D, dtype, before):
     assert got in {shares(2, 16, 4, rows, n, D, dtype) for n in range(seen, seen + 128)}
 
 
+@pytest.mark.parametrize("D", [256, 192, 160])
+@pytest.mark.parametrize("H, Hkv, rows", [(4, 1, 3000), (8, 4, 2000), (16, 8, 1000), (12, 12, 1693)])
+def test_a_windowed_prompt_is_not_shared_out_as_a_whole_one(H, Hkv, rows, D):
+    """Above 128 dims a row block under a narrow window would meet one or two of the shares that the whole prompt has."""
+    whole = shares(1, H, Hkv, rows, rows, D, fa.F32)
+    assert whole >= 3
+    assert all(shares(1, H, Hkv, rows, rows, D, fa.F32, window=w) == 0 for w in (1, 32, 128))
+    assert all(shares(1, H, Hkv, rows, rows, D, fa.F32, window=w) == whole for w in (rows - 1, rows, 2 * rows, 2 ** 40, 2 ** 63 - 1))
+
+
+@pytest.mark.parametrize("H, Hkv, rows, keys, D, window, want", [
+    # of three shares two would hold no key of a row block
+    (32, 8, 173, 1420, 80, 334, 0), (32, 8, 173, 1420, 80, 0, 3), (32, 8, 173, 1420, 80, 1400, 3),
+])
+def test_a_windowed_chunk_is_not_shared_out_as_a_whole_one(H, Hkv, rows, keys, D, window, want):
+    assert shares(3, H, Hkv, rows, keys, D, fa.F32, window=window) == want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [256, 160])
+@pytest.mark.parametrize("H, Hkv, rows, keys, window, how, want", [
+    (4, 1, 800, 800, 500, "window", 9), (4, 2, 513, 513, 300, "window", 6), (4, 1, 700, 700, 33, "window", 0), (4, 4, 640, 800, 450, "window", 9),
+    (4, 1, 650, 650, 0, "table", 7), (4, 2, 417, 417, 200, "table", 5), (4, 1, 300, 640, 0, "lens", 10), (2, 2, 129, 333, 0, "lens", 4),
+])
+def test_wide_heads_in_shares(device, H, Hkv, rows, keys, window, how, want, D):
+    """Uneven shares and their levels above 128 dims under a window, a mask tensor's interval table and lengths of two sequences (one of
+    them in the first share alone)."""
+    B = 2 if how == "lens" else 1
+    rng = np.random.default_rng(rows * 7 + D)
+    q, k, v = tensor(device, rng, fa.F32, (B, H, rows, D)), tensor(device, rng, fa.F32, (B, Hkv, keys, D)), tensor(device, rng, fa.F32, (B, Hkv, keys, D))
+    i, j = np.arange(rows)[:, None] + keys - rows, np.arange(keys)[None, :]
+    hidden = np.broadcast_to((j > i) | ((j + window <= i) if window else False), (B, rows, keys))
+    analytic = mask = lens = None
+    if how == "window":
+        analytic = (True, keys - rows, window)
+    elif how == "table":
+        m = fa.Tensor.from_numpy(device, np.where(hidden[0], -np.inf, 0.0).astype(np.float32), fa.F32)
+        mask = (m, fa.MaskKind.QKMask)
+    else:
+        counts = np.array([keys, 20], np.int32)
+        lens, hidden = fa.IntTensor(device, counts), np.broadcast_to(np.arange(keys)[None, None, :] >= counts[:, None, None], (B, rows, keys))
+    assert shares(B, H, Hkv, rows, keys, D, fa.F32, causal=how != "lens", window=window if how == "window" else 0) == want
+    out = q.flash_attention(k, v, D ** -0.5, mask, analytic=analytic, kv_lens=lens).to_numpy().astype(np.float64)
+    a, b, c = (t.to_numpy().astype(np.float64) for t in (q, k, v))
+    b, c = (np.repeat(t, H // Hkv, axis=1) for t in (b, c))
+    s = np.where(hidden[:, None], -np.inf, a @ b.transpose(0, 1, 3, 2) * D ** -0.5)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    ref = (p / p.sum(-1, keepdims=True)) @ c
+    err = np.linalg.norm(out - ref) / np.linalg.norm(ref)
+    assert err <= 7.6e-7, f"relative L2 {err:.2e}"
+
+
 def tensor(device, rng, dtype, shape):
     return fa.Tensor.from_numpy(device, rng.normal(0, 1, shape).astype(np.float32), dtype)
 
