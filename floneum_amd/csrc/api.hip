@@ -327,8 +327,9 @@ static void visible_range(const fhip_attn_args *a, int *lo0, int *len) {
 static void f32_split_plan(const fhip_attn_args *a, int cus, int *nsplit, int *chunk) {
     int lo0, len;
     visible_range(a, &lo0, &len);
-    const bool causal_square = a->analytic.enabled && a->analytic.causal && 2ll * a->q.shape[2] > len;
-    const bool uneven = causal_square || (a->mask_kind == FHIP_MASK_QK && 2ll * a->q.shape[2] > len);
+    const bool square = 2ll * a->q.shape[2] > len, causal_square = a->analytic.enabled && a->analytic.causal && square;
+    const bool uneven = prefill_f32_uneven(a->q.shape[2], len, a->q.shape[3], a->analytic.enabled && a->analytic.causal,
+                                           a->mask_kind == FHIP_MASK_QK, a->analytic.q_pos_offset - lo0, a->analytic.window);
     const int Hkv = (int)a->k.shape[1];
     prefill_f32_plan((int)a->q.shape[0], (int)a->q.shape[1], Hkv ? (int)a->q.shape[1] / Hkv : 1, (int)a->q.shape[2],
                      len, (int)a->q.shape[3], a->dtype == FHIP_F32, causal_square, uneven, a->analytic.enabled ? a->analytic.window : 0,

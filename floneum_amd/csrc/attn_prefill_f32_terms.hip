@@ -998,9 +998,8 @@ TermsForm prefill_f32_terms_form(const TermsCall &c, int ns) {
     return prefill_f32_terms_time(c, other, ns) < 0.9 * prefill_f32_terms_time(c, ordinary, ns) ? other : ordinary;
 }
 
-// (rows of a square prompt under a causal mask, for which a mask tensor is taken, see from one to all of the keys)
 static TermsCall terms_call(const AttnParams &p) {
-    const bool uneven = 2L * p.Sq > p.Skv && (p.causal || p.mask_kind == FHIP_MASK_QK);
+    const bool uneven = prefill_f32_uneven(p.Sq, p.Skv, p.D, p.analytic && p.causal, p.mask_kind == FHIP_MASK_QK, p.q_pos_offset, p.window);
     return {p.B, p.Hkv, p.G, p.Sq, p.Skv, p.D, p.cus > 0 ? p.cus : 256, uneven, p.analytic ? p.window : 0};
 }
 

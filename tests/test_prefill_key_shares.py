@@ -71,6 +71,12 @@ def test_a_windowed_chunk_is_not_shared_out_as_a_whole_one(H, Hkv, rows, keys, D
     assert shares(3, H, Hkv, rows, keys, D, fa.F32, window=window) == want
 
 
+def test_rows_behind_a_full_window_see_alike():
+    """A chunk of more rows than its window is planned as an even call from the keys on at which the first row sees a whole window."""
+    assert [shares(1, 8, 4, 1200, keys, 128, fa.F32, window=600) for keys in (1200, 1798, 1799, 4000)] == [3, 3, 0, 0]
+    assert shares(1, 4, 1, 1804, 6014, 256, fa.F32, window=1515) >= 3  # (above 128 dims uneven shares know their window)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("D", [256, 160])
 @pytest.mark.parametrize("H, Hkv, rows, keys, window, how, want", [
