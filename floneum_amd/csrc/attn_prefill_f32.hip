@@ -15,6 +15,7 @@
 //
 // Reference semantics: fusor-ml/fusor/src/composite/flash_attention.rs:141-199; this is the data
 // type kalosm-llama always calls with (models/kalosm-llama/src/raw/attention_layer.rs:400-448).
+#include <algorithm>
 #include <type_traits>
 
 #include "attn_bounds.h"
@@ -701,6 +702,18 @@ static long shares_of_least_time(const TermsCall &c, long ordinary) {
     return ordinary;
 }
 
+// Time in us of an unsplit call of more than 64 rows above head_dim 128 on the f32 matrix instruction (launch_wide): 64-row workgroups that
+// walk their rows' keys, two on a CU beyond one each.  Its tiles take longer than the terms kernel's, but its workgroups start sooner
+// and see fewer keys beside a window's: short prompts and narrow windows (us there and in terms, head_dim 256: 95 rows of 12/12 heads
+// 22.6 and 27.1, three sequences of 77 of 10/2 22.6 and 27.8, 832 of 12/12 under a window of 134 49 and 62; over 50 random such calls
+// 0.94 of the time in terms).  9 % off in the mean square over 206 calls of up to 13 tiles.
+static double wide_f32_time(const TermsCall &c) {
+    const int keys = c.window > 0 && c.window < c.Skv - 64 ? (int)c.window + 64 : c.Skv;
+    const double tile = c.D <= 192 ? 5.4 : c.uneven ? 5.75 : 6.2;
+    const long wgs = (long)c.B * c.Hkv * c.G * ((c.Sq + 63) / 64);
+    return (c.D <= 192 ? 8.5 : 6.0) + tile * ((keys + 31) / 32) * std::max(1.0, (double)wgs / c.cus);
+}
+
 // Few query rows on a long cache (a new chat turn, a prompt fed in pieces): the grid of query blocks alone leaves
 // most CUs idle, so the keys are split over workgroups as well.
 void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, bool causal_square, bool uneven, int64_t window, int compute_units,
@@ -756,8 +769,9 @@ void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, boo
         // Head dims above 128 in the terms kernel: the shares of least time (us, 16/4 heads at 256 causal, in one share and in
         // the shares taken: 148 rows on 3510 keys 584 -> 80, 300 on 700 128 -> 49, 1000 on 1000 182 -> 93, 2000 on 2000 347 -> 235; 2048 on 2048 stays at 355, its two shares
         // would be more than 64 MiB of partials).
-        const long ns = shares_of_least_time({B, H / G, G, Sq, Skv, D, compute_units, uneven, window}, 1);
-        if (ns < 2) return;
+        const TermsCall call = {B, H / G, G, Sq, Skv, D, compute_units, uneven, window};
+        const long ns = shares_of_least_time(call, 1);
+        if (ns < 2 || wide_f32_time(call) < prefill_f32_terms_time(call, {4, 1}, (int)ns)) return;
         const long c = ((Skv + ns - 1) / ns + 31) / 32 * 32;
         *chunk = (int)c;
         *nsplit = (int)((Skv + c - 1) / c);
@@ -794,15 +808,24 @@ size_t prefill_f32_workspace_bytes(int B, int H, int Sq, int D, int nsplit) {
     return (size_t)B * H * Sq * nsplit * (size_t)(D + 2) * sizeof(float);
 }
 
-// Head dims above 128 in f32: the terms kernel, but for up to 64 rows on up to 2048 keys whose shares leave CUs without a workgroup of
-// launch_wide's: a workgroup alone on its CU takes longer to split its first tile and Q into terms than the f32 instruction takes for both
-// (us, head_dim 256, here and in terms: 9 rows of 16/4 heads on 2048 keys 34.7 and 37.3, 33 rows on 1000 39.6 and 43.0; 64 rows of 4 heads
-// on 4096 50.2 and 41.1, 17 rows of 32/8 heads on 8192 108 and 70).
+// Head dims above 128 in f32: the terms kernel, but for
+//  - up to 64 rows whose shares leave CUs without a workgroup of launch_wide's, on up to 2048 keys, or above 192 dims half of the CUs: a
+//    workgroup alone on its CU takes longer to split its first tile and Q into terms than the f32 instruction takes for both
+//    (us, head_dim 256, here and in terms: 9 rows of 16/4 heads on 2048 keys 34.7 and 37.3, 33 rows on 1000 39.6 and 43.0, 16 of 4/1 on 3299
+//    39.1 and 41.2; 64 rows of 4 heads on 4096 50.2 and 41.1, 17 rows of 32/8 heads on 8192 108 and 70);
+//  - up to 64 rows whose heads leave half of the terms kernel's units empty, so that it has as many workgroups as launch_wide (40 to 50 rows of
+//    16/16 heads on 1829 keys 73.7 and 78.8, of 32/32 on 3286 283 and 306);
+//  - more rows that see few keys, unsplit (wide_f32_time).
 static bool wide_in_terms(const AttnParams &p) {
-    if (p.Sq > 64) return true;
-    const long ns = p.pf_nsplit > 1 ? p.pf_nsplit : 1, keys = ns > 1 ? ns * p.pf_chunk : p.Skv;
-    const long wgs = (long)p.B * (prefill_f32_wide_pack(p.G, p.Sq, p.D) ? p.H / 2 : p.H) * ns;
-    return keys > 2048 || wgs >= (p.cus > 0 ? p.cus : 256);
+    const int cus = p.cus > 0 ? p.cus : 256;
+    const long ns = p.pf_nsplit > 1 ? p.pf_nsplit : 1;
+    if (p.Sq > 64) {
+        const TermsCall c = prefill_f32_terms_call(p);
+        return ns > 1 || prefill_f32_terms_time(c, {4, 1}, 1) <= wide_f32_time(c);
+    }
+    const long wgs = (long)p.B * (prefill_f32_wide_pack(p.G, p.Sq, p.D) ? p.H / 2 : p.H);
+    const long of_units = (long)p.B * p.Hkv * ((p.G * ((p.Sq + 31) / 32) + 3) / 4);
+    return of_units < wgs && (wgs * ns >= cus || (p.Skv > 2048 && (p.D <= 192 || 2 * wgs * ns >= cus)));
 }
 
 template <typename T>

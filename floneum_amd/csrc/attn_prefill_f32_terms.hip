@@ -998,7 +998,7 @@ TermsForm prefill_f32_terms_form(const TermsCall &c, int ns) {
     return prefill_f32_terms_time(c, other, ns) < 0.9 * prefill_f32_terms_time(c, ordinary, ns) ? other : ordinary;
 }
 
-static TermsCall terms_call(const AttnParams &p) {
+TermsCall prefill_f32_terms_call(const AttnParams &p) {
     const bool uneven = prefill_f32_uneven(p.Sq, p.Skv, p.D, p.analytic && p.causal, p.mask_kind == FHIP_MASK_QK, p.q_pos_offset, p.window);
     return {p.B, p.Hkv, p.G, p.Sq, p.Skv, p.D, p.cus > 0 ? p.cus : 256, uneven, p.analytic ? p.window : 0};
 }
@@ -1007,7 +1007,7 @@ template <typename T, int U, int KG, int MODE>
 static int launch_form(const AttnParams &p_in, hipStream_t stream) {
     AttnParams p = p_in;
     const int cus = p.cus > 0 ? p.cus : 256;
-    const long blocks = terms_workgroups(terms_call(p), U, p.pf_nsplit);
+    const long blocks = terms_workgroups(prefill_f32_terms_call(p), U, p.pf_nsplit);
     if (blocks > 0x7fffffffL) {
         set_error("prefill f32: too many workgroups (%ld)", blocks);
         return FHIP_ERR_UNSUPPORTED;
@@ -1017,7 +1017,7 @@ static int launch_form(const AttnParams &p_in, hipStream_t stream) {
     tl.level_pitch = 0;
     // (grids of one round too: without it calls of 500 rows take 2 to 5 % longer, those of 300 1 to 2 % less; under a window the same
     // workgroups of a share still see alike: the grid's order takes 1.07 to 1.16 times as long in two to eight shares of 120 random prompts)
-    if (p.D > 128 && nks > 1 && terms_call(p).uneven) tl.level_pitch = std::max(1, (int)((int64_t)p.pf_chunk * p.G / (32 * U)));
+    if (p.D > 128 && nks > 1 && prefill_f32_terms_call(p).uneven) tl.level_pitch = std::max(1, (int)((int64_t)p.pf_chunk * p.G / (32 * U)));
     tl.g_magic = p.G > 1 ? (uint32_t)((0x100000000ull + p.G - 1) / p.G) : 0;
     const bool two_per_cu = (KG == 1 && p.D <= 128) || (U * KG == 4 && p.D <= 64);
     tl.snake = (two_per_cu && blocks > cus && blocks <= 2L * cus) ? (int)((cus + nks * groups - 1) / (nks * groups)) : 0;
@@ -1058,7 +1058,7 @@ template <typename T, int MODE>
 static int launch_terms(const AttnParams &p, hipStream_t stream) {
     // 16-bit storage takes (4, 1) always
     if constexpr (sizeof(T) == 4) {
-        const TermsForm f = prefill_f32_terms_form(terms_call(p), p.pf_nsplit > 1 ? p.pf_nsplit : 1);
+        const TermsForm f = prefill_f32_terms_form(prefill_f32_terms_call(p), p.pf_nsplit > 1 ? p.pf_nsplit : 1);
         if (f.U == 2 && f.KG == 4) return launch_form<T, 2, 4, MODE>(p, stream);
         if (f.U == 2) return launch_form<T, 2, 2, MODE>(p, stream);
         if (f.KG == 2) return launch_form<T, 4, 2, MODE>(p, stream);

@@ -87,6 +87,7 @@ struct TermsCall {
 struct TermsForm {
     int U, KG;
 };
+TermsCall prefill_f32_terms_call(const AttnParams &p);
 double prefill_f32_terms_time(const TermsCall &call, TermsForm form, int key_shares);  // us, of calls that are not uneven, or above head_dim 128
 TermsForm prefill_f32_terms_quickest(const TermsCall &call, int key_shares);           // by that time
 TermsForm prefill_f32_terms_form(const TermsCall &call, int key_shares);               // the one that runs

@@ -74,6 +74,8 @@ WIDE = {
     "even_shares": (1, 8, 4, 148, 1251, True), "uneven_shares": (1, 8, 4, 417, 417, True), "shares_some_rows_do_not_see": (1, 4, 4, 801, 801, True),
     "shares_behind_a_cache": (1, 8, 4, 500, 801, True), "shares_of_odd_heads": (2, 6, 3, 330, 330, True),
     "few_rows": (1, 4, 2, 33, 2500, True), "few_rows_in_f32": (1, 4, 2, 33, 1500, True),
+    # (few keys, unsplit, take the f32 instruction above 192 dims unless the grid is large; half-filled workgroups of units do)
+    "unsplit_of_many": (8, 16, 4, 130, 65, False), "half_filled": (2, 16, 16, 40, 700, True), "half_filled_long": (2, 4, 4, 40, 2500, True),
 }
 
 
@@ -90,7 +92,7 @@ def test_wide_heads(device, form, D):
 
 @pytest.mark.parametrize("D", [256, 160])
 @pytest.mark.parametrize("of", ["V", "Q"])
-@pytest.mark.parametrize("form", ["unsplit", "uneven_shares"])
+@pytest.mark.parametrize("form", ["unsplit", "unsplit_of_many", "uneven_shares"])
 def test_wide_heads_beyond_bf16(device, form, of, D):
     """Rows that are formed once more in f32: magnitudes at the bottom of f32's range, and an infinity that one key's V holds."""
     B, H, Hkv, Sq, Skv, causal = WIDE[form]

@@ -63,6 +63,12 @@ def test_a_windowed_prompt_is_not_shared_out_as_a_whole_one(H, Hkv, rows, D):
     assert all(shares(1, H, Hkv, rows, rows, D, fa.F32, window=w) == whole for w in (rows - 1, rows, 2 * rows, 2 ** 40, 2 ** 63 - 1))
 
 
+def test_narrow_windows_are_not_shared_out():
+    """Above 192 dims a short walk is quicker unsplit on the f32 instruction than in shares of the terms kernel."""
+    assert [shares(1, 32, 32, 396, 396, 256, fa.F32, window=w) for w in (130, 156, 200, 300)] == [0, 0, 0, 3]
+    assert [shares(1, 32, 32, 175, 175, 256, fa.F32, window=w) for w in (50, 0)] == [0, 2]
+
+
 @pytest.mark.parametrize("H, Hkv, rows, keys, D, window, want", [
     # of three shares two would hold no key of a row block
     (32, 8, 173, 1420, 80, 334, 0), (32, 8, 173, 1420, 80, 0, 3), (32, 8, 173, 1420, 80, 1400, 3),
