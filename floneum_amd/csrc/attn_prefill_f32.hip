@@ -680,7 +680,8 @@ static int launch_rows(const AttnParams &p, hipStream_t stream) {
     return FHIP_OK;
 }
 
-// Shares of the keys: the fewest within 2 % of the least time, where that is 5 % less than the time of `ordinary` ones.
+// Shares of the keys: the fewest within 2 % of the least time, where that is 5 % less than the time of `ordinary` ones; each in the form
+// that it would run in.
 static long shares_of_least_time(const TermsCall &c, long ordinary) {
     constexpr int SHARES[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48};
     const long units = (long)c.G * ((c.Sq + 31) / 32);
@@ -691,7 +692,7 @@ static long shares_of_least_time(const TermsCall &c, long ordinary) {
         if (n > 1 && (c.Skv / n < 64 || prefill_f32_workspace_bytes(c.B, c.Hkv * c.G, c.Sq, c.D, n) > ((size_t)64 << 20) ||
                       (n - 1) * (long)c.B * c.Hkv * units > 6L * c.cus))
             break;
-        times[tried] = prefill_f32_terms_time(c, prefill_f32_terms_quickest(c, n), n);
+        times[tried] = prefill_f32_terms_time(c, prefill_f32_terms_form(c, n), n);
         if (tried == 0 || times[tried] < least) least = times[tried];
         tried++;
     }
@@ -758,7 +759,7 @@ void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, boo
         // rule's; at most 64 MiB of partials (us a call: two sequences of 275 rows of 32/8
         // heads at 64 on 2911 keys 116 -> 92; 16 heads without a mask, 1156 rows at 128 148 -> 80, 2506 366 -> 285, 1147 at 80 109 -> 59; over 90
         // random calls the time is 0.91, the worst 1.03 of the rule's).  Square prompts to 768 keys keep the rule, masked or not.
-        if (!uneven && Sq > 128 && (few_rows || Skv > 768)) ns = shares_of_least_time({B, H / G, G, Sq, Skv, D, compute_units, false, window}, ns < 2 ? 1 : ns);
+        if (!uneven && Sq > 128 && (few_rows || Skv > 768)) ns = shares_of_least_time({B, H / G, G, Sq, Skv, D, compute_units, false, window, f32}, ns < 2 ? 1 : ns);
         if (ns < 2) return;
         const long c = ((Skv + ns - 1) / ns + 31) / 32 * 32;
         *chunk = (int)c;
@@ -769,7 +770,7 @@ void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, boo
         // Head dims above 128 in the terms kernel: the shares of least time (us, 16/4 heads at 256 causal, in one share and in
         // the shares taken: 148 rows on 3510 keys 584 -> 80, 300 on 700 128 -> 49, 1000 on 1000 182 -> 93, 2000 on 2000 347 -> 235; 2048 on 2048 stays at 355, its two shares
         // would be more than 64 MiB of partials).
-        const TermsCall call = {B, H / G, G, Sq, Skv, D, compute_units, uneven, window};
+        const TermsCall call = {B, H / G, G, Sq, Skv, D, compute_units, uneven, window, true};
         const long ns = shares_of_least_time(call, 1);
         if (ns < 2 || wide_f32_time(call) < prefill_f32_terms_time(call, {4, 1}, (int)ns)) return;
         const long c = ((Skv + ns - 1) / ns + 31) / 32 * 32;

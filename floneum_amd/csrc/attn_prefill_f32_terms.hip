@@ -976,7 +976,7 @@ static double wide_terms_time(const TermsCall &c, int ns) {
 }
 
 TermsForm prefill_f32_terms_quickest(const TermsCall &c, int ns) {
-    if (c.D > 128) return {4, 1};
+    if (c.D > 128 || !c.f32) return {4, 1};
     TermsForm best = {4, 1};
     double least = prefill_f32_terms_time(c, best, ns);
     for (const TermsForm f : {TermsForm{4, 2}, TermsForm{2, 2}, TermsForm{2, 4}}) {
@@ -991,16 +991,17 @@ TermsForm prefill_f32_terms_quickest(const TermsCall &c, int ns) {
 // is 10 % better (us a call: 16 heads without a mask, 1356 rows at 128 169 -> 99; 6 encoder sequences of 436 tokens 41.5 -> 30.6, 11
 // of 169 23.2 -> 18.4; at 7 % ten sequences of 154, 240 workgroups of five tiles, 16.4 -> 17.1).  Up to 128 rows the rule is as good.
 TermsForm prefill_f32_terms_form(const TermsCall &c, int ns) {
-    if (c.D > 128) return {4, 1};
+    if (c.D > 128 || !c.f32) return {4, 1};
     const TermsForm ordinary = form_by_workgroups(c, ns);
     if (c.uneven || c.Sq <= 128 || c.Skv <= 2 * PT_BN) return ordinary;
     const TermsForm other = prefill_f32_terms_quickest(c, ns);
     return prefill_f32_terms_time(c, other, ns) < 0.9 * prefill_f32_terms_time(c, ordinary, ns) ? other : ordinary;
 }
 
+// (of f32 tensors)
 TermsCall prefill_f32_terms_call(const AttnParams &p) {
     const bool uneven = prefill_f32_uneven(p.Sq, p.Skv, p.D, p.analytic && p.causal, p.mask_kind == FHIP_MASK_QK, p.q_pos_offset, p.window);
-    return {p.B, p.Hkv, p.G, p.Sq, p.Skv, p.D, p.cus > 0 ? p.cus : 256, uneven, p.analytic ? p.window : 0};
+    return {p.B, p.Hkv, p.G, p.Sq, p.Skv, p.D, p.cus > 0 ? p.cus : 256, uneven, p.analytic ? p.window : 0, true};
 }
 
 template <typename T, int U, int KG, int MODE>

@@ -83,6 +83,7 @@ struct TermsCall {
     int B, Hkv, G, Sq, Skv, D, cus;
     bool uneven;
     int64_t window;
+    bool f32;  // the tensors' type (16-bit ones run in one form)
 };
 struct TermsForm {
     int U, KG;

@@ -63,6 +63,19 @@ def test_a_windowed_prompt_is_not_shared_out_as_a_whole_one(H, Hkv, rows, D):
     assert all(shares(1, H, Hkv, rows, rows, D, fa.F32, window=w) == whole for w in (rows - 1, rows, 2 * rows, 2 ** 40, 2 ** 63 - 1))
 
 
+@pytest.mark.parametrize("H, Hkv, rows, keys, D, causal, want", [
+    (16, 4, 1500, 1500, 100, False, 2), (32, 8, 200, 3000, 100, True, 7), (32, 8, 200, 3000, 36, True, 7), (16, 8, 400, 2500, 60, True, 8),
+])
+def test_16_bit_tensors_on_the_f32_kernel_are_planned_for_their_one_form(H, Hkv, rows, keys, D, causal, want):
+    """Head dims that are no multiple of 8.  (f32 tensors have other forms, and other shares, to choose from.)"""
+    a, need = make_args(B=1, H=H, Hkv=Hkv, Sq=rows, Skv=keys, D=D, dtype=fa.F16), ctypes.c_size_t()
+    if causal:
+        a.analytic.enabled, a.analytic.causal, a.analytic.q_pos_offset = 1, 1, keys - rows
+    assert fa.lib().fhip_flash_attention_workspace_bytes(ctypes.byref(a), CUS, ctypes.byref(need)) == fa.OK
+    assert need.value == want * H * rows * (D + 2) * 4
+    assert shares(1, H, Hkv, rows, keys, D, fa.F32, causal=causal) < want
+
+
 def test_narrow_windows_are_not_shared_out():
     """Above 192 dims a short walk is quicker unsplit on the f32 instruction than in shares of the terms kernel."""
     assert [shares(1, 32, 32, 396, 396, 256, fa.F32, window=w) for w in (130, 156, 200, 300)] == [0, 0, 0, 3]
