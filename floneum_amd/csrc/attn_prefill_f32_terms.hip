@@ -917,7 +917,9 @@ double prefill_f32_terms_time(const TermsCall &c, TermsForm f, int ns) {
     else tile = 0.374 + 1.78 * dims, ends = 0.8, alone = 0.74, two_per_cu = true;
     const int chunk = ((c.Skv + ns - 1) / ns + PT_BN - 1) / PT_BN * PT_BN, n = (c.Skv + chunk - 1) / chunk;
     int tiles = chunk / PT_BN;
-    if (c.window > 0 && c.window < c.Skv) tiles = std::min(tiles, ((int)c.window + 2 * PT_BN - 1) / PT_BN + 1);
+    // (rows of a chunk see the window's keys; wider windows than 0.7 of the keys are taken for none: 32/8 heads at 128, 1100 rows under 2885
+    // of 3984 keys would stay unsplit and take 1.21 times as long)
+    if (c.window > 0 && c.window < c.Skv && 10 * (c.window + PT_BN) < 7LL * c.Skv) tiles = std::min(tiles, ((int)c.window + 2 * PT_BN - 1) / PT_BN + 1);
     const double walk = tile * ((tiles + f.KG - 1) / f.KG);
     const long wgs = terms_workgroups(c, f.U, n), slots = (two_per_cu ? 2L : 1L) * c.cus, rest = wgs % slots;
     double us = 4.9 + wgs / slots * (ends + walk);

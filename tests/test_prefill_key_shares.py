@@ -90,6 +90,11 @@ def test_a_windowed_chunk_is_not_shared_out_as_a_whole_one(H, Hkv, rows, keys, D
     assert shares(3, H, Hkv, rows, keys, D, fa.F32, window=window) == want
 
 
+def test_a_wide_window_is_planned_as_none():
+    assert [shares(1, 32, 8, 1100, 4357, 128, fa.F32, window=w) for w in (1000, 2885, 4357)] == [0, 2, 2]
+    assert shares(2, 32, 32, 728, 3304, 64, fa.F32, window=2549) == 2
+
+
 def test_rows_behind_a_full_window_see_alike():
     """A chunk of more rows than its window is planned as an even call from the keys on at which the first row sees a whole window."""
     assert [shares(1, 8, 4, 1200, keys, 128, fa.F32, window=600) for keys in (1200, 1798, 1799, 4000)] == [3, 3, 0, 0]
