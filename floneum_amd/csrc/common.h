@@ -67,13 +67,13 @@ struct AttnParams {
 
 // the key split of a tiled f32 prefill call (1 = none) and the scratch it needs
 // A square call whose rows see the keys up to their own position (a mask tensor is taken for one), some of them far fewer than others: not
-// where a window is behind them all, as in a chunk of more rows than the window (f32, us taken for uneven and not: 12/12 heads at 128,
+// where at least half a window is behind them all, as in a chunk of more rows than the window (f32, us taken for uneven and not: 12/12 heads at 128,
 // 1757 rows behind 4598 keys under a window of 803 115 and 74, 32/8 721 behind 6990 under 308 58 and 36, 16/8 at 128 905 behind
-// 140 under 137 36 and 21; over 125 random ones 0.90, the worst 1.11).  Above head_dim 128, where the model counts a window's keys by itself
+// 140 under 137 36 and 21, 32/8 at 80 642 behind 265 under 531 54 and 40; over 125 random ones 0.90, the worst 1.11).  Above head_dim 128, where the model counts a window's keys by itself
 // and takes the levels of uneven shares, such calls stay with the uneven ones (4/1 heads at 256, 1804 behind 4210 under 1515 123 and 164).
 inline bool prefill_f32_uneven(int64_t Sq, int64_t Skv, int64_t D, bool causal, bool qk_mask, int64_t first_row_at, int64_t window) {
     if (2 * Sq <= Skv) return false;
-    return qk_mask || (causal && !(D <= 128 && window > 0 && first_row_at >= window - 1));
+    return qk_mask || (causal && !(D <= 128 && window > 0 && 2 * (first_row_at + 1) >= window));
 }
 // uneven: see prefill_f32_uneven; window: rows see the last so many keys up to their position (0: all)
 void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, bool causal_square, bool uneven, int64_t window, int compute_units,
