@@ -352,7 +352,7 @@ static void mfma_split_plan(const fhip_attn_args *a, int cus, int *nsplit, int *
     if (!prefill_mfma_rows256_takes((int)a->q.shape[3], a->scale, (int)a->q.shape[0], (int)a->q.shape[1], (int)a->q.shape[2],
                                     cus > 0 ? cus : 256))  // the wide-head form: 128-row query blocks
         prefill_mfma_wide_plan((int)a->q.shape[0], (int)a->q.shape[1], Hkv ? (int)a->q.shape[1] / Hkv : 1, (int)a->q.shape[2],
-                               len, causal_square, cus > 0 ? cus : 256, nsplit, chunk);
+                               len, (int)a->q.shape[3], causal_square, uneven, cus > 0 ? cus : 256, nsplit, chunk);
     else
         prefill_mfma_plan((int)a->q.shape[0], (int)a->q.shape[1], Hkv ? (int)a->q.shape[1] / Hkv : 1, (int)a->q.shape[2], len,
                           (int)a->q.shape[3], causal_square, uneven, later_rows_see, a->analytic.enabled ? a->analytic.window : 0, cus > 0 ? cus : 256,

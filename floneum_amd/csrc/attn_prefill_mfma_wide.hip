@@ -17,6 +17,7 @@
 //
 // Reference semantics: fusor-ml/fusor/src/composite/flash_attention.rs:141-199 with the f32 accumulation of 16-bit
 // inputs of fusor-ml/core/src/composite/flash_attention.rs:186-203,323-327.
+#include <cmath>
 #include <type_traits>
 
 #include "attn_bounds.h"
@@ -474,9 +475,35 @@ int launch_wide_t(const AttnParams &p_in, hipStream_t stream) {
 
 }  // namespace
 
+// Time in us of a call above head_dim 128 whose rows all see about the same keys, by the form it takes in ns shares: rounds of
+// workgroups that walk their tiles, and parking and merging the shares.  Over 2200 timings of 330 calls (turns, chunks and images at
+// 136 to 256 dims in up to 48 shares) it is 15 % off in the mean square.
+static double prefill_wide_time(int B, int H, int G, int Sq, int Skv, int D, int compute_units, int ns) {
+    const int c = ((Skv + ns - 1) / ns + PW_KEYS - 1) / PW_KEYS * PW_KEYS, n = (Skv + c - 1) / c, tiles = c / PW_KEYS;
+    const int heads = prefill_mfma_pack(B, H, G, Sq, Skv, compute_units) ? H / 4 : H;
+    const long wgs128 = (long)B * heads * ((Sq + PW_BM - 1) / PW_BM);
+    double us = 5.0, walk;
+    if (D > 192 && heads == H && (n == 1 || Sq > 64)) {  // attn_prefill_mfma_rows32.hip
+        walk = 6.5 + 0.70 * tiles;
+        us += (wgs128 * n + compute_units - 1) / compute_units * walk;
+    } else if (heads != H || (n == 1 ? wgs128 >= 2 * compute_units : Sq > 64)) {  // 128-row workgroups
+        walk = 1.5 + 1.32 * D / 192 * tiles;
+        us += (wgs128 * n + compute_units - 1) / compute_units * walk;
+    } else {  // 64-row workgroups, two on a CU
+        const long wgs = (long)B * H * ((Sq + 63) / 64) * n, rest = wgs % (2 * compute_units);
+        const double alone = rest <= compute_units ? 0.8 : 1.0, tile = 1.15 * sqrt(D / 192.0);
+        us += wgs / (2 * compute_units) * (1.0 + tile * tiles);
+        if (rest) us += 1.0 + tile * tiles * alone;
+    }
+    if (n > 1) us += 2.0 + 0.42e-6 * prefill_mfma_workspace_bytes(B, H, Sq, D, n);
+    return us;
+}
+
 // Few query rows on a long cache: 128-row query blocks alone leave most CUs idle, so the keys are split over workgroups
 // too, down to 1024 keys per share, until there are about two workgroups per CU (the rule of the other tiled kernels).
-void prefill_mfma_wide_plan(int B, int H, int G, int Sq, int Skv, bool causal_square, int compute_units, int *nsplit, int *chunk) {
+// qk_square: a square call with a mask tensor, which is taken for a causal one.
+void prefill_mfma_wide_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_square, bool qk_square, int compute_units, int *nsplit,
+                            int *chunk) {
     *nsplit = 1;
     *chunk = Skv;
     if (causal_square) return;
@@ -485,17 +512,32 @@ void prefill_mfma_wide_plan(int B, int H, int G, int Sq, int Skv, bool causal_sq
     // places for workgroups: one per CU, two for the 64-row form that serves up to 64 rows.  A tile takes this kernel
     // microseconds whatever part of the row block is real, so a grid that leaves places empty splits its keys.
     const long places = (!pack && Sq <= 64 ? 2L : 1L) * compute_units;
-    if (wgs >= places) return;
+    if (wgs == 0 || wgs >= places) return;
     // The share count that needs the fewest tile steps: rounds of `places` workgroups, each walking its share of the
     // keys tile by tile, plus a few steps for parking and merging the partial results of a split.
-    // Shares of at least 1024 keys, or up to four of 512.
-    const long most = Skv / 1024 > 64 ? 64 : Skv / 1024 > 4 ? Skv / 1024 : Skv / 512 < 4 ? Skv / 512 : 4;
+    // Shares of at least 1024 keys; to 128 dims also up to four of 512 (186 random calls below 64 dims 0.91 of the time, the worst 1.02).
+    long most = Skv / 1024 < 64 ? Skv / 1024 : 64;
+    if (D <= 128 && most < 4) most = Skv / 512 < 4 ? Skv / 512 : 4;
     long best_ns = 1, best_cost = (Skv + PW_KEYS - 1) / PW_KEYS;
     for (long ns = 2; ns <= most; ns++) {
         const long rounds = (wgs * ns + places - 1) / places;
         const long tiles = ((Skv + ns - 1) / ns + PW_KEYS - 1) / PW_KEYS;
         const long cost = rounds * tiles + 4;
         if (cost < best_cost) best_cost = cost, best_ns = ns;
+    }
+    // Above 128 dims up to four of 512 keys where the time says that these take 5 % less: by tile steps alone, without the bytes of the
+    // partials, calls of many rows lose (us, by steps and now: 12/12 heads at 256, three sequences of 413 rows on 1858 keys 69 -> 54, two
+    // of 893 under a window on 2622 82 -> 61; 6/3 at 192, three of 1209 on 2620 115 -> 95).
+    if (D > 128 && !qk_square) {
+        double times[5] = {}, least = 0.0;
+        const int few = Skv / 512 < 4 ? Skv / 512 : 4;
+        for (int n = 1; n <= few; n++) {
+            times[n] = prefill_wide_time(B, H, G, Sq, Skv, D, compute_units, n);
+            if (n == 1 || times[n] < least) least = times[n];
+        }
+        int n = 1;
+        while (n < few && times[n] > 1.01 * least) n++;
+        if (few > 1 && times[n] < 0.95 * prefill_wide_time(B, H, G, Sq, Skv, D, compute_units, (int)best_ns)) best_ns = n;
     }
     if (best_ns < 2) return;
     long c = (Skv + best_ns - 1) / best_ns;

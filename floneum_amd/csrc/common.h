@@ -152,7 +152,8 @@ bool prefill_mfma_rows256_takes(int D, float scale, int B, int H, int Sq, int co
 int launch_prefill_mfma(const AttnParams &p, fhip_dtype dtype, hipStream_t stream);
 // the same for every multiple of 8 up to 256 (four wavefronts per workgroup, 128 query rows, 32-key tiles)
 int launch_prefill_mfma_wide(const AttnParams &p, fhip_dtype dtype, hipStream_t stream);
-void prefill_mfma_wide_plan(int B, int H, int G, int Sq, int Skv, bool causal_square, int compute_units, int *nsplit, int *chunk);
+void prefill_mfma_wide_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_square, bool qk_square, int compute_units, int *nsplit,
+                            int *chunk);
 // head dims above 192 on 128-row workgroups of four wavefronts with 32 rows each (one per SIMD, software-pipelined)
 bool prefill_mfma_rows32_takes(const AttnParams &p);
 int launch_prefill_mfma_rows32(const AttnParams &p, fhip_dtype dtype, hipStream_t stream);

@@ -38,6 +38,8 @@ def shares(B, H, Hkv, Sq, Skv, D, dtype, causal=True, window=0):
     ((1, 16, 4, 2048, 2048, 256, fa.F32), 0), ((1, 16, 4, 1024, 1024, 256, fa.F32, False), 2), ((1, 16, 4, 64, 4096, 256, fa.F32), 16),
     # above 128 dims: up to four shares of 512 keys
     ((1, 16, 4, 141, 2659, 256, fa.BF16), 4), ((1, 16, 4, 141, 1000, 256, fa.BF16), 0),
+    # but not of many rows, whose partials' bytes cost more than the rounds of tiles gain
+    ((3, 12, 12, 413, 1858, 256, fa.BF16), 0), ((2, 12, 12, 893, 2927, 256, fa.BF16, True, 1734), 0), ((3, 6, 3, 1209, 2620, 192, fa.F16), 0),
 ])
 def test_shares(call, want):
     assert shares(*call) == want
