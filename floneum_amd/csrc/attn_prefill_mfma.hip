@@ -694,7 +694,10 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(AttnPara
 // heads 46 and 39, on 4096 keys 91 and 88, 5120 113.2 and 112.9, 6144 136 and 138; 16/8 heads, 3000 rows on 3000 keys 61 and 48, 6000 125
 // and 121, 7500 158.2 and 157.4, 9000 190 and 193.  So rows that all see the same keys keep the 256-row form, and where they see
 // the keys up to their own position the line is 2.5 keys per row.  Under a window narrower than that it stays at 2, beyond which
-// the 256-row form wins by more (2048 rows on 4096 keys under a window of 2048: 68 and 78).  Sequences of different lengths in
+// the 256-row form wins by more (2048 rows on 4096 keys under a window of 2048: 68 and 78).  Rows with half a window or more behind the
+// first of them see about the same keys as well, however few the call as a whole sees (12/12 heads at 128, 3132 rows under 2512 68 and 85,
+// at 80, two sequences of 1939 under 208 22 and 26), but where the key-split form has one workgroup per CU, or little more and the first rows see less
+// than a window (12/12 at 128, 2668 behind 226 under 452 29 and 20; 8/4 at 64, 4130 behind 1313 under 2626 50 and 41).  Sequences of different lengths in
 // a batch are even grids in this sense (2 to 8 of them, 500 to 2048 keys long: 0.80 to 0.85 of the key-split form's time).
 // later_rows_see: the keys up to the last row's own where rows see the keys up to their own position, 0 where all see the same.
 int prefill_mfma_block_rows(int B, int H, int Sq, int Skv, int key_shares, int64_t later_rows_see, int64_t window, int compute_units) {
@@ -705,6 +708,12 @@ int prefill_mfma_block_rows(int B, int H, int Sq, int Skv, int key_shares, int64
     if (wgs > compute_units || nqb < 8 || later_rows_see <= 0) return PF_BM;
     const int64_t keys = later_rows_see < Skv ? later_rows_see : Skv;
     const bool narrow = window > 0 && window < keys;
+    const long of_half = (long)((Sq + PF_BM / 2 - 1) / (PF_BM / 2)) * B * H;
+    const int64_t before = later_rows_see - Sq + 1;  // keys that the first row sees without the window
+    // (before < window + 128: the keys begin where the first row's window does; they do not where the call brings lengths)
+    if (narrow && window <= Sq && before < window + 128 &&
+        (before >= window ? of_half > compute_units : 2 * before >= window && 4 * of_half > 5L * compute_units))
+        return PF_BM;
     return 2L * Sq > Skv || (!narrow && 5L * Sq >= 2 * keys) ? PF_BM / 2 : PF_BM;
 }
 

@@ -22,6 +22,20 @@ def block_rows(B, H, Sq, Skv, later_rows_see=0, window=0, compute_units=CUS):
     return rule(B, H, Sq, Skv, 1, ctypes.c_int64(later_rows_see), ctypes.c_int64(window), compute_units)
 
 
+@pytest.mark.parametrize("B, H, Sq, before, window, rows", [
+    # rows with a whole window behind the first of them, whose keys begin with that window: 256 rows a block, but for a 128-row grid of
+    # one workgroup per CU
+    (1, 16, 2364, 1398, 1399, 256), (1, 12, 3132, 2620, 2512, 256), (2, 12, 1939, 300, 208, 256), (1, 12, 2668, 451, 452, 128),
+    # half a window: 256 from one and a quarter workgroups per CU on; less than half: as a prompt
+    (1, 24, 2048, 511, 1024, 256), (1, 24, 2048, 510, 1024, 128), (1, 20, 2048, 511, 1024, 128), (1, 24, 2048, 0, 1024, 128),
+    (1, 24, 2048, 2047, 2049, 128),  # of a window longer than the rows the line of the keys per row decides
+])
+def test_which_form_under_a_window(B, H, Sq, before, window, rows):
+    first = max(0, before - window + 1) // 128 * 128
+    later = before - first + Sq
+    assert block_rows(B, H, Sq, later, later, window) == rows
+
+
 @pytest.mark.parametrize("B, H, Sq, Skv, later_rows_see, window, rows", [
     (1, 16, 4096, 4096, 0, 0, 256), (1, 32, 2048, 8192, 0, 0, 256), (1, 32, 2048, 2048, 2048, 0, 128),  # even rows; a prompt
     (1, 32, 2048, 4096, 4096, 0, 128), (1, 32, 2048, 5120, 5120, 0, 128), (1, 32, 2048, 5121, 5121, 0, 256),  # the line
