@@ -807,7 +807,7 @@ void prefill_mfma_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_
     if (causal_square) return;
     const long wgs = (long)B * (prefill_mfma_pack(B, H, G, Sq, Skv, compute_units) ? H / 4 : H) * ((Sq + PF_BM - 1) / PF_BM);
     if (wgs == 0) return;
-    // While the query blocks alone keep at least half the chip busy, parking and merging partial results costs more than it gains.
+    // By rule a grid of query blocks that keeps half the chip busy by itself is not split (the times below may find otherwise).
     const long want = (2L * compute_units + wgs - 1) / wgs;
     long most = Skv / 1024;
     // A few rows on a short cache: shares down to 512 keys, and for up to 64 rows to 256, while CUs would stay without a
@@ -827,7 +827,9 @@ void prefill_mfma_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_
     int tried = 0;
     for (const int n : SHARES) {
         if (uneven) break;
-        if (n > 1 && (Skv / n < 128 || (n - 1) * wgs > 3L * compute_units)) break;  // (three rounds gain nothing more)
+        // (three rounds gain nothing more; partials of at most 64 MiB)
+        if (n > 1 && (Skv / n < 128 || (n - 1) * wgs > 3L * compute_units || prefill_mfma_workspace_bytes(B, H, Sq, D, n) > ((size_t)64 << 20)))
+            break;
         times[tried] = prefill_mfma_time(B, H, G, Sq, Skv, D, later_rows_see, window, compute_units, n);
         if (tried == 0 || times[tried] < least) least = times[tried];
         tried++;

@@ -45,6 +45,14 @@ def test_shares(call, want):
     assert shares(*call) == want
 
 
+@pytest.mark.parametrize("call, want", [((8, 16, 4, 1278, 21043, 128), 0), ((4, 16, 16, 2363, 21840, 128), 0), ((2, 16, 16, 2826, 9136, 128), 0),
+                                        ((2, 16, 16, 2320, 14643, 80), 2), ((8, 12, 12, 458, 30160, 96), 0)])
+def test_the_partials_of_a_call_are_limited(call, want):
+    """16-bit calls: 64 MiB where the time asks for more shares than the rules (the first of these asked for 165, the next for 152)."""
+    B, H, _, rows, _, D = call
+    assert shares(*call, fa.BF16) == want and want * B * H * rows * (D + 4) * 4 <= 64 << 20
+
+
 @pytest.mark.parametrize("D, dtype", [(64, fa.F32), (96, fa.F32), (256, fa.F32), (64, fa.F16), (128, fa.BF16), (256, fa.F16)])
 @pytest.mark.parametrize("before", [0, 1, 127, 128, 4000, 20000])
 def test_a_window_is_planned_on_its_keys(D, dtype, before):
