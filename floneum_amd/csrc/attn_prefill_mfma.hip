@@ -819,9 +819,10 @@ void prefill_mfma_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_
     long ns = 2 * wgs > compute_units ? 1 : want < most ? want : most;
     if (ns < 1) ns = 1;
     // These rules count workgroups and not their rounds, nor the bytes of the partials: the shares of least time by the function
-    // above, the fewest within 1 % of it, are taken where that is 5 % less than the rules' (us a call: four sequences of 207 rows of
-    // 32/8 heads at 96 under a window of 4096 84 -> 56 in none; 189 rows of 8/4 heads at 80 on 1993 keys 23.5 -> 19, 231 of 32/8 at 64 on 14900
-    // 59 -> 48, 49 of 32/32 at 128 on 3032 36 -> 22; over 140 random calls 0.93 of the rules' time, the worst 1.06).
+    // above, the fewest within 1 % of it, are taken where that is 5 % less than the rules', or 10 % for grids that the rules do not split
+    // (us a call: four sequences of 207 rows of 32/8 heads at 96 under a window of 4096 84 -> 56 in none; 189 rows of 8/4 heads at 80 on 1993 keys 23.5 -> 19, 231 of 32/8 at 64 on 14900
+    // 59 -> 48, 49 of 32/32 at 128 on 3032 36 -> 22; over 500 random calls without lengths or a mask tensor 0.93 of the rules' time, the
+    // worst 1.11; at 5 % everywhere large ones lost up to 14 %: 32/32 heads at 80, 2859 rows on 7370 keys 209 and 238).
     constexpr int SHARES[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48};
     double times[sizeof(SHARES) / sizeof(SHARES[0])], least = 0.0;
     int tried = 0;
@@ -836,7 +837,8 @@ void prefill_mfma_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_
     }
     for (int i = 0; i < tried; i++) {
         if (times[i] > 1.01 * least) continue;
-        if (times[i] < 0.95 * prefill_mfma_time(B, H, G, Sq, Skv, D, later_rows_see, window, compute_units, (int)ns)) ns = SHARES[i];
+        const double gain = 2 * wgs > compute_units ? 0.9 : 0.95;
+        if (times[i] < gain * prefill_mfma_time(B, H, G, Sq, Skv, D, later_rows_see, window, compute_units, (int)ns)) ns = SHARES[i];
         break;
     }
     if (ns < 2) return;

@@ -53,6 +53,12 @@ def test_the_partials_of_a_call_are_limited(call, want):
     assert shares(*call, fa.BF16) == want and want * B * H * rows * (D + 4) * 4 <= 64 << 20
 
 
+@pytest.mark.parametrize("call", [(1, 32, 32, 2859, 7370, 80), (8, 16, 16, 689, 6007, 80), (8, 4, 1, 2154, 6748, 96)])
+def test_full_grids_are_split_for_a_tenth_of_their_time(call):
+    """16-bit grids of more than half the chip, which two shares slow down (us 209 -> 238, 210 -> 245, 190 -> 211)."""
+    assert shares(*call, fa.F16) == 0
+
+
 @pytest.mark.parametrize("D, dtype", [(64, fa.F32), (96, fa.F32), (256, fa.F32), (64, fa.F16), (128, fa.BF16), (256, fa.F16)])
 @pytest.mark.parametrize("before", [0, 1, 127, 128, 4000, 20000])
 def test_a_window_is_planned_on_its_keys(D, dtype, before):
