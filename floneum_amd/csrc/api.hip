@@ -322,6 +322,10 @@ static void visible_range(const fhip_attn_args *a, int *lo0, int *len) {
     *len = (int)(hi - *lo0);
 }
 
+// Calls whose rows may see far fewer keys than the host knows of: of sequences with lengths of their own, or with a mask tensor over
+// (query, key).  (A key mask over the batch is counted as padding, which most rows do not have.)
+static bool unknown_lengths(const fhip_attn_args *a) { return a->kv_lens || a->mask_kind == FHIP_MASK_QK; }
+
 // Key split of a call the f32-arithmetic tiled kernel serves (few query rows on a long cache), and where its
 // partial results go in the workspace: behind the mask scratch, 256-byte aligned.
 static void f32_split_plan(const fhip_attn_args *a, int cus, int *nsplit, int *chunk) {
@@ -333,7 +337,7 @@ static void f32_split_plan(const fhip_attn_args *a, int cus, int *nsplit, int *c
     const int Hkv = (int)a->k.shape[1];
     prefill_f32_plan((int)a->q.shape[0], (int)a->q.shape[1], Hkv ? (int)a->q.shape[1] / Hkv : 1, (int)a->q.shape[2],
                      len, (int)a->q.shape[3], a->dtype == FHIP_F32, causal_square, uneven, a->analytic.enabled ? a->analytic.window : 0,
-                     cus > 0 ? cus : 256, nsplit, chunk);
+                     unknown_lengths(a), cus > 0 ? cus : 256, nsplit, chunk);
 }
 static size_t f32_partials_offset(const fhip_attn_args *a) { return (mask_scratch_bytes(a) + 255) & ~(size_t)255; }
 static void mfma_split_plan(const fhip_attn_args *a, int cus, int *nsplit, int *chunk) {
@@ -352,11 +356,11 @@ static void mfma_split_plan(const fhip_attn_args *a, int cus, int *nsplit, int *
     if (!prefill_mfma_rows256_takes((int)a->q.shape[3], a->scale, (int)a->q.shape[0], (int)a->q.shape[1], (int)a->q.shape[2],
                                     cus > 0 ? cus : 256))  // the wide-head form: 128-row query blocks
         prefill_mfma_wide_plan((int)a->q.shape[0], (int)a->q.shape[1], Hkv ? (int)a->q.shape[1] / Hkv : 1, (int)a->q.shape[2],
-                               len, (int)a->q.shape[3], causal_square, uneven, cus > 0 ? cus : 256, nsplit, chunk);
+                               len, (int)a->q.shape[3], causal_square, uneven, unknown_lengths(a), cus > 0 ? cus : 256, nsplit, chunk);
     else
         prefill_mfma_plan((int)a->q.shape[0], (int)a->q.shape[1], Hkv ? (int)a->q.shape[1] / Hkv : 1, (int)a->q.shape[2], len,
-                          (int)a->q.shape[3], causal_square, uneven, later_rows_see, a->analytic.enabled ? a->analytic.window : 0, cus > 0 ? cus : 256,
-                          nsplit, chunk);
+                          (int)a->q.shape[3], causal_square, uneven, later_rows_see, a->analytic.enabled ? a->analytic.window : 0, unknown_lengths(a),
+                          cus > 0 ? cus : 256, nsplit, chunk);
 }
 
 // A workspace too small for the planned key split still takes the largest split that fits (shares stay multiples of 64

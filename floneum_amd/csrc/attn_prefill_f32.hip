@@ -680,9 +680,9 @@ static int launch_rows(const AttnParams &p, hipStream_t stream) {
     return FHIP_OK;
 }
 
-// Shares of the keys: the fewest within 2 % of the least time, where that is 5 % less than the time of `ordinary` ones; each in the form
+// Shares of the keys: the fewest within 2 % of the least time, where that is less than `gain` of the time of `ordinary` ones; each in the form
 // that it would run in.
-static long shares_of_least_time(const TermsCall &c, long ordinary) {
+static long shares_of_least_time(const TermsCall &c, long ordinary, double gain) {
     constexpr int SHARES[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48};
     const long units = (long)c.G * ((c.Sq + 31) / 32);
     double times[sizeof(SHARES) / sizeof(SHARES[0])], least = 0.0;
@@ -698,7 +698,7 @@ static long shares_of_least_time(const TermsCall &c, long ordinary) {
     }
     for (int i = 0; i < tried; i++) {
         if (times[i] > 1.02 * least) continue;
-        return times[i] < 0.95 * prefill_f32_terms_time(c, prefill_f32_terms_form(c, (int)ordinary), (int)ordinary) ? SHARES[i] : ordinary;
+        return times[i] < gain * prefill_f32_terms_time(c, prefill_f32_terms_form(c, (int)ordinary), (int)ordinary) ? SHARES[i] : ordinary;
     }
     return ordinary;
 }
@@ -717,8 +717,8 @@ static double wide_f32_time(const TermsCall &c) {
 
 // Few query rows on a long cache (a new chat turn, a prompt fed in pieces): the grid of query blocks alone leaves
 // most CUs idle, so the keys are split over workgroups as well.
-void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, bool causal_square, bool uneven, int64_t window, int compute_units,
-                      int *nsplit, int *chunk) {
+void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, bool causal_square, bool uneven, int64_t window,
+                      bool unknown_lengths, int compute_units, int *nsplit, int *chunk) {
     *nsplit = 1;
     *chunk = Skv;
     if (D <= 128) {
@@ -756,10 +756,10 @@ void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, boo
         constexpr size_t MOST_PARTIALS = (size_t)16 << 20;
         if (few_rows && D > 64 && prefill_f32_workspace_bytes(B, H, Sq, D, (int)ns) > MOST_PARTIALS) ns = shares(2);
         // More than 128 rows that see about the same keys (chunks, images): the shares of least time, where that is 5 % less than the
-        // rule's; at most 64 MiB of partials (us a call: two sequences of 275 rows of 32/8
+        // rule's (shares_gain); at most 64 MiB of partials (us a call: two sequences of 275 rows of 32/8
         // heads at 64 on 2911 keys 116 -> 92; 16 heads without a mask, 1156 rows at 128 148 -> 80, 2506 366 -> 285, 1147 at 80 109 -> 59; over 90
         // random calls the time is 0.91, the worst 1.03 of the rule's).  Square prompts to 768 keys keep the rule, masked or not.
-        if (!uneven && Sq > 128 && (few_rows || Skv > 768)) ns = shares_of_least_time({B, H / G, G, Sq, Skv, D, compute_units, false, window, f32}, ns < 2 ? 1 : ns);
+        if (!uneven && Sq > 128 && (few_rows || Skv > 768)) ns = shares_of_least_time({B, H / G, G, Sq, Skv, D, compute_units, false, window, f32}, ns < 2 ? 1 : ns, shares_gain(unknown_lengths));
         if (ns < 2) return;
         const long c = ((Skv + ns - 1) / ns + 31) / 32 * 32;
         *chunk = (int)c;
@@ -771,7 +771,7 @@ void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, boo
         // the shares taken: 148 rows on 3510 keys 584 -> 80, 300 on 700 128 -> 49, 1000 on 1000 182 -> 93, 2000 on 2000 347 -> 235; 2048 on 2048 stays at 355, its two shares
         // would be more than 64 MiB of partials).
         const TermsCall call = {B, H / G, G, Sq, Skv, D, compute_units, uneven, window, true};
-        const long ns = shares_of_least_time(call, 1);
+        const long ns = shares_of_least_time(call, 1, shares_gain(false));
         if (ns < 2 || wide_f32_time(call) < prefill_f32_terms_time(call, {4, 1}, (int)ns)) return;
         const long c = ((Skv + ns - 1) / ns + 31) / 32 * 32;
         *chunk = (int)c;

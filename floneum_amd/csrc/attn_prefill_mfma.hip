@@ -40,6 +40,7 @@
 // Reference semantics: fusor-ml/fusor/src/composite/flash_attention.rs:141-199, f32 accumulation
 // of 16-bit inputs as fusor-ml/core/src/composite/flash_attention.rs:186-203,323-327; head
 // mapping kv_head = head / (H / Hkv) (core :135-137,163-167).
+#include <algorithm>
 #include <type_traits>
 
 #include "attn_bounds.h"
@@ -801,7 +802,7 @@ static double prefill_mfma_time(int B, int H, int G, int Sq, int Skv, int D, int
 // uneven: a square call whose rows see the keys up to their own position (a mask tensor is taken for one): by the rules alone.
 // later_rows_see, window: as for prefill_mfma_block_rows.
 void prefill_mfma_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_square, bool uneven, int64_t later_rows_see, int64_t window,
-                       int compute_units, int *nsplit, int *chunk) {
+                       bool unknown_lengths, int compute_units, int *nsplit, int *chunk) {
     *nsplit = 1;
     *chunk = Skv;
     if (causal_square) return;
@@ -819,7 +820,7 @@ void prefill_mfma_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_
     long ns = 2 * wgs > compute_units ? 1 : want < most ? want : most;
     if (ns < 1) ns = 1;
     // These rules count workgroups and not their rounds, nor the bytes of the partials: the shares of least time by the function
-    // above, the fewest within 1 % of it, are taken where that is 5 % less than the rules', or 10 % for grids that the rules do not split
+    // above, the fewest within 1 % of it, are taken where that is 5 % less than the rules' (shares_gain), or 10 % for grids that the rules do not split
     // (us a call: four sequences of 207 rows of 32/8 heads at 96 under a window of 4096 84 -> 56 in none; 189 rows of 8/4 heads at 80 on 1993 keys 23.5 -> 19, 231 of 32/8 at 64 on 14900
     // 59 -> 48, 49 of 32/32 at 128 on 3032 36 -> 22; over 500 random calls without lengths or a mask tensor 0.93 of the rules' time, the
     // worst 1.11; at 5 % everywhere large ones lost up to 14 %: 32/32 heads at 80, 2859 rows on 7370 keys 209 and 238).
@@ -837,7 +838,7 @@ void prefill_mfma_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_
     }
     for (int i = 0; i < tried; i++) {
         if (times[i] > 1.01 * least) continue;
-        const double gain = 2 * wgs > compute_units ? 0.9 : 0.95;
+        const double gain = std::min(shares_gain(unknown_lengths), 2 * wgs > compute_units ? 0.9 : 1.0);
         if (times[i] < gain * prefill_mfma_time(B, H, G, Sq, Skv, D, later_rows_see, window, compute_units, (int)ns)) ns = SHARES[i];
         break;
     }

@@ -502,8 +502,8 @@ static double prefill_wide_time(int B, int H, int G, int Sq, int Skv, int D, int
 // Few query rows on a long cache: 128-row query blocks alone leave most CUs idle, so the keys are split over workgroups
 // too, down to 1024 keys per share, until there are about two workgroups per CU (the rule of the other tiled kernels).
 // qk_square: a square call with a mask tensor, which is taken for a causal one.
-void prefill_mfma_wide_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_square, bool qk_square, int compute_units, int *nsplit,
-                            int *chunk) {
+void prefill_mfma_wide_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_square, bool qk_square, bool unknown_lengths,
+                            int compute_units, int *nsplit, int *chunk) {
     *nsplit = 1;
     *chunk = Skv;
     if (causal_square) return;
@@ -525,7 +525,7 @@ void prefill_mfma_wide_plan(int B, int H, int G, int Sq, int Skv, int D, bool ca
         const long cost = rounds * tiles + 4;
         if (cost < best_cost) best_cost = cost, best_ns = ns;
     }
-    // Above 128 dims up to four of 512 keys where the time says that these take 5 % less: by tile steps alone, without the bytes of the
+    // Above 128 dims up to four of 512 keys where the time says that these take 5 % less (shares_gain): by tile steps alone, without the bytes of the
     // partials, calls of many rows lose (us, by steps and now: 12/12 heads at 256, three sequences of 413 rows on 1858 keys 69 -> 54, two
     // of 893 under a window on 2622 82 -> 61; 6/3 at 192, three of 1209 on 2620 115 -> 95).
     if (D > 128 && !qk_square) {
@@ -537,7 +537,7 @@ void prefill_mfma_wide_plan(int B, int H, int G, int Sq, int Skv, int D, bool ca
         }
         int n = 1;
         while (n < few && times[n] > 1.01 * least) n++;
-        if (few > 1 && times[n] < 0.95 * prefill_wide_time(B, H, G, Sq, Skv, D, compute_units, (int)best_ns)) best_ns = n;
+        if (few > 1 && times[n] < shares_gain(unknown_lengths) * prefill_wide_time(B, H, G, Sq, Skv, D, compute_units, (int)best_ns)) best_ns = n;
     }
     if (best_ns < 2) return;
     long c = (Skv + best_ns - 1) / best_ns;

@@ -76,8 +76,12 @@ inline bool prefill_f32_uneven(int64_t Sq, int64_t Skv, int64_t D, bool causal, 
     return qk_mask || (causal && !(D <= 128 && window > 0 && 2 * (first_row_at + 1) >= window));
 }
 // uneven: see prefill_f32_uneven; window: rows see the last so many keys up to their position (0: all)
-void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, bool causal_square, bool uneven, int64_t window, int compute_units,
-                      int *nsplit, int *chunk);
+void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, bool causal_square, bool uneven, int64_t window, bool unknown_lengths,
+                      int compute_units, int *nsplit, int *chunk);
+// What part of the rules' time the shares of least time have to be, by a model: 5 % less, and 30 % where the rows may see far fewer
+// keys than it counts (us, in the rules' shares and by 5 %: f16, two sequences of 84 rows of 6/3 heads at 80 on up to 1416 keys 11.2 and 14.5;
+// bf16, two of 377 of 32/8 at 256 on up to 2369 50 and 97; f32, 32/8 at 128, 360 rows that see 300 of 1844 keys by a mask tensor 56 and 65).
+inline double shares_gain(bool unknown_lengths) { return unknown_lengths ? 0.7 : 0.95; }
 // The forms of the f32 terms kernel (attn_prefill_f32_terms.hip): units and key groups per workgroup, and what a call takes in them
 struct TermsCall {
     int B, Hkv, G, Sq, Skv, D, cus;
@@ -95,7 +99,7 @@ TermsForm prefill_f32_terms_form(const TermsCall &call, int key_shares);        
 size_t prefill_f32_workspace_bytes(int B, int H, int Sq, int D, int nsplit);
 // the same for the 16-bit matrix-core prefill kernel (256-row query blocks, one workgroup per CU)
 void prefill_mfma_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_square, bool uneven, int64_t later_rows_see,
-                       int64_t window, int compute_units, int *nsplit, int *chunk);
+                       int64_t window, bool unknown_lengths, int compute_units, int *nsplit, int *chunk);
 // query heads that share one workgroup's K/V tiles (0: one head per workgroup)
 int prefill_mfma_pack(int B, int H, int G, int Sq, int Skv, int compute_units);
 size_t prefill_mfma_workspace_bytes(int B, int H, int Sq, int D, int nsplit);
@@ -152,8 +156,8 @@ bool prefill_mfma_rows256_takes(int D, float scale, int B, int H, int Sq, int co
 int launch_prefill_mfma(const AttnParams &p, fhip_dtype dtype, hipStream_t stream);
 // the same for every multiple of 8 up to 256 (four wavefronts per workgroup, 128 query rows, 32-key tiles)
 int launch_prefill_mfma_wide(const AttnParams &p, fhip_dtype dtype, hipStream_t stream);
-void prefill_mfma_wide_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_square, bool qk_square, int compute_units, int *nsplit,
-                            int *chunk);
+void prefill_mfma_wide_plan(int B, int H, int G, int Sq, int Skv, int D, bool causal_square, bool qk_square, bool unknown_lengths,
+                            int compute_units, int *nsplit, int *chunk);
 // head dims above 192 on 128-row workgroups of four wavefronts with 32 rows each (one per SIMD, software-pipelined)
 bool prefill_mfma_rows32_takes(const AttnParams &p);
 int launch_prefill_mfma_rows32(const AttnParams &p, fhip_dtype dtype, hipStream_t stream);

@@ -53,6 +53,29 @@ def test_the_partials_of_a_call_are_limited(call, want):
     assert shares(*call, fa.BF16) == want and want * B * H * rows * (D + 4) * 4 <= 64 << 20
 
 
+@pytest.mark.parametrize("call, known, unknown", [
+    ((2, 6, 3, 84, 1416, 80, fa.F16), 8, 0), ((4, 16, 4, 75, 1187, 128, fa.F16), 3, 0), ((3, 12, 12, 271, 1201, 256, fa.F16), 2, 0),
+    ((1, 32, 8, 360, 1844, 128, fa.F32), 5, 2), ((1, 16, 4, 765, 1999, 96, fa.F32), 5, 2), ((3, 16, 4, 321, 1323, 128, fa.F32), 3, 0),
+])
+def test_rows_that_may_see_fewer_keys_than_the_call_has(call, known, unknown):
+    """Sequences with lengths of their own and masks over (query, key) take more shares than by rule only for 30 % of the time."""
+    B, H, Hkv, rows, keys, D, dtype = call
+    a, need = make_args(B=B, H=H, Hkv=Hkv, Sq=rows, Skv=keys, D=D, dtype=dtype), ctypes.c_size_t()
+    per = B * H * rows * (D + (2 if dtype == fa.F32 else 4)) * 4
+
+    def asked():
+        assert fa.lib().fhip_flash_attention_workspace_bytes(ctypes.byref(a), CUS, ctypes.byref(need)) == fa.OK
+        return need.value / per
+
+    assert shares(*call, causal=False) == known and asked() == known
+    a.kv_lens = 0x1000
+    assert asked() == unknown
+    a.kv_lens = None
+    a.mask_kind, a.mask.ptr, a.mask_intervals = fa.MaskKind.QKMask, 0x10000, 0x20000
+    a.mask.shape[:], a.mask.stride[:] = (rows, keys), (keys, 1)
+    assert asked() == unknown
+
+
 @pytest.mark.parametrize("call", [(1, 32, 32, 2859, 7370, 80), (8, 16, 16, 689, 6007, 80), (8, 4, 1, 2154, 6748, 96)])
 def test_full_grids_are_split_for_a_tenth_of_their_time(call):
     """16-bit grids of more than half the chip, which two shares slow down (us 209 -> 238, 210 -> 245, 190 -> 211)."""
