@@ -1304,7 +1304,7 @@ template <typename T, int LPR, int GROUPS, int U>
 __global__ __launch_bounds__(GROUPS > 1 ? LPR * GROUPS : 256) void decode_combine_kernel(AttnParams p, int out_vec) {
     request_arguments<AttnParams, int>();
     constexpr int ROWS = GROUPS > 1 ? 1 : 256 / LPR;  // of a workgroup
-    __shared__ float parts[GROUPS > 1 ? GROUPS : 1][GROUPS > 1 ? 4 * LPR : 1];
+    __shared__ __attribute__((aligned(16))) float parts[GROUPS > 1 ? GROUPS : 1][GROUPS > 1 ? 4 * LPR : 1];  // in pieces of 16 bytes
     __shared__ float states[GROUPS > 1 ? GROUPS : 1][2];
     const uint32_t row = GROUPS > 1 ? blockIdx.x : blockIdx.x * ROWS + threadIdx.x / LPR;
     if (GROUPS == 1 && row >= (uint32_t)(p.B * p.H * p.Sq)) return;
