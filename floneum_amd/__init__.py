@@ -178,7 +178,7 @@ SYMBOLS = {
 }
 
 _LIB = None
-_native = None  # csrc/host_python.cpp, loaded with the library
+_native = None  # csrc/host_python.cpp, loaded with the library where it is built for this interpreter
 
 
 def lib():
@@ -199,12 +199,13 @@ def lib():
 
 
 def _bind_native():
-    """Loads the calls of a decode step in native code (csrc/host_python.cpp), which is built with the library."""
+    """Loads the calls of a decode step in native code (csrc/host_python.cpp), which is built with the library for the interpreter
+    that builds it.  Under another one every call goes through ctypes."""
     global _native
     try:
         from . import _host
-    except ImportError as e:
-        raise ImportError(f"{_HERE}/_host.so: {e}: run `python -m floneum_amd.build` (or __graft_entry__.build()) first") from e
+    except ModuleNotFoundError:
+        return
     _host.bind(Tensor, _View, KvCache, RopeCache, RmsNorm, IntTensor)
     _native = _host
 
@@ -584,13 +585,13 @@ class Tensor:
         counts; `out_dtype` F32 for 16-bit inputs.  Raises InvalidArgument (an AssertionError)
         where the reference panics."""
         L = _LIB or lib()
-        if out is None and len(self.shape) == 4:
-            out = Tensor.empty(self.buffer.device, self.shape, self.dtype if out_dtype is None else out_dtype)
-        rc = _native.attention(self, k, v, scale, mask, analytic, kv_lens, out_dtype, force_kernel, out)
-        if rc is not None:
-            if rc != OK:
-                check(rc)
-            return out
+        if _native is not None:
+            done = _native.attention(self, k, v, scale, mask, analytic, kv_lens, out_dtype, force_kernel, out, Buffer)
+            if done is not None:
+                if type(done) is Tensor:
+                    return done
+                check(done)
+                return out
         args = self._attn_args(k, v, scale, mask, analytic, kv_lens, out_dtype, force_kernel, out)
         dev = self.device
         need = ctypes.c_size_t()
@@ -866,7 +867,7 @@ def _kv_step(self, rope, q, k, v, start_pos, interleaved=False, q_norm=None, k_n
     """rope(norm(q)) and append(rope(norm(k)), v) in one launch; returns (q_rotated, k_all, v_all)."""
     assert k.dtype == v.dtype
     q_out = Tensor.empty(self.device, q.shape, q_out_dtype if q_out_dtype is not None else q.dtype)
-    done = _native.append(self, rope, q, q_out, k, v, start_pos, interleaved, q_norm, k_norm)
+    done = _native.append(self, rope, q, q_out, k, v, start_pos, interleaved, q_norm, k_norm) if _native is not None else None
     if done is not None:
         if done[0] != OK:
             check(done[0])

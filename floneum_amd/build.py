@@ -1,4 +1,4 @@
-"""Builds libfusor_hip.so (and libfusor_hip.a) for gfx950 from floneum_amd/csrc with hipcc, and the Python mirror's _host.so."""
+"""Builds libfusor_hip.so (and libfusor_hip.a) for gfx950 from floneum_amd/csrc with hipcc, and the Python mirror's native half (_host)."""
 import os
 import subprocess
 import sys
@@ -11,7 +11,7 @@ SOURCES = ["api.hip", "attn_generic.hip", "attn_decode.hip", "attn_prefill_mfma.
            "attn_prefill_f32.hip", "attn_prefill_f32_terms.hip",
            "kv_cache.hip", "mask_intervals.hip", "rope.hip", "calibration.hip"]
 LIB = os.path.join(HERE, "libfusor_hip.so")
-HOST = os.path.join(HERE, "_host.so")
+HOST = os.path.join(HERE, "_host" + sysconfig.get_config_var("EXT_SUFFIX"))  # (no other interpreter takes it for its own)
 STATIC = os.path.join(HERE, "libfusor_hip.a")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fno-gpu-rdc", "-Wall", "-Wno-unused-function", "-Wno-inline-asm",
@@ -43,6 +43,9 @@ def build(verbose=True):
         os.remove(STATIC)
     subprocess.check_call(["ar", "rcs", STATIC] + objs)
     # the Python mirror's native half
+    untagged = os.path.join(HERE, "_host.so")  # (any interpreter would load it)
+    if os.path.exists(untagged):
+        os.remove(untagged)
     subprocess.check_call(["g++", "-std=c++17", "-O2", "-Wall", "-Wno-missing-field-initializers", "-fPIC", "-shared", "-fvisibility=hidden",
                            "-I", sysconfig.get_paths()["include"], os.path.join(CSRC, "host_python.cpp"), "-o", HOST, "-L", HERE,
                            "-lfusor_hip", "-Wl,-rpath,$ORIGIN"])

@@ -141,11 +141,11 @@ PyObject *cache_tensor(PyObject *cache, PyObject *device, PyObject *dtype, const
     return instance(tensor, 5, tv);
 }
 
-// The descriptor of attention(q, k, v, scale, mask, analytic, kv_lens, out_dtype, force_kernel, out), without a workspace, and the
-// device (a new reference) of a plain call.
-PyObject *attention_args(PyObject *const *a, Py_ssize_t n, fhip_attn_args *args) {
+// The descriptor of attention(q, k, v, scale, mask, analytic, kv_lens, out_dtype, force_kernel, out), without a workspace (and without a
+// result where `out` is None), and the device (a new reference) of a plain call.
+PyObject *attention_args(PyObject *const *a, fhip_attn_args *args) {
     memset(args, 0, sizeof(*args));
-    if (n != 10 || Py_TYPE(a[0]) != tensor.type || !slot(tensor, a[0], 0)) return nullptr;
+    if (Py_TYPE(a[0]) != tensor.type || !slot(tensor, a[0], 0)) return nullptr;
     const Ref memory(Py_NewRef(slot(tensor, a[0], 0)));
     Ref device(PyObject_GetAttr(memory.o, n_device));
     if (!device.o) {
@@ -154,8 +154,8 @@ PyObject *attention_args(PyObject *const *a, Py_ssize_t n, fhip_attn_args *args)
     }
     int32_t dtypes[4], mask_dtype, kind;
     if (!describe<4>(a[0], &args->q, &dtypes[0], nullptr) || !describe<4>(a[1], &args->k, &dtypes[1], device.o) ||
-        !describe<4>(a[2], &args->v, &dtypes[2], device.o) || !describe<4>(a[9], &args->out, &dtypes[3], nullptr) || dtypes[1] != dtypes[0] ||
-        dtypes[2] != dtypes[0])
+        !describe<4>(a[2], &args->v, &dtypes[2], device.o) || (a[9] != Py_None && !describe<4>(a[9], &args->out, &dtypes[3], nullptr)) ||
+        dtypes[1] != dtypes[0] || dtypes[2] != dtypes[0])
         return nullptr;
     args->dtype = (fhip_dtype)dtypes[0];
     int32_t out_dtype = dtypes[0];
@@ -204,39 +204,11 @@ PyObject *attention_args(PyObject *const *a, Py_ssize_t n, fhip_attn_args *args)
     return device.o;
 }
 
-// attention(...): the library's status, or None
-PyObject *attention(PyObject *, PyObject *const *a, Py_ssize_t n) {
-    fhip_attn_args args;
-    void *stream;
-    uint64_t cus;
-    Ref device(attention_args(a, n, &args));
-    if (!device.o || !attr_handle(device.o, n_stream, &stream) || !attr_u64(device.o, n_compute_units, &cus)) Py_RETURN_NONE;
-    size_t need = 0;
-    int rc = fhip_flash_attention_workspace_bytes(&args, (int32_t)cus, &need);
-    if (rc == FHIP_OK && need) {
-        Ref bytes(PyLong_FromSize_t(need));
-        if (!bytes.o) return nullptr;
-        Ref ws(PyObject_CallMethodOneArg(device.o, n_workspace, bytes.o));
-        if (!ws.o) return nullptr;  // what the caller's own call of it would raise
-        uint64_t ptr, size;
-        if (!PyTuple_CheckExact(ws.o) || PyTuple_GET_SIZE(ws.o) != 2 || !as_u64(PyTuple_GET_ITEM(ws.o, 0), &ptr) ||
-            !as_u64(PyTuple_GET_ITEM(ws.o, 1), &size))
-            Py_RETURN_NONE;
-        args.workspace = (void *)(uintptr_t)ptr;
-        args.workspace_bytes = size;
-    }
-    if (rc == FHIP_OK) {
-        Py_BEGIN_ALLOW_THREADS
-        rc = fhip_flash_attention((fhip_stream *)stream, &args);
-        Py_END_ALLOW_THREADS
-    }
-    return PyLong_FromLong(rc);
-}
-
 // attention_descriptor(...): the bytes of what `attention` hands to the library, or None (for tests; nothing is called)
 PyObject *attention_descriptor(PyObject *, PyObject *const *a, Py_ssize_t n) {
     fhip_attn_args args;
-    Ref device(attention_args(a, n, &args));
+    if (n != 10 || a[9] == Py_None) Py_RETURN_NONE;
+    Ref device(attention_args(a, &args));
     if (!device.o) Py_RETURN_NONE;
     return PyBytes_FromStringAndSize((const char *)&args, sizeof(args));
 }
@@ -330,6 +302,53 @@ PyObject *contiguous(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (!buffer.o) return nullptr;
     PyObject *const values[5] = {buffer.o, a[3], a[4], strides.o, zero.o};
     return instance(tensor, 5, values);
+}
+
+// a Tensor of q's shape for a result of that type (a new reference, None where it is left to the general way, null with an exception)
+PyObject *result(PyObject *buffer_type, PyObject *device, PyObject *q, fhip_dtype dtype) {
+    if (dtype != FHIP_F32 && dtype != FHIP_F16 && dtype != FHIP_BF16) Py_RETURN_NONE;
+    Ref element(PyLong_FromLong(dtype == FHIP_F32 ? 4 : 2)), type(PyLong_FromLong(dtype)), shape(Py_NewRef(slot(tensor, q, 2)));
+    if (!element.o || !type.o) return nullptr;
+    PyObject *const of[5] = {buffer_type, device, element.o, type.o, shape.o};
+    return contiguous(nullptr, of, 5);
+}
+
+// attention(q, k, v, scale, mask, analytic, kv_lens, out_dtype, force_kernel, out, Buffer): the library's status, or None.  Where `out` is
+// None, the result (on memory of its own, once the arguments have been looked at) instead of the status 0.
+PyObject *attention(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    if (n != 11) Py_RETURN_NONE;
+    fhip_attn_args args;
+    void *stream;
+    uint64_t cus;
+    Ref device(attention_args(a, &args));
+    if (!device.o || !attr_handle(device.o, n_stream, &stream) || !attr_u64(device.o, n_compute_units, &cus)) Py_RETURN_NONE;
+    Ref made(a[9] == Py_None ? result(a[10], device.o, a[0], args.out_dtype) : nullptr);
+    if (a[9] == Py_None) {
+        int32_t dtype;
+        if (!made.o) return nullptr;
+        if (made.o == Py_None || !describe<4>(made.o, &args.out, &dtype, nullptr)) Py_RETURN_NONE;
+    }
+    size_t need = 0;
+    int rc = fhip_flash_attention_workspace_bytes(&args, (int32_t)cus, &need);
+    if (rc == FHIP_OK && need) {
+        Ref bytes(PyLong_FromSize_t(need));
+        if (!bytes.o) return nullptr;
+        Ref ws(PyObject_CallMethodOneArg(device.o, n_workspace, bytes.o));
+        if (!ws.o) return nullptr;  // what the caller's own call of it would raise
+        uint64_t ptr, size;
+        if (!PyTuple_CheckExact(ws.o) || PyTuple_GET_SIZE(ws.o) != 2 || !as_u64(PyTuple_GET_ITEM(ws.o, 0), &ptr) ||
+            !as_u64(PyTuple_GET_ITEM(ws.o, 1), &size))
+            Py_RETURN_NONE;
+        args.workspace = (void *)(uintptr_t)ptr;
+        args.workspace_bytes = size;
+    }
+    if (rc == FHIP_OK) {
+        Py_BEGIN_ALLOW_THREADS
+        rc = fhip_flash_attention((fhip_stream *)stream, &args);
+        Py_END_ALLOW_THREADS
+    }
+    if (rc == FHIP_OK && made.o) return Py_NewRef(made.o);
+    return PyLong_FromLong(rc);
 }
 
 bool find(Slots *s, PyObject *type, int n, const char *const *names) {

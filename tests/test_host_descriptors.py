@@ -1,6 +1,10 @@
 """Host-only checks of how the Python mirror fills the C ABI's descriptors: packed in one go, they are byte for byte what
 assigning the fields one by one gives, in every form of call and for values beyond their fields."""
 import ctypes
+import os
+import subprocess
+import sys
+import sysconfig
 
 import numpy as np
 import pytest
@@ -204,3 +208,60 @@ def test_native_tensors_are_the_mirror_s():
         assert host.contiguous(memory, dev, 2, fa.F16, shape) is None
     with pytest.raises(ZeroDivisionError):
         host.contiguous(lambda *_: 1 // 0, dev, 2, fa.F16, (1,))
+
+
+def test_the_native_half_is_for_one_interpreter():
+    """Its name says for which, so no other one loads it."""
+    fa.lib()
+    at = fa._native.__file__
+    assert os.path.basename(at) == "_host" + sysconfig.get_config_var("EXT_SUFFIX")
+    assert not os.path.exists(os.path.join(os.path.dirname(at), "_host.so"))
+
+
+def test_the_mirror_without_its_native_half():
+    """As under an interpreter that it was not built for: the library loads, and calls are described through ctypes."""
+    program = """
+import sys
+sys.modules["floneum_amd._host"] = None
+import floneum_amd as fa
+fa.lib()
+assert fa._native is None
+class Device: pass
+class Memory:
+    def __init__(self, device, ptr): self.device, self.ptr = device, ptr
+fa.Buffer = lambda device, nbytes: Memory(device, nbytes)
+one, other = Device(), Device()
+t = fa.Tensor.empty(one, (1, 2, 9, 64), fa.F16)
+assert t.buffer.ptr == 2 * 2 * 9 * 64 and t.strides == (2 * 9 * 64, 9 * 64, 64, 1)
+try:
+    t.flash_attention(fa.Tensor.empty(other, (1, 2, 9, 64), fa.F16), t, 0.125)
+except AssertionError as e:
+    assert "different devices" in str(e)
+else:
+    sys.exit("accepted")
+"""
+    done = subprocess.run([sys.executable, "-c", program], cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))), capture_output=True, text=True)
+    assert done.returncode == 0, done.stderr
+
+
+@pytest.mark.parametrize("with_native", [True, False])
+def test_no_result_is_allocated_for_a_call_that_is_refused(monkeypatch, with_native):
+    dev, other = _Device(), _Device()
+    dev.stream = other.stream = ctypes.c_void_p(0x10)  # (no call gets as far as using it)
+    _, tensor, _, _ = native(dev)
+    if not with_native:
+        monkeypatch.setattr(fa, "_native", None)
+
+    def allocated(*_):
+        raise MemoryError("a result was allocated")
+
+    monkeypatch.setattr(fa, "Buffer", allocated)
+    q, k, v = tensor(0x1000, (1, 2, 3, 64)), tensor(0x2000, (1, 2, 9, 64)), tensor(0x3000, (1, 2, 9, 64))
+    with pytest.raises(AssertionError, match="different devices"):
+        q.flash_attention(fa.Tensor(_Memory(0x2000, other), fa.F16, (1, 2, 9, 64)), v, 0.125)
+    with pytest.raises(fa.InvalidArgument, match="one element type"):
+        q.flash_attention(k, tensor(0x3000, (1, 2, 9, 64), dtype=fa.F32), 0.125)
+    with pytest.raises(fa.InvalidArgument, match="rank-4"):
+        q.flash_attention(tensor(0x2000, (2, 9, 64)), v, 0.125)
+    with pytest.raises(MemoryError):
+        q.flash_attention(k, v, 0.125)
