@@ -845,18 +845,16 @@ static void take_visible_range(const fhip_attn_args *args, AttnParams *p) {
 
 // The plan of a split-KV decode call: the visible stretch of the cache, the split, and whether the splits are merged
 // inside the main kernel (when the device's workgroups are grouped by XCD as that form needs, see probe_xcd_grouping).
-static void plan_decode_call(fhip_device *dev, const fhip_attn_args *args, AttnParams *p) {
+static void plan_decode_call(fhip_device *dev, const fhip_attn_args *args, AttnParams *p, size_t *marks_offset) {
     take_visible_range(args, p);
     int workspace_splits;
     decode_plan(p->B, p->Hkv, p->G * p->Sq, p->Skv, p->D, dev->prop.multiProcessorCount, p->kv_lens != nullptr,
                 args->dtype == FHIP_F32, &p->chunk, &p->nsplit, &p->dec_waves, &workspace_splits);
     int stride;
-    size_t marks_off;
     p->dec_fused = 0;
-    if (dev->xcd_grouped.load() && decode_fused_layout(*p, args->dtype == FHIP_F32, &stride, &marks_off)) {
+    if (dev->xcd_grouped.load() && decode_fused_layout(*p, args->dtype == FHIP_F32, &stride, marks_offset)) {
         p->dec_fused = 1;
         p->dec_unit_stride = stride;
-        p->dec_marks_offset = marks_off;
     }
 }
 
@@ -884,7 +882,8 @@ int fhip_flash_attention_decode_plan(fhip_stream *s, const fhip_attn_args *args,
     if (id != FHIP_KERNEL_DECODE_SPLITKV || output_is_empty(args) || no_keys(args)) return FHIP_OK;
     AttnParams p;
     fill_params(args, &p);
-    plan_decode_call(s->dev, args, &p);
+    size_t marks_offset = 0;
+    plan_decode_call(s->dev, args, &p, &marks_offset);
     info->is_decode = 1;
     info->nsplit = p.nsplit;
     info->chunk = p.chunk;
@@ -1023,7 +1022,8 @@ int fhip_flash_attention(fhip_stream *s, const fhip_attn_args *args) {
         case FHIP_KERNEL_PREFILL_MFMA: rc = launch_mfma_by_head_dim(p, args->dtype, s->s); break;
         case FHIP_KERNEL_PREFILL_F32: rc = launch_prefill_f32(p, args->dtype, s->s); break;
         case FHIP_KERNEL_DECODE_SPLITKV: {
-            plan_decode_call(s->dev, args, &p);
+            size_t marks_offset = 0;
+            plan_decode_call(s->dev, args, &p, &marks_offset);
             const size_t need = decode_workspace_bytes(p.B, p.H * p.Sq, p.Hkv, p.D, p.nsplit);
             if (need > 0 && (!args->workspace || args->workspace_bytes < need)) {
                 set_error("decode needs a workspace of %zu bytes, got %zu", need,
@@ -1045,7 +1045,7 @@ int fhip_flash_attention(fhip_stream *s, const fhip_attn_args *args) {
                     return FHIP_ERR_HIP;
                 }
                 if (p.dec_fused) {
-                    p.dec_marks = (uint64_t *)((char *)args->workspace + p.dec_marks_offset);
+                    p.dec_marks = (uint64_t *)((char *)args->workspace + marks_offset);
                     p.dec_trip = dev->trip_dev;
                     do p.dec_tag = mark_tag(dev->next_mark.fetch_add(1, std::memory_order_relaxed));
                     while (p.dec_tag == 0);

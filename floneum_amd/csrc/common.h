@@ -35,7 +35,6 @@ struct AttnParams {
     int32_t dec_unit_stride;  // floats between the partials of consecutive units (a multiple of 32: 128-byte lines)
     uint64_t dec_tag;         // the call's own, see decode_marks.h
     uint64_t *dec_marks;      // [units][splits] the marks of arrivals, see fused_merge_tail
-    size_t dec_marks_offset;  // host side: bytes from the workspace's start to the marks
     int32_t *dec_trip;        // host-visible word set when the workgroups of a unit turn out to run on different XCDs
     // host-side only (profiling hook).  Both set: the dispatch of the main kernel carries the two events, which then
     // hold its own begin and end timestamps.  Only main_done: recorded on the stream after the main kernel.
