@@ -692,6 +692,8 @@ static long shares_of_least_time(const TermsCall &c, long ordinary, double gain)
         if (n > 1 && (c.Skv / n < 64 || prefill_f32_workspace_bytes(c.B, c.Hkv * c.G, c.Sq, c.D, n) > ((size_t)64 << 20) ||
                       (n - 1) * (long)c.B * c.Hkv * units > 6L * c.cus))
             break;
+        // (what parking and merging alone takes grows with n)
+        if (n > 1 && prefill_f32_merge_time(c, n) > 1.02 * least) break;
         times[tried] = prefill_f32_terms_time(c, prefill_f32_terms_form(c, n), n);
         if (tried == 0 || times[tried] < least) least = times[tried];
         tried++;

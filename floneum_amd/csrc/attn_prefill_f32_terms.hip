@@ -904,6 +904,9 @@ static TermsForm form_by_workgroups(const TermsCall &c, int ns) {
 // Time of a call whose rows all see about the same keys, in us: rounds of workgroups that walk their tiles, and parking and
 // merging the shares.  Constants fitted to 210 random calls (chunks, turns, images and encoders of 8 to 32 heads at 64 to 128
 // dims, each in every form and up to 48 shares): 6 % off in the mean square.
+double prefill_f32_merge_time(const TermsCall &c, int ns) {
+    return 3.24 + 0.456e-6 * prefill_f32_workspace_bytes(c.B, c.Hkv * c.G, c.Sq, c.D, ns);
+}
 static double wide_terms_time(const TermsCall &c, int ns);
 double prefill_f32_terms_time(const TermsCall &c, TermsForm f, int ns) {
     if (c.D > 128) return wide_terms_time(c, ns);
@@ -924,7 +927,7 @@ double prefill_f32_terms_time(const TermsCall &c, TermsForm f, int ns) {
     const long wgs = terms_workgroups(c, f.U, n), slots = (two_per_cu ? 2L : 1L) * c.cus, rest = wgs % slots;
     double us = 4.9 + wgs / slots * (ends + walk);
     if (rest) us += ends + walk * (rest <= c.cus ? alone : 1.0);
-    if (n > 1) us += 3.24 + 0.456e-6 * prefill_f32_workspace_bytes(c.B, c.Hkv * c.G, c.Sq, c.D, n);
+    if (n > 1) us += prefill_f32_merge_time(c, n);
     return us;
 }
 
@@ -973,7 +976,7 @@ static double wide_terms_time(const TermsCall &c, int ns) {
         us = std::max({longest, 1.08 * load, 2.0 * time_of(c.cus + 1.0), 3.0 * time_of(2.0 * c.cus + 1.0)});
     }
     us += 4.9;
-    if (n > 1) us += 3.24 + 0.456e-6 * prefill_f32_workspace_bytes(c.B, c.Hkv * c.G, c.Sq, c.D, n);
+    if (n > 1) us += prefill_f32_merge_time(c, n);
     return us;
 }
 

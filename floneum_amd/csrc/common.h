@@ -93,6 +93,7 @@ struct TermsForm {
 };
 TermsCall prefill_f32_terms_call(const AttnParams &p);
 double prefill_f32_terms_time(const TermsCall &call, TermsForm form, int key_shares);  // us, of calls that are not uneven, or above head_dim 128
+double prefill_f32_merge_time(const TermsCall &call, int key_shares);                  // the part of it that parks and merges shares
 TermsForm prefill_f32_terms_quickest(const TermsCall &call, int key_shares);           // by that time
 TermsForm prefill_f32_terms_form(const TermsCall &call, int key_shares);               // the one that runs
 size_t prefill_f32_workspace_bytes(int B, int H, int Sq, int D, int nsplit);
