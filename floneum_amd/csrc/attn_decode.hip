@@ -114,6 +114,14 @@ void decode_plan(int B, int Hkv, int G, int Skv, int D, int compute_units, bool 
     // The workspace is reported for these splits, also where fewer are run below: calls that one workspace served (a cache
     // that grows, the same batch with and without per-sequence lengths) still share it.
     *workspace_splits = (int)n;
+    // As many splits as were asked for fill one round, to the next whole one: a few workgroups more than the chip holds, which
+    // run a round of their own, are taken back while more than 8 splits are left, but for calls with per-sequence lengths, whose
+    // workgroups are uneven anyway: beyond 8 splits the same batch is split otherwise with lengths and without (us a step:
+    // bf16, 3 sequences of 32/8 at 96, 13774 keys 30.0 -> 25.3; f16, 10 of 8/4 at 96, two rows on 10826 keys 37.2 -> 31.1).
+    if (!ragged && decode_use_mfma(D, f32, G) && (!f32 || df_shares(D, gt / 16)) && ns == (target + units - 1) / units && units * n > target) {
+        const long k = target / units, kc = k > 8 ? ((Skv + k - 1) / k + step_keys - 1) / step_keys * step_keys : 0;
+        if (kc > 0 && (Skv + kc - 1) / kc > 8) c = kc, n = (Skv + kc - 1) / kc;
+    }
     // Fewer, longer chunks where the workgroups would need a further round for the last few of them: the chip runs rounds of
     // `target` workgroups that all take as long as their chunk and about 100 keys more; merged inside the kernel (to 8 splits) a
     // unit's splits share an XCD, and the fullest XCD counts.  Taken where that is shorter by an eighth and the call's workspace does
@@ -128,17 +136,10 @@ void decode_plan(int B, int Hkv, int G, int Skv, int D, int compute_units, bool 
     //  - on the vector variant (f16, 13 of 32/8 at 48, four rows on 6032 keys: 214 -> 236);
     //  - from more than 8 splits to 8 or fewer with two workgroups per CU: merged inside the kernel, many splits of small rows
     //    take longer than with a second launch (f16, 8 of 32/8 at 32, 8946 keys: 17.7 -> 23.4);
-    //  - calls with per-sequence lengths, whose workgroups are uneven anyway (f32, 16 sequences of up to 13172 keys: 254 -> 332), and
-    //    where two workgroups share a CU and the chunks are as long as they were asked to be: such calls share their plan with those;
+    //  - calls with per-sequence lengths (f32, 16 sequences of up to 13172 keys: 254 -> 332), and where two workgroups share a CU and the
+    //    chunks are as long as they were asked to be: up to 8 splits such calls share their plan with those;
     //  - f32 calls on the kernels that round once per four keys, where longer sums lose precision (9 sequences at 128: 2.36e-7 ->
     //    2.53e-7 against 64 bits; 1.50e-7 as it is).
-    // As many splits as were asked for fill one round, to the next whole one: a few workgroups more than the chip holds, which
-    // run a round of their own, are taken back while more than 8 splits are left (us a step: bf16, 3 sequences of 32/8 at 96, 13774 keys
-    // 30.0 -> 25.3; f16, 10 of 8/4 at 96, two rows on 10826 keys 37.2 -> 31.1).
-    if (!ragged && decode_use_mfma(D, f32, G) && (!f32 || df_shares(D, gt / 16)) && ns == (target + units - 1) / units && units * n > target) {
-        const long k = target / units, kc = k > 8 ? ((Skv + k - 1) / k + step_keys - 1) / step_keys * step_keys : 0;
-        if (kc > 0 && (Skv + kc - 1) / kc > 8) c = kc, n = (Skv + kc - 1) / kc;
-    }
     const bool asked = wgs_per_cu > 1 && ns_min <= (target + units - 1) / units;
     if (!ragged && !asked && decode_use_mfma(D, f32, G) && (!f32 || df_shares(D, gt / 16)) && units * n <= 4L * compute_units) {
         auto rounds_time = [&](long splits, long keys) {

@@ -112,6 +112,19 @@ def test_calls_that_keep_their_ordinary_splits(B, H, Hkv, rows, Skv, D, dtype):
     assert planned_splits(B, H, Hkv, rows, Skv, D, dtype) == ordinary_splits(B, Hkv, H // Hkv * rows, Skv, D, dtype == fa.F32)
 
 
+@pytest.mark.parametrize("B, H, Hkv, rows, Skv, D, dtype, splits", [
+    (3, 32, 8, 1, 13774, 96, fa.BF16, 18), (10, 8, 4, 2, 10826, 96, fa.F16, 11), (9, 16, 4, 1, 9000, 128, fa.F16, 12), (3, 32, 8, 1, 13774, 96, fa.F32, 20),
+])
+def test_splits_counted_down_to_one_round(B, H, Hkv, rows, Skv, D, dtype, splits):
+    """A few workgroups beyond what the chip holds are taken back above 8 splits; calls with per-sequence lengths keep them, and both
+    report the same workspace."""
+    call = (B, H, Hkv, rows, Skv, D, dtype)
+    ordinary = ordinary_splits(B, Hkv, H // Hkv * rows, Skv, D, dtype == fa.F32)
+    assert planned_splits(*call) == splits < ordinary and B * Hkv * splits <= 2 * CUS < B * Hkv * ordinary
+    assert planned_splits(*call, lens=True) == ordinary
+    assert workspace(*call) == workspace(*call, lens=True) == bytes_of(B, H * rows, Hkv, D, ordinary)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [fa.F32, fa.F16, fa.BF16])
 @pytest.mark.parametrize("B, H, Hkv, rows, Skv, D", [(16, 8, 8, 1, 4104, 32), (17, 16, 8, 2, 4500, 32), (20, 8, 4, 1, 3000, 160)])
