@@ -95,6 +95,16 @@ def test_division_by_multiplication():
                     assert quotient(t, job.mul[1], job.shift[1]) == t // d, (t, d)
 
 
+QUARTER_BLOCKS = 3584  # blocks of a quarter of 32 / 16 / 8 rows from which on a launch takes halves
+
+
+@pytest.mark.parametrize("D, quarter", [(64, 8), (128, 4), (256, 2)])
+def test_rows_of_a_block(D, quarter):
+    """4: a quarter of 32 / 16 / 8 rows, 2: half of them (the heads of a position together where those are neighbours)."""
+    most = (QUARTER_BLOCKS - 1) * quarter
+    assert [filled((1, 1, rows, D), 0, True).few & 7 for rows in (1, most, most + 1, 10 * most)] == [4, 4, 2, 2]
+
+
 @pytest.mark.parametrize("mode, norm", [(0, False), (1, False), (2, False), (0, True), (1, True), (2, True)])
 def test_steps_of_a_row(mode, norm):
     """Steps per row: four pairs each, or four elements where nothing is rotated; and which inputs are numbered in 32 bits."""
@@ -111,12 +121,17 @@ def test_steps_of_a_row(mode, norm):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [fa.F32, fa.F16, fa.BF16])
 @pytest.mark.parametrize("D, heads, kv_heads, rows, turned", [
-    (64, 5, 1, 4779, True), (64, 5, 1, 4777, True), (64, 5, 1, 4779, False),  # 3584 blocks of eight rows and a few less
+    (64, 5, 1, 4779, True), (64, 5, 1, 4777, True), (64, 5, 1, 4779, False),
+    (64, 5, 1, 2388, True), (64, 5, 1, 2389, True), (64, 5, 1, 2389, False), (128, 7, 2, 796, True), (128, 7, 2, 797, True),  # about 3584 blocks
+    (256, 4, 2, 597, True), (256, 4, 2, 597, False), (256, 4, 2, 598, True),
     (128, 7, 2, 801, True), (256, 4, 2, 601, True), (256, 4, 2, 601, False), (128, 3, 1, 2, True),
 ])
 def test_jobs_of_a_layer(device, dtype, D, heads, kv_heads, rows, turned):
     """q, k and v of two sequences in one launch, each with blocks of its own, against the same jobs one by one; views of
     [rows, heads, D] and of [heads, rows, D], around the sizes between which blocks change their rows and their order."""
+    # q's and k's blocks of a quarter of 32 / 16 / 8 rows: so many or more of them are made of twice the rows
+    blocks = sum(-(-2 * h * rows // {64: 8, 128: 4, 256: 2}[D]) for h in (heads, kv_heads))
+    assert (blocks < QUARTER_BLOCKS) == (rows in (2, 2388, 796, 597)) and (rows == 2 or blocks > QUARTER_BLOCKS - 8)
     rng = np.random.default_rng(D + rows)
 
     def rows_of(h):
