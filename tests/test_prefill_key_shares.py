@@ -218,3 +218,24 @@ def test_shared_keys(device, dtype, B, H, Hkv, Sq, Skv, D, causal, window, out):
     ref = (p / p.sum(-1, keepdims=True)) @ c
     err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
     assert err <= {fa.F32: 7.6e-7, fa.F16: 2.0 ** -10, fa.BF16: 2.0 ** -7}[dtype], f"relative L2 {err:.2e}"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("keys, lengths", [(800, (800,)), (900, (613, )), (769, (1, )), (801, (801, 260))])
+@pytest.mark.parametrize("hidden", [-10000.0, -np.inf, float(np.finfo(np.float32).min)])
+@pytest.mark.parametrize("D", [64, 128])
+def test_padded_sequences_in_shares(device, keys, lengths, hidden, D):
+    """Squares of more than 768 keys with a key mask: the mask-adding form and the interval form in even shares, some of which a
+    sequence's keys do not reach."""
+    B, H = len(lengths), 12
+    rng = np.random.default_rng(keys + D)
+    q, k, v = (tensor(device, rng, fa.F32, (B, H, keys, D)) for _ in range(3))
+    bias = np.where(np.arange(keys)[None, :] >= np.array(lengths)[:, None], hidden, 0.0).astype(np.float32)
+    assert shares(B, H, H, keys, keys, D, fa.F32, causal=False) >= 2
+    out = q.flash_attention(k, v, D ** -0.5, (fa.Tensor.from_numpy(device, bias, fa.F32), fa.MaskKind.BatchKeyMask)).to_numpy().astype(np.float64)
+    a, b, c = (t.to_numpy().astype(np.float64) for t in (q, k, v))
+    s = a @ b.transpose(0, 1, 3, 2) * D ** -0.5 + bias.astype(np.float64)[:, None, None, :]
+    p = np.exp(s - s.max(-1, keepdims=True))
+    ref = (p / p.sum(-1, keepdims=True)) @ c
+    err = np.linalg.norm(out - ref) / np.linalg.norm(ref)
+    assert err <= 7.6e-7, f"relative L2 {err:.2e}"
