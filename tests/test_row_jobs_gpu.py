@@ -121,17 +121,12 @@ def test_steps_of_a_row(mode, norm):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [fa.F32, fa.F16, fa.BF16])
 @pytest.mark.parametrize("D, heads, kv_heads, rows, turned", [
-    (64, 5, 1, 4779, True), (64, 5, 1, 4777, True), (64, 5, 1, 4779, False),
-    (64, 5, 1, 2388, True), (64, 5, 1, 2389, True), (64, 5, 1, 2389, False), (128, 7, 2, 796, True), (128, 7, 2, 797, True),  # about 3584 blocks
-    (256, 4, 2, 597, True), (256, 4, 2, 597, False), (256, 4, 2, 598, True),
+    (64, 5, 1, 4779, True), (64, 5, 1, 4777, True), (64, 5, 1, 4779, False),  # 3584 blocks of eight rows and a few less
     (128, 7, 2, 801, True), (256, 4, 2, 601, True), (256, 4, 2, 601, False), (128, 3, 1, 2, True),
 ])
 def test_jobs_of_a_layer(device, dtype, D, heads, kv_heads, rows, turned):
     """q, k and v of two sequences in one launch, each with blocks of its own, against the same jobs one by one; views of
     [rows, heads, D] and of [heads, rows, D], around the sizes between which blocks change their rows and their order."""
-    # q's and k's blocks of a quarter of 32 / 16 / 8 rows: so many or more of them are made of twice the rows
-    blocks = sum(-(-2 * h * rows // {64: 8, 128: 4, 256: 2}[D]) for h in (heads, kv_heads))
-    assert (blocks < QUARTER_BLOCKS) == (rows in (2, 2388, 796, 597)) and (rows == 2 or blocks > QUARTER_BLOCKS - 8)
     rng = np.random.default_rng(D + rows)
 
     def rows_of(h):
@@ -156,3 +151,16 @@ def test_jobs_of_a_layer(device, dtype, D, heads, kv_heads, rows, turned):
         n = rounded(oracle.rms_norm(np.ascontiguousarray(x), rounded(q_norm.weight.to_numpy()[0], dtype), None, 1e-6), dtype)
         y = rounded(oracle.rope(n, rope.cos_host, rope.sin_host, 5 + r), dtype)
         assert np.array_equal(rounded(got[0].to_numpy(), dtype)[:, :, r:r + 1].view(np.uint32), y.view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [fa.F32, fa.F16, fa.BF16])
+@pytest.mark.parametrize("D, heads, kv_heads, rows, turned, quarters", [
+    (64, 5, 1, 2388, True, True), (64, 5, 1, 2389, True, False), (64, 5, 1, 2389, False, False), (128, 7, 2, 796, True, True),
+    (128, 7, 2, 797, True, False), (256, 4, 2, 597, True, True), (256, 4, 2, 597, False, True), (256, 4, 2, 598, True, False),
+])
+def test_jobs_of_a_layer_on_both_sides(device, dtype, D, heads, kv_heads, rows, turned, quarters):
+    """The same of two sequences whose q and k are just below and just above QUARTER_BLOCKS blocks."""
+    blocks = sum(-(-2 * h * rows // {64: 8, 128: 4, 256: 2}[D]) for h in (heads, kv_heads))
+    assert quarters == (blocks < QUARTER_BLOCKS) and abs(blocks - QUARTER_BLOCKS) < 8
+    test_jobs_of_a_layer(device, dtype, D, heads, kv_heads, rows, turned)
