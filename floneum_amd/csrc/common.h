@@ -72,7 +72,7 @@ struct AttnParams {
 // and takes the levels of uneven shares, such calls stay with the uneven ones (4/1 heads at 256, 1804 behind 4210 under 1515 123 and 164).
 inline bool prefill_f32_uneven(int64_t Sq, int64_t Skv, int64_t D, bool causal, bool qk_mask, int64_t first_row_at, int64_t window) {
     if (2 * Sq <= Skv) return false;
-    return qk_mask || (causal && !(D <= 128 && window > 0 && 2 * (first_row_at + 1) >= window));
+    return qk_mask || (causal && !(D <= 128 && window > 0 && first_row_at >= (window - 1) / 2));
 }
 // uneven: see prefill_f32_uneven; window: rows see the last so many keys up to their position (0: all)
 void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, bool causal_square, bool uneven, int64_t window, bool unknown_lengths,

@@ -140,6 +140,15 @@ def test_rows_behind_a_window_see_alike():
     assert shares(1, 4, 1, 1804, 6014, 256, fa.F32, window=1515) >= 3  # (above 128 dims uneven shares know their window)
 
 
+@pytest.mark.parametrize("at", [2 ** 20, 2 ** 62 - 2, 2 ** 62, 2 ** 63 - 1 - 1156])
+def test_rows_far_behind_the_keys_see_alike(at):
+    """Rows and a window at the end of the 64 bits: every row sees every key, as without a mask."""
+    a, need = make_args(B=1, H=16, Hkv=16, Sq=1156, Skv=1156, D=128, dtype=fa.F32), ctypes.c_size_t()
+    a.analytic.enabled, a.analytic.causal, a.analytic.q_pos_offset, a.analytic.window = 1, 1, at, at + 1156
+    assert fa.lib().fhip_flash_attention_workspace_bytes(ctypes.byref(a), CUS, ctypes.byref(need)) == fa.OK
+    assert need.value == shares(1, 16, 16, 1156, 1156, 128, fa.F32, causal=False) * 16 * 1156 * 130 * 4 > 0
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("D", [256, 160])
 @pytest.mark.parametrize("H, Hkv, rows, keys, window, how, want", [
