@@ -1,6 +1,7 @@
 // Prefill attention in f32 precision on the gfx950 f32 matrix instruction (v_mfma_f32_32x32x2_f32): calls that
 // attn_prefill_f32_terms.hip cannot address (prefill_f32_terms_takes): K or V rows that overlap, a K, V
-// or Q slice of 2 GiB and more, or grids beyond its dimensions; and of head dims above 128 short calls of few rows (wide_in_terms).
+// or Q slice of 2 GiB and more, or grids beyond its dimensions; and above head_dim 128
+// 16-bit tensors, short calls of few rows and unsplit ones whose rows see few keys (wide_in_terms, wide_f32_time).
 //
 // A workgroup of 4 wavefronts owns 128 query rows of one (batch, head), a wavefront 32 of them; K/V tiles of 32 rows pass
 // through LDS.

@@ -148,10 +148,11 @@ typedef enum {
     FHIP_KERNEL_PREFILL_MFMA = 2,/* f16/bf16, head_dim a multiple of 8 up to 256, LDS-tiled MFMA (to 128 on 256-row
                                     workgroups where they fill the chip, else the wide-head form); masks by interval
                                     (analytic, kv_lens, or a mask tensor reduced on the device) */
-    FHIP_KERNEL_PREFILL_F32 = 3, /* f32 precision, LDS-tiled: on the bf16 MFMA from three bf16 terms per value to
-                                    head_dim 128, on the f32 MFMA above: f32 tensors, and 16-bit tensors
-                                    (widened on load) the kernel above does not take; head_dim multiple of
-                                    4 up to 256; masks by interval or, up to head_dim 128, added as they are */
+    FHIP_KERNEL_PREFILL_F32 = 3, /* f32 precision, LDS-tiled: on the bf16 MFMA from three bf16 terms per value: f32
+                                    tensors, and 16-bit tensors (widened on load) the kernel above does not
+                                    take; head_dim multiple of 4 up to 256.  On the f32 MFMA where the terms
+                                    kernel cannot address a call, above head_dim 128 also short calls and
+                                    16-bit tensors; masks by interval or, up to head_dim 128, added as they are */
     FHIP_KERNEL_DECODE_SPLITKV = 4,/* 1..4 query rows per sequence, head_dim multiple of 8 up to 256: split-KV
                                       streaming + LSE combine.  Matrix cores at every head_dim that is a multiple
                                       of 32 up to 256 (the 16-bit or the f32 instruction, by the tensors' type;
