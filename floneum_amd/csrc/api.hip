@@ -322,9 +322,10 @@ static void visible_range(const fhip_attn_args *a, int *lo0, int *len) {
     *len = (int)(hi - *lo0);
 }
 
-// Calls whose rows may see far fewer keys than the host knows of: of sequences with lengths of their own, or with a mask tensor over
-// (query, key).  (A key mask over the batch is counted as padding, which most rows do not have.)
-static bool unknown_lengths(const fhip_attn_args *a) { return a->kv_lens || a->mask_kind == FHIP_MASK_QK; }
+// Calls whose rows may see far fewer keys than the host knows of: of sequences with lengths of their own.  (A key mask over the batch is
+// counted as padding, which most rows do not have; a mask over (query, key) as the causal one that it mostly is, whose plan it shares, for
+// the two give the same bits.)
+static bool unknown_lengths(const fhip_attn_args *a) { return a->kv_lens != nullptr; }
 
 // Key split of a call the f32-arithmetic tiled kernel serves (few query rows on a long cache), and where its
 // partial results go in the workspace: behind the mask scratch, 256-byte aligned.

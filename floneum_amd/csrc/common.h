@@ -79,7 +79,8 @@ void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, boo
                       int compute_units, int *nsplit, int *chunk);
 // What part of the rules' time the shares of least time have to be, by a model: 5 % less, and 30 % where the rows may see far fewer
 // keys than it counts (us, in the rules' shares and by 5 %: f16, two sequences of 84 rows of 6/3 heads at 80 on up to 1416 keys 11.2 and 14.5;
-// bf16, two of 377 of 32/8 at 256 on up to 2369 50 and 97; f32, 32/8 at 128, 360 rows that see 300 of 1844 keys by a mask tensor 56 and 65).
+// bf16, two of 377 of 32/8 at 256 on up to 2369 50 and 97).  Mask tensors that hide most keys lose by the 5 % as well (f32, 32/8 at 128, 360 rows that see 300 of 1844 keys 56 and 65),
+// but are not told from causal ones, whose plan they have to share.
 inline double shares_gain(bool unknown_lengths) { return unknown_lengths ? 0.7 : 0.95; }
 // The forms of the f32 terms kernel (attn_prefill_f32_terms.hip): units and key groups per workgroup, and what a call takes in them
 struct TermsCall {

@@ -58,7 +58,8 @@ def test_the_partials_of_a_call_are_limited(call, want):
     ((1, 32, 8, 360, 1844, 128, fa.F32), 5, 2), ((1, 16, 4, 765, 1999, 96, fa.F32), 5, 2), ((3, 16, 4, 321, 1323, 128, fa.F32), 3, 0),
 ])
 def test_rows_that_may_see_fewer_keys_than_the_call_has(call, known, unknown):
-    """Sequences with lengths of their own and masks over (query, key) take more shares than by rule only for 30 % of the time."""
+    """Sequences with lengths of their own take more shares than by rule only for 30 % of the time; masks over (query, key) are planned as
+    causal ones, whose bits they have."""
     B, H, Hkv, rows, keys, D, dtype = call
     a, need = make_args(B=B, H=H, Hkv=Hkv, Sq=rows, Skv=keys, D=D, dtype=dtype), ctypes.c_size_t()
     per = B * H * rows * (D + (2 if dtype == fa.F32 else 4)) * 4
@@ -73,7 +74,27 @@ def test_rows_that_may_see_fewer_keys_than_the_call_has(call, known, unknown):
     a.kv_lens = None
     a.mask_kind, a.mask.ptr, a.mask_intervals = fa.MaskKind.QKMask, 0x10000, 0x20000
     a.mask.shape[:], a.mask.stride[:] = (rows, keys), (keys, 1)
-    assert asked() == unknown
+    assert asked() == known == shares(*call)
+
+
+@pytest.mark.parametrize("dtype, D", [(fa.F32, 64), (fa.F32, 100), (fa.F32, 128), (fa.F32, 256), (fa.F16, 64), (fa.BF16, 128), (fa.F16, 192), (fa.F16, 256)])
+def test_a_mask_tensor_shares_the_plan_of_the_causal_mask(dtype, D):
+    """The tensor of a causal mask gives the bits of the analytic call, so chunks of a prompt are shared out alike."""
+    rng = np.random.default_rng(D)
+    for _ in range(300):
+        rows, Hkv = int(rng.integers(65, 1500)), int(rng.choice([1, 2, 4, 8]))
+        keys, B, H = 2 * rows + int(rng.integers(0, 6000)), int(rng.integers(1, 5)), Hkv * int(rng.choice([1, 2, 4]))
+        asked = []
+        for masked in (False, True):
+            a, need = make_args(B=B, H=H, Hkv=Hkv, Sq=rows, Skv=keys, D=D, dtype=dtype), ctypes.c_size_t()
+            if masked:
+                a.mask_kind, a.mask.ptr, a.mask_intervals = fa.MaskKind.QKMask, 0x10000, 0x20000
+                a.mask.shape[:], a.mask.stride[:] = (rows, keys), (keys, 1)
+            else:
+                a.analytic.enabled, a.analytic.causal, a.analytic.q_pos_offset = 1, 1, keys - rows
+            assert fa.lib().fhip_flash_attention_workspace_bytes(ctypes.byref(a), CUS, ctypes.byref(need)) == fa.OK
+            asked.append(need.value)
+        assert asked[0] == asked[1], (B, H, Hkv, rows, keys)
 
 
 @pytest.mark.parametrize("call", [(1, 32, 32, 2859, 7370, 80), (8, 16, 16, 689, 6007, 80), (8, 4, 1, 2154, 6748, 96)])
