@@ -869,9 +869,9 @@ static long terms_workgroups(const TermsCall &c, int U, int ns) {
 
 // The form by the numbers of its workgroups (measured on f32 calls, time per call in us; w2, w4: workgroups with 2 or 4 units):
 //   (4, 1)  two workgroups per CU, least splitting per tile: grids that fill the chip twice.  Head dims above 128, one workgroup per CU
-//           (106 KiB of LDS, 512 registers): a wavefront per SIMD issues its matrix and vector work in turn, 5.3 us a tile at 256 of
-//           which 2.6 are matrix instructions (16/4 heads causal, us before, on the f32 matrix instruction: 148 rows on 3510 keys
-//           192 -> 80, 1024 x 1024 181 -> 119, 3191 x 3191 826 -> 555, 1500 x 6000 1577 -> 1005)
+//           (106 KiB of LDS, 512 registers): a wavefront per SIMD issues its matrix and vector work in turn, 12200 cycles a tile
+//           at 256, 6144 of them matrix instructions (5.3 to 5.6 us by the clock; profiles/prefill_f32_terms.txt; 16/4 heads causal, us before, on the f32 matrix instruction: 148 rows on 3510 keys
+//           192 -> 80, 1024 x 1024 181 -> 119, 3191 x 3191 826 -> 555, 1500 x 6000 1577 -> 1020)
 //   (4, 2)  eight wavefronts, one workgroup per CU: D = 128 1500 rows 115 against 142 for (4, 1), 4000 rows of 8 heads
 //           262 against 348, 129 rows on 8003 keys (keys split over workgroups) 111 against 133
 //   (2, 2)  D > 64: one wavefront per SIMD with 512 registers, half the units per workgroup, for short prompts (700 rows
