@@ -337,7 +337,8 @@ static void f32_split_plan(const fhip_attn_args *a, int cus, int *nsplit, int *c
                                            a->mask_kind == FHIP_MASK_QK, a->analytic.q_pos_offset - lo0, a->analytic.window);
     const int Hkv = (int)a->k.shape[1];
     prefill_f32_plan((int)a->q.shape[0], (int)a->q.shape[1], Hkv ? (int)a->q.shape[1] / Hkv : 1, (int)a->q.shape[2],
-                     len, (int)a->q.shape[3], a->dtype == FHIP_F32, causal_square, uneven, a->analytic.enabled ? a->analytic.window : 0,
+                     len, (int)a->q.shape[3], a->dtype == FHIP_F32,
+                     (a->analytic.enabled && a->analytic.causal) || a->mask_kind == FHIP_MASK_QK, causal_square, uneven, a->analytic.enabled ? a->analytic.window : 0,
                      unknown_lengths(a), cus > 0 ? cus : 256, nsplit, chunk);
 }
 static size_t f32_partials_offset(const fhip_attn_args *a) { return (mask_scratch_bytes(a) + 255) & ~(size_t)255; }

@@ -688,6 +688,10 @@ static long shares_of_least_time(const TermsCall &c, long ordinary, double gain)
     const long units = (long)c.G * ((c.Sq + 31) / 32);
     double times[sizeof(SHARES) / sizeof(SHARES[0])], least = 0.0;
     int tried = 0;
+    auto time_in = [&](int n) {
+        const TermsForm form = prefill_f32_terms_form(c, n);
+        return n > 1 ? prefill_f32_terms_time(c, form, n) : prefill_f32_unsplit_time(c, form);
+    };
     for (const int n : SHARES) {
         // (shares that make three rounds of the smallest workgroups gain nothing more)
         if (n > 1 && (c.Skv / n < 64 || prefill_f32_workspace_bytes(c.B, c.Hkv * c.G, c.Sq, c.D, n) > ((size_t)64 << 20) ||
@@ -695,13 +699,13 @@ static long shares_of_least_time(const TermsCall &c, long ordinary, double gain)
             break;
         // (what parking and merging alone takes grows with n)
         if (n > 1 && prefill_f32_merge_time(c, n) > 1.02 * least) break;
-        times[tried] = prefill_f32_terms_time(c, prefill_f32_terms_form(c, n), n);
+        times[tried] = time_in(n);
         if (tried == 0 || times[tried] < least) least = times[tried];
         tried++;
     }
     for (int i = 0; i < tried; i++) {
         if (times[i] > 1.02 * least) continue;
-        return times[i] < gain * prefill_f32_terms_time(c, prefill_f32_terms_form(c, (int)ordinary), (int)ordinary) ? SHARES[i] : ordinary;
+        return times[i] < gain * time_in((int)ordinary) ? SHARES[i] : ordinary;
     }
     return ordinary;
 }
@@ -720,7 +724,7 @@ static double wide_f32_time(const TermsCall &c) {
 
 // Few query rows on a long cache (a new chat turn, a prompt fed in pieces): the grid of query blocks alone leaves
 // most CUs idle, so the keys are split over workgroups as well.
-void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, bool causal_square, bool uneven, int64_t window,
+void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, bool causal, bool causal_square, bool uneven, int64_t window,
                       bool unknown_lengths, int compute_units, int *nsplit, int *chunk) {
     *nsplit = 1;
     *chunk = Skv;
@@ -762,7 +766,7 @@ void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, boo
         // rule's (shares_gain); at most 64 MiB of partials (us a call: two sequences of 275 rows of 32/8
         // heads at 64 on 2911 keys 116 -> 92; 16 heads without a mask, 1156 rows at 128 148 -> 80, 2506 366 -> 285, 1147 at 80 109 -> 59; over 90
         // random calls the time is 0.91, the worst 1.03 of the rule's).  Square prompts to 768 keys keep the rule, masked or not.
-        if (!uneven && Sq > 128 && (few_rows || Skv > 768)) ns = shares_of_least_time({B, H / G, G, Sq, Skv, D, compute_units, false, window, f32}, ns < 2 ? 1 : ns, shares_gain(unknown_lengths));
+        if (!uneven && Sq > 128 && (few_rows || Skv > 768)) ns = shares_of_least_time({B, H / G, G, Sq, Skv, D, compute_units, false, window, f32, causal}, ns < 2 ? 1 : ns, shares_gain(unknown_lengths));
         if (ns < 2) return;
         const long c = ((Skv + ns - 1) / ns + 31) / 32 * 32;
         *chunk = (int)c;
@@ -773,7 +777,7 @@ void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, boo
         // Head dims above 128 in the terms kernel: the shares of least time (us, 16/4 heads at 256 causal, in one share and in
         // the shares taken: 148 rows on 3510 keys 584 -> 80, 300 on 700 128 -> 49, 1000 on 1000 182 -> 93, 2000 on 2000 347 -> 235; 2048 on 2048 stays at 355, its two shares
         // would be more than 64 MiB of partials).
-        const TermsCall call = {B, H / G, G, Sq, Skv, D, compute_units, uneven, window, true};
+        const TermsCall call = {B, H / G, G, Sq, Skv, D, compute_units, uneven, window, true, causal};
         const long ns = shares_of_least_time(call, 1, shares_gain(false));
         if (ns < 2 || wide_f32_time(call) < prefill_f32_terms_time(call, {4, 1}, (int)ns)) return;
         const long c = ((Skv + ns - 1) / ns + 31) / 32 * 32;

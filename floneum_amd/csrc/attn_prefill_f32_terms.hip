@@ -908,27 +908,52 @@ double prefill_f32_merge_time(const TermsCall &c, int ns) {
     return 3.24 + 0.456e-6 * prefill_f32_workspace_bytes(c.B, c.Hkv * c.G, c.Sq, c.D, ns);
 }
 static double wide_terms_time(const TermsCall &c, int ns);
+namespace {
+// Of a workgroup: a tile of one of its key groups, its ends, and what a tile takes where a CU has one of two workgroups.
+struct FormTimes {
+    double tile, ends, alone;
+    bool two_per_cu;
+};
+FormTimes times_of_form(int D, TermsForm f) {
+    const double dims = (D <= 64 ? 64 : D <= 96 ? 96 : 128) / 64.0;
+    if (f.U == 2 && f.KG == 2 && D <= 64) return {2.65, 1.4, 0.71, true};
+    if (f.U == 2 && f.KG == 2) return {0.38 + 1.494 * dims, 3.9, 1.0, false};
+    if (f.KG == 2) return {0.306 + 1.945 * dims, 3.45, 1.0, false};
+    if (f.KG == 4) return {2.65, 3.87, 1.0, false};
+    return {0.374 + 1.78 * dims, 0.8, 0.74, true};
+}
+}  // namespace
 double prefill_f32_terms_time(const TermsCall &c, TermsForm f, int ns) {
     if (c.D > 128) return wide_terms_time(c, ns);
-    const double dims = (c.D <= 64 ? 64 : c.D <= 96 ? 96 : 128) / 64.0;
-    double tile, ends, alone = 1.0;  // per tile of a group, per workgroup, and a tile's time where a CU has one of two workgroups
-    bool two_per_cu = false;
-    if (f.U == 2 && f.KG == 2 && c.D <= 64) tile = 2.65, ends = 1.4, alone = 0.71, two_per_cu = true;
-    else if (f.U == 2 && f.KG == 2) tile = 0.38 + 1.494 * dims, ends = 3.9;
-    else if (f.KG == 2) tile = 0.306 + 1.945 * dims, ends = 3.45;
-    else if (f.KG == 4) tile = 2.65, ends = 3.87;
-    else tile = 0.374 + 1.78 * dims, ends = 0.8, alone = 0.74, two_per_cu = true;
+    const FormTimes t = times_of_form(c.D, f);
     const int chunk = ((c.Skv + ns - 1) / ns + PT_BN - 1) / PT_BN * PT_BN, n = (c.Skv + chunk - 1) / chunk;
     int tiles = chunk / PT_BN;
     // (rows of a chunk see the window's keys; wider windows than 0.7 of the keys are taken for none: 32/8 heads at 128, 1100 rows under 2885
     // of 3984 keys would stay unsplit and take 1.21 times as long)
     if (c.window > 0 && c.window < c.Skv && 10 * (c.window + PT_BN) < 7LL * c.Skv) tiles = std::min(tiles, ((int)c.window + 2 * PT_BN - 1) / PT_BN + 1);
-    const double walk = tile * ((tiles + f.KG - 1) / f.KG);
-    const long wgs = terms_workgroups(c, f.U, n), slots = (two_per_cu ? 2L : 1L) * c.cus, rest = wgs % slots;
-    double us = 4.9 + wgs / slots * (ends + walk);
-    if (rest) us += ends + walk * (rest <= c.cus ? alone : 1.0);
+    const double walk = t.tile * ((tiles + f.KG - 1) / f.KG);
+    const long wgs = terms_workgroups(c, f.U, n), slots = (t.two_per_cu ? 2L : 1L) * c.cus, rest = wgs % slots;
+    double us = 4.9 + wgs / slots * (t.ends + walk);
+    if (rest) us += t.ends + walk * (rest <= c.cus ? t.alone : 1.0);
     if (n > 1) us += prefill_f32_merge_time(c, n);
     return us;
+}
+
+// Unsplit chunks under a causal mask that need more than one round: the rows of the later rounds see the fewest keys, and start first where rows
+// of few keys end.  1.15 times what the second (third) round's first workgroup takes twice (three times), or the mean load: 5 % off over nine
+// chunks of 272 to 376 workgroups, which as even calls were taken for 1.1 to 1.5 times their time and split for nothing (us, four sequences
+// of 1071 rows of 8/4 heads at 128 on 2216 keys 203 unsplit and 261 in two shares, three of 1832 of 8/2 at 96 on 3665 289 and 336).
+double prefill_f32_unsplit_time(const TermsCall &c, TermsForm f) {
+    const double even = prefill_f32_terms_time(c, f, 1);
+    if (c.D > 128 || !c.causal || c.window > 0) return even;
+    const FormTimes t = times_of_form(c.D, f);
+    const double walk = t.tile * (((c.Skv + PT_BN - 1) / PT_BN + f.KG - 1) / f.KG), part = (double)c.Sq / c.Skv;
+    const double wgs = (double)terms_workgroups(c, f.U, 1), slots = (t.two_per_cu ? 2.0 : 1.0) * c.cus;
+    if (wgs <= slots) return even;
+    double us = std::max(t.ends + walk, 1.08 * wgs / slots * (t.ends + walk * (1.0 - 0.5 * part)));
+    us = std::max(us, 2.0 * (t.ends + walk * (1.0 - part * slots / wgs)));
+    if (wgs > 2 * slots) us = std::max(us, 3.0 * (t.ends + walk * (1.0 - part * 2.0 * slots / wgs)));
+    return std::min(even, 4.9 + 1.15 * us);
 }
 
 // The same above head_dim 128, where the form is (4, 1) with one workgroup per CU, of uneven calls too: even shares in rounds; of uneven
@@ -1006,7 +1031,8 @@ TermsForm prefill_f32_terms_form(const TermsCall &c, int ns) {
 // (of f32 tensors)
 TermsCall prefill_f32_terms_call(const AttnParams &p) {
     const bool uneven = prefill_f32_uneven(p.Sq, p.Skv, p.D, p.analytic && p.causal, p.mask_kind == FHIP_MASK_QK, p.q_pos_offset, p.window);
-    return {p.B, p.Hkv, p.G, p.Sq, p.Skv, p.D, p.cus > 0 ? p.cus : 256, uneven, p.analytic ? p.window : 0, true};
+    return {p.B, p.Hkv, p.G, p.Sq, p.Skv, p.D, p.cus > 0 ? p.cus : 256, uneven, p.analytic ? p.window : 0, true,
+            (p.analytic && p.causal) || p.mask_kind == FHIP_MASK_QK};
 }
 
 template <typename T, int U, int KG, int MODE>

@@ -74,9 +74,9 @@ inline bool prefill_f32_uneven(int64_t Sq, int64_t Skv, int64_t D, bool causal, 
     if (2 * Sq <= Skv) return false;
     return qk_mask || (causal && !(D <= 128 && window > 0 && first_row_at >= (window - 1) / 2));
 }
-// uneven: see prefill_f32_uneven; window: rows see the last so many keys up to their position (0: all)
-void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, bool causal_square, bool uneven, int64_t window, bool unknown_lengths,
-                      int compute_units, int *nsplit, int *chunk);
+// causal: see TermsCall; uneven: see prefill_f32_uneven; window: rows see the last so many keys up to their position (0: all)
+void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, bool causal, bool causal_square, bool uneven, int64_t window,
+                      bool unknown_lengths, int compute_units, int *nsplit, int *chunk);
 // What part of the rules' time the shares of least time have to be, by a model: 5 % less, and 30 % where the rows may see far fewer
 // keys than it counts (us, in the rules' shares and by 5 %: f16, two sequences of 84 rows of 6/3 heads at 80 on up to 1416 keys 11.2 and 14.5;
 // bf16, two of 377 of 32/8 at 256 on up to 2369 50 and 97).  Mask tensors that hide most keys lose by the 5 % as well (f32, 32/8 at 128, 360 rows that see 300 of 1844 keys 56 and 65),
@@ -88,12 +88,14 @@ struct TermsCall {
     bool uneven;
     int64_t window;
     bool f32;  // the tensors' type (16-bit ones run in one form)
+    bool causal;  // rows see keys up to their own position (a mask tensor over (query, key) is taken for one that says so)
 };
 struct TermsForm {
     int U, KG;
 };
 TermsCall prefill_f32_terms_call(const AttnParams &p);
 double prefill_f32_terms_time(const TermsCall &call, TermsForm form, int key_shares);  // us, of calls that are not uneven, or above head_dim 128
+double prefill_f32_unsplit_time(const TermsCall &call, TermsForm form);                // the same of one share, of causal chunks as well
 double prefill_f32_merge_time(const TermsCall &call, int key_shares);                  // the part of it that parks and merges shares
 TermsForm prefill_f32_terms_quickest(const TermsCall &call, int key_shares);           // by that time
 TermsForm prefill_f32_terms_form(const TermsCall &call, int key_shares);               // the one that runs

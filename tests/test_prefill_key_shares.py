@@ -123,6 +123,13 @@ def test_a_windowed_prompt_is_not_shared_out_as_a_whole_one(H, Hkv, rows, D):
     assert all(shares(1, H, Hkv, rows, rows, D, fa.F32, window=w) == whole for w in (rows - 1, rows, 2 * rows, 2 ** 40, 2 ** 63 - 1))
 
 
+@pytest.mark.parametrize("call", [(4, 8, 4, 1071, 2216, 128), (1, 32, 8, 1494, 2990, 96), (3, 8, 2, 1832, 3665, 96), (1, 16, 4, 2436, 5021, 80)])
+def test_long_chunks_are_not_split_for_rows_that_see_few_keys(call):
+    """Chunks of more than a round of workgroups, whose later rounds see the fewest keys under a causal mask (us unsplit and in the two shares
+    that calls without one take: 203 and 257, 245 and 284, 287 and 339, 348 and 433)."""
+    assert shares(*call, fa.F32) == 0 and shares(*call, fa.F32, causal=False) >= 2
+
+
 @pytest.mark.parametrize("H, Hkv, rows, keys, D, causal, want", [
     (16, 4, 1500, 1500, 100, False, 2), (32, 8, 200, 3000, 100, True, 7), (32, 8, 200, 3000, 36, True, 7), (16, 8, 400, 2500, 60, True, 8),
 ])
