@@ -681,17 +681,19 @@ static int launch_rows(const AttnParams &p, hipStream_t stream) {
     return FHIP_OK;
 }
 
-// Shares of the keys: the fewest within 2 % of the least time, where that is less than `gain` of the time of `ordinary` ones; each in the form
-// that it would run in.
+// Shares of the keys: the fewest within 2 % of the least time, where that is less than `gain` of the time of `ordinary` ones.  The times
+// are those of a number's quickest form, although f32 tensors keep the form of the workgroups' numbers unless it is 10 % better
+// (prefill_f32_terms_form): in the form that runs the model takes fewer or more shares for a few per cent that it is off itself (60 calls whose shares
+// differ: 0.92 to 1.20 of the time, 1.03 in the mean; 8/4 heads at 64, 162 rows on 390 keys 12.8 -> 14.6 us).  Only causal chunks of more than a
+// round, which lose by half a round too many, go by the form that runs (prefill_f32_unsplit_time).  16-bit tensors have one form.
 static long shares_of_least_time(const TermsCall &c, long ordinary, double gain) {
     constexpr int SHARES[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48};
     const long units = (long)c.G * ((c.Sq + 31) / 32);
     double times[sizeof(SHARES) / sizeof(SHARES[0])], least = 0.0;
     int tried = 0;
-    auto time_in = [&](int n) {
-        const TermsForm form = prefill_f32_terms_form(c, n);
-        return n > 1 ? prefill_f32_terms_time(c, form, n) : prefill_f32_unsplit_time(c, form);
-    };
+    const TermsForm whole = prefill_f32_terms_form(c, 1);
+    const bool by_form = prefill_f32_unsplit_time(c, whole) < prefill_f32_terms_time(c, whole, 1);
+    auto time_in = [&](TermsForm form, int n) { return n > 1 ? prefill_f32_terms_time(c, form, n) : prefill_f32_unsplit_time(c, form); };
     for (const int n : SHARES) {
         // (shares that make three rounds of the smallest workgroups gain nothing more)
         if (n > 1 && (c.Skv / n < 64 || prefill_f32_workspace_bytes(c.B, c.Hkv * c.G, c.Sq, c.D, n) > ((size_t)64 << 20) ||
@@ -699,13 +701,13 @@ static long shares_of_least_time(const TermsCall &c, long ordinary, double gain)
             break;
         // (what parking and merging alone takes grows with n)
         if (n > 1 && prefill_f32_merge_time(c, n) > 1.02 * least) break;
-        times[tried] = time_in(n);
+        times[tried] = time_in(by_form ? prefill_f32_terms_form(c, n) : prefill_f32_terms_quickest(c, n), n);
         if (tried == 0 || times[tried] < least) least = times[tried];
         tried++;
     }
     for (int i = 0; i < tried; i++) {
         if (times[i] > 1.02 * least) continue;
-        return times[i] < gain * time_in((int)ordinary) ? SHARES[i] : ordinary;
+        return times[i] < gain * time_in(prefill_f32_terms_form(c, (int)ordinary), (int)ordinary) ? SHARES[i] : ordinary;
     }
     return ordinary;
 }

@@ -123,6 +123,12 @@ def test_a_windowed_prompt_is_not_shared_out_as_a_whole_one(H, Hkv, rows, D):
     assert all(shares(1, H, Hkv, rows, rows, D, fa.F32, window=w) == whole for w in (rows - 1, rows, 2 * rows, 2 ** 40, 2 ** 63 - 1))
 
 
+@pytest.mark.parametrize("call, want", [((1, 8, 4, 162, 390, 64), 4), ((1, 16, 4, 154, 445, 64), 4), ((8, 8, 2, 516, 2456, 64), 2), ((8, 32, 8, 180, 2905, 64), 2)])
+def test_f32_tensors_are_shared_out_by_the_quickest_form(call, want):
+    """(us, in these shares and in those of the least time of the form that runs: 12.8 and 14.6, 13.3 and 14.9, 143 and 162, 199 and 238)"""
+    assert shares(*call, fa.F32) == want
+
+
 @pytest.mark.parametrize("call", [(4, 8, 4, 1071, 2216, 128), (1, 32, 8, 1494, 2990, 96), (3, 8, 2, 1832, 3665, 96), (1, 16, 4, 2436, 5021, 80)])
 def test_long_chunks_are_not_split_for_rows_that_see_few_keys(call):
     """Chunks of more than a round of workgroups, whose later rounds see the fewest keys under a causal mask (us unsplit and in the two shares
