@@ -928,9 +928,11 @@ double prefill_f32_terms_time(const TermsCall &c, TermsForm f, int ns) {
     const FormTimes t = times_of_form(c.D, f);
     const int chunk = ((c.Skv + ns - 1) / ns + PT_BN - 1) / PT_BN * PT_BN, n = (c.Skv + chunk - 1) / chunk;
     int tiles = chunk / PT_BN;
-    // (rows of a chunk see the window's keys; wider windows than 0.7 of the keys are taken for none: 32/8 heads at 128, 1100 rows under 2885
-    // of 3984 keys would stay unsplit and take 1.21 times as long)
-    if (c.window > 0 && c.window < c.Skv && 10 * (c.window + PT_BN) < 7LL * c.Skv) tiles = std::min(tiles, ((int)c.window + 2 * PT_BN - 1) / PT_BN + 1);
+    // (a workgroup's rows see the window's keys and as many more as there are rows: counted for 32 rows in every form, ungrouped heads took
+    // four units too often, 16 heads at 96, three sequences of 156 rows under 32 21.7 us for 13.9, over 110 chunks 1.09 of the time; wider windows
+    // than 0.7 of the keys are taken for none: 32/8 heads at 128, 1100 rows under 2885 of 3984 keys would stay unsplit and take 1.21 times as long)
+    const int rows = 32 * ((f.U + c.G - 1) / c.G);
+    if (c.window > 0 && c.window < c.Skv && 10 * (c.window + PT_BN) < 7LL * c.Skv) tiles = std::min(tiles, ((int)c.window + rows + PT_BN - 1) / PT_BN + 1);
     const double walk = t.tile * ((tiles + f.KG - 1) / f.KG);
     const long wgs = terms_workgroups(c, f.U, n), slots = (t.two_per_cu ? 2L : 1L) * c.cus, rest = wgs % slots;
     double us = 4.9 + wgs / slots * (t.ends + walk);

@@ -123,6 +123,26 @@ def test_a_windowed_prompt_is_not_shared_out_as_a_whole_one(H, Hkv, rows, D):
     assert all(shares(1, H, Hkv, rows, rows, D, fa.F32, window=w) == whole for w in (rows - 1, rows, 2 * rows, 2 ** 40, 2 ** 63 - 1))
 
 
+class TermsCall(ctypes.Structure):  # floneum_amd/csrc/common.h
+    _fields_ = [(n, ctypes.c_int) for n in ("B", "Hkv", "G", "Sq", "Skv", "D", "cus")] + [
+        ("uneven", ctypes.c_bool), ("window", ctypes.c_int64), ("f32", ctypes.c_bool), ("causal", ctypes.c_bool)]
+
+
+@pytest.mark.parametrize("call, want", [
+    # workgroups of half the units, or of two key groups, see fewer keys beside a window's (us in those of four units and now: 21.7 and
+    # 13.9, 19.2 and 13.4, 14.2 and 10.4, 18.3 and 13.6, 16.4 and 13.4, 27.1 and 24.0)
+    ((3, 16, 1, 156, 314, 96, 32), (2, 2)), ((1, 16, 1, 228, 319, 80, 24), (2, 2)), ((1, 8, 2, 224, 249, 80, 25), (2, 2)),
+    ((1, 16, 1, 1558, 1580, 64, 27), (2, 2)), ((1, 4, 2, 155, 309, 96, 29), (2, 2)), ((4, 16, 1, 273, 444, 96, 82), (4, 2)),
+    ((1, 32, 1, 1000, 1063, 128, 64), (4, 1)),
+])
+def test_forms_under_a_narrow_window(call, want):
+    """The form of an unsplit f32 chunk (batch, KV heads, heads each, rows, keys seen, head_dim, window), from what the launcher asks."""
+    rule = fa.lib()._ZN4fhip22prefill_f32_terms_formERKNS_9TermsCallEi
+    rule.restype, rule.argtypes = ctypes.c_uint64, [ctypes.POINTER(TermsCall), ctypes.c_int]
+    form = rule(ctypes.byref(TermsCall(*call[:6], CUS, False, call[6], True, True)), 1)
+    assert (form & 0xffffffff, form >> 32) == want
+
+
 @pytest.mark.parametrize("call, want", [((1, 8, 4, 162, 390, 64), 4), ((1, 16, 4, 154, 445, 64), 4), ((8, 8, 2, 516, 2456, 64), 2), ((8, 32, 8, 180, 2905, 64), 2)])
 def test_f32_tensors_are_shared_out_by_the_quickest_form(call, want):
     """(us, in these shares and in those of the least time of the form that runs: 12.8 and 14.6, 13.3 and 14.9, 143 and 162, 199 and 238)"""
