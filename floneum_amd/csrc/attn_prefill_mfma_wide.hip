@@ -528,9 +528,13 @@ void prefill_mfma_wide_plan(int B, int H, int G, int Sq, int Skv, int D, bool ca
     // Above 128 dims up to four of 512 keys where the time says that these take 5 % less (shares_gain): by tile steps alone, without the bytes of the
     // partials, calls of many rows lose (us, by steps and now: 12/12 heads at 256, three sequences of 413 rows on 1858 keys 69 -> 54, two
     // of 893 under a window on 2622 82 -> 61; 6/3 at 192, three of 1209 on 2620 115 -> 95).
-    if (D > 128 && !qk_square) {
+    // Of a square call with a mask tensor, whose rows may see from one to all of the keys, only shares that fit one round, where the longest
+    // workgroup counts (us, unsplit and in these: 4/4 heads at 160, 1768 rows 56.7 and 45.5; at 192, 1985 rows 73.7 and 58.4; 70 such calls of 400
+    // to 2800 rows 0.98 of the time, the worst 1.06).
+    if (D > 128) {
         double times[5] = {}, least = 0.0;
-        const int few = Skv / 512 < 4 ? Skv / 512 : 4;
+        int few = Skv / 512 < 4 ? Skv / 512 : 4;
+        while (qk_square && few > 1 && few * wgs > compute_units) few--;
         for (int n = 1; n <= few; n++) {
             times[n] = prefill_wide_time(B, H, G, Sq, Skv, D, compute_units, n);
             if (n == 1 || times[n] < least) least = times[n];

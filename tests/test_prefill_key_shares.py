@@ -123,6 +123,18 @@ def test_a_windowed_prompt_is_not_shared_out_as_a_whole_one(H, Hkv, rows, D):
     assert all(shares(1, H, Hkv, rows, rows, D, fa.F32, window=w) == whole for w in (rows - 1, rows, 2 * rows, 2 ** 40, 2 ** 63 - 1))
 
 
+@pytest.mark.parametrize("call, want", [((1, 4, 4, 1768, 1768, 160), 3), ((1, 4, 4, 1985, 1985, 192), 3), ((1, 6, 3, 1603, 2289, 160), 3),
+                                        ((3, 12, 12, 413, 700, 256), 0), ((2, 16, 4, 1205, 1205, 160), 0), ((1, 6, 3, 1256, 1256, 256), 2)])
+def test_squares_with_a_mask_tensor_are_split_to_one_round(call, want):
+    """16-bit calls above head_dim 128 whose rows may see from one to all of the keys."""
+    B, H, Hkv, rows, keys, D = call
+    a, need = make_args(B=B, H=H, Hkv=Hkv, Sq=rows, Skv=keys, D=D, dtype=fa.F16), ctypes.c_size_t()
+    a.mask_kind, a.mask.ptr, a.mask_intervals = fa.MaskKind.QKMask, 0x10000, 0x20000
+    a.mask.shape[:], a.mask.stride[:] = (rows, keys), (keys, 1)
+    assert fa.lib().fhip_flash_attention_workspace_bytes(ctypes.byref(a), CUS, ctypes.byref(need)) == fa.OK
+    assert need.value == want * B * H * rows * (D + 4) * 4
+
+
 class TermsCall(ctypes.Structure):  # floneum_amd/csrc/common.h
     _fields_ = [(n, ctypes.c_int) for n in ("B", "Hkv", "G", "Sq", "Skv", "D", "cus")] + [
         ("uneven", ctypes.c_bool), ("window", ctypes.c_int64), ("f32", ctypes.c_bool), ("causal", ctypes.c_bool)]
