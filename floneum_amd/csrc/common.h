@@ -68,7 +68,8 @@ struct AttnParams {
 // A square call whose rows see the keys up to their own position (a mask tensor is taken for one), some of them far fewer than others: not
 // where at least half a window is behind them all, as in a chunk of more rows than the window (f32, us taken for uneven and not: 12/12 heads at 128,
 // 1757 rows behind 4598 keys under a window of 803 115 and 74, 32/8 721 behind 6990 under 308 58 and 36, 16/8 at 128 905 behind
-// 140 under 137 36 and 21, 32/8 at 80 642 behind 265 under 531 54 and 40; over 125 random ones 0.90, the worst 1.11).  Above head_dim 128, where the model counts a window's keys by itself
+// 140 under 137 36 and 21, 32/8 at 80 642 behind 265 under 531 54 and 40; over 125 random ones 0.90, the worst 1.11).  Above head_dim 128, where
+// the model counts a window's keys by itself
 // and takes the levels of uneven shares, such calls stay with the uneven ones (4/1 heads at 256, 1804 behind 4210 under 1515 123 and 164).
 inline bool prefill_f32_uneven(int64_t Sq, int64_t Skv, int64_t D, bool causal, bool qk_mask, int64_t first_row_at, int64_t window) {
     if (2 * Sq <= Skv) return false;
@@ -79,7 +80,8 @@ void prefill_f32_plan(int B, int H, int G, int Sq, int Skv, int D, bool f32, boo
                       bool unknown_lengths, int compute_units, int *nsplit, int *chunk);
 // What part of the rules' time the shares of least time have to be, by a model: 5 % less, and 30 % where the rows may see far fewer
 // keys than it counts (us, in the rules' shares and by 5 %: f16, two sequences of 84 rows of 6/3 heads at 80 on up to 1416 keys 11.2 and 14.5;
-// bf16, two of 377 of 32/8 at 256 on up to 2369 50 and 97).  Mask tensors that hide most keys lose by the 5 % as well (f32, 32/8 at 128, 360 rows that see 300 of 1844 keys 56 and 65),
+// bf16, two of 377 of 32/8 at 256 on up to 2369 50 and 97).  Mask tensors that hide most keys lose by the 5 % as well (f32, 32/8 at 128, 360
+// rows that see 300 of 1844 keys 56 and 65),
 // but are not told from causal ones, whose plan they have to share.
 inline double shares_gain(bool unknown_lengths) { return unknown_lengths ? 0.7 : 0.95; }
 // The forms of the f32 terms kernel (attn_prefill_f32_terms.hip): units and key groups per workgroup, and what a call takes in them
